@@ -85,7 +85,7 @@ def draw(rng):
                      "ssd_forward", "ssd_step", "ssd_step"])
     dtype = rng.choice(["bf16", "bf16", "bf16", "f32"])
     if op.startswith("ema"):
-        room = _MAX_EMA // (1 if dtype == "bf16" else 2) // (2 if op == "ema_stages" else 1)
+        room = _MAX_EMA * 7 // 8 // (1 if dtype == "bf16" else 2) // (2 if op == "ema_stages" else 1)
         d = 8 * _log(rng, 4, 256)
         nh = rng.choice([0, 1, 2, 3, 4])
         if op == "ema_decode":
