@@ -1,0 +1,32 @@
+"""The split per-row dots and column sums of the stage launchers, at the sizes where they can go wrong."""
+import pytest
+import torch
+
+from oracle import ema_oracle as O
+from parity_util import announce, check_close
+
+pytestmark = pytest.mark.gpu
+
+F32, BF16 = torch.float32, torch.bfloat16
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("N,L,T,Q", [(1, 64, 64, 64), (2, 130, 72, 128), (1, 500, 8, 512), (3, 2048, 1032, 1000)])
+def test_row_dots_and_column_sums_split_over_workgroups(N, L, T, Q, dtype, device):
+    """Few chunks: several workgroups per chunk (rows past the end, a span that does not divide the chunk)."""
+    from kernels.ema_kernels.ema_state_fwd import _ema_chunk_state_fwd
+    from kernels.ema_kernels_bwd.ema_chunk_scan_bwd_dc import _ema_chunk_scan_bwd_dC
+    from kernels.ema_kernels_bwd.ema_chunk_state_bwd_db import _ema_chunk_state_bwd_db
+    from kernels.ema_kernels_bwd.ema_scan_bwd import _ema_chunk_scan_bwd_dstates
+    from parity_util import flat_case, oracle_intermediates
+
+    announce(f"split dots N={N} L={L} T={T} Q={Q} {dtype}")
+    A, X, dy = flat_case(N, L, T, 3, dtype)
+    o = oracle_intermediates(A, X, dy, Q)
+    d = lambda t: t.to(device)
+    # the states are bfloat16 sums of the inputs held in float32: the float32 bar applies to all of these
+    check_close("states", _ema_chunk_state_fwd(d(X), d(o["cs"])), O.chunk_state(X.float(), o["cs"]), F32)
+    check_close("dstates", _ema_chunk_scan_bwd_dstates(d(o["cs"]), d(dy)), o["ds"], F32)
+    check_close("db", _ema_chunk_state_bwd_db(d(X), d(o["cs"]), d(o["g"])), O.bwd_db(X.float(), o["cs"], o["g"]), F32)
+    check_close("dc", _ema_chunk_scan_bwd_dC(d(o["prev"]), d(o["cs"]), d(dy)),
+                O.bwd_dc(o["prev"], o["cs"], dy.float()), F32)

@@ -72,6 +72,9 @@ inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s);
 // ---------------------------------------------------------------- launch helpers
 
 // prob = 1: the input holds probabilities p and the sums are of log(1 - p).
+// Workgroups that fill the chip in the streaming kernels: four on each of 256 compute units.
+constexpr int64_t kFillWorkgroups = 1024;
+
 int launch_cumsum(const float* A, SeqStrides sa, float* cs, const Dims& d, hipStream_t st, int prob = 0) {
   const int64_t total = d.N * d.C;
   const unsigned grid = (unsigned)((total + 3) / 4);
@@ -88,6 +91,9 @@ int launch_chunk_reduce(const void* x, SeqStrides sx, int dtype, const float* cs
   int cg_log2 = 0;
   while ((1 << cg_log2) < vecs && cg_log2 < 6) ++cg_log2;
   const int cg = 1 << cg_log2;
+  // Narrower column tiles (down to 256 bytes of a row) while the workgroups do not fill the chip: at b4 nh2
+  // d1024 L4096 chunk 256 bf16, 256 workgroups of 1 KB rows take 16.3 us, 1024 of 256 bytes 13.9.
+  while (cg_log2 > 4 && d.N * d.C * ((vecs + (1 << cg_log2) - 1) >> cg_log2) < kFillWorkgroups) --cg_log2;
   const int ntiles = (int)((vecs + cg - 1) / cg);
   const int64_t grid = d.N * d.C * ntiles;
   if (grid > 0x7fffffff) return EMA_ERR_SHAPE;
@@ -163,19 +169,29 @@ int launch_chunk_gemm(const void* in, SeqStrides si, int dtype, const float* cs,
   if (dtype == EMA_BF16)
     return launch_chunk_scan_t<bf16_t, kWalkBnBf16, REVERSE>(in, si, cs, vec, out, so, d, st);
   return launch_chunk_scan_t<float, kWalkBnF32, REVERSE>(in, si, cs, vec, out, so, d, st);
+// Workgroups per chunk: one where the chunks alone fill the chip (four workgroups of eight waves on each of
+// 256 compute units), else as many as fill it, as long as each has rows for a full turn of its waves.
 }
 
 template <int MODE>
 int launch_row_dot(const void* x, SeqStrides sx, int dtype, const float* vec, const float* cs,
                    float* out, int raw, const Dims& d, hipStream_t st) {
-  const unsigned grid = (unsigned)(d.N * d.C);
+  const int64_t chunks = d.N * d.C;
+  int64_t split = 1;
+  while (split * chunks < kFillWorkgroups && d.Q >= 2 * split * kRowDotStep) split *= 2;
+  const int64_t span = split == 1 ? d.Q : (int64_t)align_up((size_t)((d.Q + split - 1) / split), kRowDotStep);
+  const dim3 grid((unsigned)chunks, (unsigned)((d.Q + span - 1) / span));
   if (dtype == EMA_BF16)
-    hipLaunchKernelGGL((row_dot_kernel<bf16_t, MODE>), dim3(grid), dim3(kRowDotThreads), 0, st,
+    hipLaunchKernelGGL((row_dot_kernel<bf16_t, MODE>), grid, dim3(kRowDotThreads), 0, st,
                        (const bf16_t*)x, sx, vec, cs, out, (int)d.nh, (int)d.L, (int)d.T, (int)d.Q,
-                       (int)d.C, raw);
+                       (int)d.C, raw, (int)span);
   else
-    hipLaunchKernelGGL((row_dot_kernel<float, MODE>), dim3(grid), dim3(kRowDotThreads), 0, st, (const float*)x,
-                       sx, vec, cs, out, (int)d.nh, (int)d.L, (int)d.T, (int)d.Q, (int)d.C, raw);
+    hipLaunchKernelGGL((row_dot_kernel<float, MODE>), grid, dim3(kRowDotThreads), 0, st, (const float*)x,
+                       sx, vec, cs, out, (int)d.nh, (int)d.L, (int)d.T, (int)d.Q, (int)d.C, raw, (int)span);
+  if (MODE == 0 && !raw && grid.y > 1) {
+    EMA_TRY(launched());
+    hipLaunchKernelGGL(row_scan_kernel, dim3((unsigned)((chunks + 3) / 4)), dim3(256), 0, st, out, (int)d.Q, chunks);
+  }
   return launched();
 }
 
@@ -487,9 +503,8 @@ int launch_da_flat(const void* x, SeqStrides sx, const void* dy, SeqStrides sd, 
   }
 }
 
-// B6.  Every chunk goes through the factored form first; the kernel that forms the product and its
-// finish then take the chunks in which the cumsum rises somewhere (none, for decays) and the finish
-// of the factored form the others.
+// B6.  Every chunk goes through the factored form first; the kernel that forms the product then takes
+// the chunks in which the cumsum rises somewhere (none, for decays), and one finish ends both forms.
 int launch_da(const void* x, SeqStrides sx, const void* dy, SeqStrides sd, int dtype,
               const float* cs, float* ddA_intra, const DaWs& w, const Dims& d, hipStream_t st) {
   const int MT = (int)((d.Q + kBM - 1) / kBM);
@@ -517,13 +532,7 @@ int launch_da(const void* x, SeqStrides sx, const void* dy, SeqStrides sd, int d
   EMA_TRY(launched());
   const int64_t total = d.N * d.C;
   hipLaunchKernelGGL(da_finish_kernel<kBM>, dim3((unsigned)((total + 3) / 4)), dim3(256), 0, st, w.part,
-                     w.rowsum, ddA_intra, (int)d.Q, MT, total, only);
-  if (flat) {
-    EMA_TRY(launched());
-    const int64_t n = total * d.Q;
-    hipLaunchKernelGGL(da_flat_finish_kernel<256>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, w.flat, w.steep,
-                       ddA_intra, (int)d.Q, da_flat_tiles(d, dtype), n);
-  }
+                     w.rowsum, w.flat, da_flat_tiles(d, dtype), only, ddA_intra, (int)d.Q, MT, total);
   return launched();
 }
 

@@ -175,19 +175,32 @@ __global__ __launch_bounds__(256, 2) void da_gemm_kernel(const T* __restrict__ x
   }
 }
 
-// B6, second part: ddA_intra[j] = sum_{i<j} (colsum[i] - rowsum[i]) with
-// colsum[i] = sum over the row tiles mt >= i / 128 of part[mt][i].  One wave per (n, c).
-// only (may be null): the chunks whose entry is 0 are left alone.
+// B6, second part, one wave per (n, c).  Where the chunk went through the factored form (steep is given and
+// its entry is 0) the per-column-tile dots only have to be added up:
+//   ddA_intra[q] = sum over the ntiles column tiles of flat[(chunk*ntiles + tile)*Q + q];
+// otherwise ddA_intra[j] = sum_{i<j} (colsum[i] - rowsum[i]) with
+//   colsum[i] = sum over the row tiles mt >= i / BM of part[mt][i].
+// Both forms in one launch: a launch that mostly finds nothing to do costs as much as one that works (4.5 and 4.7 us
+// at b4 nh2 d1024 L4096 chunk 256; 6.4 together).
 template <int BM>
 __global__ __launch_bounds__(256) void da_finish_kernel(const float* __restrict__ part,
                                                         const float* __restrict__ rowsum,
+                                                        const float* __restrict__ flat, int ntiles,
+                                                        const int* __restrict__ steep,
                                                         float* __restrict__ ddA_intra, int Q,
-                                                        int MT, int64_t total_chunks,
-                                                        const int* __restrict__ only = nullptr) {
+                                                        int MT, int64_t total_chunks) {
   const int lane = threadIdx.x & 63;
   const int64_t chunk_id = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (chunk_id >= total_chunks) return;
-  if (only && only[chunk_id] == 0) return;
+  if (steep && steep[chunk_id] == 0) {
+    const float* fp = flat + chunk_id * ntiles * (int64_t)Q;
+    for (int q = lane; q < Q; q += 64) {
+      float s = 0.f;
+      for (int ct = 0; ct < ntiles; ++ct) s += fp[ct * (int64_t)Q + q];
+      ddA_intra[chunk_id * Q + q] = s;
+    }
+    return;
+  }
   const int per = (Q + 63) >> 6;
   const int q0 = lane * per;
   auto val = [&](int q) {
@@ -206,24 +219,6 @@ __global__ __launch_bounds__(256) void da_finish_kernel(const float* __restrict_
       run += val(q);
     }
   }
-}
-
-// The same for the factored form, whose per-column-tile dots only have to be added up:
-// ddA_intra[chunk][q] = sum over the ntiles column tiles of flat[(chunk*ntiles + tile)*Q + q], for
-// the chunks whose entry in steep is 0.  One thread per (chunk, q).
-template <int BLOCK>
-__global__ __launch_bounds__(BLOCK) void da_flat_finish_kernel(const float* __restrict__ flat,
-                                                             const int* __restrict__ steep,
-                                                             float* __restrict__ ddA_intra, int Q,
-                                                             int ntiles, int64_t total) {
-  const int64_t i = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
-  if (i >= total) return;
-  const int64_t chunk_id = i / Q;
-  if (steep[chunk_id] != 0) return;
-  const int q = (int)(i - chunk_id * Q);
-  float s = 0.f;
-  for (int ct = 0; ct < ntiles; ++ct) s += flat[(chunk_id * ntiles + ct) * (int64_t)Q + q];
-  ddA_intra[i] = s;
 }
 
 }  // namespace ema

@@ -366,9 +366,15 @@ __global__ __launch_bounds__(256) void state_passing_bwd_finish_kernel(
 //                chunk limit give 0; out[0] = 0, out[j] = r[j-1] (raw) or
 //                out[j] = sum_{m<j} r[m] (cumulative).
 //   MODE 1 (dc): out[m] = exp(cs[m]) * <dy[n,cQ+m], prev[n,c]>, 0 past the limit.
-// One workgroup of kRowDotThreads per (n, c); wave w takes rows R*w + R*NWV*i + {0..R-1}; a wave
-// covers the feature axis with 16-byte loads per lane (R of them in flight per lane and column
-// step) and reduces with DPP.
+// gridDim.y workgroups of kRowDotThreads share one (n, c), `span` rows each (a multiple of R * NWV unless it
+// is the whole chunk); wave w takes rows R*w + R*NWV*i + {0..R-1} of its workgroup's; a wave covers the feature
+// axis with 16-byte loads per lane (R of them in flight per lane and column step) and reduces with DPP.
+// The dots are independent of each other, so how a chunk is split only changes who computes them; the running
+// sum of the cumulative form needs the whole chunk: with gridDim.y > 1 the kernel leaves r[m] in out[m] and
+// row_scan_kernel turns it into out[j] in place.
+// Bound by HBM once the chip is filled.  At b4 nh2 d1024 L4096 chunk 256 bf16 there are 128 chunks for 256
+// compute units: one workgroup per chunk 41 us (db and dc alike), eight per chunk 13.6 us (db, and 3.8 for
+// its running sum) and 14.1 us (dc).
 // ------------------------------------------------------------------------------------
 constexpr int kRowDotThreads = 512;
 template <typename T, int MODE>
@@ -376,7 +382,7 @@ __global__ __launch_bounds__(kRowDotThreads) void row_dot_kernel(const T* __rest
                                                                  const float* __restrict__ vec,
                                                                  const float* __restrict__ cs,
                                                                  float* __restrict__ out, int nh, int L,
-                                                                 int Tdim, int Q, int C, int raw) {
+                                                                 int Tdim, int Q, int C, int raw, int span) {
   constexpr int VEC = Vec16<T>::N;
   constexpr int NWV = kRowDotThreads / 64;
   __shared__ float rbuf[EMA_MAX_CHUNK_DEV];
@@ -390,14 +396,36 @@ __global__ __launch_bounds__(kRowDotThreads) void row_dot_kernel(const T* __rest
   const int limit = min(Q, L - c * Q);
   const float* csp = cs + chunk_id * Q;
   const float cs_last = csp[Q - 1];
+constexpr int kRowDotRows = 2;  // rows per wave and turn
+constexpr int kRowDotStep = kRowDotThreads / 64 * kRowDotRows;  // rows per workgroup and turn
+
+// out[j] = sum_{m<j} r[m] by one wave: lane l owns positions l*per .. l*per+per-1 (out may be r).
+__device__ __forceinline__ void row_exclusive_sum(const float* r, float* out, int Q, int lane) {
+  const int per = (Q + 63) >> 6;
+  const int q0 = lane * per;
+  float local = 0.f;
+  for (int i = 0; i < per; ++i)
+    if (q0 + i < Q) local += r[q0 + i];
+  float run = wave_exclusive_scan(local);
+  for (int i = 0; i < per; ++i) {
+    const int q = q0 + i;
+    if (q < Q) {
+      const float v = r[q];
+      out[q] = run;
+      run += v;
+    }
+  }
+}
+
   const float* vp = vec + chunk_id * Tdim;
   const T* xp = x + b * sx.sb + h * sx.sh + (int64_t)c * Q * sx.sl;
 
   // rows per wave and turn.  Measured at b16 nh2 d1024 L4096 chunk 128 (db / dc, us): 8 rows 50 / 49, 4 rows
   // 47.5 / 47, 2 rows 44.7 / 44.5, 1 row 47.7 / 47.5, 16 rows 58 / 56: fewer registers per wave keep more waves
   // resident, and two 16-byte loads per lane and column step are enough to cover the latency with them.
-  constexpr int R = 2;
-  for (int m0 = wave * R; m0 < Q; m0 += NWV * R) {
+  constexpr int R = kRowDotRows;
+  const int mbeg = (int)blockIdx.y * span, mend = min(mbeg + span, Q);
+  for (int m0 = mbeg + wave * R; m0 < mend; m0 += NWV * R) {
     float acc[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) acc[r] = 0.f;
@@ -423,7 +451,7 @@ __global__ __launch_bounds__(kRowDotThreads) void row_dot_kernel(const T* __rest
     for (int r = 0; r < R; ++r) {
       const float s = wave_sum(acc[r]);
       const int m = m0 + r;
-      if (lane == 0 && m < Q) {
+      if (lane == 0 && m < mend) {
         float w = 0.f;
         if (m < limit) w = MODE == 0 ? __expf(fminf(cs_last - csp[m], 0.f)) : __expf(csp[m]);
         rbuf[m] = w * s;
@@ -432,25 +460,14 @@ __global__ __launch_bounds__(kRowDotThreads) void row_dot_kernel(const T* __rest
   }
   __syncthreads();
   float* op = out + chunk_id * Q;
-  if (MODE == 1) {
-    for (int m = tid; m < Q; m += kRowDotThreads) op[m] = rbuf[m];
+  if (MODE == 1 || (!raw && gridDim.y > 1)) {
+    for (int m = mbeg + tid; m < mend; m += kRowDotThreads) op[m] = rbuf[m];
   } else if (raw) {
-    for (int m = tid; m < Q; m += kRowDotThreads) op[m] = m == 0 ? 0.f : rbuf[m - 1];
+    if (mbeg == 0 && tid == 0) op[0] = 0.f;
+    for (int m = mbeg + tid; m < mend; m += kRowDotThreads)
+      if (m + 1 < Q) op[m + 1] = rbuf[m];
   } else if (wave == 0) {
-    // out[j] = sum_{m<j} r[m]: exclusive scan, lane l owns positions l*per .. l*per+per-1
-    const int per = (Q + 63) >> 6;
-    const int q0 = lane * per;
-    float local = 0.f;
-    for (int i = 0; i < per; ++i)
-      if (q0 + i < Q) local += rbuf[q0 + i];
-    float run = wave_exclusive_scan(local);
-    for (int i = 0; i < per; ++i) {
-      const int q = q0 + i;
-      if (q < Q) {
-        op[q] = run;
-        run += rbuf[q];
-      }
-    }
+    row_exclusive_sum(rbuf, op, Q, lane);
   }
 }
 
@@ -473,6 +490,14 @@ __global__ __launch_bounds__(256) void combine_dA_kernel(const float* __restrict
   const int per = (Q + 63) >> 6;
   const int p0 = lane * per;
   const float* sp = sraw + chunk_id * Q;
+// The running sum of row_dot_kernel<T, 0> where several workgroups share a chunk: one wave per chunk, in place.
+__global__ __launch_bounds__(256) void row_scan_kernel(float* __restrict__ v, int Q, int64_t chunks) {
+  const int64_t chunk = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (chunk >= chunks) return;
+  float* p = v + chunk * Q;
+  row_exclusive_sum(p, p, Q, threadIdx.x & 63);
+}
+
   const float extra = ddA_chunk[chunk_id];
   float local = 0.f;
   for (int i = 0; i < per; ++i) {

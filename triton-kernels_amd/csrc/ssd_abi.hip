@@ -803,7 +803,7 @@ int ssd_chunk_scan_bwd_ddAcs(const void* x, int64_t x_sb, int64_t x_sl, int64_t 
   SSD_TRY(launched());
   const int64_t total = batch * nheads * d.C;
   hipLaunchKernelGGL(ema::da_finish_kernel<ema::kBM>, dim3((unsigned)((total + 3) / 4)), dim3(256), 0, st, part,
-                     rowsum, ddA_cumsum, (int)chunk, MT, total);
+                     rowsum, (const float*)nullptr, 0, (const int*)nullptr, ddA_cumsum, (int)chunk, MT, total);
   return launched();
 }
 
