@@ -1,0 +1,43 @@
+"""The chunk scan in one tile per chunk (chunks of 64 and 128 rows), at the sizes where it can go wrong."""
+import pytest
+import torch
+
+from oracle import ssd_oracle as S
+from parity_util import announce, check_close
+
+F32, BF16 = torch.float32, torch.bfloat16
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["decay", "rise", "mixed"])
+@pytest.mark.parametrize("nh,g,P,dtype", [(4, 1, 64, BF16), (6, 3, 64, BF16), (2, 1, 128, BF16), (3, 1, 64, F32),
+                                          (2, 2, 128, F32)])
+@pytest.mark.parametrize("Q,L", [(128, 257), (128, 128), (128, 33), (64, 190), (64, 64), (64, 1)])
+def test_chunk_scan_one_tile_vs_oracle(Q, L, nh, g, P, dtype, kind, device):
+    """L one row past a chunk, exact and shorter than a 32-row block; dA falling, rising and both (the weights
+    then take the exact form everywhere)."""
+    from kernels.mamba_kernels.mamba_scan_fwd import _chunk_scan_fwd
+
+    announce(f"chunk scan Q={Q} L={L} nh={nh} g={g} P={P} {dtype} {kind}")
+    N, b = 64 if P == 128 else 128, 2
+    gen = torch.Generator().manual_seed(Q + L + nh)
+    r = lambda *s: torch.randn(*s, generator=gen)
+    x, C, z = r(b, L, nh, P).to(dtype), r(b, L, g, N).to(dtype), r(b, L, nh, P).to(dtype)
+    dt = torch.rand(b, L, nh, generator=gen) * 0.5
+    A = -torch.rand(nh, generator=gen) - 0.1
+    if kind == "rise":
+        A = -A
+    elif kind == "mixed":
+        dt = dt - 0.25
+    dA, dto = S.chunk_cumsum(dt, A, Q)
+    nc = -(-L // Q)
+    cb = r(b, nc, g, Q, Q) * 0.3
+    states = r(b, nc, nh, P, N).to(dtype)
+    D = r(nh)
+    for zz in (None, z):
+        ref, ref_x = S.chunk_scan(cb, x, dto, dA, C, states, D=D, z=zz, round_to=dtype)
+        got, got_x = _chunk_scan_fwd(*(t.to(device) for t in (cb, x, dto, dA, C, states)), D=D.to(device),
+                                     z=None if zz is None else zz.to(device))
+        check_close("out", got, ref, dtype, regrouped=True)
+        if zz is not None:
+            check_close("out_x", got_x, ref_x, dtype, regrouped=True)

@@ -196,18 +196,56 @@ struct ScanLaunch {
                        (const T*)x, sx, (const T*)z, sz, dt, dA, (const T*)C, sC, (const TS*)prev, D, d_has_hdim,
                        (T*)out, so, (T*)out_x, (int)d.nh, (int)(d.nh / d.g), (int)d.g, (int)d.L, (int)d.Q, (int)d.C,
                        stiles, seq);
+  template <typename T, int P, int N, typename TS, int HP, int ST>
+  int launch_mid() const {
+    auto kernel = ssd_chunk_scan_mid_kernel<T, P, N, TS, HP, ST>;
+    constexpr int smem = MidSmem<T, P * HP, N, ST>::bytes_for(HP);
+    static_assert(smem <= kLdsBytes, "the tile must fit the LDS of a compute unit");
+    SSD_TRY(allow_smem(kernel, smem));
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(d.batch * d.C * (d.nh / HP))), dim3(256), smem, st, cb,
+                       (const T*)x, sx, (const T*)z, sz, dt, dA, (const T*)C, sC, (const TS*)prev, D, d_has_hdim,
+                       (T*)out, so, (T*)out_x, (int)d.nh, (int)(d.nh / d.g), (int)d.g, (int)d.L, (int)d.C, seq);
+    return launched();
+  }
+  // Whether a chunk's rows sit at 32-bit byte offsets from its first one.
+  bool near(const Strides3& s) const { return forward_strides(s) && d.Q * s.sl < (int64_t(1) << 28); }
+  // Chunks of 64 or 128 rows in one tile.  Two adjacent heads of a group per workgroup where they are adjacent
+  // in memory too (dense heads of 64 features): they share the fragments of cb and the rows of C.  A single
+  // bfloat16 head of 64 features leaves each wave one column block for the weights it forms, and the 64-row
+  // kernel is the faster one (17 heads, L 4096, b2, chunk 128: 29.0 against 32.4 us).  Against the 64-row
+  // kernel otherwise, us at dstate 128: bfloat16 b8 nh32 L8192 hdim 64 chunk 128 437 -> 260, chunk 64
+  // 334 -> 240; b2 nh16 L4096 hdim 128 chunk 128 42 -> 38; float32 b1 nh16 L4096 chunk 128 hdim 64 35 -> 25,
+  // hdim 128 70 -> 40.
+  template <typename T, int P, int N, typename TS, int ST>
+  int launch_mid_pairs(bool* taken) const {
+    *taken = true;
+    if constexpr (P == 64 && sizeof(T) == 2) {
+      const bool dense = sx.sh == P && so.sh == P && (!z || sz.sh == P);
+      if (dense && (d.nh / d.g) % 2 == 0) return launch_mid<T, P, N, TS, 2, ST>();
+      *taken = false;
+      return SSD_OK;
+    } else {
+      return launch_mid<T, P, N, TS, 1, ST>();
+    }
+  }
     return launched();
   }
   template <typename T, int P, int N, typename TS>
   int run_as() const {
     constexpr int wide_smem = WideSmem<T, P, N>::kBytes;
-    if (d.Q % 256 == 0 && wide_smem <= kLdsBytes) {  // 256-row super-tiles, no barrier inside the k loop
+    const bool close = near(sx) && near(sC) && near(so) && (!z || near(sz));
+    if (d.Q % 256 == 0 && wide_smem <= kLdsBytes && close) {  // 256-row super-tiles, no barrier inside the k loop
       // Two adjacent heads of a group per workgroup where they are adjacent in memory too (dense
       // heads of 64 features): they share the fragments of cb and the rows of C.
       if constexpr (P == 64 && WideSmem<T, 128, N>::bytes_for(2) <= kLdsBytes / 2) {
         const bool dense = sx.sh == P && so.sh == P && (!z || sz.sh == P);
         if (dense && (d.nh / d.g) % 2 == 0) return launch_wide<T, P, N, TS, 2>();
       }
+    if ((d.Q == 64 || d.Q == 128) && close) {
+      bool taken;
+      const int status = d.Q == 128 ? launch_mid_pairs<T, P, N, TS, 128>(&taken) : launch_mid_pairs<T, P, N, TS, 64>(&taken);
+      if (taken) return status;
+    }
       return launch_wide<T, P, N, TS, 1>();
     }
     auto kernel = ssd_chunk_scan_kernel<T, P, N, TS>;

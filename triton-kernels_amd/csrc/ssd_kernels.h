@@ -211,6 +211,18 @@ __device__ __forceinline__ void stage_rows(T* tile, const T* __restrict__ g, int
     }
   }
 }
+// 16 bytes at a 32-bit byte offset from a base that is the same for the whole wave.
+template <bool STREAM = false, typename T>
+__device__ __forceinline__ Vec16<T> load16_at(const T* base, unsigned bytes) {
+  const T* p = reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + bytes);
+  return STREAM ? load16_stream(p) : load16(p);
+}
+template <typename T>
+__device__ __forceinline__ T* at_bytes(T* base, unsigned bytes) {
+  using Byte = std::conditional_t<std::is_const<T>::value, const char, char>;
+  return reinterpret_cast<T*>(reinterpret_cast<Byte*>(base) + bytes);
+}
+
 // The two halves of stage_rows for tiles of at most eight 16-byte pieces per thread: the loads
 // (into registers) and, later, the scaling, masking and LDS stores.  A kernel that has the next
 // tile's loads in flight while it works on the current one calls them apart.  Up to two float32
@@ -237,6 +249,16 @@ struct RowPieces {
       if (BOTH || aux1) a1[i] = aux1[row];
     }
   }
+  // The same from byte offsets that fit 32 bits (the caller has checked): one address register per piece
+  // instead of two, the base stays in scalar registers.
+  template <bool STREAM = false>
+  __device__ __forceinline__ void load32(const T* __restrict__ g, unsigned row_bytes, int row0, int limit, int tid) {
+#pragma unroll
+    for (int i = 0; i < CNT; ++i) {
+      const int idx = tid + 256 * i;
+      v[i] = load16_at<STREAM>(g, (unsigned)min(row0 + idx / VPR, limit - 1) * row_bytes + (idx % VPR) * 16u);
+    }
+  }
   // scale(row, aux0[row], aux1[row]) multiplies the row; NoScale leaves it
   template <typename F>
   __device__ __forceinline__ void store(T* tile, int row0, int limit, int tid, F scale) {
@@ -258,6 +280,44 @@ struct RowPieces {
     }
   }
 };
+
+template <bool STREAM>
+__device__ __forceinline__ float4 state_load4(const float* p);
+template <bool STREAM>
+__device__ __forceinline__ float4 state_load4(const bf16_t* p);
+
+// Rows [row0, row0 + ROWS) into an LDS tile of the given pitch, through registers in groups of at most eight
+// pieces per thread, from 32-bit byte offsets.
+template <typename T, int ROWS, int COLS, int PITCH, bool STREAM>
+__device__ __forceinline__ void stage_rows32(T* tile, const T* __restrict__ g, unsigned row_bytes, int row0, int limit,
+                                             int tid) {
+  constexpr int VPR = COLS / Vec16<T>::N, RP = ROWS * VPR / 256 <= 8 ? ROWS : 2048 / VPR;
+  static_assert(ROWS % RP == 0, "load groups must divide the tile");
+#pragma unroll
+  for (int r = 0; r < ROWS; r += RP) {
+    RowPieces<T, RP, COLS, PITCH> part;
+    part.template load32<STREAM>(g, row_bytes, row0 + r, limit, tid);
+    asm volatile("" ::: "memory");  // all loads of a group go out before its first LDS store
+    part.store(tile + r * PITCH, row0 + r, limit, tid, NoScale());
+  }
+}
+// A carried state (ROWS x N, dense) into an LDS tile in the operand type.
+template <typename T, typename TS, int ROWS, int N, int PITCH>
+__device__ __forceinline__ void stage_state(T* tile, const TS* __restrict__ g, int tid) {
+  if constexpr (std::is_same<T, TS>::value) {
+    stage_rows32<T, ROWS, N, PITCH, true>(tile, g, N * sizeof(T), 0, ROWS, tid);
+  } else {
+    constexpr int VPR = N / 4;
+#pragma unroll
+    for (int i = 0; i < ROWS * VPR / 256; ++i) {
+      const int idx = tid + 256 * i;
+      const int r = idx / VPR, cv = (idx % VPR) * 4;
+      const float4 v = state_load4<true>(at_bytes(g, (unsigned)(r * N + cv) * (unsigned)sizeof(TS)));
+      T* d = tile + r * PITCH + cv;
+      d[0] = (T)v.x, d[1] = (T)v.y, d[2] = (T)v.z, d[3] = (T)v.w;
+    }
+  }
+}
 
 // ------------------------------------------------------------------------------------
 // chunk_cumsum.  One workgroup per (b, c, group of HT heads), HT a power of two up to 8.  dt is
@@ -1903,7 +1963,7 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_scan_wide_kernel(
   static_assert(S::kPrev <= (ST / 2) * S::PX * (int)sizeof(T), "the carried state must leave the upper half of the x tile free");
   constexpr bool kEarly = (ST / 2) * (PW / EPL) / 256 <= 8;  // (eight pieces per thread travel in registers)
   RowPieces<T, kEarly ? ST / 2 : 32, kEarly ? PW : EPL * 8, S::PX> upper;
-  if constexpr (kEarly) upper.template load<true>(xg, sx.sl, ST / 2, limit, tid);
+  if constexpr (kEarly) upper.template load32<true>(xg, xrow, ST / 2, limit, tid);
   // ---- phase A: C . prev, scaled by exp(dA_m)
   {
     constexpr int VPR = N / 4;
@@ -1917,6 +1977,7 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_scan_wide_kernel(
     }
   }
   {
+  const unsigned xrow = (unsigned)(sx.sl * sizeof(T));
     const ChunkSeq sq = chunk_seq(seq, b, c, Q);
     const bool live = !sq.on() || sq.at(min(m0 + tid, limit - 1)) == sq.entering(c);
 #pragma unroll
@@ -1976,7 +2037,7 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_scan_wide_kernel(
       float am[HP];
 #pragma unroll
       for (int hh = 0; hh < HP; ++hh) am[hh] = dAp[hh][m0 + mloc];
-      const float* cbrow = cbg + (int64_t)(m0 + mloc) * Q + k0 + EPL * half;
+      const unsigned cbrow = 4u * ((unsigned)(m0 + mloc) * Q + k0 + EPL * half);
       const int kend = diag ? mrow[mb] + 32 : ST;
       // NS steps at a time (the step count is even): their cb fragments are all requested before
       // the first is used, so the wave waits for memory once per NS steps.  Only where the
@@ -1988,7 +2049,7 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_scan_wide_kernel(
         for (int u = 0; u < NS; ++u)
 #pragma unroll
           for (int e = 0; e < EPL; e += 4) {
-            const float4 c4 = *reinterpret_cast<const float4*>(cbrow + kk0 + KG * u + e);
+            const float4 c4 = *reinterpret_cast<const float4*>(at_bytes(cbg + kk0 + KG * u + e, cbrow));
             w[u][e] = c4.x, w[u][e + 1] = c4.y, w[u][e + 2] = c4.z, w[u][e + 3] = c4.w;
           }
         // the group of 32 positions that holds the diagonal takes the exact, masked form
@@ -2108,6 +2169,250 @@ __device__ __forceinline__ void store_dD_partial(float* __restrict__ slot, float
 template <typename T, int P, int N, typename TS>
 __global__ __launch_bounds__(256) void ssd_chunk_scan_bwd_dx_kernel(
     const float* __restrict__ cb, const T* __restrict__ x, Strides3 sx, const T* __restrict__ dout, Strides3 sd,
+// ------------------------------------------------------------------------------------
+// chunk_scan for chunks of ST = 64 or 128 rows.  One workgroup of four waves per (b, c, head or pair of heads).  PW = HP * hdim columns (two adjacent heads of
+// a group share the rows of C and the fragments of cb, as in ssd_chunk_scan_wide_kernel); wave w owns the
+// columns of half w & 1 (one head of a pair) and the 32-row blocks w >> 1 and ST/32 - 1 - (w >> 1) of the tile
+// (one block where the tile has two), which balances the causal sum.  What a lane needs of C and of cb comes
+// straight from global memory, cb one group of 32 positions ahead; LDS holds what the waves share: the
+// carried state, then the chunk's rows of x (requested before the state's product).
+//
+// The weight of (m, k) below the diagonal group is split at the last position r of k's group of 32 as in the
+// 256-row kernel, which equals the clamped exponential of the definition where dA does not rise; the
+// workgroup looks at the dA it uses, and where it rises anywhere (dt of mixed sign) every group takes the
+// exact form.
+//
+// Latency bound: a tile is a short chain of dependent loads, so what counts is how many of them a compute unit
+// has under way.  A wave holds half the accumulators of the 256-row kernel, so three workgroups fit instead
+// of two.  b8 nh32 L8192 hdim 64 dstate 128 bf16: chunk 128 437 us by the 64-row kernel, 260
+// here (3.2 TB/s); chunk 64 334 and 240 us.
+// ------------------------------------------------------------------------------------
+template <typename T, int PW, int N, int ST>
+struct MidSmem {
+  static constexpr int PX = Tile<T>::kpitch(PW), PC = Tile<T>::pitch(N), PO = PW / 2 + 4;
+  static constexpr int kX = ST * PX * (int)sizeof(T);
+  static constexpr int kPrev = PW * PC * (int)sizeof(T);
+  static constexpr int kOut = 4 * 32 * PO * (int)sizeof(float);  // one block per wave
+  static constexpr int kXP = kX > kPrev ? kX : kPrev;
+  static constexpr int kMain = kXP > kOut ? kXP : kOut;          // the three are live one after the other
+  static constexpr int bytes_for(int heads) { return kMain + heads * 4 * ST * (int)sizeof(float); }
+};
+
+template <typename T, int P, int N, typename TS, int HP, int ST>
+__global__ __launch_bounds__(256, (P * HP * (int)sizeof(T) > 256 ? 2 : 3)) void ssd_chunk_scan_mid_kernel(
+    const float* __restrict__ cb, const T* __restrict__ x, Strides3 sx, const T* __restrict__ z, Strides3 sz,
+    const float* __restrict__ dt, const float* __restrict__ dA_cs, const T* __restrict__ Cm, Strides3 sC,
+    const TS* __restrict__ prev, const float* __restrict__ D, int d_has_hdim, T* __restrict__ out,
+    Strides3 so, T* __restrict__ out_x, int nh, int heads_per_group, int ngroups, int L, int C,
+    SeqIdx seq) {
+  constexpr int PW = P * HP, PH = PW / 2;  // columns of the tile and of a wave
+  using S = MidSmem<T, PW, N, ST>;
+  constexpr int EPL = Vec16<T>::N, KG = Tile<T>::KG, PB = PH / 32, MB = ST / 64, NK = N / KG;
+  constexpr int GS = 32 / KG;  // steps of a group of 32 positions
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  T* Xs = reinterpret_cast<T*>(smem);
+  T* Pv = reinterpret_cast<T*>(smem);
+  float* Os = reinterpret_cast<float*>(smem);
+  float* vec = reinterpret_cast<float*>(smem + S::kMain);  // per head: dA_k, dt_k, factor of k, exp(dA_m)
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, half = lane >> 5;
+  const int bid = xcd_local_index((int)blockIdx.x, (int)gridDim.x);
+  const int nhp = nh / HP;
+  const int h0 = (bid % nhp) * HP;  // first head of the workgroup
+  const int c = (bid / nhp) % C;
+  const int64_t b = bid / ((int64_t)nhp * C);
+  constexpr int Q = ST;
+  const int limit = min(Q, L - c * Q);
+  const int g = h0 / heads_per_group;
+  const int cw = wave & 1, hw = HP == 2 ? cw : 0;  // the wave's column half and head
+  const T* xg = x + b * sx.sb + (int64_t)c * Q * sx.sl + h0 * sx.sh;
+  const T* Cg = Cm + b * sC.sb + (int64_t)c * Q * sC.sl + g * sC.sh;
+  const TS* pg = prev + (((b * C + c) * nh + h0) * (int64_t)P) * N;
+  const float* cbg = cb + (((b * C + c) * ngroups + g) * (int64_t)Q) * Q;
+  const int64_t row0 = ((b * nh + h0) * C + c) * (int64_t)Q;  // dA, dt of head h0; the next head C * Q further
+  const unsigned xrow = (unsigned)(sx.sl * sizeof(T));
+
+  int mrow[MB];
+  mrow[0] = 32 * (wave >> 1);
+  if constexpr (MB == 2) mrow[1] = 32 * (3 - (wave >> 1));
+  floatx16 acc[MB][PB];
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int pb = 0; pb < PB; ++pb) zero_acc(acc[mb][pb]);
+
+  // ---- everything the first two phases need is requested up front
+  constexpr bool kEarly = ST * (PW / EPL) / 256 <= 8;  // (eight pieces per thread travel in registers)
+  RowPieces<T, kEarly ? ST : 32, kEarly ? PW : EPL * 8, S::PX> xt;
+  if constexpr (kEarly) xt.template load32<true>(xg, xrow, 0, limit, tid);
+  const unsigned Crow = (unsigned)(sC.sl * sizeof(T));
+  auto c_frag = [&](int mb, int i) {
+    return load16_at(Cg + KG * i, (unsigned)min(mrow[mb] + l32, limit - 1) * Crow + 16u * half);
+  };
+  constexpr int CA = NK < 4 ? NK : 4;  // fragments of C under way
+  Vec16<T> cf[CA];
+#pragma unroll
+  for (int i = 0; i < CA; ++i) cf[i] = c_frag(0, i);
+  stage_state<T, TS, PW, N, S::PC>(Pv, pg, tid);
+  bool rises = false;
+  if (tid < HP * ST) {
+    const int hh = tid / ST, i = tid % ST;
+    const ChunkSeq sq = chunk_seq(seq, b, c, Q);
+    const bool live = !sq.on() || sq.at(min(i, limit - 1)) == sq.entering(c);
+    const float* dAp = dA_cs + row0 + (int64_t)hh * C * Q;
+    const float ak = dAp[i], ar = dAp[i | 31], tk = dt[row0 + (int64_t)hh * C * Q + i];
+    float* d = vec + (4 * hh) * ST + i;
+    d[0] = ak, d[ST] = tk, d[2 * ST] = __expf(fminf(ar - ak, 0.f)) * tk, d[3 * ST] = live ? __expf(ak) : 0.f;
+    rises = i + 1 < ST && !(dAp[i + 1] <= ak);  // (a NaN counts as a rise)
+  }
+  rises = __syncthreads_or(rises);
+
+  // ---- phase A: C . prev, scaled by exp(dA_m).  (Rows past the sequence hold a copy of the last row's C:
+  // no row of the product reaches another, and theirs are not stored.)
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) {
+#pragma unroll
+    for (int i = 0; i < NK; ++i) {
+      const Vec16<T> a = cf[i % CA];
+      const int nx = mb * NK + i + CA;
+      if (nx < MB * NK) cf[i % CA] = c_frag(nx / NK, nx % NK);
+#pragma unroll
+      for (int pb = 0; pb < PB; ++pb) mma_group(a, frag_rows(Pv, S::PC, PH * cw + 32 * pb, KG * i, lane), acc[mb][pb]);
+    }
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const float sc = vec[(4 * hw + 3) * ST + mrow[mb] + acc_row(v, lane)];
+#pragma unroll
+      for (int pb = 0; pb < PB; ++pb) acc[mb][pb][v] *= sc;
+    }
+  }
+
+  // ---- phase B: the causal sum
+  const float* dAk = vec + (4 * hw) * ST;
+  const float* dtk = dAk + ST;
+  const float* fk = dAk + 2 * ST;
+  unsigned cbrow[MB];  // byte offset of the lane's piece of its row of cb
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) cbrow[mb] = 4u * ((unsigned)(mrow[mb] + l32) * Q + EPL * half);
+  float wn[GS][EPL];  // the cb fragments of the next group
+  auto request = [&](unsigned at) {
+#pragma unroll
+    for (int u = 0; u < GS; ++u)
+#pragma unroll
+      for (int e = 0; e < EPL; e += 4) {
+        const float4 c4 = *reinterpret_cast<const float4*>(at_bytes(cbg + KG * u + e, at));
+        wn[u][e] = c4.x, wn[u][e + 1] = c4.y, wn[u][e + 2] = c4.z, wn[u][e + 3] = c4.w;
+      }
+  };
+  request(cbrow[0]);
+  __syncthreads();  // the x tile takes the place of the carried state
+  if constexpr (kEarly) {
+    xt.store(Xs, 0, limit, tid, NoScale());
+  } else {
+    stage_rows32<T, ST, PW, S::PX, true>(Xs, xg, xrow, 0, limit, tid);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) {
+    const int mloc = mrow[mb] + l32;
+    const float am = dAk[mloc];
+    for (int kg = 0; kg <= mrow[mb]; kg += 32) {
+      float w[GS][EPL];
+#pragma unroll
+      for (int u = 0; u < GS; ++u)
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) w[u][e] = wn[u][e];
+      request(kg < mrow[mb] ? cbrow[mb] + 4u * (kg + 32) : cbrow[MB - 1]);
+      const bool diag = kg == mrow[mb], exact = rises || diag;
+      const float gm = __expf(fminf(am - dAk[kg + 31], 0.f));
+#pragma unroll
+      for (int u = 0; u < GS; ++u) {
+        const int kb = kg + KG * u + EPL * half;
+        Vec16<T> a;
+        float wf[EPL];
+        if (exact) {
+#pragma unroll
+          for (int e = 0; e < EPL; ++e) {
+            const float f = w[u][e] * __expf(fminf(am - dAk[kb + e], 0.f)) * dtk[kb + e];
+            wf[e] = kb + e > mloc ? 0.f : f;
+          }
+        } else {
+#pragma unroll
+          for (int e = 0; e < EPL; ++e) wf[e] = w[u][e] * fk[kb + e] * gm;
+        }
+        a.set_all(wf);
+#pragma unroll
+        for (int pb = 0; pb < PB; ++pb)
+          mma_group(a, frag_cols(Xs, S::PX, kg + KG * u, PH * cw + 32 * pb, lane), acc[mb][pb]);
+      }
+    }
+    if (D) {
+#pragma unroll
+      for (int pb = 0; pb < PB; ++pb) {
+        const int col = PH * cw + 32 * pb + l32;  // column of the tile = feature of head h0 + col / P
+        const float dv = d_has_hdim ? D[h0 * P + col] : D[h0 + hw];
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          acc[mb][pb][v] = fmaf(dv, (float)Xs[(mrow[mb] + acc_row(v, lane)) * S::PX + col], acc[mb][pb][v]);
+      }
+    }
+  }
+  __syncthreads();
+
+  // ---- phase C: each wave moves its blocks through its own staging area, gate on the way (the rows of z are
+  // requested before the accumulators go to LDS)
+  float* mine = Os + wave * 32 * S::PO;
+  constexpr int VPR = PH / EPL, NI = 32 * VPR / 64;
+  const int col0 = HP == 2 ? 0 : PH * cw;
+  const T* zg = z ? z + b * sz.sb + (int64_t)c * Q * sz.sl + (h0 + hw) * sz.sh + col0 : nullptr;
+  const int64_t ob = b * so.sb + (int64_t)c * Q * so.sl + (h0 + hw) * so.sh + col0;
+  const unsigned zrow = (unsigned)(sz.sl * sizeof(T)), orow = (unsigned)(so.sl * sizeof(T));
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) {
+    Vec16<T> zv[NI];
+    if (z) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int idx = lane + 64 * i;
+        zv[i] = load16_at<true>(zg, (unsigned)min(mrow[mb] + idx / VPR, limit - 1) * zrow + (idx % VPR) * 16u);
+      }
+    }
+#pragma unroll
+    for (int pb = 0; pb < PB; ++pb)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) mine[acc_row(v, lane) * S::PO + 32 * pb + l32] = acc[mb][pb][v];
+    // the wave's own writes are visible to its own reads once the LDS counter has drained
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int idx = lane + 64 * i;
+      const int r = idx / VPR, cv = (idx % VPR) * EPL;
+      const int m = mrow[mb] + r;
+      if (m < limit) {
+        const unsigned at = (unsigned)m * orow + cv * (unsigned)sizeof(T);
+        float v[EPL];
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) v[e] = mine[r * S::PO + cv + e];
+        Vec16<T> o;
+        if (z) {
+          if (out_x) {
+            o.set_all(v);
+            store16(at_bytes(out_x + ob, at), o);
+          }
+#pragma unroll
+          for (int e = 0; e < EPL; ++e) {
+            const float zf = zv[i].get(e);
+            v[e] *= zf / (1.f + __expf(-zf));
+          }
+        }
+        o.set_all(v);
+        store16_stream(at_bytes(out + ob, at), o);
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+  }
+}
+
     const float* __restrict__ dt, const float* __restrict__ dA_cs, const T* __restrict__ Bm, Strides3 sB,
     const TS* __restrict__ dstates, const float* __restrict__ D, int d_has_hdim, T* __restrict__ dx,
     Strides3 sdx, float* __restrict__ ddt, int nh, int heads_per_group, int ngroups, int L, int Q, int C,
