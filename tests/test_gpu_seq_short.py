@@ -1,4 +1,5 @@
-"""The split per-row dots and column sums of the stage launchers, at the sizes where they can go wrong."""
+"""The forward over a few rows and the split per-row dots, at the sizes
+where they can go wrong."""
 import pytest
 import torch
 
@@ -8,6 +9,31 @@ from parity_util import announce, check_close
 pytestmark = pytest.mark.gpu
 
 F32, BF16 = torch.float32, torch.bfloat16
+
+
+@pytest.mark.parametrize("form", ["log_decay", "probability"])
+@pytest.mark.parametrize("dtype", [F32, BF16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("b,nh,d", [(1, 1, 8), (3, 2, 264)])
+@pytest.mark.parametrize("L", [1, 7, 8, 9, 15, 16, 17])  # the turn of eight rows and the last row count taken
+def test_short_forward_vs_oracle(L, b, nh, d, dtype, form, device):
+    from kernels.ema_seq import ema_seq_fwd
+
+    announce(f"short forward L={L} b={b} nh={nh} d={d} {dtype} {form}")
+    gen = torch.Generator().manual_seed(L * 31 + d)
+    x = torch.randn(b, L, nh, d, generator=gen).to(dtype)
+    coef = torch.rand(b, L, nh, generator=gen)
+    coef = -2 * coef if form == "log_decay" else coef
+    flat = lambda t: t.permute(0, 2, 1, 3).reshape(b * nh, L, d)
+    cf = coef.permute(0, 2, 1).reshape(b * nh, L)
+    for init in (None, torch.randn(b, nh, d, generator=gen)):
+        ref = O.ema_seq_loop(flat(x.float()), cf, form, None if init is None else init.reshape(b * nh, d))
+        ref = ref[0] if isinstance(ref, tuple) else ref
+        y, final, prev = ema_seq_fwd(coef.to(device), x.to(device), form,
+                                     initial_states=None if init is None else init.to(device))
+        check_close("y", flat(y), ref, dtype)
+        check_close("final", final.reshape(b * nh, d), ref[:, -1], F32)
+        entering = torch.zeros(b * nh, 1, d) if init is None else init.reshape(b * nh, 1, d)
+        assert torch.equal(prev.cpu(), entering)
 
 
 @pytest.mark.parametrize("dtype", [F32, BF16], ids=["f32", "bf16"])

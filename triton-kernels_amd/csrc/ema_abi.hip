@@ -322,6 +322,24 @@ int launch_fwd_tile_t(const void* x, SeqStrides sx, const float* A, SeqStrides s
   if (total > 0x7fffffff) return EMA_ERR_SHAPE;
   if (!ready) EMA_TRY(launch_clear(chain_base, chain_ws_bytes(di), st));
   const ChainWs w = chain_carve(chain_base, di);
+// Rows up to which a thread per 16 bytes running down all rows beats the tile kernel, whose tickets, barriers and
+// chained state cost the same whatever the rows.  Short / tile kernel, us: b8 nh2 d1024 bf16, 1 row 5.6 / 12.4,
+// 16 rows 9.3 / 13.6, 32 rows 13.5 / 13.6; b1 nh1 d64 float32, 16 rows 6.7 / 9.3, 32 rows 10.0 / 9.0; b256 nh4
+// d2048 bf16, 1 row 14.9 / 126, 16 rows 36 / 139, 32 rows 65 / 140.  (Between 16 and 32 rows it depends on how
+// many columns there are; the line is where no size loses.)
+constexpr int kShortRows = 16;
+
+template <typename T, bool XP>
+int launch_fwd_short(const void* x, SeqStrides sx, const float* A, SeqStrides sa, void* y, SeqStrides sy,
+                     float* prev, float* fin, const float* init, const Dims& d, hipStream_t st, void* ev0,
+                     void* ev1) {
+  const int64_t vecs = d.T / Vec16<T>::N, total = d.N * vecs;
+  EMA_TRY(launch_timed(fwd_short_kernel<T, XP>, dim3((unsigned)((total + 255) / 256)), dim3(256), st, ev0, ev1,
+                       (const T*)x, sx, A, sa, (T*)y, sy, prev, fin, init, (int)d.nh, (int)d.L, (int)d.T, (int)vecs,
+                       (int)total));
+  return launched();
+}
+
   auto kernel = fwd_tile_kernel<T, S::FWD_CPL, S::FWD_RPL, S::FWD_MINW, XP>;
   const int64_t cap = resident_blocks(kernel, NT, 0);
   EMA_TRY(launch_timed(kernel, dim3((unsigned)(total < cap ? total : cap)), dim3(NT), st, ev0, ev1, (const T*)x,
@@ -1022,6 +1040,13 @@ static int seq_fwd_impl(int form, const float* coef, int64_t c_sb, int64_t c_sl,
   EMA_TRY(check_form(form));
   EMA_TRY(check_dims(batch, nheads, seqlen, dim, kTileRows, true, &d));
   EMA_TRY(check_dtype(dtype));
+  if (d.L <= kShortRows && d.N * d.T < (int64_t)1 << 31) {
+    // (the workspace is not used, but a caller that passes it as not ready may pass it as ready from now on)
+    if (!ready) EMA_TRY(launch_clear(w.chain, chain_ws_bytes(d), st));
+    auto run = [&](auto launch) { return launch(x, sx, coef, sc, y, sy, prev128, final_state, init, d, st, ev_start, ev_stop); };
+    if (dtype == EMA_BF16) return xp ? run(launch_fwd_short<bf16_t, true>) : run(launch_fwd_short<bf16_t, false>);
+    return xp ? run(launch_fwd_short<float, true>) : run(launch_fwd_short<float, false>);
+  }
   EMA_TRY(check_seq(x, x_sb, x_sl, x_sh, dtype, dim));
   EMA_TRY(check_seq(y, y_sb, y_sl, y_sh, dtype, dim));
   if (!coef || !prev128) return EMA_ERR_NULL;

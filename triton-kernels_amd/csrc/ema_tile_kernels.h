@@ -269,6 +269,62 @@ __device__ __forceinline__ float tile_keep(float coef) {
 }
 
 // ------------------------------------------------------------------------------------
+// Forward over a few rows: decoding, one or a handful of positions per call with the
+// state carried by the caller.  One thread per 16 bytes of a row runs the recurrence down all rows, eight
+// requested at a time; nothing is chained, nothing is shared, so there is no workspace, no ticket and no
+// barrier.  Bound by the latency of one load and one store: b64 nh2 d1024 bf16, one row,
+// 5.5 us where the tile kernel takes 20.1.
+// The recurrence is fwd_tile_kernel's final pass from the same state, so the values are the same.
+// ------------------------------------------------------------------------------------
+template <typename T, bool XP>
+__global__ __launch_bounds__(256) void fwd_short_kernel(const T* __restrict__ x, SeqStrides sx,
+                                                        const float* __restrict__ A, SeqStrides sa,
+                                                        T* __restrict__ y, SeqStrides sy, float* __restrict__ prev,
+                                                        float* __restrict__ final_state,
+                                                        const float* __restrict__ init, int nh, int L, int Tdim,
+                                                        int vecs, int total) {
+  constexpr int VEC = Vec16<T>::N, U = 8;
+  const int id = (int)blockIdx.x * 256 + (int)threadIdx.x;
+  if (id >= total) return;
+  const int n = id / vecs, col = (id - n * vecs) * VEC;
+  const int b = n / nh, h = n - b * nh;
+  const T* xp = x + (int64_t)b * sx.sb + (int64_t)h * sx.sh + col;
+  T* yp = y + (int64_t)b * sy.sb + (int64_t)h * sy.sh + col;
+  const float* ap = A + (int64_t)b * sa.sb + (int64_t)h * sa.sh;
+  const int64_t so = (int64_t)n * Tdim + col;
+  float s[VEC];
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) {
+    s[e] = init ? init[so + e] : 0.f;
+    prev[so + e] = s[e];
+  }
+  for (int l0 = 0; l0 < L; l0 += U) {
+    Vec16<T> v[U];
+    float a[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {  // unconditional loads from rows clamped into the sequence
+      const int64_t l = min(l0 + u, L - 1);
+      v[u] = load16_stream(xp + l * sx.sl);
+      a[u] = ap[l * sa.sl];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (l0 + u >= L) break;
+      const float c = XP ? a[u] : __expf(fminf(a[u], 0.f));
+      float o[VEC];
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) o[e] = s[e] = tile_step<XP>(c, s[e], v[u].get(e));
+      v[u].set_all(o);
+      store16(yp + (int64_t)(l0 + u) * sy.sl, v[u]);
+    }
+  }
+  if (final_state) {
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) final_state[so + e] = s[e];
+  }
+}
+
+// ------------------------------------------------------------------------------------
 // Forward.  Writes y, prev[n,c,:] (state entering each 128-row chunk), optionally a copy at
 // a coarser chunking and the final state.  init (may be null): the state before the first row,
 // (N, T).  hdr / decw / status: the chained-scan workspace (zero-filled once, see
