@@ -13,6 +13,7 @@
 #include "ema_chain_kernels.h"
 #include "ema_tile_kernels.h"
 #include "ema_flat_kernels.h"
+#include "launch_facts.h"
 
 using namespace ema;
 
@@ -136,14 +137,11 @@ int launch_state_passing_bwd(const float* prev, const float* cs_last, int64_t cl
   return launched();
 }
 
-// Kernels that ask for more dynamic LDS than the default limit must opt in once.
+// Kernels that ask for more dynamic LDS than the default limit must opt in, once per device.
 template <typename K>
 int allow_smem(K kernel, int bytes) {
   if (bytes <= 48 * 1024) return EMA_OK;
-  return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess
-             ? EMA_OK
-             : EMA_ERR_LAUNCH;
+  return launch_facts::smem(reinterpret_cast<const void*>(kernel), bytes) ? EMA_OK : EMA_ERR_LAUNCH;
 }
 
 constexpr int kWalkBnBf16 = 128;  // column tile of the per-stage intra-chunk kernels, bf16
@@ -237,14 +235,7 @@ int launch_timed(void (*kernel)(Args...), dim3 grid, dim3 block, hipStream_t st,
 #endif
 template <typename K>
 int resident_blocks(K kernel, int threads, int smem) {
-  int dev = 0, ncu = 0, per_cu = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 256;
-  if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) ncu = 256;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kernel),
-                                                   threads, smem) != hipSuccess || per_cu < 1)
-    per_cu = 1;
-  if (per_cu > EMA_MAX_WGS_PER_CU) per_cu = EMA_MAX_WGS_PER_CU;
-  return ncu * per_cu;
+  return launch_facts::resident(reinterpret_cast<const void*>(kernel), threads, smem, EMA_MAX_WGS_PER_CU);
 }
 
 inline int64_t padded_dim(int64_t T) { return (T + 255) / 256 * 256; }

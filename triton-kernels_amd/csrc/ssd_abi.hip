@@ -7,6 +7,7 @@
 #include <type_traits>
 
 #include "ema_gemm_kernels.h"
+#include "launch_facts.h"
 #include "ssd_kernels.h"
 
 using namespace ssd;
@@ -73,10 +74,7 @@ constexpr int kLdsBytes = 160 * 1024;  // LDS of one CU
 template <typename K>
 int allow_smem(K kernel, int bytes) {
   if (bytes <= 64 * 1024) return SSD_OK;
-  return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                             bytes) == hipSuccess
-             ? SSD_OK
-             : SSD_ERR_LAUNCH;
+  return launch_facts::smem(reinterpret_cast<const void*>(kernel), bytes) ? SSD_OK : SSD_ERR_LAUNCH;
 }
 
 // Calls f.template run<T, P, N>() for the runtime (dtype, hdim, dstate).

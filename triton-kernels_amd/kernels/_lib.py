@@ -5,6 +5,7 @@ operators raise.  There is no CPU or PyTorch fallback.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_void_p
@@ -142,7 +143,16 @@ def require_gpu(*tensors: torch.Tensor) -> torch.device:
 
 
 def stream_ptr(dev: torch.device) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
+    """Handle of the current stream of `dev` (without building a torch.cuda.Stream around it)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if dev.index is None else dev.index)
+
+
+_HERE = contextlib.nullcontext()
+
+
+def on_device(dev: torch.device):
+    """Context in which `dev` is the current device; switches only where it is not already."""
+    return _HERE if dev.index is None or torch.cuda.current_device() == dev.index else torch.cuda.device(dev)
 
 
 def seq_view(x: torch.Tensor):
@@ -153,9 +163,11 @@ def seq_view(x: torch.Tensor):
         x = x.contiguous()
     if x.dim() == 3:
         B, L, T = x.shape
-        return x, [x.data_ptr(), x.stride(0), x.stride(1), 0], B, 1, L, T
+        sb, sl, _ = x.stride()
+        return x, [x.data_ptr(), sb, sl, 0], B, 1, L, T
     b, L, nh, d = x.shape
-    return x, [x.data_ptr(), x.stride(0), x.stride(1), x.stride(2)], b, nh, L, d
+    sb, sl, sh, _ = x.stride()
+    return x, [x.data_ptr(), sb, sl, sh], b, nh, L, d
 
 
 def decay_view(A: torch.Tensor):
@@ -163,8 +175,10 @@ def decay_view(A: torch.Tensor):
     assert A.dim() in (2, 3), "expected (B, L) or (b, L, nh)"
     assert A.dtype == torch.float32, "log-decay must be float32"
     if A.dim() == 2:
-        return [A.data_ptr(), A.stride(0), A.stride(1), 0], A.shape[0], 1, A.shape[1]
-    return [A.data_ptr(), A.stride(0), A.stride(1), A.stride(2)], A.shape[0], A.shape[2], A.shape[1]
+        b, L = A.shape
+        return [A.data_ptr(), *A.stride(), 0], b, 1, L
+    b, L, nh = A.shape
+    return [A.data_ptr(), *A.stride()], b, nh, L
 
 
 def event_ptrs(events):
@@ -225,7 +239,7 @@ def private_workspaces(on: bool) -> None:
 
 
 def _clear(buf: torch.Tensor, dev: torch.device) -> None:
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(lib().ema_workspace_clear(buf.data_ptr(), buf.numel(), stream_ptr(dev)), "ema_workspace_clear")
 
 

@@ -38,7 +38,7 @@ def _ema_matmul_scan_combined_fwd(A_ema, X_ema, chunk_size, dtype=torch.float32,
     L = _lib.lib()
     ws_bytes = L.ema_fwd_workspace_bytes(batch, nh, seqlen, token_dim, chunk_size)
     ws, ready = _lib.workspace(dev, ws_bytes, batch, nh, seqlen, token_dim)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = L.ema_fwd(
             *a_args, *x_args, _lib.dtype_code(x), *y_args, cs.data_ptr(), prev.data_ptr(),
             final.data_ptr(), None if prev128 is None or prev128 is prev else prev128.data_ptr(),

@@ -14,7 +14,7 @@ def ema_chunk_cumsum_fwd(A: torch.Tensor, chunk_size: int):
     a_args, batch, nh, seqlen = _lib.decay_view(A)
     nchunks = math.ceil(seqlen / chunk_size)
     dA_cumsum = torch.empty(batch * nh, nchunks, chunk_size, device=dev, dtype=torch.float32)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = _lib.lib().ema_chunk_cumsum_fwd(
             *a_args, dA_cumsum.data_ptr(), batch, nh, seqlen, chunk_size, _lib.stream_ptr(dev)
         )

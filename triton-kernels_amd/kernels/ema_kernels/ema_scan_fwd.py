@@ -21,7 +21,7 @@ def _ema_scan_fwd(x, A_cumsum, states):
     prev = _lib.f32c(states)
     out = torch.empty(x.shape, device=dev, dtype=x.dtype)
     _, y_args, *_ = _lib.seq_view(out)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = _lib.lib().ema_scan_fwd(
             *x_args, _lib.dtype_code(x), cs.data_ptr(), prev.data_ptr(), *y_args,
             batch, nh, seqlen, token_dim, chunk_size, _lib.stream_ptr(dev),

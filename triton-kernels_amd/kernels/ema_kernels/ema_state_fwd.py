@@ -28,7 +28,7 @@ def _ema_chunk_state_fwd(x, A_cumsum, seq_idx=None, states=None, states_in_fp32=
             out = states
     if out is None:
         out = torch.empty((batch * nh, nchunks, token_dim), device=dev, dtype=torch.float32)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = _lib.lib().ema_chunk_state_fwd(
             *x_args, _lib.dtype_code(x), A_cumsum.data_ptr(), out.data_ptr(),
             batch, nh, seqlen, token_dim, chunk_size, _lib.stream_ptr(dev),

@@ -21,7 +21,7 @@ def _ema_state_passing_fwd(states, A_cs_last, initial_states=None, chunk_size=No
     st_in = _lib.f32c(states)
     out = torch.empty((batch, nchunks, token_dim), device=dev, dtype=torch.float32)
     final_states = torch.empty((batch, token_dim), device=dev, dtype=torch.float32)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = _lib.lib().ema_state_passing_fwd(
             st_in.data_ptr(), A_cs_last.data_ptr(), A_cs_last.stride(0), A_cs_last.stride(1),
             out.data_ptr(), final_states.data_ptr(), batch, nchunks, token_dim,

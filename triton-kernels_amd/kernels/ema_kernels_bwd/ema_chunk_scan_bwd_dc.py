@@ -19,7 +19,7 @@ def _ema_chunk_scan_bwd_dC(prev_states, dA_cumsum, dout, seq_idx=None, C=None, n
     cs = _lib.f32c(dA_cumsum)
     prev = _lib.f32c(prev_states)
     ddA_cumsum = torch.empty(batch * nh, nchunks, chunk_size, device=dev, dtype=torch.float32)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = _lib.lib().ema_chunk_scan_bwd_dc(
             *d_args, _lib.dtype_code(dout), prev.data_ptr(), cs.data_ptr(), ddA_cumsum.data_ptr(),
             batch, nh, seqlen, token_dim, chunk_size, _lib.stream_ptr(dev),

@@ -25,7 +25,7 @@ def _chunk_scan_chunk_state_bwd_dx(x, dA_cumsum, dout, dstates, D=None, seq_idx=
     _, dx_args, *_ = _lib.seq_view(dx)
     cs = _lib.f32c(dA_cumsum)
     g = _lib.f32c(dstates)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = _lib.lib().ema_chunk_scan_chunk_state_bwd_dx(
             *d_args, _lib.dtype_code(dout), cs.data_ptr(), g.data_ptr(), *dx_args,
             batch, nh, seqlen, token_dim, chunk_size, _lib.stream_ptr(dev),

@@ -21,7 +21,7 @@ def _ema_chunk_state_bwd_db(x, dA_cumsum, dstates, seq_idx=None, B=None, ngroups
     cs = _lib.f32c(dA_cumsum)
     g = _lib.f32c(dstates)
     ddA_cumsum = torch.empty(batch * nh, nchunks, chunk_size, device=dev, dtype=torch.float32)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = _lib.lib().ema_chunk_state_bwd_db(
             *x_args, _lib.dtype_code(x), cs.data_ptr(), g.data_ptr(), ddA_cumsum.data_ptr(),
             1 if raw_scale_gradient else 0, batch, nh, seqlen, token_dim, chunk_size,

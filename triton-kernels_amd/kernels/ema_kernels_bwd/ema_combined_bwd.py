@@ -43,7 +43,7 @@ def _ema_chunk_scan_combined_bwd(dout, x, A, chunk_size, dt_limit=(0.0, float("i
     L = _lib.lib()
     ws_bytes = L.ema_bwd_workspace_bytes(batch, nh, seqlen, token_dim, chunk_size)
     ws, ready = _lib.workspace(dev, ws_bytes, batch, nh, seqlen, token_dim)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = L.ema_bwd(
             *d_args, *x_args, *a_args, None if prev128 is None else prev128.data_ptr(),
             _lib.dtype_code(x), *dx_args, ddA.data_ptr(), *y_args,
@@ -83,7 +83,7 @@ def _ema_bwd_dx_dA_fused(x, dA_cumsum, dout, prev_states, dstates, recompute_out
     ws_bytes = L.ema_bwd_dx_dA_fused_workspace_bytes(batch, nh, seqlen, token_dim)
     assert ws_bytes > 0, "unsupported shape"
     ws = torch.empty(ws_bytes, device=dev, dtype=torch.uint8)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = L.ema_bwd_dx_dA_fused(
             *x_args, *d_args, _lib.dtype_code(x), cs.data_ptr(), prev.data_ptr(), g.data_ptr(),
             *dx_args, ddA.data_ptr(), *y_args, ws.data_ptr(), ws_bytes, batch, nh, seqlen,

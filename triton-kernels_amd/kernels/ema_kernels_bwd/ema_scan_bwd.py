@@ -19,7 +19,7 @@ def _ema_chunk_scan_bwd_dstates(dA_cumsum, dout, seq_idx=None, dtype=None):
     dtype = dA_cumsum.dtype if dtype is None else dtype
     cs = _lib.f32c(dA_cumsum)
     ds = torch.empty(batch * nh, nchunks, token_dim, device=dev, dtype=torch.float32)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = _lib.lib().ema_chunk_scan_bwd_dstates(
             *d_args, _lib.dtype_code(dout), cs.data_ptr(), ds.data_ptr(),
             batch, nh, seqlen, token_dim, chunk_size, _lib.stream_ptr(dev),

@@ -25,7 +25,7 @@ def _ema_chunk_scan_bwd_ddAcs_stable(x, dA_cumsum, dout):
     )
     assert ws_bytes > 0, "unsupported shape"
     ws = torch.empty(ws_bytes, device=dev, dtype=torch.uint8)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = L.ema_chunk_scan_bwd_ddAcs(
             *x_args, *d_args, _lib.dtype_code(x), cs.data_ptr(), ddA_cumsum.data_ptr(),
             ws.data_ptr(), ws_bytes, batch, nh, seqlen, token_dim, chunk_size, _lib.stream_ptr(dev),

@@ -37,7 +37,7 @@ def _ema_state_passing_bwd(
     L = _lib.lib()
     ws_bytes = L.ema_state_passing_bwd_workspace_bytes(batch, nchunks, token_dim)
     ws = torch.empty(ws_bytes, device=dev, dtype=torch.uint8)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = L.ema_state_passing_bwd(
             prev.data_ptr(), dA_chunk_cumsum.data_ptr(), dA_chunk_cumsum.stride(0),
             dA_chunk_cumsum.stride(1), ds.data_ptr(), g.data_ptr(), ddA.data_ptr(),

@@ -42,21 +42,20 @@ def ema_seq_fwd(coef, x, form="log_decay", initial_states=None, kernel_events=No
     N = batch * nh
     y = torch.empty_like(x)
     _, ys, *_ = _lib.seq_view(y)
-    final = torch.empty(N, T, dtype=torch.float32, device=dev)
+    final = torch.empty((batch, T) if x.dim() == 3 else (batch, nh, T), dtype=torch.float32, device=dev)
     prev128 = torch.empty(N, -(-L // 128), T, dtype=torch.float32, device=dev)
     init = None if initial_states is None else _state_2d(initial_states, batch, nh, T, "initial_states")
     nbytes = lib.ema_seq_fwd_workspace_bytes(batch, nh, L, T)
     ws, ready = _lib.workspace(dev, nbytes, batch, nh, L, T) if workspace is None else workspace
     assert ws.numel() >= nbytes
     ev0, ev1 = _lib.event_ptrs(kernel_events)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         _lib.check(
             lib.ema_seq_fwd(FORMS[form], *cs_, *xs, _lib.dtype_code(x), *ys,
                             None if init is None else init.data_ptr(), final.data_ptr(),
                             prev128.data_ptr(), ws.data_ptr(), ws.numel(), ready, batch, nh, L, T,
                             _lib.stream_ptr(dev), ev0, ev1),
             "ema_seq_fwd")
-    final = final.reshape(batch, T) if x.dim() == 3 else final.reshape(batch, nh, T)
     return y, final, prev128
 
 
@@ -80,20 +79,20 @@ def ema_seq_bwd(dy, x, coef, prev128, form="log_decay", dfinal_states=None, want
     dcoef = torch.empty_like(coef)
     dcs, *_ = _lib.decay_view(dcoef)
     dfin = None if dfinal_states is None else _state_2d(dfinal_states, batch, nh, T, "dfinal_states")
-    dinit = torch.empty(N, T, dtype=torch.float32, device=dev) if want_dinit else None
+    dinit = None
+    if want_dinit:
+        dinit = torch.empty((batch, T) if x.dim() == 3 else (batch, nh, T), dtype=torch.float32, device=dev)
     nbytes = lib.ema_seq_bwd_workspace_bytes(batch, nh, L, T)
     ws, ready = _lib.workspace(dev, nbytes, batch, nh, L, T) if workspace is None else workspace
     assert ws.numel() >= nbytes
     ev0, ev1 = _lib.event_ptrs(kernel_events)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         _lib.check(
             lib.ema_seq_bwd(FORMS[form], *ds, *xs, *cs_, prev128.data_ptr(),
                             None if dfin is None else dfin.data_ptr(), _lib.dtype_code(x), *dxs, *dcs,
                             None if dinit is None else dinit.data_ptr(), ws.data_ptr(), ws.numel(),
                             ready, batch, nh, L, T, _lib.stream_ptr(dev), ev0, ev1),
             "ema_seq_bwd")
-    if dinit is not None:
-        dinit = dinit.reshape(batch, T) if x.dim() == 3 else dinit.reshape(batch, nh, T)
     return dx, dcoef, dinit
 
 

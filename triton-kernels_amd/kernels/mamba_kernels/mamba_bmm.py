@@ -35,7 +35,7 @@ def _bmm_chunk_fwd(a, b, chunk_size, seq_idx=None, causal=False, output_dtype=No
     out_dtype = a.dtype if output_dtype is None else output_dtype
     kernel_out = torch.float32 if out_dtype != a4.dtype else out_dtype
     out = torch.empty(batch, nchunks, ngroups, chunk_size, chunk_size, device=dev, dtype=kernel_out)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         _lib.check(
             _lib.lib().ssd_bmm_chunk_fwd(*sa, *sb, _lib.dtype_code(a4), out.data_ptr(), _lib.dtype_code(out), batch,
                                          seqlen, ngroups, k, chunk_size, *ids, _lib.stream_ptr(dev)),

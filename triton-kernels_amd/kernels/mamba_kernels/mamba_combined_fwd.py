@@ -38,7 +38,7 @@ def _chunk_state_passing_fwd(B, x, dt, dA_cumsum, initial_states=None, out_dtype
     init = None if initial_states is None else _lib.f32c(initial_states)
     states = torch.empty(batch, nchunks, nheads, headdim, dstate, device=dev, dtype=out_dtype)
     final_states = torch.empty(batch, nheads, headdim, dstate, device=dev, dtype=torch.float32)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         _lib.check(
             _lib.lib().ssd_chunk_state_passing_fwd(*bs, *xs, _lib.dtype_code(x), dt_f.data_ptr(), dA_f.data_ptr(),
                                                    None if init is None else init.data_ptr(), states.data_ptr(),

@@ -23,7 +23,7 @@ def _chunk_cumsum_fwd(dt, A, chunk_size, dt_bias=None, dt_softplus=False, dt_lim
     dA_cumsum = torch.empty(batch, nheads, nchunks, chunk_size, device=dev, dtype=torch.float32)
     Af = _lib.f32c(A)
     bias = None if dt_bias is None else _lib.f32c(dt_bias)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         _lib.check(
             _lib.lib().ssd_chunk_cumsum_fwd(
                 dt.data_ptr(), _lib.dtype_code(dt), dt.stride(0), dt.stride(1), dt.stride(2), Af.data_ptr(),

@@ -44,7 +44,7 @@ def _chunk_scan_fwd(cb, x, dt, dA_cumsum, C, states, D=None, z=None, seq_idx=Non
     cb_f = _lib.f32c(cb)
     dt_f = _lib.f32c(dt)
     dA_cumsum_f = _lib.f32c(dA_cumsum)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         _lib.check(
             _lib.lib().ssd_chunk_scan_fwd(
                 cb_f.data_ptr(), *xs, *zs, _lib.dtype_code(x), dt_f.data_ptr(),

@@ -37,7 +37,7 @@ def _chunk_state_fwd(B, x, dt, dA_cumsum, seq_idx=None, states=None, states_in_f
     # float32 views / copies are bound to names so that they outlive the launch below
     dt_f = _lib.f32c(dt)
     dA_cumsum_f = _lib.f32c(dA_cumsum)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         _lib.check(
             _lib.lib().ssd_chunk_state_fwd(*bs, *xs, _lib.dtype_code(x), dt_f.data_ptr(),
                                            dA_cumsum_f.data_ptr(), out.data_ptr(), batch, seqlen, nheads,
@@ -80,7 +80,7 @@ def chunk_state_varlen(B, x, dt, dA_cumsum, cu_seqlens, chunk_states):
     # float32 views / copies are bound to names so that they outlive the launch below
     dt_f = _lib.f32c(dt)
     dA_cumsum_f = _lib.f32c(dA_cumsum)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         _lib.check(
             _lib.lib().ssd_chunk_state_varlen(B.data_ptr(), B.stride(0), B.stride(1), x.data_ptr(), x.stride(0),
                                               x.stride(1), _lib.dtype_code(x), dt_f.data_ptr(),

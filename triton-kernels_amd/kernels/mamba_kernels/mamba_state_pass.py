@@ -34,7 +34,7 @@ def _state_passing_fwd(states, dA_chunk_cumsum, initial_states=None, seq_idx=Non
     native = out_dtype if out_dtype in (torch.float32, torch.bfloat16) else torch.float32
     out = torch.empty(batch, nchunks, nheads, dim, device=dev, dtype=native)
     final_states = torch.empty(batch, nheads, dim, device=dev, dtype=torch.float32)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         _lib.check(
             _lib.lib().ssd_state_passing_fwd(st.data_ptr(), da.data_ptr(), da.stride(0), da.stride(1), da.stride(2),
                                              None if init is None else init.data_ptr(), out.data_ptr(),

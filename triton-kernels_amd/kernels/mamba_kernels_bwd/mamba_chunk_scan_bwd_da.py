@@ -33,7 +33,7 @@ def _chunk_scan_bwd_ddAcs_stable(x, dt, dA_cumsum, dout, cb):
     dt_f = _lib.f32c(dt)
     dA_cumsum_f = _lib.f32c(dA_cumsum)
     cb_f = _lib.f32c(cb)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         _lib.check(
             lib.ssd_chunk_scan_bwd_ddAcs(*xs, *ds, _lib.dtype_code(x), dt_f.data_ptr(),
                                          dA_cumsum_f.data_ptr(), cb_f.data_ptr(),

@@ -51,7 +51,7 @@ def _chunk_scan_chunk_state_bwd_dx(x, dt, dA_cumsum, B, CB, dout, dstates, D=Non
     CB_f = _lib.f32c(CB)
     dt_f = _lib.f32c(dt)
     dA_cumsum_f = _lib.f32c(dA_cumsum)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         _lib.check(
             _lib.lib().ssd_chunk_scan_chunk_state_bwd_dx(
                 CB_f.data_ptr(), *xs, *ds, _lib.dtype_code(x), dt_f.data_ptr(),

@@ -37,7 +37,7 @@ def _chunk_state_bwd_db(x, dt, dA_cumsum, dstates, seq_idx=None, B=None, ngroups
     # float32 views / copies are bound to names so that they outlive the launch below
     dt_f = _lib.f32c(dt)
     dA_cumsum_f = _lib.f32c(dA_cumsum)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         _lib.check(
             _lib.lib().ssd_chunk_state_bwd_db(*xs, _lib.dtype_code(x), dt_f.data_ptr(),
                                               dA_cumsum_f.data_ptr(), dstates.data_ptr(), ds_code, *bs,

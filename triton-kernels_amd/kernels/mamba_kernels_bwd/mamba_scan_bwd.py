@@ -32,7 +32,7 @@ def _chunk_scan_bwd_dstates(C, dA_cumsum, dout, seq_idx=None, dtype=None):
     out = torch.empty(batch, nchunks, nheads, headdim, dstate, device=dev, dtype=native)
     # float32 views / copies are bound to names so that they outlive the launch below
     dA_cumsum_f = _lib.f32c(dA_cumsum)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         _lib.check(
             _lib.lib().ssd_chunk_scan_bwd_dstates(*cs, *ds, _lib.dtype_code(dout), dA_cumsum_f.data_ptr(),
                                                   out.data_ptr(), _lib.dtype_code(out), batch, seqlen, nheads, ngroups, headdim, dstate,

@@ -43,7 +43,7 @@ def _state_passing_bwd(states, dA_chunk_cumsum, dout, dfinal_states=None, seq_id
     dinit = torch.empty(batch, nheads, dim, device=dev, dtype=torch.float32) if has_initial_states else None
     nbytes = lib.ssd_state_passing_bwd_workspace_bytes(batch, nchunks, nheads, dim)
     ws = torch.empty(max(nbytes, 16), device=dev, dtype=torch.uint8)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         _lib.check(
             lib.ssd_state_passing_bwd(st.data_ptr(), st_code, da.data_ptr(), da.stride(0), da.stride(1), da.stride(2),
                                       do.data_ptr(), do_code, None if dfin is None else dfin.data_ptr(),
