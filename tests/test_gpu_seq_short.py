@@ -1,4 +1,4 @@
-"""The forward over a few rows and the split per-row dots, at the sizes
+"""The forward over a few rows, the one-launch packing of coefficients and the split per-row dots, at the sizes
 where they can go wrong."""
 import pytest
 import torch
@@ -34,6 +34,42 @@ def test_short_forward_vs_oracle(L, b, nh, d, dtype, form, device):
         check_close("final", final.reshape(b * nh, d), ref[:, -1], F32)
         entering = torch.zeros(b * nh, 1, d) if init is None else init.reshape(b * nh, 1, d)
         assert torch.equal(prev.cpu(), entering)
+
+
+@pytest.mark.parametrize("form", ["log_decay", "probability"])
+@pytest.mark.parametrize("layout", ["flat", "headed", "permuted", "expanded"])
+def test_packing_in_one_launch_equals_tensor_operations(layout, form, device):
+    """int32 ids take the one-launch packing, int64 ids the tensor operations: same outputs, same gradients,
+    for every layout of the coefficient and of the ids."""
+    from kernels.ema_seq import ema_seq_scan
+
+    announce(f"packing {layout} {form}")
+    b, L, nh, d = 2, 150, 3, 16
+    gen = torch.Generator().manual_seed(5)
+    base = torch.rand(b, L, nh, generator=gen)
+    base = -base if form == "log_decay" else base
+    x = torch.randn(b, L, nh, d, generator=gen)
+    if layout == "flat":
+        base, x = base[..., 0].contiguous(), x[:, :, 0].contiguous()
+    ids = (torch.rand(b, L, generator=gen) < 0.1).to(torch.int32).cumsum(1, dtype=torch.int32)
+    dy = torch.randn(x.shape, generator=gen)
+    res = []
+    for id_type in (torch.int32, torch.int64):
+        if layout == "permuted":
+            leaf = base.permute(2, 0, 1).contiguous().to(device).requires_grad_()
+            coef, seq = leaf.permute(1, 2, 0), ids.t().contiguous().to(device, id_type).t()
+        elif layout == "expanded":
+            leaf = base[..., :1].contiguous().to(device).requires_grad_()
+            coef, seq = leaf.expand(b, L, nh), ids[:1].to(device, id_type).expand(b, L)
+        else:
+            leaf = base.to(device).requires_grad_()
+            coef, seq = leaf, ids.to(device, id_type)
+        xg = x.to(device).requires_grad_()
+        y, final = ema_seq_scan(coef, xg, form=form, return_final_states=True, seq_idx=seq)
+        torch.autograd.backward((y, final), (dy.to(device), torch.ones_like(final)))
+        res.append((y.detach(), final.detach(), xg.grad, leaf.grad))
+    for name, a, c in zip(("y", "final", "dx", "dcoef"), *res):
+        check_close(name, a, c.cpu(), F32)
 
 
 @pytest.mark.parametrize("dtype", [F32, BF16], ids=["f32", "bf16"])

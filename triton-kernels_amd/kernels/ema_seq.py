@@ -147,9 +147,55 @@ def pack_probability(p, seq_idx):
     return torch.where(start, -p, p)
 
 
+def _coef_starts(src, seq_idx, form, gradient, dst=None):
+    """One launch of what pack_log_decay / pack_probability (gradient=False) and their backward do."""
+    dst = torch.empty_like(src) if dst is None else dst
+    dev = _lib.require_gpu(src, dst, seq_idx)
+    ss, batch, nh, L = _lib.decay_view(src)
+    ds, *_ = _lib.decay_view(dst)
+    with _lib.on_device(dev):
+        _lib.check(
+            _lib.lib().ema_coef_starts(FORMS[form], int(gradient), *ss, *ds, seq_idx.data_ptr(), *seq_idx.stride(),
+                                       batch, nh, L, _lib.stream_ptr(dev)),
+            "ema_coef_starts")
+    return dst
+
+
+class EMASeqPackedFn(torch.autograd.Function):
+    """EMASeqFn on the packed form of coef, with the packing and its gradient in one launch each."""
+
+    @staticmethod
+    def forward(ctx, coef, x, initial_states, form, seq_idx):
+        packed = _coef_starts(coef, seq_idx, form, gradient=False)
+        y, final, prev128 = ema_seq_fwd(packed, x, form, initial_states)
+        ctx.save_for_backward(packed, x, prev128, seq_idx)
+        ctx.form = form
+        ctx.has_init = initial_states is not None
+        ctx.init_dtype = None if initial_states is None else initial_states.dtype
+        ctx.set_materialize_grads(False)
+        return y, final
+
+    @staticmethod
+    def backward(ctx, dy, dfinal):
+        packed, x, prev128, seq_idx = ctx.saved_tensors
+        if dy is None:
+            dy = torch.zeros_like(x)
+        dx, dcoef, dinit = ema_seq_bwd(dy.contiguous(), x, packed, prev128, ctx.form, dfinal_states=dfinal,
+                                       want_dinit=ctx.has_init)
+        dcoef = _coef_starts(dcoef, seq_idx, ctx.form, gradient=True, dst=dcoef)
+        if dinit is not None:
+            dinit = dinit.to(ctx.init_dtype)
+        return dcoef, dx, dinit, None, None
+
+
 def ema_seq_scan(coef, x, form="log_decay", initial_states=None, return_final_states=False, seq_idx=None):
     """Differentiable in coef, x and initial_states (and through the final states).  seq_idx
     (batch, L) marks packed sequences: the state is reset where it changes."""
+    if seq_idx is not None and seq_idx.dtype == torch.int32 and coef.dtype == torch.float32 and coef.is_cuda \
+            and seq_idx.device == coef.device and form in FORMS:
+        assert seq_idx.shape == coef.shape[:2], "seq_idx must be (batch, seqlen)"
+        y, final = EMASeqPackedFn.apply(coef, x, initial_states, form, seq_idx)
+        return (y, final) if return_final_states else y
     if seq_idx is not None:
         coef = pack_log_decay(coef, seq_idx) if form == "log_decay" else pack_probability(coef, seq_idx)
     y, final = EMASeqFn.apply(coef, x, initial_states, form)
