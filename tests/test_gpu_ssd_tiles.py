@@ -1,4 +1,5 @@
-"""The chunk scan in one tile per chunk (chunks of 64 and 128 rows), at the sizes where it can go wrong."""
+"""The chunk scan in one tile per chunk (chunks of 64 and 128 rows) and the states at the ends of packed
+sequences, at the sizes where they can go wrong."""
 import pytest
 import torch
 
@@ -41,3 +42,24 @@ def test_chunk_scan_one_tile_vs_oracle(Q, L, nh, g, P, dtype, kind, device):
         check_close("out", got, ref, dtype, regrouped=True)
         if zz is not None:
             check_close("out_x", got_x, ref_x, dtype, regrouped=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [F32, BF16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("P,N", [(64, 64), (128, 128), (64, 128)])
+def test_varlen_states_at_stage_edges(P, N, dtype, device):
+    """Sequences that end one row into a chunk, on and around the 64-row stages, and an empty one."""
+    from kernels.ema_chunk_state import chunk_state_varlen
+
+    announce(f"varlen stages P={P} N={N} {dtype}")
+    Q, nh, g = 256, 4, 2
+    cu = torch.tensor([0, 1, 64, 129, 129, 257, 320, 511, 577], dtype=torch.int32)
+    L = int(cu[-1])
+    gen = torch.Generator().manual_seed(9)
+    r = lambda *s: torch.randn(*s, generator=gen)
+    x, B = r(L, nh, P).to(dtype), r(L, g, N).to(dtype)
+    dA, dt = S.chunk_cumsum(torch.rand(1, L, nh, generator=gen) * 0.5, -torch.rand(nh, generator=gen), Q)
+    prev = r(-(-L // Q), nh, P, N).to(dtype)
+    ref = S.chunk_state_varlen(B, x, dt[0], dA[0], cu, prev, dtype)
+    got = chunk_state_varlen(*(t.to(device) for t in (B, x, dt[0], dA[0], cu, prev)))
+    check_close("varlen states", got, ref, dtype, regrouped=True)

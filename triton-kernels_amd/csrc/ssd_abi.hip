@@ -194,6 +194,8 @@ struct ScanLaunch {
                        (const T*)x, sx, (const T*)z, sz, dt, dA, (const T*)C, sC, (const TS*)prev, D, d_has_hdim,
                        (T*)out, so, (T*)out_x, (int)d.nh, (int)(d.nh / d.g), (int)d.g, (int)d.L, (int)d.Q, (int)d.C,
                        stiles, seq);
+    return launched();
+  }
   template <typename T, int P, int N, typename TS, int HP, int ST>
   int launch_mid() const {
     auto kernel = ssd_chunk_scan_mid_kernel<T, P, N, TS, HP, ST>;
@@ -226,8 +228,6 @@ struct ScanLaunch {
       return launch_mid<T, P, N, TS, 1, ST>();
     }
   }
-    return launched();
-  }
   template <typename T, int P, int N, typename TS>
   int run_as() const {
     constexpr int wide_smem = WideSmem<T, P, N>::kBytes;
@@ -239,12 +239,12 @@ struct ScanLaunch {
         const bool dense = sx.sh == P && so.sh == P && (!z || sz.sh == P);
         if (dense && (d.nh / d.g) % 2 == 0) return launch_wide<T, P, N, TS, 2>();
       }
+      return launch_wide<T, P, N, TS, 1>();
+    }
     if ((d.Q == 64 || d.Q == 128) && close) {
       bool taken;
       const int status = d.Q == 128 ? launch_mid_pairs<T, P, N, TS, 128>(&taken) : launch_mid_pairs<T, P, N, TS, 64>(&taken);
       if (taken) return status;
-    }
-      return launch_wide<T, P, N, TS, 1>();
     }
     auto kernel = ssd_chunk_scan_kernel<T, P, N, TS>;
     constexpr int smem = ScanSmem<T, P, N>::kBytes;
@@ -843,35 +843,46 @@ int ssd_chunk_scan_bwd_ddAcs(const void* x, int64_t x_sb, int64_t x_sl, int64_t 
   return launched();
 }
 
-int ssd_chunk_state_varlen(const void* B, int64_t b_sl, int64_t b_sg, const void* x, int64_t x_sl, int64_t x_sh,
-                           int dtype, const float* dt, const float* dA_cumsum, const void* chunk_states,
-                           int states_dtype, const int32_t* cu_seqlens, float* states, int64_t nseq, int64_t seqlen, int64_t nheads,
-                           int64_t ngroups, int64_t hdim, int64_t dstate, int64_t chunk, void* stream) {
+namespace {
+// The states at the sequence ends in float32 or, with states_dtype bfloat16, rounded to it.
+int varlen_states(const void* B, int64_t b_sl, int64_t b_sg, const void* x, int64_t x_sl, int64_t x_sh, int dtype,
+                  const float* dt, const float* dA_cumsum, const void* chunk_states, int states_dtype,
+                  const int32_t* cu_seqlens, void* states, int out_dtype, int64_t nseq, int64_t seqlen,
+                  int64_t nheads, int64_t ngroups, int64_t hdim, int64_t dstate, int64_t chunk, void* stream) {
   Dims d;
   SSD_TRY(check_dims(1, seqlen, nheads, ngroups, hdim, dstate, chunk, &d));
   SSD_TRY(check_dtype(dtype));
   if (nseq <= 0 || nseq > 65535 || hdim <= 0 || dstate <= 0 || hdim > 4096 || dstate > 4096) return SSD_ERR_SHAPE;
   if (states_dtype != SSD_F32 && states_dtype != dtype) return SSD_ERR_DTYPE;
+  if (out_dtype != SSD_F32 && out_dtype != states_dtype) return SSD_ERR_DTYPE;
   if (!B || !x || !dt || !dA_cumsum || !chunk_states || !cu_seqlens || !states) return SSD_ERR_NULL;
   const int64_t tiles = ((hdim + 63) / 64) * ((dstate + 63) / 64);
   const dim3 grid((unsigned)tiles, (unsigned)nseq, (unsigned)nheads);
   const int hpg = (int)(nheads / ngroups);
-  if (dtype == SSD_BF16 && states_dtype == SSD_BF16)
-    hipLaunchKernelGGL((ssd_chunk_state_varlen_kernel<bf16_t, bf16_t>), grid, dim3(256), 0, as_stream(stream),
-                       (const bf16_t*)x, x_sl, x_sh, (const bf16_t*)B, b_sl, b_sg, dt, dA_cumsum,
-                       (const bf16_t*)chunk_states, cu_seqlens, states, (int)seqlen, (int)nheads, hpg, (int)hdim,
-                       (int)dstate, (int)chunk, (int)d.C);
-  else if (dtype == SSD_BF16)
-    hipLaunchKernelGGL((ssd_chunk_state_varlen_kernel<bf16_t, float>), grid, dim3(256), 0, as_stream(stream),
-                       (const bf16_t*)x, x_sl, x_sh, (const bf16_t*)B, b_sl, b_sg, dt, dA_cumsum,
-                       (const float*)chunk_states, cu_seqlens, states, (int)seqlen, (int)nheads, hpg, (int)hdim,
-                       (int)dstate, (int)chunk, (int)d.C);
-  else
-    hipLaunchKernelGGL((ssd_chunk_state_varlen_kernel<float, float>), grid, dim3(256), 0, as_stream(stream),
-                       (const float*)x, x_sl, x_sh, (const float*)B, b_sl, b_sg, dt, dA_cumsum,
-                       (const float*)chunk_states, cu_seqlens, states, (int)seqlen, (int)nheads, hpg, (int)hdim,
-                       (int)dstate, (int)chunk, (int)d.C);
+  // the matrix kernel takes whole 64 x 64 tiles of the state and rows in 16-byte pieces; anything else is
+  // multiplied out in float32
+  const bool mma = hdim % 64 == 0 && dstate % 64 == 0 && check_vec(x, 0, x_sl, x_sh, dtype, hdim) == SSD_OK &&
+                   check_vec(B, 0, b_sl, b_sg, dtype, dstate) == SSD_OK;
+#define SSD_VARLEN_LAUNCH(T, TS, TO)                                                                                   \
+  hipLaunchKernelGGL((mma ? ssd_chunk_state_varlen_mma_kernel<T, TS, TO> : ssd_chunk_state_varlen_kernel<T, TS, TO>),  \
+                     grid, dim3(256), 0, as_stream(stream), (const T*)x, x_sl, x_sh, (const T*)B, b_sl, b_sg, dt,      \
+                     dA_cumsum, (const TS*)chunk_states, cu_seqlens, (TO*)states, (int)seqlen, (int)nheads, hpg,       \
+                     (int)hdim, (int)dstate, (int)chunk, (int)d.C)
+  if (dtype != SSD_BF16) SSD_VARLEN_LAUNCH(float, float, float);
+  else if (states_dtype != SSD_BF16) SSD_VARLEN_LAUNCH(bf16_t, float, float);
+  else if (out_dtype == SSD_BF16) SSD_VARLEN_LAUNCH(bf16_t, bf16_t, bf16_t);
+  else SSD_VARLEN_LAUNCH(bf16_t, bf16_t, float);
+#undef SSD_VARLEN_LAUNCH
   return launched();
+}
+}  // namespace
+
+int ssd_chunk_state_varlen(const void* B, int64_t b_sl, int64_t b_sg, const void* x, int64_t x_sl, int64_t x_sh,
+                           int dtype, const float* dt, const float* dA_cumsum, const void* chunk_states,
+                           int states_dtype, const int32_t* cu_seqlens, float* states, int64_t nseq, int64_t seqlen, int64_t nheads,
+                           int64_t ngroups, int64_t hdim, int64_t dstate, int64_t chunk, void* stream) {
+  return varlen_states(B, b_sl, b_sg, x, x_sl, x_sh, dtype, dt, dA_cumsum, chunk_states, states_dtype, cu_seqlens,
+                       states, SSD_F32, nseq, seqlen, nheads, ngroups, hdim, dstate, chunk, stream);
 }
 
 #ifdef SSD_TIMING

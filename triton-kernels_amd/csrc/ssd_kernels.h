@@ -2998,11 +2998,11 @@ __global__ __launch_bounds__(256, (P == 64 ? 3 : 2)) void ssd_chunk_scan_bwd_dx_
 // Grid (P tiles * N tiles, sequences, heads).  The weighted B is rounded to T before the product,
 // as the reference does; an empty or out-of-range sequence gives zeros.
 // ------------------------------------------------------------------------------------
-template <typename T, typename TS>
+template <typename T, typename TS, typename TO>
 __global__ __launch_bounds__(256) void ssd_chunk_state_varlen_kernel(
     const T* __restrict__ x, int64_t x_sl, int64_t x_sh, const T* __restrict__ Bm, int64_t b_sl, int64_t b_sg,
     const float* __restrict__ dt, const float* __restrict__ dA_cs, const TS* __restrict__ chunk_states,
-    const int32_t* __restrict__ cu_seqlens, float* __restrict__ out, int L, int nh, int hpg, int P, int N, int Q,
+    const int32_t* __restrict__ cu_seqlens, TO* __restrict__ out, int L, int nh, int hpg, int P, int N, int Q,
     int C) {
   constexpr int TP = 64, TN = 64, KB = 32;
   __shared__ float sx[KB][TP];
@@ -3066,9 +3066,87 @@ __global__ __launch_bounds__(256) void ssd_chunk_state_varlen_kernel(
       if (p < P && n < N) {
         float v = acc[i][j];
         if (carried) v = fmaf((float)chunk_states[(((int64_t)c * nh + h) * P + p) * N + n], keep, v);
-        out[(((int64_t)s * nh + h) * P + p) * N + n] = v;
+        out[(((int64_t)s * nh + h) * P + p) * N + n] = (TO)v;
       }
     }
 }
 
 }  // namespace ssd
+// ------------------------------------------------------------------------------------
+// The same on the matrix units, for state tiles of 64 x 64 that divide the state and rows that can be read 16
+// bytes at a time.  Wave w owns one 32 x 32 block of the tile; 64 positions per stage, the next stage's rows
+// under way while this one is multiplied.  Bound by the chain of its loads (a handful of workgroups per compute
+// unit, two stages each): b1 nh24 hdim 64 dstate 128 chunk 128, 6 sequences, 27.1 us by
+// the kernel above, 13.2 here.
+// ------------------------------------------------------------------------------------
+template <typename T, typename TS, typename TO>
+__global__ __launch_bounds__(256) void ssd_chunk_state_varlen_mma_kernel(
+    const T* __restrict__ x, int64_t x_sl, int64_t x_sh, const T* __restrict__ Bm, int64_t b_sl, int64_t b_sg,
+    const float* __restrict__ dt, const float* __restrict__ dA_cs, const TS* __restrict__ chunk_states,
+    const int32_t* __restrict__ cu_seqlens, TO* __restrict__ out, int L, int nh, int hpg, int P, int N, int Q,
+    int C) {
+  constexpr int KT = 64, W = 64, PITCH = Tile<T>::kpitch(W), EPL = Vec16<T>::N, KG = Tile<T>::KG;
+  constexpr int VPR = W / EPL, CNT = KT * VPR / 256;
+  __shared__ __attribute__((aligned(16))) T xs[KT * PITCH];
+  __shared__ __attribute__((aligned(16))) T bs[KT * PITCH];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tiles_n = N / W;
+  const int p0 = (blockIdx.x / tiles_n) * W, n0 = (blockIdx.x % tiles_n) * W;
+  const int s = blockIdx.y, h = blockIdx.z;
+  const int start = cu_seqlens[s];
+  const int end = min(cu_seqlens[s + 1], L);
+  const bool live = start >= 0 && end > start;  // uniform over the workgroup
+  const int c = live ? (end - 1) / Q : 0;
+  const int limit = live ? end - c * Q : 0;     // positions of chunk c up to the sequence's end
+  const int first = max(start - c * Q, 0);      // first position of chunk c that belongs to s
+  const int64_t row = ((int64_t)h * C + c) * Q;  // dt, dA_cumsum are (nheads, nchunks, Q)
+  const float dA_last = live ? dA_cs[row + limit - 1] : 0.f;
+  const T* xg = x + (int64_t)c * Q * x_sl + (int64_t)h * x_sh + p0;
+  const T* bg = Bm + (int64_t)c * Q * b_sl + (int64_t)(h / hpg) * b_sg + n0;
+  Vec16<T> xv[CNT], bv[CNT];
+  float w[CNT];
+  auto request = [&](int k0) {
+#pragma unroll
+    for (int i = 0; i < CNT; ++i) {
+      const int idx = tid + 256 * i, k = k0 + idx / VPR, kc = min(k, limit - 1), cv = (idx % VPR) * EPL;
+      xv[i] = load16(xg + (int64_t)kc * x_sl + cv);
+      bv[i] = load16(bg + (int64_t)kc * b_sl + cv);
+      const float f = __expf(fminf(dA_last - dA_cs[row + kc], 0.f)) * dt[row + kc];
+      w[i] = k >= first && k < limit ? f : 0.f;
+    }
+  };
+  floatx16 acc;
+  zero_acc(acc);
+  const int mi = wave & 1, ni = wave >> 1;
+  const int kbeg = first / KT * KT;
+  if (kbeg < limit) request(kbeg);
+  for (int k0 = kbeg; k0 < limit; k0 += KT) {
+    __syncthreads();  // every wave is done with the stage that is overwritten now
+#pragma unroll
+    for (int i = 0; i < CNT; ++i) {
+      const int idx = tid + 256 * i, at = idx / VPR * PITCH + (idx % VPR) * EPL;
+      float t[EPL];
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) t[e] = bv[i].get(e) * w[i];
+      bv[i].set_all(t);
+      if (w[i] == 0.f) xv[i].zero(), bv[i].zero();  // whatever another sequence holds there
+      store16(xs + at, xv[i]);
+      store16(bs + at, bv[i]);
+    }
+    __syncthreads();
+    if (k0 + KT < limit) request(k0 + KT);
+#pragma unroll
+    for (int kk = 0; kk < KT; kk += KG)
+      mma_group(frag_cols(xs, PITCH, kk, 32 * mi, lane), frag_cols(bs, PITCH, kk, 32 * ni, lane), acc);
+  }
+  const bool carried = live && start < c * Q;  // the sequence began before chunk c
+  const float keep = carried ? __expf(dA_last) : 0.f;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    const int64_t at = (int64_t)(p0 + 32 * mi + acc_row(v, lane)) * N + n0 + 32 * ni + (lane & 31);
+    float r = acc[v];
+    if (carried) r = fmaf((float)chunk_states[((int64_t)c * nh + h) * P * N + at], keep, r);
+    out[((int64_t)s * nh + h) * P * N + at] = (TO)r;
+  }
+}
+
