@@ -72,10 +72,10 @@ inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s);
 
 // ---------------------------------------------------------------- launch helpers
 
-// prob = 1: the input holds probabilities p and the sums are of log(1 - p).
 // Workgroups that fill the chip in the streaming kernels: four on each of 256 compute units.
 constexpr int64_t kFillWorkgroups = 1024;
 
+// prob = 1: the input holds probabilities p and the sums are of log(1 - p).
 int launch_cumsum(const float* A, SeqStrides sa, float* cs, const Dims& d, hipStream_t st, int prob = 0) {
   const int64_t total = d.N * d.C;
   const unsigned grid = (unsigned)((total + 3) / 4);
@@ -91,10 +91,10 @@ int launch_chunk_reduce(const void* x, SeqStrides sx, int dtype, const float* cs
   const int64_t vecs = d.T / epl;
   int cg_log2 = 0;
   while ((1 << cg_log2) < vecs && cg_log2 < 6) ++cg_log2;
-  const int cg = 1 << cg_log2;
   // Narrower column tiles (down to 256 bytes of a row) while the workgroups do not fill the chip: at b4 nh2
   // d1024 L4096 chunk 256 bf16, 256 workgroups of 1 KB rows take 16.3 us, 1024 of 256 bytes 13.9.
   while (cg_log2 > 4 && d.N * d.C * ((vecs + (1 << cg_log2) - 1) >> cg_log2) < kFillWorkgroups) --cg_log2;
+  const int cg = 1 << cg_log2;
   const int ntiles = (int)((vecs + cg - 1) / cg);
   const int64_t grid = d.N * d.C * ntiles;
   if (grid > 0x7fffffff) return EMA_ERR_SHAPE;
@@ -167,10 +167,10 @@ int launch_chunk_gemm(const void* in, SeqStrides si, int dtype, const float* cs,
   if (dtype == EMA_BF16)
     return launch_chunk_scan_t<bf16_t, kWalkBnBf16, REVERSE>(in, si, cs, vec, out, so, d, st);
   return launch_chunk_scan_t<float, kWalkBnF32, REVERSE>(in, si, cs, vec, out, so, d, st);
-// Workgroups per chunk: one where the chunks alone fill the chip (four workgroups of eight waves on each of
-// 256 compute units), else as many as fill it, as long as each has rows for a full turn of its waves.
 }
 
+// Workgroups per chunk: one where the chunks alone fill the chip (four workgroups of eight waves on each of
+// 256 compute units), else as many as fill it, as long as each has rows for a full turn of its waves.
 template <int MODE>
 int launch_row_dot(const void* x, SeqStrides sx, int dtype, const float* vec, const float* cs,
                    float* out, int raw, const Dims& d, hipStream_t st) {
@@ -313,6 +313,15 @@ int launch_fwd_tile_t(const void* x, SeqStrides sx, const float* A, SeqStrides s
   if (total > 0x7fffffff) return EMA_ERR_SHAPE;
   if (!ready) EMA_TRY(launch_clear(chain_base, chain_ws_bytes(di), st));
   const ChainWs w = chain_carve(chain_base, di);
+  auto kernel = fwd_tile_kernel<T, S::FWD_CPL, S::FWD_RPL, S::FWD_MINW, XP>;
+  const int64_t cap = resident_blocks(kernel, NT, 0);
+  EMA_TRY(launch_timed(kernel, dim3((unsigned)(total < cap ? total : cap)), dim3(NT), st, ev0, ev1, (const T*)x,
+                       sx, A, sa, (T*)y, sy, prev128, prev_coarse, ratio, fin, init, w.hdr, w.decw, w.status,
+                       (int)di.nh, (int)di.L, (int)di.T, (int)di.C, ntiles, (int)cols, (int)total,
+                       make_order(di, ntiles)));
+  return launched();
+}
+
 // Rows up to which a thread per 16 bytes running down all rows beats the tile kernel, whose tickets, barriers and
 // chained state cost the same whatever the rows.  Short / tile kernel, us: b8 nh2 d1024 bf16, 1 row 5.6 / 12.4,
 // 16 rows 9.3 / 13.6, 32 rows 13.5 / 13.6; b1 nh1 d64 float32, 16 rows 6.7 / 9.3, 32 rows 10.0 / 9.0; b256 nh4
@@ -328,15 +337,6 @@ int launch_fwd_short(const void* x, SeqStrides sx, const float* A, SeqStrides sa
   EMA_TRY(launch_timed(fwd_short_kernel<T, XP>, dim3((unsigned)((total + 255) / 256)), dim3(256), st, ev0, ev1,
                        (const T*)x, sx, A, sa, (T*)y, sy, prev, fin, init, (int)d.nh, (int)d.L, (int)d.T, (int)vecs,
                        (int)total));
-  return launched();
-}
-
-  auto kernel = fwd_tile_kernel<T, S::FWD_CPL, S::FWD_RPL, S::FWD_MINW, XP>;
-  const int64_t cap = resident_blocks(kernel, NT, 0);
-  EMA_TRY(launch_timed(kernel, dim3((unsigned)(total < cap ? total : cap)), dim3(NT), st, ev0, ev1, (const T*)x,
-                       sx, A, sa, (T*)y, sy, prev128, prev_coarse, ratio, fin, init, w.hdr, w.decw, w.status,
-                       (int)di.nh, (int)di.L, (int)di.T, (int)di.C, ntiles, (int)cols, (int)total,
-                       make_order(di, ntiles)));
   return launched();
 }
 
@@ -1031,13 +1031,6 @@ static int seq_fwd_impl(int form, const float* coef, int64_t c_sb, int64_t c_sl,
   EMA_TRY(check_form(form));
   EMA_TRY(check_dims(batch, nheads, seqlen, dim, kTileRows, true, &d));
   EMA_TRY(check_dtype(dtype));
-  if (d.L <= kShortRows && d.N * d.T < (int64_t)1 << 31) {
-    // (the workspace is not used, but a caller that passes it as not ready may pass it as ready from now on)
-    if (!ready) EMA_TRY(launch_clear(w.chain, chain_ws_bytes(d), st));
-    auto run = [&](auto launch) { return launch(x, sx, coef, sc, y, sy, prev128, final_state, init, d, st, ev_start, ev_stop); };
-    if (dtype == EMA_BF16) return xp ? run(launch_fwd_short<bf16_t, true>) : run(launch_fwd_short<bf16_t, false>);
-    return xp ? run(launch_fwd_short<float, true>) : run(launch_fwd_short<float, false>);
-  }
   EMA_TRY(check_seq(x, x_sb, x_sl, x_sh, dtype, dim));
   EMA_TRY(check_seq(y, y_sb, y_sl, y_sh, dtype, dim));
   if (!coef || !prev128) return EMA_ERR_NULL;
@@ -1047,6 +1040,13 @@ static int seq_fwd_impl(int form, const float* coef, int64_t c_sb, int64_t c_sl,
   const SeqWs w = carve_seq(workspace, d, false);
   const SeqStrides sx{x_sb, x_sl, x_sh}, sy{y_sb, y_sl, y_sh}, sc{c_sb, c_sl, c_sh};
   const bool xp = form == EMA_FORM_PROBABILITY, ready = workspace_ready != 0;
+  if (d.L <= kShortRows && d.N * d.T < (int64_t)1 << 31) {
+    // (the workspace is not used, but a caller that passes it as not ready may pass it as ready from now on)
+    if (!ready) EMA_TRY(launch_clear(w.chain, chain_ws_bytes(d), st));
+    auto run = [&](auto launch) { return launch(x, sx, coef, sc, y, sy, prev128, final_state, init, d, st, ev_start, ev_stop); };
+    if (dtype == EMA_BF16) return xp ? run(launch_fwd_short<bf16_t, true>) : run(launch_fwd_short<bf16_t, false>);
+    return xp ? run(launch_fwd_short<float, true>) : run(launch_fwd_short<float, false>);
+  }
   if (dtype == EMA_BF16) {
     if (xp)
       return launch_fwd_tile_t<bf16_t, TileBf16, true>(x, sx, coef, sc, y, sy, prev128, nullptr, 1, final_state,

@@ -377,25 +377,6 @@ __global__ __launch_bounds__(256) void state_passing_bwd_finish_kernel(
 // its running sum) and 14.1 us (dc).
 // ------------------------------------------------------------------------------------
 constexpr int kRowDotThreads = 512;
-template <typename T, int MODE>
-__global__ __launch_bounds__(kRowDotThreads) void row_dot_kernel(const T* __restrict__ x, SeqStrides sx,
-                                                                 const float* __restrict__ vec,
-                                                                 const float* __restrict__ cs,
-                                                                 float* __restrict__ out, int nh, int L,
-                                                                 int Tdim, int Q, int C, int raw, int span) {
-  constexpr int VEC = Vec16<T>::N;
-  constexpr int NWV = kRowDotThreads / 64;
-  __shared__ float rbuf[EMA_MAX_CHUNK_DEV];
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63;
-  const int64_t chunk_id = blockIdx.x;
-  const int64_t n = chunk_id / C;
-  const int c = (int)(chunk_id - n * C);
-  const int64_t b = n / nh;
-  const int h = (int)(n - b * nh);
-  const int limit = min(Q, L - c * Q);
-  const float* csp = cs + chunk_id * Q;
-  const float cs_last = csp[Q - 1];
 constexpr int kRowDotRows = 2;  // rows per wave and turn
 constexpr int kRowDotStep = kRowDotThreads / 64 * kRowDotRows;  // rows per workgroup and turn
 
@@ -417,6 +398,25 @@ __device__ __forceinline__ void row_exclusive_sum(const float* r, float* out, in
   }
 }
 
+template <typename T, int MODE>
+__global__ __launch_bounds__(kRowDotThreads) void row_dot_kernel(const T* __restrict__ x, SeqStrides sx,
+                                                                 const float* __restrict__ vec,
+                                                                 const float* __restrict__ cs,
+                                                                 float* __restrict__ out, int nh, int L,
+                                                                 int Tdim, int Q, int C, int raw, int span) {
+  constexpr int VEC = Vec16<T>::N;
+  constexpr int NWV = kRowDotThreads / 64;
+  __shared__ float rbuf[EMA_MAX_CHUNK_DEV];
+  const int tid = threadIdx.x;
+  const int wave = tid >> 6, lane = tid & 63;
+  const int64_t chunk_id = blockIdx.x;
+  const int64_t n = chunk_id / C;
+  const int c = (int)(chunk_id - n * C);
+  const int64_t b = n / nh;
+  const int h = (int)(n - b * nh);
+  const int limit = min(Q, L - c * Q);
+  const float* csp = cs + chunk_id * Q;
+  const float cs_last = csp[Q - 1];
   const float* vp = vec + chunk_id * Tdim;
   const T* xp = x + b * sx.sb + h * sx.sh + (int64_t)c * Q * sx.sl;
 
@@ -471,6 +471,14 @@ __device__ __forceinline__ void row_exclusive_sum(const float* r, float* out, in
   }
 }
 
+// The running sum of row_dot_kernel<T, 0> where several workgroups share a chunk: one wave per chunk, in place.
+__global__ __launch_bounds__(256) void row_scan_kernel(float* __restrict__ v, int Q, int64_t chunks) {
+  const int64_t chunk = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (chunk >= chunks) return;
+  float* p = v + chunk * Q;
+  row_exclusive_sum(p, p, Q, threadIdx.x & 63);
+}
+
 // ------------------------------------------------------------------------------------
 // Final sum of the log-decay gradient, one wave per (n, c):
 //   ddA[j] = intra[j] + next[j] + sum_{m>=j} (s[m] + [m == Q-1] * ddA_chunk)
@@ -490,14 +498,6 @@ __global__ __launch_bounds__(256) void combine_dA_kernel(const float* __restrict
   const int per = (Q + 63) >> 6;
   const int p0 = lane * per;
   const float* sp = sraw + chunk_id * Q;
-// The running sum of row_dot_kernel<T, 0> where several workgroups share a chunk: one wave per chunk, in place.
-__global__ __launch_bounds__(256) void row_scan_kernel(float* __restrict__ v, int Q, int64_t chunks) {
-  const int64_t chunk = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (chunk >= chunks) return;
-  float* p = v + chunk * Q;
-  row_exclusive_sum(p, p, Q, threadIdx.x & 63);
-}
-
   const float extra = ddA_chunk[chunk_id];
   float local = 0.f;
   for (int i = 0; i < per; ++i) {
@@ -516,7 +516,6 @@ __global__ __launch_bounds__(256) void row_scan_kernel(float* __restrict__ v, in
   }
 }
 
-}  // namespace ema
 // ------------------------------------------------------------------------------------
 // The coefficients of a packed batch with the state dropped where the sequence id changes (MODE 0), and the
 // gradient with respect to the given coefficients from that of the packed ones (MODE 1, may run in place):
@@ -542,3 +541,4 @@ __global__ __launch_bounds__(256) void coef_starts_kernel(const float* src, SeqS
   dst[b * sd.sb + (int64_t)l * sd.sl + h * sd.sh] = v;
 }
 
+}  // namespace ema

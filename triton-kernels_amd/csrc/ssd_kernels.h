@@ -1947,6 +1947,7 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_scan_wide_kernel(
   const TS* pg = prev + (((b * C + c) * nh + h) * (int64_t)P) * N;
   const float* cbg = cb + (((b * C + c) * ngroups + g) * (int64_t)Q) * Q;
 
+  const unsigned xrow = (unsigned)(sx.sl * sizeof(T));
   int mrow[2];
   mrow[0] = 32 * wave;
   mrow[1] = 32 * (7 - wave);
@@ -1977,7 +1978,6 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_scan_wide_kernel(
     }
   }
   {
-  const unsigned xrow = (unsigned)(sx.sl * sizeof(T));
     const ChunkSeq sq = chunk_seq(seq, b, c, Q);
     const bool live = !sq.on() || sq.at(min(m0 + tid, limit - 1)) == sq.entering(c);
 #pragma unroll
@@ -2139,36 +2139,6 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_scan_wide_kernel(
   SSD_TSTAMP(7);
 }
 
-// Partial sums for the gradient of the skip weight D: a lane holds, for its EPL adjacent features
-// cv .. (cv = EPL * (lane % VPR)), the sum of dout * x over the rows it handled; the lanes of a
-// wave that share cv are added up and the wave's hdim sums go to its slot.  The caller adds the
-// slots of all waves, chunks and batch elements.
-template <int EPL, int VPR>
-__device__ __forceinline__ void store_dD_partial(float* __restrict__ slot, float* dsum, int lane) {
-#pragma unroll
-  for (int off = VPR; off < 64; off <<= 1)
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) dsum[e] += __shfl_xor(dsum[e], off);
-  if (lane < VPR) {
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) slot[lane * EPL + e] = dsum[e];
-  }
-}
-
-// ------------------------------------------------------------------------------------
-// Backward of chunk_scan and chunk_state with respect to x (and the explicit dt factors).
-// One workgroup per (b, c, h, tile of 64 rows m):
-//   acc[m][p] = exp(min(dA_last - dA_m, 0)) * sum_n B[m][n] * round_T(dstates[p][n])
-//             + sum_{k >= m, k < limit} round_T(cb[k][m] * exp(min(dA_k - dA_m, 0))) * dout[k][p]
-//   dx[m][p] = acc * dt_m + D * dout[m][p],    ddt[m] = sum_p acc[m][p] * x[m][p]
-// The mirror image of ssd_chunk_scan_kernel: the k tiles run from the diagonal one to the end
-// of the chunk, and the weights are staged transposed (k-major), so that cb is still read along
-// its rows.  In a packed batch the dstates term only reaches the rows whose id equals that of the
-// chunk's last position.
-// ------------------------------------------------------------------------------------
-template <typename T, int P, int N, typename TS>
-__global__ __launch_bounds__(256) void ssd_chunk_scan_bwd_dx_kernel(
-    const float* __restrict__ cb, const T* __restrict__ x, Strides3 sx, const T* __restrict__ dout, Strides3 sd,
 // ------------------------------------------------------------------------------------
 // chunk_scan for chunks of ST = 64 or 128 rows.  One workgroup of four waves per (b, c, head or pair of heads).  PW = HP * hdim columns (two adjacent heads of
 // a group share the rows of C and the fragments of cb, as in ssd_chunk_scan_wide_kernel); wave w owns the
@@ -2413,6 +2383,36 @@ __global__ __launch_bounds__(256, (P * HP * (int)sizeof(T) > 256 ? 2 : 3)) void 
   }
 }
 
+// Partial sums for the gradient of the skip weight D: a lane holds, for its EPL adjacent features
+// cv .. (cv = EPL * (lane % VPR)), the sum of dout * x over the rows it handled; the lanes of a
+// wave that share cv are added up and the wave's hdim sums go to its slot.  The caller adds the
+// slots of all waves, chunks and batch elements.
+template <int EPL, int VPR>
+__device__ __forceinline__ void store_dD_partial(float* __restrict__ slot, float* dsum, int lane) {
+#pragma unroll
+  for (int off = VPR; off < 64; off <<= 1)
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) dsum[e] += __shfl_xor(dsum[e], off);
+  if (lane < VPR) {
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) slot[lane * EPL + e] = dsum[e];
+  }
+}
+
+// ------------------------------------------------------------------------------------
+// Backward of chunk_scan and chunk_state with respect to x (and the explicit dt factors).
+// One workgroup per (b, c, h, tile of 64 rows m):
+//   acc[m][p] = exp(min(dA_last - dA_m, 0)) * sum_n B[m][n] * round_T(dstates[p][n])
+//             + sum_{k >= m, k < limit} round_T(cb[k][m] * exp(min(dA_k - dA_m, 0))) * dout[k][p]
+//   dx[m][p] = acc * dt_m + D * dout[m][p],    ddt[m] = sum_p acc[m][p] * x[m][p]
+// The mirror image of ssd_chunk_scan_kernel: the k tiles run from the diagonal one to the end
+// of the chunk, and the weights are staged transposed (k-major), so that cb is still read along
+// its rows.  In a packed batch the dstates term only reaches the rows whose id equals that of the
+// chunk's last position.
+// ------------------------------------------------------------------------------------
+template <typename T, int P, int N, typename TS>
+__global__ __launch_bounds__(256) void ssd_chunk_scan_bwd_dx_kernel(
+    const float* __restrict__ cb, const T* __restrict__ x, Strides3 sx, const T* __restrict__ dout, Strides3 sd,
     const float* __restrict__ dt, const float* __restrict__ dA_cs, const T* __restrict__ Bm, Strides3 sB,
     const TS* __restrict__ dstates, const float* __restrict__ D, int d_has_hdim, T* __restrict__ dx,
     Strides3 sdx, float* __restrict__ ddt, int nh, int heads_per_group, int ngroups, int L, int Q, int C,
@@ -3071,7 +3071,6 @@ __global__ __launch_bounds__(256) void ssd_chunk_state_varlen_kernel(
     }
 }
 
-}  // namespace ssd
 // ------------------------------------------------------------------------------------
 // The same on the matrix units, for state tiles of 64 x 64 that divide the state and rows that can be read 16
 // bytes at a time.  Wave w owns one 32 x 32 block of the tile; 64 positions per stage, the next stage's rows
@@ -3150,3 +3149,4 @@ __global__ __launch_bounds__(256) void ssd_chunk_state_varlen_mma_kernel(
   }
 }
 
+}  // namespace ssd
