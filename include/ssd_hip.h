@@ -274,6 +274,23 @@ int ssd_chunk_state_varlen(const void* B, int64_t b_sl, int64_t b_sg, const void
                            int states_dtype, const int32_t* cu_seqlens, float* states, int64_t nseq, int64_t seqlen, int64_t nheads,
                            int64_t ngroups, int64_t hdim, int64_t dstate, int64_t chunk, void* stream);
 
+/* The five forward stages one after the other, each as its own entry point above runs it: cumsum; chunk states
+ * and state passing (one walk per head, or, with local_states (batch, C, nheads, hdim, dstate) float32 given, the
+ * two launchers; packed batches need it); bmm; chunk scan; and, with varlen_out given (batch 1), the states at the
+ * sequence ends cu_seqlens names.  x, z, B, C, states and varlen_out are of `dtype`, final_states float32.  One
+ * call from the host instead of five or six.  A refused stage ends the call with its status; the stages before
+ * it have been enqueued by then. */
+int ssd_combined_fwd(const void* x, int64_t x_sb, int64_t x_sl, int64_t x_sh, int dtype, const void* dt, int dt_dtype,
+                     int64_t dt_sb, int64_t dt_sl, int64_t dt_sh, const float* A, const float* dt_bias,
+                     int dt_softplus, float dt_min, float dt_max, const void* B, int64_t b_sb, int64_t b_sl,
+                     int64_t b_sg, const void* C, int64_t c_sb, int64_t c_sl, int64_t c_sg, const float* D,
+                     int d_has_hdim, const void* z, int64_t z_sb, int64_t z_sl, int64_t z_sh, const float* initial,
+                     const int32_t* seq_idx, int64_t seq_sb, int64_t seq_sl, const int32_t* cu_seqlens, int64_t nseq,
+                     float* dt_out, float* dA_cumsum, float* local_states, void* states, float* final_states,
+                     float* cb, void* out, int64_t o_sb, int64_t o_sl, int64_t o_sh, void* out_x, void* varlen_out,
+                     int64_t batch, int64_t seqlen, int64_t nheads, int64_t ngroups, int64_t hdim, int64_t dstate,
+                     int64_t chunk, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

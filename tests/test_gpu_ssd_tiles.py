@@ -1,8 +1,9 @@
-"""The chunk scan in one tile per chunk (chunks of 64 and 128 rows) and the states at the ends of packed
-sequences, at the sizes where they can go wrong."""
+"""The chunk scan in one tile per chunk (chunks of 64 and 128 rows) and the choice between the state walk and
+the two launchers, at the sizes where they can go wrong."""
 import pytest
 import torch
 
+from kernels.mamba_kernels._shapes import walk_pays
 from oracle import ssd_oracle as S
 from parity_util import announce, check_close
 
@@ -42,6 +43,44 @@ def test_chunk_scan_one_tile_vs_oracle(Q, L, nh, g, P, dtype, kind, device):
         check_close("out", got, ref, dtype, regrouped=True)
         if zz is not None:
             check_close("out_x", got_x, ref_x, dtype, regrouped=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nchunks", [1, 4, 5, 8, 9, 17])
+def test_state_passing_turns(nchunks, device):
+    """Chunk counts around one and two turns of the prefetch, plain and packed, both directions."""
+    from kernels.mamba_kernels.mamba_state_pass import _state_passing_fwd
+    from kernels.mamba_kernels_bwd.mamba_state_passing_bwd_dstates import _state_passing_bwd
+
+    announce(f"state passing, {nchunks} chunks")
+    b, nh, dim, Q = 2, 3, 200, 4
+    L = nchunks * Q - 1
+    gen = torch.Generator().manual_seed(nchunks)
+    st, dout = torch.randn(b, nchunks, nh, dim, generator=gen), torch.randn(b, nchunks, nh, dim, generator=gen)
+    da = -torch.rand(b, nh, nchunks, generator=gen)
+    ids = (torch.rand(b, L, generator=gen) < 0.15).to(torch.int32).cumsum(1, dtype=torch.int32)
+    d = lambda t: t.to(device)
+    for seq in (None, ids):
+        kw = {} if seq is None else dict(seq_idx=seq, chunk_size=Q)
+        dkw = {} if seq is None else dict(seq_idx=d(seq), chunk_size=Q)
+        ref, rfin = S.state_passing(st, da, **kw)
+        got, fin = _state_passing_fwd(d(st), d(da), out_dtype=F32, **dkw)
+        check_close("states", got, ref, F32)
+        check_close("final", fin, rfin, F32)
+        rd, rdda, _ = S.state_passing_bwd(ref, da, dout, **kw)
+        gd, gdda, _ = _state_passing_bwd(d(ref), d(da), d(dout), dstates_dtype=F32, **dkw)
+        check_close("dstates", gd, rd, F32)
+        check_close("ddA", gdda, rdda, F32)
+
+
+def test_walk_choice():
+    """Few heads or long chunks: the two launchers; a head per compute unit: the walk."""
+    assert not walk_pays(1, 32, 4096, 256, 64, 128, 2)
+    assert not walk_pays(1, 4, 512, 64, 64, 64, 4)
+    assert walk_pays(8, 32, 8192, 256, 64, 128, 2) and walk_pays(8, 32, 8192, 256, 64, 128, 2, backward=True)
+    assert walk_pays(4, 32, 512, 64, 64, 128, 2)
+    for heads in (8, 64, 128):  # monotone: more heads never turn the walk away
+        assert walk_pays(1, heads, 8192, 256, 64, 128, 2) <= walk_pays(1, 2 * heads, 8192, 256, 64, 128, 2)
 
 
 @pytest.mark.gpu

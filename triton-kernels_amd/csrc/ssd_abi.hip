@@ -885,6 +885,41 @@ int ssd_chunk_state_varlen(const void* B, int64_t b_sl, int64_t b_sg, const void
                        states, SSD_F32, nseq, seqlen, nheads, ngroups, hdim, dstate, chunk, stream);
 }
 
+int ssd_combined_fwd(const void* x, int64_t x_sb, int64_t x_sl, int64_t x_sh, int dtype, const void* dt, int dt_dtype,
+                     int64_t dt_sb, int64_t dt_sl, int64_t dt_sh, const float* A, const float* dt_bias,
+                     int dt_softplus, float dt_min, float dt_max, const void* B, int64_t b_sb, int64_t b_sl,
+                     int64_t b_sg, const void* C, int64_t c_sb, int64_t c_sl, int64_t c_sg, const float* D,
+                     int d_has_hdim, const void* z, int64_t z_sb, int64_t z_sl, int64_t z_sh, const float* initial,
+                     const int32_t* seq_idx, int64_t seq_sb, int64_t seq_sl, const int32_t* cu_seqlens, int64_t nseq,
+                     float* dt_out, float* dA_cumsum, float* local_states, void* states, float* final_states,
+                     float* cb, void* out, int64_t o_sb, int64_t o_sl, int64_t o_sh, void* out_x, void* varlen_out,
+                     int64_t batch, int64_t seqlen, int64_t nheads, int64_t ngroups, int64_t hdim, int64_t dstate,
+                     int64_t chunk, void* stream) {
+  SSD_TRY(ssd_chunk_cumsum_fwd(dt, dt_dtype, dt_sb, dt_sl, dt_sh, A, dt_bias, dA_cumsum, dt_out, batch, seqlen,
+                               nheads, chunk, dt_softplus, dt_min, dt_max, stream));
+  const int64_t C_ = (seqlen + chunk - 1) / chunk;
+  if (local_states) {
+    SSD_TRY(ssd_chunk_state_fwd(B, b_sb, b_sl, b_sg, x, x_sb, x_sl, x_sh, dtype, dt_out, dA_cumsum, local_states,
+                                batch, seqlen, nheads, ngroups, hdim, dstate, chunk, seq_idx, seq_sb, seq_sl, stream));
+    SSD_TRY(ssd_state_passing_fwd(local_states, dA_cumsum + (chunk - 1), nheads * C_ * chunk, C_ * chunk, chunk,
+                                  initial, states, dtype, final_states, batch, C_, nheads, hdim * dstate, seq_idx,
+                                  seq_sb, seq_sl, seqlen, chunk, stream));
+  } else {
+    if (seq_idx) return SSD_ERR_UNSUPPORTED;  // the walk knows no packed batches
+    SSD_TRY(ssd_chunk_state_passing_fwd(B, b_sb, b_sl, b_sg, x, x_sb, x_sl, x_sh, dtype, dt_out, dA_cumsum, initial,
+                                        states, dtype, final_states, batch, seqlen, nheads, ngroups, hdim, dstate,
+                                        chunk, stream));
+  }
+  SSD_TRY(ssd_bmm_chunk_fwd(C, c_sb, c_sl, c_sg, B, b_sb, b_sl, b_sg, dtype, cb, SSD_F32, batch, seqlen, ngroups,
+                            dstate, chunk, seq_idx, seq_sb, seq_sl, stream));
+  SSD_TRY(ssd_chunk_scan_fwd(cb, x, x_sb, x_sl, x_sh, z, z_sb, z_sl, z_sh, dtype, dt_out, dA_cumsum, C, c_sb, c_sl,
+                             c_sg, states, dtype, D, d_has_hdim, out, o_sb, o_sl, o_sh, out_x, batch, seqlen, nheads,
+                             ngroups, hdim, dstate, chunk, seq_idx, seq_sb, seq_sl, stream));
+  if (!varlen_out) return SSD_OK;
+  return varlen_states(B, b_sl, b_sg, x, x_sl, x_sh, dtype, dt_out, dA_cumsum, states, dtype, cu_seqlens, varlen_out,
+                       dtype, nseq, seqlen, nheads, ngroups, hdim, dstate, chunk, stream);
+}
+
 #ifdef SSD_TIMING
 // Development aid, only in builds with -DSSD_TIMING: installs the per-workgroup timestamp buffer.
 int ssd_debug_set_timing(void* buf) {

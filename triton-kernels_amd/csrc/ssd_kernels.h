@@ -602,27 +602,43 @@ __global__ __launch_bounds__(256) void ssd_state_passing_kernel(
   StateVec<E> s;
 #pragma unroll
   for (int i = 0; i < E; ++i) s.v[i] = initial ? initial[(b * nh + h) * (int64_t)dim + e + i] : 0.f;
-  constexpr int U = 4;
-  for (int c0 = 0; c0 < C; c0 += U) {
-    StateVec<E> nv[U];
-    float a[U];
-    // unconditional loads from chunk indices clamped into the tensor
+  constexpr int U = 4;  // chunks per turn; the next turn's are requested before this turn's are used
+  StateVec<E> nv[2][U];
+  float a[2][U];
+  int id[2][U];
+  const int* ids = seq.p ? seq.p + b * seq.sb : nullptr;
+  int id_before = 0;
+  // unconditional loads from chunk indices clamped into the tensor
+  auto request = [&](int c0, StateVec<E>* v, float* w, int* last_id) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int c = min(c0 + u, C - 1);
-      nv[u] = state_load<E>(src + c * chunk_stride);
-      a[u] = __expf(da[(int64_t)c * da_sc]);
-      if (!chunk_keeps_state(seq, b, c, Q, L)) a[u] = 0.f;
+      v[u] = state_load<E>(src + c * chunk_stride);
+      w[u] = da[(int64_t)c * da_sc];
+      if (ids) last_id[u] = ids[(int64_t)(min((c + 1) * Q, L) - 1) * seq.sl];
     }
+  };
+  auto turn = [&](int c0, const StateVec<E>* v, const float* w, const int* last_id) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int c = c0 + u;
       if (c < C) {
         state_store<E>(dst + c * chunk_stride, s);
+        // (the state survives a chunk whose last position has the id of the previous chunk's last, see
+        // chunk_keeps_state)
+        const float keep = !ids || last_id[u] == id_before ? __expf(w[u]) : 0.f;
+        if (ids) id_before = last_id[u];
 #pragma unroll
-        for (int i = 0; i < E; ++i) s.v[i] = fmaf(a[u], s.v[i], nv[u].v[i]);
+        for (int i = 0; i < E; ++i) s.v[i] = fmaf(keep, s.v[i], v[u].v[i]);
       }
     }
+  };
+  request(0, nv[0], a[0], id[0]);
+  for (int c0 = 0; c0 < C; c0 += 2 * U) {
+    request(c0 + U, nv[1], a[1], id[1]);
+    turn(c0, nv[0], a[0], id[0]);
+    request(c0 + 2 * U, nv[0], a[0], id[0]);
+    turn(c0 + U, nv[1], a[1], id[1]);
   }
 #pragma unroll
   for (int i = 0; i < E; ++i) final_states[(b * nh + h) * (int64_t)dim + e + i] = s.v[i];
@@ -1178,19 +1194,25 @@ __global__ __launch_bounds__(256) void ssd_state_passing_bwd_kernel(
   StateVec<E> G;
 #pragma unroll
   for (int i = 0; i < E; ++i) G.v[i] = (dfinal && ok) ? dfinal[(b * nh + h) * (int64_t)dim + e + i] : 0.f;
-  constexpr int U = 4;
-  for (int c1 = C - 1; c1 >= 0; c1 -= U) {
-    StateVec<E> sv[U], dv[U];
-    float a[U];
-    // unconditional loads from chunk indices clamped into the tensor; what lies outside is zeroed
+  constexpr int U = 4;  // chunks per turn; the next turn's are requested before this turn's are used
+  StateVec<E> sv[2][U], dv[2][U];
+  float a[2][U];
+  int id[2][U + 1];  // ids at the ends of the turn's chunks, and of the chunk before them
+  const int* ids = seq.p ? seq.p + b * seq.sb : nullptr;
+  // unconditional loads from chunk indices clamped into the tensor; what lies outside is not used
+  auto request = [&](int c1, StateVec<E>* s, StateVec<E>* d, float* w, int* end_id) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int c = max(c1 - u, 0);
-      sv[u] = state_load<E>(states + base + c * chunk_stride);
-      dv[u] = state_load<E>(dout + base + c * chunk_stride);
-      a[u] = __expf(da[(int64_t)c * da_sc]);
-      if (!chunk_keeps_state(seq, b, c, Q, L)) a[u] = 0.f;
+      s[u] = state_load<E>(states + base + c * chunk_stride);
+      d[u] = state_load<E>(dout + base + c * chunk_stride);
+      w[u] = da[(int64_t)c * da_sc];
     }
+    if (ids)
+#pragma unroll
+      for (int u = 0; u <= U; ++u) end_id[u] = c1 - u >= 0 ? ids[(int64_t)(min((c1 - u + 1) * Q, L) - 1) * seq.sl] : 0;
+  };
+  auto turn = [&](int c1, const StateVec<E>* s, const StateVec<E>* d, const float* w, const int* end_id) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int c = c1 - u;
@@ -1198,13 +1220,21 @@ __global__ __launch_bounds__(256) void ssd_state_passing_bwd_kernel(
         if (ok) state_store<E>(dstates + base + c * chunk_stride, G);
         float dot = 0.f;
 #pragma unroll
-        for (int i = 0; i < E; ++i) dot = fmaf(sv[u].v[i], G.v[i], dot);
+        for (int i = 0; i < E; ++i) dot = fmaf(s[u].v[i], G.v[i], dot);
         dot = ema::wave_sum(ok ? dot : 0.f);
         if (lane == 0) part[((b * nh + h) * C + c) * (int64_t)nw + wave_id] = dot;
+        const float keep = !ids || end_id[u] == end_id[u + 1] ? __expf(w[u]) : 0.f;  // (see chunk_keeps_state)
 #pragma unroll
-        for (int i = 0; i < E; ++i) G.v[i] = fmaf(a[u], G.v[i], dv[u].v[i]);
+        for (int i = 0; i < E; ++i) G.v[i] = fmaf(keep, G.v[i], d[u].v[i]);
       }
     }
+  };
+  request(C - 1, sv[0], dv[0], a[0], id[0]);
+  for (int c1 = C - 1; c1 >= 0; c1 -= 2 * U) {
+    request(c1 - U, sv[1], dv[1], a[1], id[1]);
+    turn(c1, sv[0], dv[0], a[0], id[0]);
+    request(c1 - 2 * U, sv[0], dv[0], a[0], id[0]);
+    turn(c1 - U, sv[1], dv[1], a[1], id[1]);
   }
   if (dinit && ok) {
 #pragma unroll

@@ -107,3 +107,38 @@ class Plan:
             return None
         b, C, nhs = t.shape[:3]
         return t.reshape(b, C, nhs // self.split, self.hd_pad, self.N)[..., : self.hd, : self.ds]
+
+
+def walk_pays(batch, nheads, seqlen, chunk, headdim, dstate, itemsize, backward=False):
+    """Whether the kernel in which one workgroup per (batch, head) walks the whole sequence is faster than
+    the two launchers it stands for, which spread the chunks over the chip and carry the chunk-local
+    float32 states through memory.  Both give the same states bit for bit.
+
+    The walk is a serial chain of 64-row stages whose time does not depend on how many of the 256 compute
+    units work (MI355X, hdim 64, dstate 128, bfloat16: 0.97 us a stage forward, 1.17 backward; other shapes
+    stage their rows through registers), the two launchers are bound by the bytes they move (5 TB/s; in
+    float32 by their matrix instructions as well).  Measured walk / two launchers, us, hdim 64, dstate 128:
+      bfloat16 forward,  chunk 256, seqlen 8192:  32 heads 127 /  31, 128 heads 129 / 101, 160 heads 130 / 123,
+                                                  192 heads 130 / 146, 256 heads 139 / 193
+                         chunk 256, seqlen 2048: 128 heads  35 /  32, 160 heads  37 /  40
+                         chunk  64, seqlen  512:  32 heads  14 /  12,  64 heads  14 /  17
+      bfloat16 backward, chunk 256, seqlen 8192: 160 heads 160 / 139, 192 heads 160 / 165
+      float32 forward,   chunk 256, seqlen 2048:  32 heads 130 /  24, 256 heads 145 / 139."""
+    heads = batch * nheads
+    stages = -(-seqlen // 64)
+    nchunks = -(-seqlen // chunk)
+    state = headdim * dstate
+    rel = state / 8192
+    if itemsize == 4:
+        stage_us = 1.0 + 3.0 * rel
+    elif headdim == 64 and dstate == 128:
+        stage_us = 1.17 if backward else 0.97
+    else:
+        stage_us = 0.5 + 0.85 * rel
+    walk_us = 4.0 + stages * stage_us * -(-heads // 256)
+    # chunk-local states written and read in float32, the carried ones written (and read, backward)
+    nbytes = heads * (nchunks * state * (8 + itemsize * (2 if backward else 1)) + seqlen * headdim * itemsize)
+    pair_us = 6.0 + nbytes / 5e6
+    if itemsize == 4:
+        pair_us += 2 * heads * seqlen * state / 100e6
+    return walk_us < pair_us
