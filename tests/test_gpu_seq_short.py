@@ -92,3 +92,24 @@ def test_row_dots_and_column_sums_split_over_workgroups(N, L, T, Q, dtype, devic
     check_close("db", _ema_chunk_state_bwd_db(d(X), d(o["cs"]), d(o["g"])), O.bwd_db(X.float(), o["cs"], o["g"]), F32)
     check_close("dc", _ema_chunk_scan_bwd_dC(d(o["prev"]), d(o["cs"]), d(dy)),
                 O.bwd_dc(o["prev"], o["cs"], dy.float()), F32)
+
+
+@pytest.mark.parametrize("C", [1, 7, 8, 9, 16, 17, 25])  # the turns of eight chunks of the inter-chunk recurrences
+def test_state_passing_turns(C, device):
+    from kernels.ema_kernels.ema_state_pass import _ema_state_passing_fwd
+    from kernels.ema_kernels_bwd.ema_state_passing_bwd_dstates import _ema_state_passing_bwd
+
+    announce(f"state passing, {C} chunks")
+    gen = torch.Generator().manual_seed(C)
+    N, T = 3, 260
+    st, ds = torch.randn(N, C, T, generator=gen), torch.randn(N, C, T, generator=gen)
+    cs_last = -torch.rand(N, C, generator=gen)
+    d = lambda t: t.to(device)
+    prev, final = O.state_passing(st, cs_last)
+    got_prev, got_final = _ema_state_passing_fwd(d(st), d(cs_last), out_dtype=F32)
+    check_close("prev", got_prev, prev, F32)
+    check_close("final", got_final, final, F32)
+    g, ddA = O.state_passing_bwd(prev, cs_last, ds)
+    got = _ema_state_passing_bwd(d(prev), d(cs_last), d(ds))
+    check_close("g", got[0], g, F32)
+    check_close("ddA_chunk", got[1], ddA, F32)
