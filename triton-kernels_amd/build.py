@@ -1,5 +1,5 @@
 """Builds lib/libema_hip.so (gfx950) from csrc/ with hipcc: the EMA scan (ema_abi.hip) and the
-SSD stages (ssd_abi.hip).  The translation units are compiled side by side and then linked.
+SSD stages (ssd_abi.hip, ssd_scan_abi.hip).  The translation units are compiled side by side and then linked.
 Usage: python build.py"""
 import os
 import subprocess
@@ -7,7 +7,7 @@ import sys
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-SRC = [os.path.join(HERE, "csrc", "ema_abi.hip"), os.path.join(HERE, "csrc", "ssd_abi.hip")]
+SRC = [os.path.join(HERE, "csrc", f) for f in ("ema_abi.hip", "ssd_abi.hip", "ssd_scan_abi.hip")]
 OUT = os.path.join(HERE, "lib", "libema_hip.so")
 OBJ_DIR = os.path.join(HERE, "build")
 

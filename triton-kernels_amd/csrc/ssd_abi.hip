@@ -1,96 +1,16 @@
-// C ABI of the SSD forward stages: argument validation and kernel launches.  Declarations and
-// the reference launcher each entry point replaces are in include/ssd_hip.h.
+// C ABI of the SSD stages other than the chunk scan (ssd_scan_abi.hip): argument validation and kernel launches.
+// Declarations and the reference launcher each entry point replaces are in include/ssd_hip.h.
 #include "../../include/ssd_hip.h"
-
-#include <hip/hip_runtime.h>
 
 #include <type_traits>
 
 #include "ema_gemm_kernels.h"
-#include "launch_facts.h"
+#include "ssd_host.h"
 #include "ssd_kernels.h"
 
 using namespace ssd;
 
 namespace {
-
-#define SSD_TRY(expr)            \
-  do {                           \
-    int _s = (expr);             \
-    if (_s != SSD_OK) return _s; \
-  } while (0)
-
-inline int launched() { return hipGetLastError() == hipSuccess ? SSD_OK : SSD_ERR_LAUNCH; }
-inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
-inline int esize(int dtype) { return dtype == SSD_BF16 ? 2 : 4; }
-inline int check_dtype(int dtype) { return (dtype == SSD_F32 || dtype == SSD_BF16) ? SSD_OK : SSD_ERR_DTYPE; }
-
-// A tensor read or written in 16-byte pieces along its dense last axis of `inner` elements.
-int check_vec(const void* p, int64_t sb, int64_t sl, int64_t sh, int dtype, int64_t inner) {
-  if (!p) return SSD_ERR_NULL;
-  const int epl = 16 / esize(dtype);
-  if (inner % epl || sb % epl || sl % epl || sh % epl) return SSD_ERR_ALIGN;
-  if (reinterpret_cast<uintptr_t>(p) % 16) return SSD_ERR_ALIGN;
-  return SSD_OK;
-}
-int check_f32(const void* p) {
-  if (!p) return SSD_ERR_NULL;
-  return reinterpret_cast<uintptr_t>(p) % 16 ? SSD_ERR_ALIGN : SSD_OK;
-}
-
-// The kernels that copy their operands straight into LDS form 32-bit unsigned byte offsets from
-// the strides: tensors addressed with a negative stride go to the register-staged kernels.
-inline bool forward_strides(const Strides3& s) { return s.sb >= 0 && s.sl >= 0 && s.sh >= 0; }
-
-// A carried-state tensor is float32 or of the inputs' type (16-byte aligned either way).
-int check_state(const void* p, int state_dtype, int dtype) {
-  if (state_dtype != SSD_F32 && state_dtype != dtype) return SSD_ERR_DTYPE;
-  return check_f32(p);
-}
-
-struct Dims {
-  int64_t batch, L, nh, g, P, N, Q, C;
-};
-int check_dims(int64_t batch, int64_t L, int64_t nh, int64_t g, int64_t P, int64_t N, int64_t Q, Dims* d) {
-  if (batch <= 0 || L <= 0 || nh <= 0 || g <= 0 || Q <= 0) return SSD_ERR_SHAPE;
-  if (nh % g) return SSD_ERR_SHAPE;
-  if (Q > 1024 || Q % 4) return SSD_ERR_UNSUPPORTED;
-  if (batch > (1 << 20) || nh > (1 << 16) || L > ((int64_t)1 << 30)) return SSD_ERR_SHAPE;
-  *d = Dims{batch, L, nh, g, P, N, Q, (L + Q - 1) / Q};
-  if (batch * nh * d->C > ((int64_t)1 << 28)) return SSD_ERR_SHAPE;
-  return SSD_OK;
-}
-inline bool dim_ok(int64_t v) { return v == 64 || v == 128; }
-// The state-passing entries take the chunking only to locate the last position of each chunk of
-// a packed batch; without seq_idx both numbers are ignored.
-inline int check_seq_chunks(const int32_t* seq_idx, int64_t seqlen, int64_t chunk, int64_t nchunks) {
-  if (!seq_idx) return SSD_OK;
-  if (seqlen <= 0 || chunk <= 0 || seqlen > ((int64_t)1 << 30)) return SSD_ERR_SHAPE;
-  return (seqlen + chunk - 1) / chunk == nchunks ? SSD_OK : SSD_ERR_SHAPE;
-}
-inline SeqIdx as_seq(const int32_t* p, int64_t sb, int64_t sl) { return SeqIdx{p, sb, sl}; }
-constexpr int kLdsBytes = 160 * 1024;  // LDS of one CU
-
-template <typename K>
-int allow_smem(K kernel, int bytes) {
-  if (bytes <= 64 * 1024) return SSD_OK;
-  return launch_facts::smem(reinterpret_cast<const void*>(kernel), bytes) ? SSD_OK : SSD_ERR_LAUNCH;
-}
-
-// Calls f.template run<T, P, N>() for the runtime (dtype, hdim, dstate).
-template <typename F>
-int dispatch_tpn(int dtype, int64_t P, int64_t N, F f) {
-  if (dtype == SSD_BF16) {
-    if (P == 64 && N == 64) return f.template run<bf16_t, 64, 64>();
-    if (P == 64 && N == 128) return f.template run<bf16_t, 64, 128>();
-    if (P == 128 && N == 64) return f.template run<bf16_t, 128, 64>();
-    return f.template run<bf16_t, 128, 128>();
-  }
-  if (P == 64 && N == 64) return f.template run<float, 64, 64>();
-  if (P == 64 && N == 128) return f.template run<float, 64, 128>();
-  if (P == 128 && N == 64) return f.template run<float, 128, 64>();
-  return f.template run<float, 128, 128>();
-}
 
 template <int MODE>
 struct StateLaunch {
@@ -161,99 +81,6 @@ struct WalkLaunch {
     hipLaunchKernelGGL(kernel, dim3((unsigned)(d.batch * d.nh * NSPLIT)), dim3(256), smem, st, (const T*)x, sx,
                        (const T*)B, sB, dt, dA, initial, (TO*)out, final_states, (int)d.nh, (int)(d.nh / d.g),
                        (int)d.L, (int)d.Q, (int)d.C);
-    return launched();
-  }
-};
-
-struct ScanLaunch {
-  const float* cb;
-  const void *x, *z, *C;
-  Strides3 sx, sz, sC, so;
-  const float *dt, *dA;
-  const void* prev;
-  int prev_dtype;
-  const float* D;
-  int d_has_hdim;
-  void *out, *out_x;
-  Dims d;
-  SeqIdx seq;
-  hipStream_t st;
-  template <typename T, int P, int N>
-  int run() const {
-    if constexpr (!std::is_same<T, float>::value)
-      if (prev_dtype != SSD_F32) return run_as<T, P, N, T>();
-    return run_as<T, P, N, float>();
-  }
-  template <typename T, int P, int N, typename TS, int HP>
-  int launch_wide() const {
-    auto kernel = ssd_chunk_scan_wide_kernel<T, P, N, TS, HP>;
-    constexpr int smem = WideSmem<T, P * HP, N>::bytes_for(HP);
-    SSD_TRY(allow_smem(kernel, smem));
-    const int stiles = (int)(d.Q / 256);
-    hipLaunchKernelGGL(kernel, dim3((unsigned)(d.batch * d.C * (d.nh / HP) * stiles)), dim3(256), smem, st, cb,
-                       (const T*)x, sx, (const T*)z, sz, dt, dA, (const T*)C, sC, (const TS*)prev, D, d_has_hdim,
-                       (T*)out, so, (T*)out_x, (int)d.nh, (int)(d.nh / d.g), (int)d.g, (int)d.L, (int)d.Q, (int)d.C,
-                       stiles, seq);
-    return launched();
-  }
-  template <typename T, int P, int N, typename TS, int HP, int ST>
-  int launch_mid() const {
-    auto kernel = ssd_chunk_scan_mid_kernel<T, P, N, TS, HP, ST>;
-    constexpr int smem = MidSmem<T, P * HP, N, ST>::bytes_for(HP);
-    static_assert(smem <= kLdsBytes, "the tile must fit the LDS of a compute unit");
-    SSD_TRY(allow_smem(kernel, smem));
-    hipLaunchKernelGGL(kernel, dim3((unsigned)(d.batch * d.C * (d.nh / HP))), dim3(256), smem, st, cb,
-                       (const T*)x, sx, (const T*)z, sz, dt, dA, (const T*)C, sC, (const TS*)prev, D, d_has_hdim,
-                       (T*)out, so, (T*)out_x, (int)d.nh, (int)(d.nh / d.g), (int)d.g, (int)d.L, (int)d.C, seq);
-    return launched();
-  }
-  // Whether a chunk's rows sit at 32-bit byte offsets from its first one.
-  bool near(const Strides3& s) const { return forward_strides(s) && d.Q * s.sl < (int64_t(1) << 28); }
-  // Chunks of 64 or 128 rows in one tile.  Two adjacent heads of a group per workgroup where they are adjacent
-  // in memory too (dense heads of 64 features): they share the fragments of cb and the rows of C.  A single
-  // bfloat16 head of 64 features leaves each wave one column block for the weights it forms, and the 64-row
-  // kernel is the faster one (17 heads, L 4096, b2, chunk 128: 29.0 against 32.4 us).  Against the 64-row
-  // kernel otherwise, us at dstate 128: bfloat16 b8 nh32 L8192 hdim 64 chunk 128 437 -> 260, chunk 64
-  // 334 -> 240; b2 nh16 L4096 hdim 128 chunk 128 42 -> 38; float32 b1 nh16 L4096 chunk 128 hdim 64 35 -> 25,
-  // hdim 128 70 -> 40.
-  template <typename T, int P, int N, typename TS, int ST>
-  int launch_mid_pairs(bool* taken) const {
-    *taken = true;
-    if constexpr (P == 64 && sizeof(T) == 2) {
-      const bool dense = sx.sh == P && so.sh == P && (!z || sz.sh == P);
-      if (dense && (d.nh / d.g) % 2 == 0) return launch_mid<T, P, N, TS, 2, ST>();
-      *taken = false;
-      return SSD_OK;
-    } else {
-      return launch_mid<T, P, N, TS, 1, ST>();
-    }
-  }
-  template <typename T, int P, int N, typename TS>
-  int run_as() const {
-    constexpr int wide_smem = WideSmem<T, P, N>::kBytes;
-    const bool close = near(sx) && near(sC) && near(so) && (!z || near(sz));
-    if (d.Q % 256 == 0 && wide_smem <= kLdsBytes && close) {  // 256-row super-tiles, no barrier inside the k loop
-      // Two adjacent heads of a group per workgroup where they are adjacent in memory too (dense
-      // heads of 64 features): they share the fragments of cb and the rows of C.
-      if constexpr (P == 64 && WideSmem<T, 128, N>::bytes_for(2) <= kLdsBytes / 2) {
-        const bool dense = sx.sh == P && so.sh == P && (!z || sz.sh == P);
-        if (dense && (d.nh / d.g) % 2 == 0) return launch_wide<T, P, N, TS, 2>();
-      }
-      return launch_wide<T, P, N, TS, 1>();
-    }
-    if ((d.Q == 64 || d.Q == 128) && close) {
-      bool taken;
-      const int status = d.Q == 128 ? launch_mid_pairs<T, P, N, TS, 128>(&taken) : launch_mid_pairs<T, P, N, TS, 64>(&taken);
-      if (taken) return status;
-    }
-    auto kernel = ssd_chunk_scan_kernel<T, P, N, TS>;
-    constexpr int smem = ScanSmem<T, P, N>::kBytes;
-    SSD_TRY(allow_smem(kernel, smem));
-    const int mtiles = (int)((d.Q + 63) / 64);
-    hipLaunchKernelGGL(kernel, dim3((unsigned)(d.batch * d.C * d.nh * mtiles)), dim3(256), smem, st, cb,
-                       (const T*)x, sx, (const T*)z, sz, dt, dA, (const T*)C, sC, (const TS*)prev, D, d_has_hdim,
-                       (T*)out, so, (T*)out_x, (int)d.nh, (int)(d.nh / d.g), (int)d.g, (int)d.L, (int)d.Q, (int)d.C, mtiles,
-                       seq);
     return launched();
   }
 };
@@ -513,34 +340,6 @@ int ssd_bmm_chunk_fwd(const void* a, int64_t a_sb, int64_t a_sl, int64_t a_sg, c
   }
   return k == 64 ? launch_bmm<float, float, 64>(a, sa, bm, sb, out, d, seq, st)
                  : launch_bmm<float, float, 128>(a, sa, bm, sb, out, d, seq, st);
-}
-
-int ssd_chunk_scan_fwd(const float* cb, const void* x, int64_t x_sb, int64_t x_sl, int64_t x_sh,
-                       const void* z, int64_t z_sb, int64_t z_sl, int64_t z_sh, int dtype,
-                       const float* dt, const float* dA_cumsum, const void* C, int64_t c_sb, int64_t c_sl,
-                       int64_t c_sg, const void* prev_states, int states_dtype, const float* D, int d_has_hdim,
-                       void* out, int64_t o_sb, int64_t o_sl, int64_t o_sh, void* out_x, int64_t batch,
-                       int64_t seqlen, int64_t nheads, int64_t ngroups, int64_t hdim, int64_t dstate,
-                       int64_t chunk, const int32_t* seq_idx, int64_t seq_sb, int64_t seq_sl, void* stream) {
-  Dims d;
-  SSD_TRY(check_dims(batch, seqlen, nheads, ngroups, hdim, dstate, chunk, &d));
-  SSD_TRY(check_dtype(dtype));
-  if (!dim_ok(hdim) || !dim_ok(dstate)) return SSD_ERR_UNSUPPORTED;
-  SSD_TRY(check_vec(x, x_sb, x_sl, x_sh, dtype, hdim));
-  SSD_TRY(check_vec(out, o_sb, o_sl, o_sh, dtype, hdim));
-  SSD_TRY(check_vec(C, c_sb, c_sl, c_sg, dtype, dstate));
-  if (z) SSD_TRY(check_vec(z, z_sb, z_sl, z_sh, dtype, hdim));
-  if (out_x && reinterpret_cast<uintptr_t>(out_x) % 16) return SSD_ERR_ALIGN;
-  if (!dt || !dA_cumsum) return SSD_ERR_NULL;
-  SSD_TRY(check_f32(cb));
-  SSD_TRY(check_state(prev_states, states_dtype, dtype));
-  if (batch * d.C * nheads * ((chunk + 63) / 64) > 0x7fffffff) return SSD_ERR_SHAPE;
-  return dispatch_tpn(dtype, hdim, dstate,
-                      ScanLaunch{cb, x, z, C, Strides3{x_sb, x_sl, x_sh}, Strides3{z_sb, z_sl, z_sh},
-                                 Strides3{c_sb, c_sl, c_sg}, Strides3{o_sb, o_sl, o_sh}, dt, dA_cumsum,
-                                 prev_states, states_dtype, D, d_has_hdim, out, out_x, d,
-                                 as_seq(seq_idx, seq_sb, seq_sl),
-                                 as_stream(stream)});
 }
 
 int ssd_chunk_scan_bwd_dstates(const void* C, int64_t c_sb, int64_t c_sl, int64_t c_sg, const void* dout,

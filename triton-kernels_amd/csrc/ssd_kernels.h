@@ -1242,7 +1242,7 @@ __global__ __launch_bounds__(256) void ssd_state_passing_bwd_kernel(
   }
 }
 
-__global__ __launch_bounds__(256) void ssd_state_passing_bwd_finish_kernel(
+static __global__ __launch_bounds__(256) void ssd_state_passing_bwd_finish_kernel(
     const float* __restrict__ part, const float* __restrict__ dA_chunk, int64_t da_sb, int64_t da_sh,
     int64_t da_sc, float* __restrict__ ddA, int nh, int C, int nw, int has_init, int64_t total, SeqIdx seq,
     int L, int Q) {
@@ -1260,7 +1260,7 @@ __global__ __launch_bounds__(256) void ssd_state_passing_bwd_finish_kernel(
 
 // In-place inclusive cumsum along the last axis of a dense (rows, Q) float32 array; one wave
 // per row, lane l owns ceil(Q/64) consecutive positions.
-__global__ __launch_bounds__(256) void ssd_row_cumsum_kernel(float* __restrict__ v, int Q, int64_t rows) {
+static __global__ __launch_bounds__(256) void ssd_row_cumsum_kernel(float* __restrict__ v, int Q, int64_t rows) {
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= rows) return;
@@ -2170,12 +2170,12 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_scan_wide_kernel(
 }
 
 // ------------------------------------------------------------------------------------
-// chunk_scan for chunks of ST = 64 or 128 rows.  One workgroup of four waves per (b, c, head or pair of heads).  PW = HP * hdim columns (two adjacent heads of
-// a group share the rows of C and the fragments of cb, as in ssd_chunk_scan_wide_kernel); wave w owns the
-// columns of half w & 1 (one head of a pair) and the 32-row blocks w >> 1 and ST/32 - 1 - (w >> 1) of the tile
-// (one block where the tile has two), which balances the causal sum.  What a lane needs of C and of cb comes
-// straight from global memory, cb one group of 32 positions ahead; LDS holds what the waves share: the
-// carried state, then the chunk's rows of x (requested before the state's product).
+// chunk_scan for chunks of ST = 64 or 128 rows.  One workgroup of four waves per (b, c, head or pair of heads).
+// PW = HP * hdim columns (two adjacent heads of a group share the rows of C and the fragments of cb, as in
+// ssd_chunk_scan_wide_kernel); wave w owns the columns of half w & 1 (one head of a pair) and the 32-row blocks
+// w >> 1 and ST/32 - 1 - (w >> 1) of the tile (one block where the tile has two), which balances the causal sum.
+// What a lane needs of C and of cb comes straight from global memory, cb one group of 32 positions ahead; LDS
+// holds what the waves share: the carried state, then the chunk's rows of x (requested before the state's product).
 //
 // The weight of (m, k) below the diagonal group is split at the last position r of k's group of 32 as in the
 // 256-row kernel, which equals the clamped exponential of the definition where dA does not rise; the
@@ -2184,8 +2184,8 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_scan_wide_kernel(
 //
 // Latency bound: a tile is a short chain of dependent loads, so what counts is how many of them a compute unit
 // has under way.  A wave holds half the accumulators of the 256-row kernel, so three workgroups fit instead
-// of two.  b8 nh32 L8192 hdim 64 dstate 128 bf16: chunk 128 437 us by the 64-row kernel, 260
-// here (3.2 TB/s); chunk 64 334 and 240 us.
+// of two.  us by the 64-row kernel and here, b8 nh32 L8192 hdim 64 dstate 128 bf16: chunk 128 437 -> 260 (3.2
+// TB/s), chunk 64 334 -> 240 (4.6 TB/s).
 // ------------------------------------------------------------------------------------
 template <typename T, int PW, int N, int ST>
 struct MidSmem {
