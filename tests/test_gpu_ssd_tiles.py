@@ -21,7 +21,9 @@ def test_chunk_scan_one_tile_vs_oracle(Q, L, nh, g, P, dtype, kind, device):
     from kernels.mamba_kernels.mamba_scan_fwd import _chunk_scan_fwd
 
     announce(f"chunk scan Q={Q} L={L} nh={nh} g={g} P={P} {dtype} {kind}")
-    N, b = 64 if P == 128 else 128, 2
+    N = 64 if P == 128 else 128
+    # in bfloat16 the kernel takes over at 384 workgroups (pairs of heads of 64 features, single heads of 128)
+    b = 2 if dtype == F32 else -(-384 // (-(-L // Q) * (nh // 2 if P == 64 else nh)))
     gen = torch.Generator().manual_seed(Q + L + nh)
     r = lambda *s: torch.randn(*s, generator=gen)
     x, C, z = r(b, L, nh, P).to(dtype), r(b, L, g, N).to(dtype), r(b, L, nh, P).to(dtype)
@@ -102,3 +104,41 @@ def test_varlen_states_at_stage_edges(P, N, dtype, device):
     ref = S.chunk_state_varlen(B, x, dt[0], dA[0], cu, prev, dtype)
     got = chunk_state_varlen(*(t.to(device) for t in (B, x, dt[0], dA[0], cu, prev)))
     check_close("varlen states", got, ref, dtype, regrouped=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["decay", "rise", "mixed"])
+@pytest.mark.parametrize("nh,g,N", [(4, 1, 128), (6, 3, 64)])
+@pytest.mark.parametrize("Q,L", [(128, 257), (128, 128), (128, 33), (64, 190), (64, 64), (64, 1)])
+def test_dx_one_tile_vs_oracle(Q, L, nh, g, N, kind, device):
+    """Pairs of bfloat16 heads: dx, ddt and dD (all its slots) at the same edges, the ddt of rows past the end zero."""
+    from kernels.mamba_kernels_bwd.mamba_chunk_scan_chunk_state_bwd_dx import _chunk_scan_chunk_state_bwd_dx
+
+    announce(f"dx Q={Q} L={L} nh={nh} g={g} N={N} {kind}")
+    P, dtype = 64, BF16
+    b = -(-384 // (-(-L // Q) * (nh // 2)))  # the kernel takes over at 384 pairs of heads
+    gen = torch.Generator().manual_seed(Q + L + nh)
+    r = lambda *s: torch.randn(*s, generator=gen)
+    x, dout, B = r(b, L, nh, P).to(dtype), r(b, L, nh, P).to(dtype), r(b, L, g, N).to(dtype)
+    dt = torch.rand(b, L, nh, generator=gen) * 0.5
+    A = -torch.rand(nh, generator=gen) - 0.1
+    if kind == "rise":
+        A = -A
+    elif kind == "mixed":
+        dt = dt - 0.25
+    dA, dto = S.chunk_cumsum(dt, A, Q)
+    nc = -(-L // Q)
+    cb = r(b, nc, g, Q, Q) * 0.3
+    if L % Q:  # what lies past the sequence must not be looked at
+        cb[:, -1, :, L % Q:, :] = float("nan")
+    ref_cb = torch.nan_to_num(cb)
+    ds = r(b, nc, nh, P, N).to(dtype)
+    d = lambda t: t.to(device)
+    for D in (None, r(nh), r(nh, P)):
+        ref = S.chunk_scan_chunk_state_bwd_dx(x, dto, dA, B, ref_cb, dout, ds, D=D, round_to=dtype)
+        got = _chunk_scan_chunk_state_bwd_dx(d(x), d(dto), d(dA), d(B), d(cb), d(dout), d(ds),
+                                             D=None if D is None else d(D))
+        check_close("dx", got[0], ref[0], dtype, regrouped=True)
+        check_close("ddt", got[1], ref[1], dtype, loose=True)
+        if D is not None:
+            check_close("dD", got[2], ref[2], F32)

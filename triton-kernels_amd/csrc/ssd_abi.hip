@@ -111,6 +111,16 @@ struct DxLaunch {
       if (states_dtype != SSD_F32) return run_as<T, P, N, T>();
     return run_as<T, P, N, float>();
   }
+  template <typename T, int P, int N, typename TS, int ST>
+  int launch_mid() const {
+    auto kernel = ssd_chunk_scan_bwd_dx_mid_kernel<T, P, N, TS, ST>;
+    constexpr int smem = MidSmem<T, 2 * P, N, ST>::bytes_for(2);
+    SSD_TRY(allow_smem(kernel, smem));
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(d.batch * d.C * (d.nh / 2))), dim3(256), smem, st, cb, (const T*)x, sx,
+                       (const T*)dout, sd, dt, dA, (const T*)B, sB, (const TS*)dstates, D, d_has_hdim, (T*)dx, sdx, ddt,
+                       (int)d.nh, (int)(d.nh / d.g), (int)d.g, (int)d.L, (int)d.C, seq, dD_part, 4 * (ST / 64));
+    return launched();
+  }
   template <typename T, int P, int N, typename TS>
   int run_as() const {
     constexpr int wide_smem = WideSmem<T, P, N>::kBytes;
@@ -123,6 +133,18 @@ struct DxLaunch {
                          d_has_hdim, (T*)dx, sdx, ddt, (int)d.nh, (int)(d.nh / d.g), (int)d.g, (int)d.L, (int)d.Q,
                          (int)d.C, stiles, seq, dD_part);
       return launched();
+    }
+    if constexpr (P == 64 && sizeof(T) == 2) {
+      // Chunks of 64 or 128 rows with two adjacent dense heads of a group per workgroup, rows at 32-bit byte offsets,
+      // and enough of them.  The 64-row kernel / this one, us, dstate 128: b8 nh32 L8192 chunk
+      // 128 443 / 279, chunk 64 352 / 274; b1 nh24 L5000 chunk 128 (480 pairs) 26 / 20; b1 nh8 L2000 chunk 64
+      // dstate 64 (128 pairs) 6.6 / 7.7.
+      auto near = [&](const Strides3& s) { return forward_strides(s) && s.sl * d.Q < (int64_t(1) << 28); };
+      const bool dense = sx.sh == P && sd.sh == P && sdx.sh == P && (d.nh / d.g) % 2 == 0;
+      if (dense && near(sx) && near(sd) && near(sB) && near(sdx) && d.batch * d.C * (d.nh / 2) >= kMidWorkgroups) {
+        if (d.Q == 128) return launch_mid<T, P, N, TS, 128>();
+        if (d.Q == 64) return launch_mid<T, P, N, TS, 64>();
+      }
     }
     auto kernel = ssd_chunk_scan_bwd_dx_kernel<T, P, N, TS>;
     constexpr int smem = ScanSmem<T, P, N>::kBytes;

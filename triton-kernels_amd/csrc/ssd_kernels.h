@@ -2606,6 +2606,227 @@ __global__ __launch_bounds__(256) void ssd_chunk_scan_bwd_dx_kernel(
 }
 
 // ------------------------------------------------------------------------------------
+// dx / ddt for chunks of ST = 64 or 128 rows and two adjacent heads of a group per workgroup: the mirror image
+// of ssd_chunk_scan_mid_kernel.  Wave w owns head w & 1 of the pair (all its columns, so a row of ddt is summed
+// inside the wave) and the 32-row blocks w >> 1 and ST/32 - 1 - (w >> 1); the groups of 32 positions k run from
+// the block's own to the chunk's last.  The weight of (m, k) past the diagonal group is split at the first position
+// of k's group as in the 256-row kernel; groups that reach past the sequence, and all groups where dA rises in the
+// chunk, take the exact, masked form.  cb is read along its columns, one 4-byte load per k that is contiguous
+// across the lanes, a group ahead.  Latency bound like its forward twin; us by the 64-row kernel and here, b8 nh32
+// L8192 dstate 128 bf16: chunk 128 443 -> 279, chunk 64 352 -> 274.
+// ------------------------------------------------------------------------------------
+template <typename T, int P, int N, typename TS, int ST>
+__global__ __launch_bounds__(256, 3) void ssd_chunk_scan_bwd_dx_mid_kernel(
+    const float* __restrict__ cb, const T* __restrict__ x, Strides3 sx, const T* __restrict__ dout, Strides3 sd,
+    const float* __restrict__ dt, const float* __restrict__ dA_cs, const T* __restrict__ Bm, Strides3 sB,
+    const TS* __restrict__ dstates, const float* __restrict__ D, int d_has_hdim, T* __restrict__ dx,
+    Strides3 sdx, float* __restrict__ ddt, int nh, int heads_per_group, int ngroups, int L, int C, SeqIdx seq,
+    float* __restrict__ dD_part, int slots) {
+  constexpr int HP = 2, PW = P * HP, Q = ST;
+  using S = MidSmem<T, PW, N, ST>;
+  constexpr int EPL = Vec16<T>::N, KG = Tile<T>::KG, PB = P / 32, NB = ST / 32, MB = NB / 2, NK = N / KG;
+  constexpr int GS = 32 / KG;  // steps of a group of 32 positions
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  T* Ds = reinterpret_cast<T*>(smem);
+  T* Pv = reinterpret_cast<T*>(smem);
+  float* Os = reinterpret_cast<float*>(smem);
+  float* vec = reinterpret_cast<float*>(smem + S::kMain);  // per head: dA_k, dt_k, factor of k, decay to the end
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, half = lane >> 5;
+  const int bid = xcd_local_index((int)blockIdx.x, (int)gridDim.x);
+  const int nhp = nh / HP;
+  const int h0 = (bid % nhp) * HP;  // first head of the workgroup
+  const int c = (bid / nhp) % C;
+  const int64_t b = bid / ((int64_t)nhp * C);
+  const int limit = min(Q, L - c * Q);
+  const int g = h0 / heads_per_group;
+  const int hw = wave & 1, wj = wave >> 1, h = h0 + hw;  // the wave's head and its share of the rows
+  const T* dg = dout + b * sd.sb + (int64_t)c * Q * sd.sl + h0 * sd.sh;
+  const T* Bg = Bm + b * sB.sb + (int64_t)c * Q * sB.sl + g * sB.sh;
+  const TS* sg = dstates + (((b * C + c) * nh + h0) * (int64_t)P) * N;
+  const float* cbg = cb + (((b * C + c) * ngroups + g) * (int64_t)Q) * Q;
+  const int64_t row0 = ((b * nh + h0) * C + c) * (int64_t)Q;  // dA, dt of head h0; the next head C * Q further
+  const unsigned drow = (unsigned)(sd.sl * sizeof(T));
+
+  int mrow[MB];
+  mrow[0] = 32 * wj;
+  if constexpr (MB == 2) mrow[1] = 32 * (NB - 1 - wj);
+  floatx16 acc[MB][PB];
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int pb = 0; pb < PB; ++pb) zero_acc(acc[mb][pb]);
+
+  // ---- everything the first two phases need is requested up front
+  RowPieces<T, ST, PW, S::PX> dtile;
+  dtile.template load32<false>(dg, drow, 0, limit, tid);  // (the epilogue reads these rows again)
+  const unsigned Brow = (unsigned)(sB.sl * sizeof(T));
+  auto b_frag = [&](int mb, int i) {
+    return load16_at(Bg + KG * i, (unsigned)min(mrow[mb] + l32, limit - 1) * Brow + 16u * half);
+  };
+  constexpr int CA = NK < 4 ? NK : 4;  // fragments of B under way
+  Vec16<T> bf[CA];
+#pragma unroll
+  for (int i = 0; i < CA; ++i) bf[i] = b_frag(0, i);
+  stage_state<T, TS, PW, N, S::PC>(Pv, sg, tid);
+  bool rises = false;
+  if (tid < HP * ST) {
+    const int hh = tid / ST, i = tid % ST;
+    const ChunkSeq sq = chunk_seq(seq, b, c, Q);
+    const bool live = !sq.on() || sq.at(min(i, limit - 1)) == sq.at(limit - 1);
+    const float* dAp = dA_cs + row0 + (int64_t)hh * C * Q;
+    const float ak = dAp[i], ar = dAp[i & ~31];
+    float* d = vec + (4 * hh) * ST + i;
+    d[0] = ak, d[ST] = dt[row0 + (int64_t)hh * C * Q + i], d[2 * ST] = __expf(fminf(ak - ar, 0.f));
+    d[3 * ST] = live ? __expf(fminf(dAp[Q - 1] - ak, 0.f)) : 0.f;
+    rises = i + 1 < ST && !(dAp[i + 1] <= ak);  // (a NaN counts as a rise)
+  }
+  rises = __syncthreads_or(rises);
+
+  // ---- phase A: B . dstates, scaled by the decay to the end of the chunk.  (Rows past the sequence hold a copy of
+  // the last row's B: no row of the product reaches another, and theirs are not stored.)
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) {
+#pragma unroll
+    for (int i = 0; i < NK; ++i) {
+      const Vec16<T> a = bf[i % CA];
+      const int nx = mb * NK + i + CA;
+      if (nx < MB * NK) bf[i % CA] = b_frag(nx / NK, nx % NK);
+#pragma unroll
+      for (int pb = 0; pb < PB; ++pb) mma_group(a, frag_rows(Pv, S::PC, P * hw + 32 * pb, KG * i, lane), acc[mb][pb]);
+    }
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const float sc = vec[(4 * hw + 3) * ST + mrow[mb] + acc_row(v, lane)];
+#pragma unroll
+      for (int pb = 0; pb < PB; ++pb) acc[mb][pb][v] *= sc;
+    }
+  }
+
+  // ---- phase B: the causal sum over k >= m
+  const float* dAk = vec + (4 * hw) * ST;
+  const float* dtk = dAk + ST;
+  const float* fk = dAk + 2 * ST;
+  float wn[GS][EPL];  // the cb pieces of the next group
+  auto request = [&](int kg, int mb) {
+    const unsigned at = 4u * (unsigned)(EPL * half * Q + mrow[mb] + l32);  // cb[kg + EPL * half][m]
+#pragma unroll
+    for (int u = 0; u < GS; ++u)
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) wn[u][e] = *at_bytes(cbg + (kg + KG * u + e) * Q, at);
+  };
+  request(mrow[0], 0);
+  __syncthreads();  // the dout tile takes the place of dstates
+  dtile.store(Ds, 0, limit, tid, NoScale());
+  __syncthreads();
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) {
+    const int mloc = mrow[mb] + l32;
+    const float am = dAk[mloc];
+    for (int kg = mrow[mb]; kg < ST; kg += 32) {
+      float w[GS][EPL];
+#pragma unroll
+      for (int u = 0; u < GS; ++u)
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) w[u][e] = wn[u][e];
+      if (kg + 32 < ST) request(kg + 32, mb);
+      else if (mb + 1 < MB) request(mrow[MB - 1], MB - 1);
+      const bool exact = rises || kg == mrow[mb] || kg + 32 > limit;
+      const float gm = __expf(fminf(dAk[kg] - am, 0.f));
+#pragma unroll
+      for (int u = 0; u < GS; ++u) {
+        const int kb = kg + KG * u + EPL * half;
+        Vec16<T> a;
+        float wf[EPL];
+        if (exact) {
+#pragma unroll
+          for (int e = 0; e < EPL; ++e) {
+            const float f = w[u][e] * __expf(fminf(dAk[kb + e] - am, 0.f));
+            wf[e] = (kb + e < mloc || kb + e >= limit) ? 0.f : f;
+          }
+        } else {
+#pragma unroll
+          for (int e = 0; e < EPL; ++e) wf[e] = w[u][e] * fk[kb + e] * gm;
+        }
+        a.set_all(wf);
+#pragma unroll
+        for (int pb = 0; pb < PB; ++pb)
+          mma_group(a, frag_cols(Ds, S::PX, kg + KG * u, P * hw + 32 * pb, lane), acc[mb][pb]);
+      }
+    }
+  }
+  __syncthreads();
+
+  // ---- phase C: each wave moves its blocks through its own staging area; dx = acc * dt + D * dout, ddt = <acc, x>
+  // per row.  The rows of x and dout are requested before the accumulators go to LDS.
+  float* mine = Os + wave * 32 * S::PO;
+  constexpr int VPR = P / EPL, NI = 32 * VPR / 64;
+  const T* xh = x + b * sx.sb + (int64_t)c * Q * sx.sl + h * sx.sh;
+  const T* dh = dout + b * sd.sb + (int64_t)c * Q * sd.sl + h * sd.sh;
+  T* oh = dx + b * sdx.sb + (int64_t)c * Q * sdx.sl + h * sdx.sh;
+  const unsigned xrow = (unsigned)(sx.sl * sizeof(T)), orow = (unsigned)(sdx.sl * sizeof(T));
+  float* ddtp = ddt + row0 + (int64_t)hw * C * Q;
+  float dsum[EPL];
+#pragma unroll
+  for (int e = 0; e < EPL; ++e) dsum[e] = 0.f;
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) {
+    Vec16<T> xv[NI], dv[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int idx = lane + 64 * i;
+      const unsigned m = (unsigned)min(mrow[mb] + idx / VPR, limit - 1), cv = (idx % VPR) * 16u;
+      xv[i] = load16_at<true>(xh, m * xrow + cv);
+      if (D) dv[i] = load16_at(dh, m * drow + cv);
+    }
+#pragma unroll
+    for (int pb = 0; pb < PB; ++pb)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) mine[acc_row(v, lane) * S::PO + 32 * pb + l32] = acc[mb][pb][v];
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int idx = lane + 64 * i;
+      const int r = idx / VPR, cv = (idx % VPR) * EPL;
+      const int m = mrow[mb] + r;
+      const float dtm = dtk[m];
+      float dot = 0.f, v[EPL];
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) {
+        v[e] = mine[r * S::PO + cv + e];
+        dot = fmaf(v[e], xv[i].get(e), dot);
+        v[e] *= dtm;
+      }
+      if (m >= limit) dot = 0.f;
+      if (D) {
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) {
+          v[e] = fmaf(d_has_hdim ? D[h * P + cv + e] : D[h], dv[i].get(e), v[e]);
+          if (m < limit) dsum[e] = fmaf(dv[i].get(e), xv[i].get(e), dsum[e]);
+        }
+      }
+      if (m < limit) {
+        Vec16<T> o;
+        o.set_all(v);
+        store16_stream(at_bytes(oh, (unsigned)m * orow + cv * (unsigned)sizeof(T)), o);
+      }
+#pragma unroll
+      for (int off = 1; off < VPR; off <<= 1) dot += __shfl_xor(dot, off);
+      if ((idx % VPR) == 0) ddtp[m] = dot;
+    }
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+  }
+  if (dD_part) {  // the head's two waves fill two of its slots, the others are zero
+    float* base = dD_part + (((b * C + c) * nh + h) * (int64_t)slots) * P;
+    store_dD_partial<EPL, VPR>(base + wj * P, dsum, lane);
+    if (lane < VPR)
+      for (int sl = wj + 2; sl < slots; sl += 2)
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) base[sl * P + lane * EPL + e] = 0.f;
+  }
+}
+
+// ------------------------------------------------------------------------------------
 // Gradient of the causal term of the chunk scan with respect to the per-position dA, for chunk
 // sizes of 64, 128 or 256.  One workgroup per (b, c, h).  With
 //   W[m][n] = <dout[m], x[n]> * dt_n * cb[m][n] * exp(min(dA_m - dA_n, 0))   for n < m < limit,

@@ -54,16 +54,18 @@ struct ScanLaunch {
   // Chunks of 64 or 128 rows in one tile.  Two adjacent heads of a group per workgroup where they are adjacent
   // in memory too (dense heads of 64 features): they share the fragments of cb and the rows of C.  A single
   // bfloat16 head of 64 features leaves each wave one column block for the weights it forms, and the 64-row
-  // kernel is the faster one (17 heads, L 4096, b2, chunk 128: 29.0 against 32.4 us).  Against the 64-row
-  // kernel otherwise, us at dstate 128: bfloat16 b8 nh32 L8192 hdim 64 chunk 128 437 -> 260, chunk 64
-  // 334 -> 240; b2 nh16 L4096 hdim 128 chunk 128 42 -> 38; float32 b1 nh16 L4096 chunk 128 hdim 64 35 -> 25,
-  // hdim 128 70 -> 40.
+  // kernel is the faster one (17 heads, L 4096, b2, chunk 128: 29.0 against 32.4 us); so it is in bfloat16 while
+  // the workgroups do not fill the chip (b1 nh8 L2000 chunk 128, 64 pairs: 8.0 against 9.6 us; b2 nh16 L1092 chunk
+  // 64, 288 pairs: 8.7 against 9.7; b1 nh24 L5000 chunk 128, 480 pairs: 27 against 17).  The 64-row kernel / this
+  // one otherwise, us at dstate 128: bfloat16 b8 nh32 L8192 hdim 64 chunk 128 437 / 260, chunk 64 334 / 240; b2
+  // nh16 L4096 hdim 128 chunk 128 41 / 38; float32 b1 nh16 L4096 chunk 128 hdim 64 35 / 26, hdim 128 70 / 40.
   template <typename T, int P, int N, typename TS, int ST>
   int launch_mid_pairs(bool* taken) const {
     *taken = true;
-    if constexpr (P == 64 && sizeof(T) == 2) {
-      const bool dense = sx.sh == P && so.sh == P && (!z || sz.sh == P);
-      if (dense && (d.nh / d.g) % 2 == 0) return launch_mid<T, P, N, TS, 2, ST>();
+    if constexpr (sizeof(T) == 2) {
+      constexpr int HP = P == 64 ? 2 : 1;
+      const bool pairs = sx.sh == P && so.sh == P && (!z || sz.sh == P) && (d.nh / d.g) % 2 == 0;
+      if ((HP == 1 || pairs) && d.batch * d.C * (d.nh / HP) >= kMidWorkgroups) return launch_mid<T, P, N, TS, HP, ST>();
       *taken = false;
       return SSD_OK;
     } else {
