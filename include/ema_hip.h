@@ -326,11 +326,12 @@ int ema_seq_fwd(int form, const float* coef, int64_t c_sb, int64_t c_sl, int64_t
 /* Coefficients of a packed batch: dst = src, except at the first position of every sequence but a row's first
  * (seq_idx int32 (batch, seqlen), where it differs from the position before), which drops the state in
  * ema_seq_fwd / ema_seq_bwd: -src in the probability form (the sign bit is the reset), -inf in the log-decay
- * form.  gradient = 1: the gradient with respect to src from that with respect to the packed coefficients
- * (-src, or 0).  dst may be src. */
+ * form; starts (dense (batch, seqlen, nheads) bytes) notes where.  gradient = 1: the gradient with respect to src
+ * from that with respect to the packed coefficients (-src, or 0, at the noted positions; seq_idx is not read and may
+ * be NULL).  dst may be src. */
 int ema_coef_starts(int form, int gradient, const float* src, int64_t s_sb, int64_t s_sl, int64_t s_sh, float* dst,
                     int64_t d_sb, int64_t d_sl, int64_t d_sh, const int32_t* seq_idx, int64_t seq_sb, int64_t seq_sl,
-                    int64_t batch, int64_t nheads, int64_t seqlen, void* stream);
+                    uint8_t* starts, int64_t batch, int64_t nheads, int64_t seqlen, void* stream);
 
 /* Backward of ema_seq_fwd in one pass over x and dy.  With r the reverse scan of dy,
  * r[t] = dy[t] + a[t+1] * r[t+1], started from dfinal (N,T) float32 (may be NULL = zero), the

@@ -66,6 +66,7 @@ def test_packing_in_one_launch_equals_tensor_operations(layout, form, device):
             coef, seq = leaf, ids.to(device, id_type)
         xg = x.to(device).requires_grad_()
         y, final = ema_seq_scan(coef, xg, form=form, return_final_states=True, seq_idx=seq)
+        seq = seq if layout == "expanded" else seq.zero_()  # the ids are the caller's again after the forward
         torch.autograd.backward((y, final), (dy.to(device), torch.ones_like(final)))
         res.append((y.detach(), final.detach(), xg.grad, leaf.grad))
     for name, a, c in zip(("y", "final", "dx", "dcoef"), *res):

@@ -1124,17 +1124,17 @@ size_t ema_seq_bwd_workspace_bytes(int64_t batch, int64_t nheads, int64_t seqlen
 
 int ema_coef_starts(int form, int gradient, const float* src, int64_t s_sb, int64_t s_sl, int64_t s_sh, float* dst,
                     int64_t d_sb, int64_t d_sl, int64_t d_sh, const int32_t* seq_idx, int64_t seq_sb, int64_t seq_sl,
-                    int64_t batch, int64_t nheads, int64_t seqlen, void* stream) {
+                    uint8_t* starts, int64_t batch, int64_t nheads, int64_t seqlen, void* stream) {
   Dims d;
   EMA_TRY(check_form(form));
   EMA_TRY(check_dims(batch, nheads, seqlen, 1, kTileRows, false, &d));
-  if (!src || !dst || !seq_idx) return EMA_ERR_NULL;
+  if (!src || !dst || !starts || (!gradient && !seq_idx)) return EMA_ERR_NULL;
   const int64_t total = d.N * d.L;
   if ((total + 255) / 256 > 0x7fffffff) return EMA_ERR_SHAPE;
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, as_stream(stream), src,
                        SeqStrides{s_sb, s_sl, s_sh}, dst, SeqStrides{d_sb, d_sl, d_sh}, (const int*)seq_idx, seq_sb,
-                       seq_sl, form == EMA_FORM_PROBABILITY ? 1 : 0, (int)d.nh, (int)d.L, total);
+                       seq_sl, (unsigned char*)starts, form == EMA_FORM_PROBABILITY ? 1 : 0, (int)d.nh, (int)d.L, total);
   };
   if (gradient) launch(coef_starts_kernel<1>);
   else launch(coef_starts_kernel<0>);

@@ -542,6 +542,8 @@ __global__ __launch_bounds__(256) void combine_dA_kernel(const float* __restrict
 // gradient with respect to the given coefficients from that of the packed ones (MODE 1, may run in place):
 //   probability form  -v at the first position of a sequence, either way (the sign bit is the reset);
 //   log-decay form    -inf at the first position (decay 0), and gradient 0 there.
+// MODE 0 notes in starts (dense (batch, L, nh) bytes) where it did so and MODE 1 goes by that, so that the gradient
+// does not depend on what becomes of the ids in between.
 // One thread per (batch, position, head).  Bound by its launch: it stands for the eleven elementwise launches that
 // a forward and backward need in tensor operations (b6 nh2 L1777: 4.4 and 3.3 us
 // in place of 35 us of kernels and eleven times the host's part of a launch).
@@ -549,16 +551,23 @@ __global__ __launch_bounds__(256) void combine_dA_kernel(const float* __restrict
 template <int MODE>
 __global__ __launch_bounds__(256) void coef_starts_kernel(const float* src, SeqStrides ss, float* dst, SeqStrides sd,
                                                           const int* __restrict__ ids, int64_t id_sb, int64_t id_sl,
-                                                          int prob, int nh, int L, int64_t total) {
+                                                          unsigned char* __restrict__ starts, int prob, int nh, int L, int64_t total) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= total) return;
   const int h = (int)(i % nh);
   const int64_t bl = i / nh;
   const int64_t b = bl / L;
   const int l = (int)(bl - b * L);
-  const int* id = ids + b * id_sb + (int64_t)l * id_sl;
   float v = src[b * ss.sb + (int64_t)l * ss.sl + h * ss.sh];
-  if (l > 0 && id[0] != id[-id_sl]) v = prob ? -v : (MODE == 0 ? -INFINITY : 0.f);
+  bool start;
+  if (MODE == 0) {
+    const int* id = ids + b * id_sb + (int64_t)l * id_sl;
+    start = l > 0 && id[0] != id[-id_sl];
+    starts[i] = start;
+  } else {
+    start = starts[i] != 0;
+  }
+  if (start) v = prob ? -v : (MODE == 0 ? -INFINITY : 0.f);
   dst[b * sd.sb + (int64_t)l * sd.sl + h * sd.sh] = v;
 }
 

@@ -58,7 +58,7 @@ _SIGNATURES = {
     "ema_seq_fwd_static_error": (c_int, [_P, _P]),
     "ema_seq_fwd_static_reset": (c_int, [_P]),
     "ema_seq_fwd_static": (c_int, [c_int] + _SEQ + _SEQ + [c_int] + _SEQ + [_P, _P, _P, _I, _I, _I, _I, _P]),
-    "ema_coef_starts": (c_int, [c_int, c_int] + _SEQ + _SEQ + _IDS + [_I, _I, _I, _P]),
+    "ema_coef_starts": (c_int, [c_int, c_int] + _SEQ + _SEQ + _IDS + [_P, _I, _I, _I, _P]),
     # SSD forward stages (include/ssd_hip.h)
     "ssd_chunk_cumsum_fwd": (c_int, [_P, c_int, _I, _I, _I, _P, _P, _P, _P, _I, _I, _I, _I, c_int, c_float, c_float, _P]),
     "ssd_chunk_state_fwd": (c_int, _SEQ + _SEQ + [c_int, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I] + _IDS + [_P]),

@@ -147,16 +147,18 @@ def pack_probability(p, seq_idx):
     return torch.where(start, -p, p)
 
 
-def _coef_starts(src, seq_idx, form, gradient, dst=None):
-    """One launch of what pack_log_decay / pack_probability (gradient=False) and their backward do."""
+def _coef_starts(src, starts, form, seq_idx=None, dst=None):
+    """One launch of what pack_log_decay / pack_probability do (with seq_idx; the first positions are noted in
+    starts), or of their backward (without)."""
     dst = torch.empty_like(src) if dst is None else dst
-    dev = _lib.require_gpu(src, dst, seq_idx)
+    dev = _lib.require_gpu(src, dst, starts)
     ss, batch, nh, L = _lib.decay_view(src)
     ds, *_ = _lib.decay_view(dst)
+    ids = [None, 0, 0] if seq_idx is None else [seq_idx.data_ptr(), *seq_idx.stride()]
     with _lib.on_device(dev):
         _lib.check(
-            _lib.lib().ema_coef_starts(FORMS[form], int(gradient), *ss, *ds, seq_idx.data_ptr(), *seq_idx.stride(),
-                                       batch, nh, L, _lib.stream_ptr(dev)),
+            _lib.lib().ema_coef_starts(FORMS[form], int(seq_idx is None), *ss, *ds, *ids, starts.data_ptr(), batch, nh,
+                                       L, _lib.stream_ptr(dev)),
             "ema_coef_starts")
     return dst
 
@@ -166,9 +168,10 @@ class EMASeqPackedFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, coef, x, initial_states, form, seq_idx):
-        packed = _coef_starts(coef, seq_idx, form, gradient=False)
+        starts = torch.empty(coef.shape, dtype=torch.uint8, device=coef.device)
+        packed = _coef_starts(coef, starts, form, seq_idx=seq_idx)
         y, final, prev128 = ema_seq_fwd(packed, x, form, initial_states)
-        ctx.save_for_backward(packed, x, prev128, seq_idx)
+        ctx.save_for_backward(packed, x, prev128, starts)
         ctx.form = form
         ctx.has_init = initial_states is not None
         ctx.init_dtype = None if initial_states is None else initial_states.dtype
@@ -177,12 +180,12 @@ class EMASeqPackedFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dy, dfinal):
-        packed, x, prev128, seq_idx = ctx.saved_tensors
+        packed, x, prev128, starts = ctx.saved_tensors
         if dy is None:
             dy = torch.zeros_like(x)
         dx, dcoef, dinit = ema_seq_bwd(dy.contiguous(), x, packed, prev128, ctx.form, dfinal_states=dfinal,
                                        want_dinit=ctx.has_init)
-        dcoef = _coef_starts(dcoef, seq_idx, ctx.form, gradient=True, dst=dcoef)
+        dcoef = _coef_starts(dcoef, starts, ctx.form, dst=dcoef)
         if dinit is not None:
             dinit = dinit.to(ctx.init_dtype)
         return dcoef, dx, dinit, None, None
