@@ -580,7 +580,9 @@ __device__ __forceinline__ void state_store(bf16_t* p, const StateVec<E>& s) {
 // ------------------------------------------------------------------------------------
 // state_passing.  out[b, c] = state entering chunk c, state <- exp(dA_chunk[c]) * state +
 // states[b, c]; the value after the last chunk goes to final.  One thread per four adjacent
-// state elements, the running state in registers, chunks fetched four ahead.
+// state elements, the running state in registers; the next four chunks are requested before the current four are
+// used.  Bound by that chain of loads while few workgroups run (b1 nh24 hdim 64 dstate 128, 40 chunks: 19.8 us
+// with one turn of four under way, 13.1 with two), by HBM otherwise.
 // states / out are (b, C, nh, dim) dense float32; dA_chunk is addressed by strides (it is the
 // last column of dA_cumsum).  In a packed batch the state is dropped across a chunk whose last
 // position has another id than the previous chunk's last position.
