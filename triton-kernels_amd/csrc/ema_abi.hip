@@ -539,8 +539,10 @@ int launch_da(const void* x, SeqStrides sx, const void* dy, SeqStrides sd, int d
                        (const float*)x, sx, (const float*)dy, sd, cs, w.part, w.rowsum, (int)d.nh,
                        (int)d.L, (int)d.T, (int)d.Q, (int)d.C, MT, nullptr, nullptr, 1, 1, only);
   EMA_TRY(launched());
+  // one wave per chunk, or, where the factored form runs, one per 64 of its positions
   const int64_t total = d.N * d.C;
-  hipLaunchKernelGGL(da_finish_kernel<kBM>, dim3((unsigned)((total + 3) / 4)), dim3(256), 0, st, w.part,
+  const unsigned parts = flat ? (unsigned)((d.Q + 63) / 64) : 1;
+  hipLaunchKernelGGL(da_finish_kernel<kBM>, dim3((unsigned)((total + 3) / 4), parts), dim3(256), 0, st, w.part,
                      w.rowsum, w.flat, da_flat_tiles(d, dtype), only, ddA_intra, (int)d.Q, MT, total);
   return launched();
 }

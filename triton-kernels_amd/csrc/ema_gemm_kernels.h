@@ -175,13 +175,14 @@ __global__ __launch_bounds__(256, 2) void da_gemm_kernel(const T* __restrict__ x
   }
 }
 
-// B6, second part, one wave per (n, c).  Where the chunk went through the factored form (steep is given and
-// its entry is 0) the per-column-tile dots only have to be added up:
+// B6, second part.  Where the chunk went through the factored form (steep is given and its entry is 0) the
+// per-column-tile dots only have to be added up, gridDim.y waves per chunk with a position per lane:
 //   ddA_intra[q] = sum over the ntiles column tiles of flat[(chunk*ntiles + tile)*Q + q];
-// otherwise ddA_intra[j] = sum_{i<j} (colsum[i] - rowsum[i]) with
+// otherwise ddA_intra[j] = sum_{i<j} (colsum[i] - rowsum[i]) by the first of the chunk's waves, with
 //   colsum[i] = sum over the row tiles mt >= i / BM of part[mt][i].
-// Both forms in one launch: a launch that mostly finds nothing to do costs as much as one that works (4.5 and 4.7 us
-// at b4 nh2 d1024 L4096 chunk 256; 6.4 together).
+// Both forms in one launch: a launch that mostly finds nothing to do costs as much as one that works.  The chain
+// of ntiles loads bounds it where chunks are few, so the positions of a chunk are spread over its waves: one wave
+// for all of them made the whole of B6 28 -> 75 us at N1 L500 d2048 chunk 512 float32 (16 column tiles).
 template <int BM>
 __global__ __launch_bounds__(256) void da_finish_kernel(const float* __restrict__ part,
                                                         const float* __restrict__ rowsum,
@@ -193,14 +194,15 @@ __global__ __launch_bounds__(256) void da_finish_kernel(const float* __restrict_
   const int64_t chunk_id = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (chunk_id >= total_chunks) return;
   if (steep && steep[chunk_id] == 0) {
-    const float* fp = flat + chunk_id * ntiles * (int64_t)Q;
-    for (int q = lane; q < Q; q += 64) {
-      float s = 0.f;
-      for (int ct = 0; ct < ntiles; ++ct) s += fp[ct * (int64_t)Q + q];
-      ddA_intra[chunk_id * Q + q] = s;
-    }
+    const int q = (int)blockIdx.y * 64 + lane;
+    if (q >= Q) return;
+    const float* fp = flat + chunk_id * ntiles * (int64_t)Q + q;
+    float s = 0.f;
+    for (int ct = 0; ct < ntiles; ++ct) s += fp[ct * (int64_t)Q];
+    ddA_intra[chunk_id * Q + q] = s;
     return;
   }
+  if (blockIdx.y != 0) return;
   const int per = (Q + 63) >> 6;
   const int q0 = lane * per;
   auto val = [&](int q) {
