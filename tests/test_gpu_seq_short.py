@@ -114,3 +114,18 @@ def test_state_passing_turns(C, device):
     got = _ema_state_passing_bwd(d(prev), d(cs_last), d(ds))
     check_close("g", got[0], g, F32)
     check_close("ddA_chunk", got[1], ddA, F32)
+
+
+@pytest.mark.parametrize("C", [1, 8, 9, 17, 31, 32, 33])  # more than 1024 workgroups: guarded loads up to 31 chunks
+def test_state_passing_backward_with_the_chip_filled(C, device):
+    from kernels.ema_kernels_bwd.ema_state_passing_bwd_dstates import _ema_state_passing_bwd
+
+    announce(f"state passing backward, 1100 sequences, {C} chunks")
+    gen = torch.Generator().manual_seed(C)
+    N, T = 1100, 12
+    prev, ds = torch.randn(N, C, T, generator=gen), torch.randn(N, C, T, generator=gen)
+    cs_last = -torch.rand(N, C, generator=gen)
+    g, ddA = O.state_passing_bwd(prev, cs_last, ds)
+    got = _ema_state_passing_bwd(*(t.to(device) for t in (prev, cs_last, ds)))
+    check_close("g", got[0], g, F32)
+    check_close("ddA_chunk", got[1], ddA, F32)

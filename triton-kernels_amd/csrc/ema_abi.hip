@@ -123,14 +123,19 @@ int launch_state_passing_bwd(const float* prev, const float* cs_last, int64_t cl
                              float* part, int64_t N, int64_t C, int64_t T, hipStream_t st) {
   const int tiles = (int)((T + 255) / 256);
   const int nw = (int)((T + 63) / 64);
-  if (!ddA_chunk) {  // only the recurrence; no <prev, g> products
-    hipLaunchKernelGGL(state_passing_bwd_kernel<false>, dim3((unsigned)(N * tiles)), dim3(256), 0,
-                       st, prev, cs_last, cl_sn, cl_sc, ds, g, part, (int)C, (int)T, tiles, nw);
+  // Loads ahead of the turn that uses them, from clamped indices, unless the workgroups fill the chip and a turn of
+  // eight chunks is more than a quarter of all: what is then loaded twice costs more than the wait.  Guarded loads /
+  // ahead, us: 32 sequences d1024, 47 chunks 19.3 / 14.1; 2048 sequences d1024, 1 chunk 15.3 / 17.3, 9 chunks 37.5 /
+  // 40.4, 47 chunks 168 / 155.
+  const bool ahead = N * tiles <= kFillWorkgroups || C >= 32;
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(N * tiles)), dim3(256), 0, st, prev, cs_last, cl_sn, cl_sc, ds, g, part,
+                       (int)C, (int)T, tiles, nw);
     return launched();
-  }
-  hipLaunchKernelGGL(state_passing_bwd_kernel<true>, dim3((unsigned)(N * tiles)), dim3(256), 0, st,
-                     prev, cs_last, cl_sn, cl_sc, ds, g, part, (int)C, (int)T, tiles, nw);
-  EMA_TRY(launched());
+  };
+  if (!ddA_chunk)  // only the recurrence; no <prev, g> products
+    return ahead ? launch(state_passing_bwd_kernel<false, true>) : launch(state_passing_bwd_kernel<false, false>);
+  EMA_TRY(ahead ? launch(state_passing_bwd_kernel<true, true>) : launch(state_passing_bwd_kernel<true, false>));
   const int64_t total = N * C;
   hipLaunchKernelGGL(state_passing_bwd_finish_kernel, dim3((unsigned)((total + 255) / 256)),
                      dim3(256), 0, st, part, cs_last, cl_sn, cl_sc, ddA_chunk, (int)C, nw, total);

@@ -306,9 +306,17 @@ __global__ __launch_bounds__(256) void state_passing_fwd_kernel(
     }
   };
   request(0, s[0], a[0]);
-  for (int c0 = 0; c0 < C; c0 += 2 * U) {
+  for (int c0 = 0;; c0 += 2 * U) {  // (nothing is requested past the last turn)
+    if (c0 + U >= C) {
+      turn(c0, s[0], a[0]);
+      break;
+    }
     request(c0 + U, s[1], a[1]);
     turn(c0, s[0], a[0]);
+    if (c0 + 2 * U >= C) {
+      turn(c0 + U, s[1], a[1]);
+      break;
+    }
     request(c0 + 2 * U, s[0], a[0]);
     turn(c0 + U, s[1], a[1]);
   }
@@ -320,7 +328,7 @@ __global__ __launch_bounds__(256) void state_passing_fwd_kernel(
 // wave writes its partial of <prev[n,c], g[n,c]> to part[(n*C + c) * nw + wave_of_t]; the
 // partials are summed (and scaled by exp(cs_last)) by state_passing_bwd_finish_kernel.
 // ------------------------------------------------------------------------------------
-template <bool DOTS>
+template <bool DOTS, bool AHEAD>
 __global__ __launch_bounds__(256) void state_passing_bwd_kernel(
     const float* __restrict__ prev, const float* __restrict__ cs_last, int64_t cl_sn,
     int64_t cl_sc, const float* __restrict__ ds, float* __restrict__ g,
@@ -334,13 +342,15 @@ __global__ __launch_bounds__(256) void state_passing_bwd_kernel(
   const int64_t base = n * (int64_t)C * Tdim + (ok ? t : 0);
   const float* cl = cs_last + n * cl_sn;
   float cur = 0.f;
-  constexpr int U = 8;  // chunks per turn; the next turn's are requested before this turn's are used
+  constexpr int U = 8;  // chunks per turn
   float d[2][U], p[2][U], a[2][U];
-  // unconditional loads from chunk indices clamped into the tensor (a thread past the last column reads column 0)
+  // AHEAD: unconditional loads from chunk indices clamped into the tensor (a thread past the last column reads
+  // column 0)
   auto request = [&](int c1, float* dv, float* pvv, float* w) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int c = max(c1 - u, 0);
+      const int c = AHEAD ? max(c1 - u, 0) : c1 - u;
+      if (!AHEAD && c < 0) break;
       dv[u] = ds[base + (int64_t)c * Tdim];
       if (DOTS) pvv[u] = prev[base + (int64_t)c * Tdim];
       w[u] = cl[(int64_t)c * cl_sc];
@@ -360,10 +370,25 @@ __global__ __launch_bounds__(256) void state_passing_bwd_kernel(
       }
     }
   };
+  if constexpr (!AHEAD) {
+    for (int c1 = C - 1; c1 >= 0; c1 -= U) {
+      request(c1, d[0], p[0], a[0]);
+      turn(c1, d[0], p[0], a[0]);
+    }
+    return;
+  }
   request(C - 1, d[0], p[0], a[0]);
-  for (int c1 = C - 1; c1 >= 0; c1 -= 2 * U) {
+  for (int c1 = C - 1;; c1 -= 2 * U) {  // (nothing is requested past the first chunk)
+    if (c1 < U) {
+      turn(c1, d[0], p[0], a[0]);
+      break;
+    }
     request(c1 - U, d[1], p[1], a[1]);
     turn(c1, d[0], p[0], a[0]);
+    if (c1 < 2 * U) {
+      turn(c1 - U, d[1], p[1], a[1]);
+      break;
+    }
     request(c1 - 2 * U, d[0], p[0], a[0]);
     turn(c1 - U, d[1], p[1], a[1]);
   }
