@@ -75,6 +75,36 @@ def test_state_passing_turns(nchunks, device):
         check_close("ddA", gdda, rdda, F32)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [F32, BF16], ids=["f32", "bf16"])  # bfloat16: eight elements per thread backward
+@pytest.mark.parametrize("nchunks", [4, 5, 8, 9])
+def test_state_passing_with_the_chip_filled(nchunks, dtype, device):
+    """More workgroups than the form with two turns of loads under way takes, plain and packed, both directions."""
+    from kernels.mamba_kernels.mamba_state_pass import _state_passing_fwd
+    from kernels.mamba_kernels_bwd.mamba_state_passing_bwd_dstates import _state_passing_bwd
+
+    announce(f"state passing, 1040 heads, {nchunks} chunks {dtype}")
+    b, nh, dim, Q = 2, 520, 16, 4
+    L = nchunks * Q - 1
+    gen = torch.Generator().manual_seed(nchunks)
+    st, dout = (torch.randn(b, nchunks, nh, dim, generator=gen).to(dtype) for _ in range(2))
+    da = -torch.rand(b, nh, nchunks, generator=gen)
+    ids = (torch.rand(b, L, generator=gen) < 0.15).to(torch.int32).cumsum(1, dtype=torch.int32)
+    d = lambda t: t.to(device)
+    for seq in (None, ids):
+        kw = {} if seq is None else dict(seq_idx=seq, chunk_size=Q)
+        dkw = {} if seq is None else dict(seq_idx=d(seq), chunk_size=Q)
+        ref, rfin = S.state_passing(st.float(), da, **kw)
+        got, fin = _state_passing_fwd(d(st), d(da), out_dtype=dtype, **dkw)
+        check_close("states", got, ref, dtype)
+        check_close("final", fin, rfin, F32)
+        carried = ref.to(dtype)
+        rd, rdda, _ = S.state_passing_bwd(carried.float(), da, dout.float(), **kw)
+        gd, gdda, _ = _state_passing_bwd(d(carried), d(da), d(dout), dstates_dtype=dtype, **dkw)
+        check_close("dstates", gd, rd, dtype)
+        check_close("ddA", gdda, rdda, F32)
+
+
 def test_walk_choice():
     """Few heads or long chunks: the two launchers; a head per compute unit: the walk."""
     assert not walk_pays(1, 32, 4096, 256, 64, 128, 2)

@@ -222,6 +222,15 @@ int launch_row_cumsum(float* v, int64_t Q, int64_t rows, hipStream_t st) {
   return launched();
 }
 
+// Whether the state-passing kernels keep two turns of chunks under way: where there is more than one turn and the
+// workgroups leave the chip latency bound, up to four on each of 256 compute units with four state elements per
+// thread (two with eight, which hold twice the registers).  One turn / two, us, 40 chunks: 64 workgroups 12.8 / 9.3
+// (backward 26.2 / 18.6), 384 20.2 / 18.5 (40.6 / 35.4), 1024 44.7 / 45.5 (65.4 / 64.7); 8 chunks: 192 workgroups
+// 4.9 / 4.4, 4096 41.9 / 44.9 (61.1 / 65.1).  Eight elements, backward, 40 chunks: 512 workgroups 41.7 / 38.3, 768 53 / 63.
+inline bool passing_ahead(int64_t nchunks, int64_t workgroups, int per_thread) {
+  return nchunks > 4 && workgroups * per_thread <= 4 * 1024;
+}
+
 template <typename T, typename TO, int K>
 int launch_bmm(const void* a, Strides3 sa, const void* bm, Strides3 sb, void* out, const Dims& d, SeqIdx seq,
                hipStream_t st) {
@@ -327,12 +336,15 @@ int ssd_state_passing_fwd(const float* states, const float* dA_chunk, int64_t da
   const int tiles = (int)((dim + 1023) / 1024);
   const int64_t grid = batch * nheads * tiles;
   if (grid > 0x7fffffff || dim > (1 << 24)) return SSD_ERR_SHAPE;
-#define SSD_SP_LAUNCH(TO)                                                                                          \
-  hipLaunchKernelGGL((ssd_state_passing_kernel<TO, 4>), dim3((unsigned)grid), dim3(256), 0, as_stream(stream), states, \
+  const bool ahead = passing_ahead(nchunks, grid, 4);
+#define SSD_SP_LAUNCH(TO, AHEAD)                                                                                   \
+  hipLaunchKernelGGL((ssd_state_passing_kernel<TO, 4, AHEAD>), dim3((unsigned)grid), dim3(256), 0, as_stream(stream), states, \
                      dA_chunk, da_sb, da_sh, da_sc, initial, (TO*)out, final_states, (int)nheads, (int)nchunks,      \
                      (int)dim, tiles, as_seq(seq_idx, seq_sb, seq_sl), (int)seqlen, (int)chunk)
-  if (out_dtype == SSD_BF16) SSD_SP_LAUNCH(bf16_t);
-  else SSD_SP_LAUNCH(float);
+  if (out_dtype == SSD_BF16 && ahead) SSD_SP_LAUNCH(bf16_t, true);
+  else if (out_dtype == SSD_BF16) SSD_SP_LAUNCH(bf16_t, false);
+  else if (ahead) SSD_SP_LAUNCH(float, true);
+  else SSD_SP_LAUNCH(float, false);
 #undef SSD_SP_LAUNCH
   return launched();
 }
@@ -419,13 +431,21 @@ int ssd_state_passing_bwd(const void* states, int states_dtype, const float* dA_
   hipStream_t st = as_stream(stream);
   float* part = static_cast<float*>(workspace);
   // the three tensors are float32 or bfloat16 independently of each other
+  const bool ahead = passing_ahead(nchunks, grid, wide ? 8 : 4);
+  auto launch_as = [&](auto kernel, auto ts, auto td, auto tg) {
+    using TS = decltype(ts);
+    using TD = decltype(td);
+    using TG = decltype(tg);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(256), 0, st,
+                       (const TS*)states, dA_chunk, da_sb, da_sh, da_sc, (const TD*)dout, dfinal, (TG*)dstates, part,
+                       dinit, (int)nheads, (int)nchunks, (int)dim, tiles, seq, (int)seqlen, (int)chunk);
+  };
   auto launch = [&](auto ts, auto td, auto tg) {
     using TS = decltype(ts);
     using TD = decltype(td);
     using TG = decltype(tg);
-    hipLaunchKernelGGL((ssd_state_passing_bwd_kernel<TS, TD, TG, 4>), dim3((unsigned)grid), dim3(256), 0, st,
-                       (const TS*)states, dA_chunk, da_sb, da_sh, da_sc, (const TD*)dout, dfinal, (TG*)dstates, part,
-                       dinit, (int)nheads, (int)nchunks, (int)dim, tiles, seq, (int)seqlen, (int)chunk);
+    if (ahead) launch_as(ssd_state_passing_bwd_kernel<TS, TD, TG, 4, true>, ts, td, tg);
+    else launch_as(ssd_state_passing_bwd_kernel<TS, TD, TG, 4, false>, ts, td, tg);
   };
   auto pick_g = [&](auto ts, auto td) {
     if (dstates_dtype == SSD_BF16) launch(ts, td, bf16_t());
@@ -435,11 +455,8 @@ int ssd_state_passing_bwd(const void* states, int states_dtype, const float* dA_
     if (dout_dtype == SSD_BF16) pick_g(ts, bf16_t());
     else pick_g(ts, float());
   };
-  if (wide)
-    hipLaunchKernelGGL((ssd_state_passing_bwd_kernel<bf16_t, bf16_t, bf16_t, 8>), dim3((unsigned)grid), dim3(256), 0,
-                       st, (const bf16_t*)states, dA_chunk, da_sb, da_sh, da_sc, (const bf16_t*)dout, dfinal,
-                       (bf16_t*)dstates, part, dinit, (int)nheads, (int)nchunks, (int)dim, tiles, seq, (int)seqlen,
-                       (int)chunk);
+  if (wide && ahead) launch_as(ssd_state_passing_bwd_kernel<bf16_t, bf16_t, bf16_t, 8, true>, bf16_t(), bf16_t(), bf16_t());
+  else if (wide) launch_as(ssd_state_passing_bwd_kernel<bf16_t, bf16_t, bf16_t, 8, false>, bf16_t(), bf16_t(), bf16_t());
   else if (states_dtype == SSD_BF16) pick_d(bf16_t());
   else pick_d(float());
   SSD_TRY(launched());

@@ -580,14 +580,15 @@ __device__ __forceinline__ void state_store(bf16_t* p, const StateVec<E>& s) {
 // ------------------------------------------------------------------------------------
 // state_passing.  out[b, c] = state entering chunk c, state <- exp(dA_chunk[c]) * state +
 // states[b, c]; the value after the last chunk goes to final.  One thread per four adjacent
-// state elements, the running state in registers; the next four chunks are requested before the current four are
-// used.  Bound by that chain of loads while few workgroups run (b1 nh24 hdim 64 dstate 128, 40 chunks: 19.8 us
-// with one turn of four under way, 13.1 with two), by HBM otherwise.
+// state elements, the running state in registers, four chunks requested at a time.  Bound by that chain of loads
+// while few workgroups run: AHEAD requests the next four before it uses the current four (b1 nh24 hdim 64 dstate
+// 128, 40 chunks: 13.3 -> 11.8 us).  Bound by HBM once they fill the chip, where the registers of the second turn cost
+// more than they bring, and with no second turn there is nothing to request: passing_ahead() chooses.
 // states / out are (b, C, nh, dim) dense float32; dA_chunk is addressed by strides (it is the
 // last column of dA_cumsum).  In a packed batch the state is dropped across a chunk whose last
 // position has another id than the previous chunk's last position.
 // ------------------------------------------------------------------------------------
-template <typename TO, int E>
+template <typename TO, int E, bool AHEAD>
 __global__ __launch_bounds__(256) void ssd_state_passing_kernel(
     const float* __restrict__ states, const float* __restrict__ dA_chunk, int64_t da_sb, int64_t da_sh,
     int64_t da_sc, const float* __restrict__ initial, TO* __restrict__ out, float* __restrict__ final_states,
@@ -604,10 +605,10 @@ __global__ __launch_bounds__(256) void ssd_state_passing_kernel(
   StateVec<E> s;
 #pragma unroll
   for (int i = 0; i < E; ++i) s.v[i] = initial ? initial[(b * nh + h) * (int64_t)dim + e + i] : 0.f;
-  constexpr int U = 4;  // chunks per turn; the next turn's are requested before this turn's are used
-  StateVec<E> nv[2][U];
-  float a[2][U];
-  int id[2][U];
+  constexpr int U = 4, TURNS = AHEAD ? 2 : 1;  // chunks per turn, turns under way
+  StateVec<E> nv[TURNS][U];
+  float a[TURNS][U];
+  int id[TURNS][U];
   const int* ids = seq.p ? seq.p + b * seq.sb : nullptr;
   int id_before = 0;
   // unconditional loads from chunk indices clamped into the tensor
@@ -636,11 +637,27 @@ __global__ __launch_bounds__(256) void ssd_state_passing_kernel(
     }
   };
   request(0, nv[0], a[0], id[0]);
-  for (int c0 = 0; c0 < C; c0 += 2 * U) {
-    request(c0 + U, nv[1], a[1], id[1]);
-    turn(c0, nv[0], a[0], id[0]);
-    request(c0 + 2 * U, nv[0], a[0], id[0]);
-    turn(c0 + U, nv[1], a[1], id[1]);
+  if constexpr (AHEAD) {
+    for (int c0 = 0;; c0 += 2 * U) {  // (nothing is requested past the last turn)
+      if (c0 + U >= C) {
+        turn(c0, nv[0], a[0], id[0]);
+        break;
+      }
+      request(c0 + U, nv[1], a[1], id[1]);
+      turn(c0, nv[0], a[0], id[0]);
+      if (c0 + 2 * U >= C) {
+        turn(c0 + U, nv[1], a[1], id[1]);
+        break;
+      }
+      request(c0 + 2 * U, nv[0], a[0], id[0]);
+      turn(c0 + U, nv[1], a[1], id[1]);
+    }
+  } else {
+    turn(0, nv[0], a[0], id[0]);
+    for (int c0 = U; c0 < C; c0 += U) {
+      request(c0, nv[0], a[0], id[0]);
+      turn(c0, nv[0], a[0], id[0]);
+    }
   }
 #pragma unroll
   for (int i = 0; i < E; ++i) final_states[(b * nh + h) * (int64_t)dim + e + i] = s.v[i];
@@ -1177,7 +1194,7 @@ __device__ __forceinline__ float half_wave_sum(float v) {
 // The finish kernel sums the wave partials: ddA[b,h,c] = exp(dA_chunk[c]) * sum, and 0 for
 // c = 0 when there is no initial state.
 // ------------------------------------------------------------------------------------
-template <typename TS, typename TD, typename TG, int E>
+template <typename TS, typename TD, typename TG, int E, bool AHEAD>
 __global__ __launch_bounds__(256) void ssd_state_passing_bwd_kernel(
     const TS* __restrict__ states, const float* __restrict__ dA_chunk, int64_t da_sb, int64_t da_sh,
     int64_t da_sc, const TD* __restrict__ dout, const float* __restrict__ dfinal,
@@ -1196,10 +1213,10 @@ __global__ __launch_bounds__(256) void ssd_state_passing_bwd_kernel(
   StateVec<E> G;
 #pragma unroll
   for (int i = 0; i < E; ++i) G.v[i] = (dfinal && ok) ? dfinal[(b * nh + h) * (int64_t)dim + e + i] : 0.f;
-  constexpr int U = 4;  // chunks per turn; the next turn's are requested before this turn's are used
-  StateVec<E> sv[2][U], dv[2][U];
-  float a[2][U];
-  int id[2][U + 1];  // ids at the ends of the turn's chunks, and of the chunk before them
+  constexpr int U = 4, TURNS = AHEAD ? 2 : 1;  // chunks per turn, turns under way (see ssd_state_passing_kernel)
+  StateVec<E> sv[TURNS][U], dv[TURNS][U];
+  float a[TURNS][U];
+  int id[TURNS][U + 1];  // ids at the ends of the turn's chunks, and of the chunk before them
   const int* ids = seq.p ? seq.p + b * seq.sb : nullptr;
   // unconditional loads from chunk indices clamped into the tensor; what lies outside is not used
   auto request = [&](int c1, StateVec<E>* s, StateVec<E>* d, float* w, int* end_id) {
@@ -1232,11 +1249,27 @@ __global__ __launch_bounds__(256) void ssd_state_passing_bwd_kernel(
     }
   };
   request(C - 1, sv[0], dv[0], a[0], id[0]);
-  for (int c1 = C - 1; c1 >= 0; c1 -= 2 * U) {
-    request(c1 - U, sv[1], dv[1], a[1], id[1]);
-    turn(c1, sv[0], dv[0], a[0], id[0]);
-    request(c1 - 2 * U, sv[0], dv[0], a[0], id[0]);
-    turn(c1 - U, sv[1], dv[1], a[1], id[1]);
+  if constexpr (AHEAD) {
+    for (int c1 = C - 1;; c1 -= 2 * U) {  // (nothing is requested past the first chunk)
+      if (c1 < U) {
+        turn(c1, sv[0], dv[0], a[0], id[0]);
+        break;
+      }
+      request(c1 - U, sv[1], dv[1], a[1], id[1]);
+      turn(c1, sv[0], dv[0], a[0], id[0]);
+      if (c1 < 2 * U) {
+        turn(c1 - U, sv[1], dv[1], a[1], id[1]);
+        break;
+      }
+      request(c1 - 2 * U, sv[0], dv[0], a[0], id[0]);
+      turn(c1 - U, sv[1], dv[1], a[1], id[1]);
+    }
+  } else {
+    turn(C - 1, sv[0], dv[0], a[0], id[0]);
+    for (int c1 = C - 1 - U; c1 >= 0; c1 -= U) {
+      request(c1, sv[0], dv[0], a[0], id[0]);
+      turn(c1, sv[0], dv[0], a[0], id[0]);
+    }
   }
   if (dinit && ok) {
 #pragma unroll
