@@ -111,8 +111,35 @@ def test_walk_choice():
     assert not walk_pays(1, 4, 512, 64, 64, 64, 4)
     assert walk_pays(8, 32, 8192, 256, 64, 128, 2) and walk_pays(8, 32, 8192, 256, 64, 128, 2, backward=True)
     assert walk_pays(4, 32, 512, 64, 64, 128, 2)
-    for heads in (8, 64, 128):  # monotone: more heads never turn the walk away
+    for heads in (8, 64, 128):  # up to a workgroup per compute unit more heads never turn the walk away
         assert walk_pays(1, heads, 8192, 256, 64, 128, 2) <= walk_pays(1, 2 * heads, 8192, 256, 64, 128, 2)
+    # 256 heads fill the chip; a few more make the walk take twice as long, many more make up for it
+    assert walk_pays(1, 256, 8192, 256, 64, 128, 2) and not walk_pays(1, 264, 8192, 256, 64, 128, 2)
+    assert walk_pays(1, 512, 8192, 256, 64, 128, 2)
+
+
+@pytest.mark.parametrize("heads,L,Q,P,N,itemsize,backward,walk,pair", [  # measured on an MI355X, us
+    (192, 500, 512, 64, 128, 2, False, 12.9, 21.1),  # one chunk: nothing to spread, eight stages in a row either way
+    (16, 500, 512, 64, 64, 2, False, 9.0, 13.3),
+    (192, 1024, 512, 64, 128, 2, False, 20.2, 25.4),
+    (192, 500, 512, 128, 64, 2, False, 15.0, 20.2),
+    (128, 500, 512, 64, 128, 2, True, 14.8, 19.6),
+    (64, 8192, 64, 128, 128, 2, False, 393, 267),
+    (128, 8192, 64, 64, 128, 4, False, 579, 431),
+    (32, 8192, 256, 64, 128, 2, False, 126, 31),
+    (192, 8192, 256, 64, 128, 2, False, 124, 147),
+    (264, 8192, 256, 64, 128, 2, False, 235, 201),
+    (512, 8192, 256, 64, 128, 2, False, 256, 358),
+    (768, 8192, 256, 64, 128, 2, False, 371, 538),
+    (128, 8192, 256, 64, 128, 2, True, 151, 117),
+    (192, 8192, 256, 64, 128, 2, True, 154, 167),
+    (512, 2048, 64, 64, 64, 4, False, 174, 220),
+    (32, 2048, 256, 128, 128, 4, False, 207, 39),
+])
+def test_walk_choice_against_measured_times(heads, L, Q, P, N, itemsize, backward, walk, pair):
+    """What the rule takes is never more than 12 % (the error of its estimates) behind the other form."""
+    taken = walk if walk_pays(1, heads, L, Q, P, N, itemsize, backward=backward) else pair
+    assert taken <= 1.12 * min(walk, pair)
 
 
 @pytest.mark.gpu

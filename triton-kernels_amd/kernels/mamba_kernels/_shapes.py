@@ -111,34 +111,47 @@ class Plan:
 
 def walk_pays(batch, nheads, seqlen, chunk, headdim, dstate, itemsize, backward=False):
     """Whether the kernel in which one workgroup per (batch, head) walks the whole sequence is faster than
-    the two launchers it stands for, which spread the chunks over the chip and carry the chunk-local
-    float32 states through memory.  Both give the same states bit for bit.
+    the two launchers it stands for, which spread the chunks over the chip and carry the chunk-local states
+    through memory in float32 (4 * batch * nheads * nchunks * headdim * dstate bytes of scratch, which the walk
+    does not need).  Both give the same states bit for bit.
 
-    The walk is a serial chain of 64-row stages whose time does not depend on how many of the 256 compute
-    units work (MI355X, hdim 64, dstate 128, bfloat16: 0.97 us a stage forward, 1.17 backward; other shapes
-    stage their rows through registers), the two launchers are bound by the bytes they move (5 TB/s; in
-    float32 by their matrix instructions as well).  Measured walk / two launchers, us, hdim 64, dstate 128:
-      bfloat16 forward,  chunk 256, seqlen 8192:  32 heads 127 /  31, 128 heads 129 / 101, 160 heads 130 / 123,
-                                                  192 heads 130 / 146, 256 heads 139 / 193
-                         chunk 256, seqlen 2048: 128 heads  35 /  32, 160 heads  37 /  40
-                         chunk  64, seqlen  512:  32 heads  14 /  12,  64 heads  14 /  17
-      bfloat16 backward, chunk 256, seqlen 8192: 160 heads 160 / 139, 192 heads 160 / 165
-      float32 forward,   chunk 256, seqlen 2048:  32 heads 130 /  24, 256 heads 145 / 139."""
+    The walk is a serial chain of 64-row stages, a workgroup per compute unit: 256 heads at a time, and its time
+    does not depend on how many of them there are.  The two launchers are bound by the chain of stages inside one
+    chunk while there are few heads, by the bytes they move (6 TB/s) and, in float32, by their matrix instructions.
+    The coefficients are fitted to 1840 measured points (MI355X; 2 to 768 heads, seqlen 500 to 8192, chunk 64 to
+    512, all four head and state sizes) with a root mean square error of 4 to 12 %.  Some of them, walk / two
+    launchers in us, hdim 64, dstate 128:
+      bfloat16 forward,  chunk 256, seqlen 8192:  32 heads 126 /  31, 128 heads 123 / 102, 192 heads 124 / 147,
+                                                  256 heads 129 / 187, 264 heads 235 / 201, 320 heads 236 / 244,
+                                                  512 heads 256 / 358, 768 heads 371 / 538
+                         chunk  64, seqlen  500:  32 heads  14 /  12,  64 heads  14 /  16
+                         chunk 512, seqlen  500:  32 heads  12 /  15, 192 heads  13 /  21
+      bfloat16 backward, chunk 256, seqlen 8192: 128 heads 151 / 117, 192 heads 154 / 167, 264 heads 291 / 223
+      float32 forward,   chunk 256, seqlen 2048:  32 heads 131 /  25, 256 heads 138 / 132, 384 heads 266 / 191.
+    Backward the two launchers take the host 25 us a call and the walk 20, so that a walk of less is kept."""
     heads = batch * nheads
     stages = -(-seqlen // 64)
     nchunks = -(-seqlen // chunk)
+    rounds = -(-heads // 256)
     state = headdim * dstate
     rel = state / 8192
-    if itemsize == 4:
-        stage_us = 1.0 + 3.0 * rel
-    elif headdim == 64 and dstate == 128:
-        stage_us = 1.17 if backward else 0.97
-    else:
-        stage_us = 0.5 + 0.85 * rel
-    walk_us = 4.0 + stages * stage_us * -(-heads // 256)
-    # chunk-local states written and read in float32, the carried ones written (and read, backward)
+    inner = -(-min(chunk, seqlen) // 64)  # stages of one chunk
+    # carried states: written forward; read and written backward
     nbytes = heads * (nchunks * state * (8 + itemsize * (2 if backward else 1)) + seqlen * headdim * itemsize)
-    pair_us = 6.0 + nbytes / 5e6
+    work = heads * seqlen * rel * 1e-6
     if itemsize == 4:
-        pair_us += 2 * heads * seqlen * state / 100e6
-    return walk_us < pair_us
+        walk_us = 5.8 + rounds * (stages * (0.41 + 2.95 * rel) + nchunks * 0.88 * rel)
+        pair_us = 5.5 + inner * (0.46 + 2.18 * rel) + nchunks * 0.11 + nbytes / 6.7e6 + 97 * work
+        if rel > 1:  # 128 x 128: fewer workgroups per compute unit
+            pair_us += heads * nchunks * 0.0144
+    else:
+        if headdim == 64 and dstate == 128:  # rows copied straight into LDS; other shapes go through registers
+            walk_us = 6.6 + rounds * (stages * 0.96 + nchunks * 0.9) if backward else \
+                5.0 + rounds * (stages * 0.87 + nchunks * 0.48)
+        else:
+            walk_us = 5.3 + rounds * (stages * (0.15 + 0.85 * rel) + nchunks * 0.81 * rel)
+        if backward:
+            pair_us = 9.5 + inner * 0.75 + nchunks * 0.17 + nbytes / 5.9e6 + 7.9 * work
+        else:
+            pair_us = 5.3 + inner * (0.73 + 0.32 * rel) + nchunks * 0.1 + nbytes / 6.1e6 + 5.3 * work
+    return walk_us < (max(pair_us, 25.0) if backward else pair_us)
