@@ -50,6 +50,34 @@ def _chunk_state_passing_fwd(B, x, dt, dA_cumsum, initial_states=None, out_dtype
     return states, final_states
 
 
+def _carried_states(B, x, dt, dA_cumsum, initial_states, seq_idx, out_dtype):
+    """(states entering each chunk, final_states) by the form that walk_pays() expects to be the faster, by the walk
+    also where there is no room for the chunk-local states of the two launchers."""
+    batch, seqlen, nheads, headdim = x.shape
+    chunk_size, dstate = dt.shape[-1], B.shape[-1]
+
+    def walk():
+        if seq_idx is not None or out_dtype not in (torch.float32, torch.bfloat16):
+            return None
+        return _chunk_state_passing_fwd(B, x, dt, dA_cumsum, initial_states=initial_states, out_dtype=out_dtype)
+
+    def two_launches():
+        states = _chunk_state_fwd(B, x, dt, dA_cumsum, seq_idx=seq_idx, states_in_fp32=True)
+        init = None if initial_states is None else initial_states.reshape(batch, nheads, headdim * dstate)
+        states, final_states = _state_passing_fwd(states.reshape(batch, -1, nheads, headdim * dstate),
+                                                  dA_cumsum[:, :, :, -1], initial_states=init, seq_idx=seq_idx,
+                                                  chunk_size=chunk_size, out_dtype=out_dtype)
+        return (states.reshape(batch, -1, nheads, headdim, dstate),
+                final_states.reshape(batch, nheads, headdim, dstate))
+
+    if not walk_pays(batch, nheads, seqlen, chunk_size, headdim, dstate, x.element_size()):
+        try:
+            return two_launches()
+        except torch.cuda.OutOfMemoryError:
+            pass
+    return walk() or two_launches()
+
+
 def _one_call(x, dt, B, C, z, chunk_size):
     """Whether the five stages run behind one entry point: one type throughout and shapes the kernels take."""
     return (x.dtype in (torch.float32, torch.bfloat16) and B.dtype == x.dtype and C.dtype == x.dtype
@@ -116,10 +144,13 @@ def _combined_one_call(x, dt, A, B, C, chunk_size, D, z, dt_bias, initial_states
 def _mamba_chunk_scan_combined_fwd(x, dt, A, B, C, chunk_size, D=None, z=None, dt_bias=None,
                                    initial_states=None, seq_idx=None, cu_seqlens=None, dt_softplus=False,
                                    dt_limit=(0.0, float("inf")), want_out_x=True):
-    """want_out_x=False leaves out_x (the result ahead of the gate) unwritten and returns None for it.  Returns (out, out_x, dt_out, dA_cumsum, states, final_states), states (the state entering
+    """Returns (out, out_x, dt_out, dA_cumsum, states, final_states), states (the state entering
     each chunk) in the dtype of C as in kernels/ema_combined.py:48-50, and as a seventh item the state
     at the end of each packed sequence when cu_seqlens is given (batch must be 1 then; the boundaries
-    are the ones seq_idx marks), as kernels/ema_combined.py:56-62 of the reference does."""
+    are the ones seq_idx marks), as kernels/ema_combined.py:56-62 of the reference does.
+    want_out_x=False returns None for out_x (the result ahead of the gate), which need not be written then.
+    Where walk_pays() chooses the two launchers, the chunk-local states take four bytes per state element of
+    scratch; if there is no room for them, the walk runs."""
     batch, seqlen, nheads, headdim = x.shape
     _, _, ngroups, dstate = B.shape
     assert nheads % ngroups == 0
@@ -130,26 +161,18 @@ def _mamba_chunk_scan_combined_fwd(x, dt, A, B, C, chunk_size, D=None, z=None, d
     if cu_seqlens is not None:
         assert batch == 1, "passing cu_seqlens to get the varlen states is only supported if batch dimension is 1"
     if _one_call(x, dt, B, C, z, chunk_size):
-        return _combined_one_call(x, dt, A, B, C, chunk_size, D, z, dt_bias, initial_states, seq_idx, cu_seqlens,
-                                  dt_softplus, dt_limit, want_out_x)
+        try:
+            return _combined_one_call(x, dt, A, B, C, chunk_size, D, z, dt_bias, initial_states, seq_idx, cu_seqlens,
+                                      dt_softplus, dt_limit, want_out_x)
+        except torch.cuda.OutOfMemoryError:
+            pass  # it holds everything at once (nothing is enqueued yet); the stages return their scratch one by one
     dA_cumsum, dt_out = _chunk_cumsum_fwd(dt, A, chunk_size, dt_bias=dt_bias, dt_softplus=dt_softplus,
                                           dt_limit=dt_limit)
-    fused = None
-    if (seq_idx is None and C.dtype in (torch.float32, torch.bfloat16)
-            and walk_pays(batch, nheads, seqlen, chunk_size, headdim, dstate, x.element_size())):
-        fused = _chunk_state_passing_fwd(B, x, dt_out, dA_cumsum, initial_states=initial_states, out_dtype=C.dtype)
-    if fused is not None:
-        states, final_states = fused
-    else:
-        states = _chunk_state_fwd(B, x, dt_out, dA_cumsum, seq_idx=seq_idx, states_in_fp32=True)
-        init = None if initial_states is None else initial_states.reshape(batch, nheads, headdim * dstate)
-        states, final_states = _state_passing_fwd(states.reshape(batch, -1, nheads, headdim * dstate),
-                                                  dA_cumsum[:, :, :, -1], initial_states=init, seq_idx=seq_idx,
-                                                  chunk_size=chunk_size, out_dtype=C.dtype)
-        states = states.reshape(batch, -1, nheads, headdim, dstate)
-        final_states = final_states.reshape(batch, nheads, headdim, dstate)
+    states, final_states = _carried_states(B, x, dt_out, dA_cumsum, initial_states, seq_idx, C.dtype)
     CB = _bmm_chunk_fwd(C, B, chunk_size, seq_idx=seq_idx, output_dtype=torch.float32)
     out, out_x = _chunk_scan_fwd(CB, x, dt_out, dA_cumsum, C, states, D=D, z=z, seq_idx=seq_idx)
+    if not want_out_x:
+        out_x = None
     if cu_seqlens is None:
         return out, out_x, dt_out, dA_cumsum, states, final_states
     varlen_states = chunk_state_varlen(B.squeeze(0), x.squeeze(0), dt_out.squeeze(0), dA_cumsum.squeeze(0),

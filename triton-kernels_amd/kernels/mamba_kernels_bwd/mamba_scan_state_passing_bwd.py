@@ -62,8 +62,8 @@ def _fused(C, dA_cumsum, dout, states, dfinal_states, has_initial_states, out_dt
 
 
 def _two_launches(C, dA_cumsum, dout, states, dfinal_states, has_initial_states, out_dtype):
-    """The same results from the two stages' own kernels with a float32 tensor between them (dstates bit for
-    bit), or None where _fused does not apply either."""
+    """The same results from the two stages' own kernels with a float32 tensor the size of states between them
+    (dstates bit for bit), or None where _fused does not apply either."""
     prep = _prepare(C, dA_cumsum, dout, states, dfinal_states, has_initial_states, out_dtype)
     if prep is None:
         return None
@@ -110,8 +110,15 @@ def _chunk_scan_state_passing_bwd(C, dA_cumsum, dout, states, dfinal_states=None
     out_dtype = dstates_dtype if dstates_dtype is not None else states.dtype
     if seq_idx is None:
         walk = walk_pays(batch, nheads, seqlen, chunk_size, headdim, dstate, dout.element_size(), backward=True)
-        both = (_fused if walk else _two_launches)(C, dA_cumsum, dout, states, dfinal_states, has_initial_states,
-                                                   out_dtype)
+        args = (C, dA_cumsum, dout, states, dfinal_states, has_initial_states, out_dtype)
+        both = None
+        if not walk:
+            try:
+                both = _two_launches(*args)
+            except torch.cuda.OutOfMemoryError:  # no room for the float32 tensor between the two: the walk needs none
+                walk = True
+        if walk:
+            both = _fused(*args)
         if both is not None:
             return both
     dim = headdim * dstate
