@@ -278,8 +278,8 @@ int ssd_chunk_state_varlen(const void* B, int64_t b_sl, int64_t b_sg, const void
  * and state passing (one walk per head, or, with local_states (batch, C, nheads, hdim, dstate) float32 given, the
  * two launchers; packed batches need it); bmm; chunk scan; and, with varlen_out given (batch 1), the states at the
  * sequence ends cu_seqlens names.  x, z, B, C, states and varlen_out are of `dtype`, final_states float32.  One
- * call from the host instead of five or six.  A refused stage ends the call with its status; the stages before
- * it have been enqueued by then. */
+ * call from the host instead of five or six.  Arguments that a stage would refuse are refused before the first
+ * one is enqueued. */
 int ssd_combined_fwd(const void* x, int64_t x_sb, int64_t x_sl, int64_t x_sh, int dtype, const void* dt, int dt_dtype,
                      int64_t dt_sb, int64_t dt_sl, int64_t dt_sh, const float* A, const float* dt_bias,
                      int dt_softplus, float dt_min, float dt_max, const void* B, int64_t b_sb, int64_t b_sl,

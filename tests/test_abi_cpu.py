@@ -152,6 +152,48 @@ def test_ssd_validation_happens_before_any_launch():
     assert rwalk(dout=[fake, 64 * 2 * 64, -2 * 64, 64]) == -5  # a reversed view: byte offsets are formed unsigned
 
 
+def test_one_call_forward_refuses_before_any_stage():
+    """Without a GPU the first launch fails with -6: any other status was found ahead of it."""
+    handle = _lib.lib()
+    fake = 0x1000
+
+    def fwd(dtype=1, dt=fake, dt_dtype=0, A=fake, x=fake, x_sl=2 * 64, B=fake, C=fake, z=None, initial=None, seq_idx=None,
+            cu=None, nseq=0, dt_out=fake, dA=fake, local=fake, states=fake, final=fake, cb=fake, out=fake, out_x=None,
+            varlen=None, batch=1, seqlen=64, nheads=2, ngroups=1, hdim=64, dstate=64, chunk=64):
+        seq = [64 * 2 * 64, 2 * 64, 64]
+        return handle.ssd_combined_fwd(
+            x, seq[0], x_sl, seq[2], dtype, dt, dt_dtype, 128, 2, 1, A, None, 0, 0.0, 1.0, B, 64 * 64, 64, 64, C,
+            64 * 64, 64, 64, None, 0, z, *seq, initial, seq_idx, 64, 1, cu, nseq, dt_out, dA, local, states, final, cb, out,
+            *seq, out_x, varlen, batch, seqlen, nheads, ngroups, hdim, dstate, chunk, None)
+
+    # the states at sequence ends: one packed row, its boundaries, as many sequences as a grid takes
+    ends = dict(varlen=fake, cu=fake, nseq=3)
+    assert fwd(**{**ends, "batch": 2}) == -2 and fwd(**{**ends, "cu": None}) == -1
+    assert fwd(**{**ends, "nseq": 0}) == -2 and fwd(**{**ends, "nseq": 65536}) == -2
+    # the walk: no packed batches, whole stages
+    assert fwd(local=None, seq_idx=fake) == -5 and fwd(local=None, chunk=48) == -5
+    # what the later stages refuse
+    assert fwd(hdim=96) == -5 and fwd(dstate=256) == -5 and fwd(chunk=62) == -5 and fwd(chunk=2048) == -5
+    assert fwd(nheads=3, ngroups=2) == -2 and fwd(dtype=7) == -4 and fwd(dt_dtype=7) == -4
+    assert fwd(x_sl=130) == -3 and fwd(z=fake + 2) == -3 and fwd(out_x=fake + 8) == -3 and fwd(initial=fake + 4) == -3
+    for name in ("dt", "A", "x", "B", "C", "dt_out", "dA", "states", "final", "cb", "out"):
+        assert fwd(**{name: None}) == -1, name
+    for name in ("x", "B", "C", "dt_out", "dA", "local", "states", "final", "cb", "out"):
+        assert fwd(**{name: fake + 4}) == -3, name
+
+
+def test_coefficient_packing_refuses_before_any_launch():
+    handle = _lib.lib()
+    fake = 0x1000
+
+    def pack(form=0, gradient=0, src=fake, dst=fake, ids=fake, starts=fake, batch=1, nheads=2, seqlen=8):
+        return handle.ema_coef_starts(form, gradient, src, 16, 2, 1, dst, 16, 2, 1, ids, 8, 1, starts, batch, nheads,
+                                      seqlen, None)
+
+    assert pack(form=5) == -5 and pack(batch=0) == -2 and pack(seqlen=0) == -2 and pack(nheads=0) == -2
+    assert pack(src=None) == -1 and pack(dst=None) == -1 and pack(starts=None) == -1 and pack(ids=None) == -1
+
+
 def test_error_mapping():
     with pytest.raises(AssertionError):
         _lib.check(-2, "x")

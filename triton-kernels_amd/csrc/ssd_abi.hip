@@ -733,9 +733,33 @@ int ssd_combined_fwd(const void* x, int64_t x_sb, int64_t x_sl, int64_t x_sh, in
                      float* cb, void* out, int64_t o_sb, int64_t o_sl, int64_t o_sh, void* out_x, void* varlen_out,
                      int64_t batch, int64_t seqlen, int64_t nheads, int64_t ngroups, int64_t hdim, int64_t dstate,
                      int64_t chunk, void* stream) {
+  // everything that a stage would refuse, before the first one is enqueued
+  Dims d;
+  SSD_TRY(check_dims(batch, seqlen, nheads, ngroups, hdim, dstate, chunk, &d));
+  SSD_TRY(check_dtype(dtype));
+  SSD_TRY(check_dtype(dt_dtype));
+  if (!dim_ok(hdim) || !dim_ok(dstate)) return SSD_ERR_UNSUPPORTED;
+  // the walk knows no packed batches and takes whole 64-row stages
+  if (!local_states && (seq_idx || chunk % 64)) return SSD_ERR_UNSUPPORTED;
+  if (varlen_out && (batch != 1 || nseq <= 0 || nseq > 65535)) return SSD_ERR_SHAPE;
+  if (varlen_out && !cu_seqlens) return SSD_ERR_NULL;
+  if (!dt || !A) return SSD_ERR_NULL;
+  SSD_TRY(check_vec(x, x_sb, x_sl, x_sh, dtype, hdim));
+  SSD_TRY(check_vec(B, b_sb, b_sl, b_sg, dtype, dstate));
+  SSD_TRY(check_vec(C, c_sb, c_sl, c_sg, dtype, dstate));
+  SSD_TRY(check_vec(out, o_sb, o_sl, o_sh, dtype, hdim));
+  if (z) SSD_TRY(check_vec(z, z_sb, z_sl, z_sh, dtype, hdim));
+  if (out_x && reinterpret_cast<uintptr_t>(out_x) % 16) return SSD_ERR_ALIGN;
+  for (const void* p : {(const void*)dt_out, (const void*)dA_cumsum, (const void*)states, (const void*)final_states, (const void*)cb})
+    SSD_TRY(check_f32(p));
+  if (local_states) SSD_TRY(check_f32(local_states));
+  if (initial) SSD_TRY(check_f32(initial));
+  const int64_t C_ = d.C, tiles = (chunk + 63) / 64;
+  if (batch * C_ * nheads * tiles > 0x7fffffff || batch * C_ * ngroups * tiles * tiles > 0x7fffffff ||
+      batch * nheads * ((hdim * dstate + 1023) / 1024) > 0x7fffffff)
+    return SSD_ERR_SHAPE;
   SSD_TRY(ssd_chunk_cumsum_fwd(dt, dt_dtype, dt_sb, dt_sl, dt_sh, A, dt_bias, dA_cumsum, dt_out, batch, seqlen,
                                nheads, chunk, dt_softplus, dt_min, dt_max, stream));
-  const int64_t C_ = (seqlen + chunk - 1) / chunk;
   if (local_states) {
     SSD_TRY(ssd_chunk_state_fwd(B, b_sb, b_sl, b_sg, x, x_sb, x_sl, x_sh, dtype, dt_out, dA_cumsum, local_states,
                                 batch, seqlen, nheads, ngroups, hdim, dstate, chunk, seq_idx, seq_sb, seq_sl, stream));
@@ -743,7 +767,6 @@ int ssd_combined_fwd(const void* x, int64_t x_sb, int64_t x_sl, int64_t x_sh, in
                                   initial, states, dtype, final_states, batch, C_, nheads, hdim * dstate, seq_idx,
                                   seq_sb, seq_sl, seqlen, chunk, stream));
   } else {
-    if (seq_idx) return SSD_ERR_UNSUPPORTED;  // the walk knows no packed batches
     SSD_TRY(ssd_chunk_state_passing_fwd(B, b_sb, b_sl, b_sg, x, x_sb, x_sl, x_sh, dtype, dt_out, dA_cumsum, initial,
                                         states, dtype, final_states, batch, seqlen, nheads, ngroups, hdim, dstate,
                                         chunk, stream));
