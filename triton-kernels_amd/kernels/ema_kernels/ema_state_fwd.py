@@ -24,7 +24,7 @@ def _ema_chunk_state_fwd(x, A_cumsum, seq_idx=None, states=None, states_in_fp32=
     out = None
     if states is not None:
         assert states.shape == (batch * nh, nchunks, token_dim)
-        if states.dtype == torch.float32 and states.is_contiguous():
+        if states.dtype == torch.float32 and states.is_contiguous() and states.device == dev:
             out = states
     if out is None:
         out = torch.empty((batch * nh, nchunks, token_dim), device=dev, dtype=torch.float32)

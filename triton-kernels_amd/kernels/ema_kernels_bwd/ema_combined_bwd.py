@@ -19,7 +19,7 @@ def _ema_chunk_scan_combined_bwd(dout, x, A, chunk_size, dt_limit=(0.0, float("i
     Returns (dx, ddA) with ddA (N, nchunks, chunk_size) float32, ddA[n, c, q] = dL/dA at
     position c * chunk_size + q of sequence n; with recompute_output also the forward
     output."""
-    dev = _lib.require_gpu(dout, x, A)
+    dev = _lib.require_gpu(dout, x, A, prev128)
     x, x_args, batch, nh, seqlen, token_dim = _lib.seq_view(x)
     if dout.dtype != x.dtype:
         dout = dout.to(x.dtype)

@@ -34,7 +34,7 @@ def ema_seq_fwd(coef, x, form="log_decay", initial_states=None, kernel_events=No
     """Forward pass.  Returns (y, final_states, prev128); prev128 (N, ceil(L/128), T) float32 is
     what ema_seq_bwd needs from the forward.  workspace: optional (uint8 buffer, ready flag) to
     use instead of the device's shared one."""
-    dev = _lib.require_gpu(x, coef)
+    dev = _lib.require_gpu(x, coef, initial_states)
     x, xs, batch, nh, L, T = _lib.seq_view(x)
     cs_, cb, cnh, cL = _lib.decay_view(coef)
     assert (cb, cnh, cL) == (batch, nh, L), "coefficient and x disagree in (batch, heads, length)"
@@ -63,7 +63,7 @@ def ema_seq_bwd(dy, x, coef, prev128, form="log_decay", dfinal_states=None, want
                 kernel_events=None, workspace=None):
     """Backward pass.  Returns (dx, dcoef, dinitial_states or None).  workspace: optional
     (uint8 buffer, ready flag) to use instead of the device's shared one."""
-    dev = _lib.require_gpu(dy, x, coef, prev128)
+    dev = _lib.require_gpu(dy, x, coef, prev128, dfinal_states)
     x, xs, batch, nh, L, T = _lib.seq_view(x)
     if dy.dtype != x.dtype:
         dy = dy.to(x.dtype)

@@ -29,7 +29,7 @@ def _chunk_state_passing_fwd(B, x, dt, dA_cumsum, initial_states=None, out_dtype
     if (chunk_size % 64 or headdim not in (64, 128) or dstate not in (64, 128)
             or x.dtype not in (torch.float32, torch.bfloat16) or out_dtype not in (torch.float32, torch.bfloat16)):
         return None
-    dev = _lib.require_gpu(x, B, dt, dA_cumsum)
+    dev = _lib.require_gpu(x, B, dt, dA_cumsum, initial_states)
     if B.dtype != x.dtype:
         B = B.to(x.dtype)
     x, xs = _lib.strided4(x)
@@ -96,7 +96,7 @@ def _combined_one_call(x, dt, A, B, C, chunk_size, D, z, dt_bias, initial_states
         assert dt_bias.shape == (nheads,)
     if D is not None:
         assert D.shape == (nheads, headdim) or D.shape == (nheads,)
-    dev = _lib.require_gpu(x, dt, A, B, C)
+    dev = _lib.require_gpu(x, dt, A, B, C, D, z, dt_bias, initial_states)
     ids, id_args = _lib.seq_ids(seq_idx, batch, seqlen, dev)
     x, xs = _lib.strided4(x)
     B, bs = _lib.strided4(B)

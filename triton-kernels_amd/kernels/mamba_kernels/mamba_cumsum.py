@@ -15,7 +15,7 @@ def _chunk_cumsum_fwd(dt, A, chunk_size, dt_bias=None, dt_softplus=False, dt_lim
     assert A.shape == (nheads,)
     if dt_bias is not None:
         assert dt_bias.shape == (nheads,)
-    dev = _lib.require_gpu(dt, A)
+    dev = _lib.require_gpu(dt, A, dt_bias)
     if dt.dtype not in (torch.float32, torch.bfloat16):
         dt = dt.float()
     nchunks = math.ceil(seqlen / chunk_size)

@@ -27,7 +27,7 @@ def _chunk_scan_fwd(cb, x, dt, dA_cumsum, C, states, D=None, z=None, seq_idx=Non
         out, out_x = _chunk_scan_fwd(cb, plan.x(x), plan.per_head(dt), plan.per_head(dA_cumsum), plan.bc(C),
                                      plan.states(states), D=plan.D(D), z=plan.x(z), seq_idx=seq_idx)
         return plan.x_back(out), plan.x_back(out_x)
-    dev = _lib.require_gpu(x, cb, dt, dA_cumsum, C, states)
+    dev = _lib.require_gpu(x, cb, dt, dA_cumsum, C, states, D, z)
     seq_idx, ids = _lib.seq_ids(seq_idx, batch, seqlen, dev)
     x, xs = _lib.strided4(x)
     if C.dtype != x.dtype:

@@ -19,7 +19,7 @@ def _state_passing_fwd(states, dA_chunk_cumsum, initial_states=None, seq_idx=Non
                                         None if initial_states is None else F.pad(initial_states, pad),
                                         seq_idx=seq_idx, chunk_size=chunk_size, out_dtype=out_dtype)
         return out[..., :dim], final[..., :dim]
-    dev = _lib.require_gpu(states, dA_chunk_cumsum)
+    dev = _lib.require_gpu(states, dA_chunk_cumsum, initial_states)
     seqlen = 0
     if seq_idx is not None:
         assert chunk_size is not None

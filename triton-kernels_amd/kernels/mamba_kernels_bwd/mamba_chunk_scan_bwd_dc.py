@@ -23,7 +23,7 @@ def _chunk_scan_bwd_dC(prev_states, dA_cumsum, dout, seq_idx=None, C=None, ngrou
         if C is None:
             return plan.bc_back(res)
         return plan.bc_back(res[0]), plan.per_head_sum(res[1])
-    dev = _lib.require_gpu(prev_states, dA_cumsum, dout)
+    dev = _lib.require_gpu(prev_states, dA_cumsum, dout, C)
     seq_idx, ids = _lib.seq_ids(seq_idx, batch, seqlen, dev)
     dout, ds = _lib.strided4(dout)
     cs = [None, 0, 0, 0]

@@ -30,7 +30,7 @@ def _chunk_scan_chunk_state_bwd_dx(x, dt, dA_cumsum, B, CB, dout, dstates, D=Non
         return plan.x_back(dxs), plan.per_head_sum(ddt), plan.dD_back(dD, D)
     if D is not None:
         assert D.shape == (nheads, headdim) or D.shape == (nheads,)
-    dev = _lib.require_gpu(x, dt, dA_cumsum, B, CB, dout, dstates)
+    dev = _lib.require_gpu(x, dt, dA_cumsum, B, CB, dout, dstates, D, dx)
     seq_idx, ids = _lib.seq_ids(seq_idx, batch, seqlen, dev)
     x, xs = _lib.strided4(x)
     dout, ds = _lib.strided4(dout.to(x.dtype))

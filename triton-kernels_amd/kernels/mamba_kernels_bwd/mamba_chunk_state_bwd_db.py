@@ -23,7 +23,7 @@ def _chunk_state_bwd_db(x, dt, dA_cumsum, dstates, seq_idx=None, B=None, ngroups
         if B is None:
             return plan.bc_back(res)
         return plan.bc_back(res[0]), plan.per_head_sum(res[1])
-    dev = _lib.require_gpu(x, dt, dA_cumsum, dstates)
+    dev = _lib.require_gpu(x, dt, dA_cumsum, dstates, B)
     seq_idx, ids = _lib.seq_ids(seq_idx, batch, seqlen, dev)
     x, xs = _lib.strided4(x)
     bs = [None, 0, 0, 0]

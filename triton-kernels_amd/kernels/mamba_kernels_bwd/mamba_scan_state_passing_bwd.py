@@ -21,7 +21,7 @@ def _prepare(C, dA_cumsum, dout, states, dfinal_states, has_initial_states, out_
     if (headdim != 64 or dstate != 128 or chunk_size % 64 or chunk_size < 128 or dout.dtype != torch.bfloat16
             or states.dtype != torch.bfloat16 or out_dtype not in (torch.float32, torch.bfloat16)):
         return None
-    dev = _lib.require_gpu(C, dA_cumsum, dout, states)
+    dev = _lib.require_gpu(C, dA_cumsum, dout, states, dfinal_states)
     if C.dtype != dout.dtype:
         C = C.to(dout.dtype)
     dout, ds = _lib.strided4(dout)

@@ -25,7 +25,7 @@ def _state_passing_bwd(states, dA_chunk_cumsum, dout, dfinal_states=None, seq_id
         return (cut(res[0]), res[1], cut(res[2])) + tuple(cut(t) for t in res[3:])
     if dfinal_states is not None:
         assert dfinal_states.shape == (batch, nheads, dim)
-    dev = _lib.require_gpu(states, dA_chunk_cumsum, dout)
+    dev = _lib.require_gpu(states, dA_chunk_cumsum, dout, dfinal_states)
     lib = _lib.lib()
     seqlen = 0
     if seq_idx is not None:
