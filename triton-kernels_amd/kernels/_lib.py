@@ -150,12 +150,12 @@ def stream_ptr(dev: torch.device) -> int:
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if dev.index is None else dev.index)
 
 
-_HERE = contextlib.nullcontext()
+_NO_SWITCH = contextlib.nullcontext()
 
 
 def on_device(dev: torch.device):
     """Context in which `dev` is the current device; switches only where it is not already."""
-    return _HERE if dev.index is None or torch.cuda.current_device() == dev.index else torch.cuda.device(dev)
+    return _NO_SWITCH if dev.index is None or torch.cuda.current_device() == dev.index else torch.cuda.device(dev)
 
 
 def seq_view(x: torch.Tensor):
