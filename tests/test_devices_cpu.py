@@ -1,5 +1,6 @@
-"""Every tensor whose address reaches a kernel must be on the GPU of the others.  Fake tensors stand for those on
-the GPU, so that the refusals (which come ahead of any use of an address) can be exercised without one."""
+"""Every tensor whose address reaches a kernel must be on the GPU of the others and of the shape the kernel assumes.
+Fake tensors stand for those on the GPU, so that the refusals (which come ahead of any use of an address) can be
+exercised without one."""
 import pytest
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
@@ -109,3 +110,30 @@ def test_a_tensor_left_on_the_host_is_refused(call, name):
     with FakeTensorMode(), pytest.raises(AssertionError, match="same device"):
         call(operand)
     assert name in seen
+
+
+@pytest.mark.parametrize("wrong,shape", [("C", (1, 256, g, N)), ("C", (2, 192, g, N)), ("dA", (1, nh, 2, 128)),
+                                         ("dA", (1, nh, 1, 256)), ("dA", (2, nh, 3, 128))])
+def test_reverse_walk_refuses_operands_of_other_shapes(wrong, shape):
+    """The kernels index C and dA_cumsum by dout's batch, length and heads."""
+    from kernels.mamba_kernels_bwd.mamba_scan_state_passing_bwd import _chunk_scan_state_passing_bwd
+
+    shapes = dict(C=(2, 256, g, N), dA=(2, nh, 2, 128))
+    shapes[wrong] = shape
+    with FakeTensorMode(), pytest.raises(AssertionError):
+        o = lambda *s, dtype=BF16: torch.empty(*s, dtype=dtype, device="cuda:0")
+        _chunk_scan_state_passing_bwd(o(*shapes["C"]), o(*shapes["dA"], dtype=F32), o(2, 256, nh, P),
+                                      o(2, shapes["dA"][2], nh, P, N))
+
+
+@pytest.mark.parametrize("wrong,shape", [("B", (1, 256, g, N)), ("B", (2, 192, g, N)), ("dt", (2, nh, 2, 64)),
+                                         ("dt", (1, nh, 4, 64)), ("init", (1, nh, P, N))])
+def test_state_walk_refuses_operands_of_other_shapes(wrong, shape):
+    from kernels.mamba_kernels.mamba_combined_fwd import _chunk_state_passing_fwd
+
+    shapes = dict(B=(2, 256, g, N), dt=(2, nh, 4, 64), init=(2, nh, P, N))
+    shapes[wrong] = shape
+    with FakeTensorMode(), pytest.raises(AssertionError):
+        o = lambda *s: torch.empty(*s, device="cuda:0")
+        _chunk_state_passing_fwd(o(*shapes["B"]), o(2, 256, nh, P), o(*shapes["dt"]), o(2, nh, 4, 64),
+                                 initial_states=o(*shapes["init"]))

@@ -25,6 +25,11 @@ def _chunk_state_passing_fwd(B, x, dt, dA_cumsum, initial_states=None, out_dtype
     batch, seqlen, nheads, headdim = x.shape
     _, _, nchunks, chunk_size = dt.shape
     _, _, ngroups, dstate = B.shape
+    assert nheads % ngroups == 0 and nchunks == -(-seqlen // chunk_size)
+    assert B.shape == (batch, seqlen, ngroups, dstate)
+    assert dt.shape == (batch, nheads, nchunks, chunk_size) and dA_cumsum.shape == dt.shape
+    if initial_states is not None:
+        assert initial_states.shape == (batch, nheads, headdim, dstate)
     out_dtype = torch.float32 if out_dtype is None else out_dtype
     if (chunk_size % 64 or headdim not in (64, 128) or dstate not in (64, 128)
             or x.dtype not in (torch.float32, torch.bfloat16) or out_dtype not in (torch.float32, torch.bfloat16)):

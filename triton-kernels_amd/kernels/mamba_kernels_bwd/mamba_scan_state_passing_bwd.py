@@ -104,6 +104,9 @@ def _chunk_scan_state_passing_bwd(C, dA_cumsum, dout, states, dfinal_states=None
     batch, seqlen, nheads, headdim = dout.shape
     _, _, nchunks, chunk_size = dA_cumsum.shape
     _, _, ngroups, dstate = C.shape
+    assert nheads % ngroups == 0 and nchunks == -(-seqlen // chunk_size)
+    assert C.shape == (batch, seqlen, ngroups, dstate)
+    assert dA_cumsum.shape == (batch, nheads, nchunks, chunk_size)
     assert states.shape == (batch, nchunks, nheads, headdim, dstate)
     if dfinal_states is not None:
         assert dfinal_states.shape == (batch, nheads, headdim, dstate)
