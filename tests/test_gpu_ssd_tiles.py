@@ -10,6 +10,13 @@ from parity_util import announce, check_close
 F32, BF16 = torch.float32, torch.bfloat16
 
 
+def one_tile_batch(Q, L, nh, P, dtype):
+    """The batch at which the kernels of one tile per chunk take over: more than 128 chunks in float32; in bfloat16 384
+    single heads of 128 features or pairs of heads of 64, more than 512 pairs with chunks of 64 rows."""
+    from_ = 129 if dtype == F32 else 513 if Q == 64 and P == 64 else 384
+    return -(-from_ // (-(-L // Q) * (nh // 2 if P == 64 and dtype == BF16 else nh)))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["decay", "rise", "mixed"])
 @pytest.mark.parametrize("nh,g,P,dtype", [(4, 1, 64, BF16), (6, 3, 64, BF16), (2, 1, 128, BF16), (3, 1, 64, F32),
@@ -22,8 +29,7 @@ def test_chunk_scan_one_tile_vs_oracle(Q, L, nh, g, P, dtype, kind, device):
 
     announce(f"chunk scan Q={Q} L={L} nh={nh} g={g} P={P} {dtype} {kind}")
     N = 64 if P == 128 else 128
-    # in bfloat16 the kernel takes over at 384 workgroups (pairs of heads of 64 features, single heads of 128)
-    b = 2 if dtype == F32 else -(-384 // (-(-L // Q) * (nh // 2 if P == 64 else nh)))
+    b = one_tile_batch(Q, L, nh, P, dtype)
     gen = torch.Generator().manual_seed(Q + L + nh)
     r = lambda *s: torch.randn(*s, generator=gen)
     x, C, z = r(b, L, nh, P).to(dtype), r(b, L, g, N).to(dtype), r(b, L, nh, P).to(dtype)
@@ -173,7 +179,7 @@ def test_dx_one_tile_vs_oracle(Q, L, nh, g, N, kind, device):
 
     announce(f"dx Q={Q} L={L} nh={nh} g={g} N={N} {kind}")
     P, dtype = 64, BF16
-    b = -(-384 // (-(-L // Q) * (nh // 2)))  # the kernel takes over at 384 pairs of heads
+    b = one_tile_batch(Q, L, nh, P, dtype)
     gen = torch.Generator().manual_seed(Q + L + nh)
     r = lambda *s: torch.randn(*s, generator=gen)
     x, dout, B = r(b, L, nh, P).to(dtype), r(b, L, nh, P).to(dtype), r(b, L, g, N).to(dtype)

@@ -136,14 +136,15 @@ struct DxLaunch {
     }
     if constexpr (P == 64 && sizeof(T) == 2) {
       // Chunks of 64 or 128 rows with two adjacent dense heads of a group per workgroup, rows at 32-bit byte offsets,
-      // and enough of them.  The 64-row kernel / this one, us, dstate 128: b8 nh32 L8192 chunk
-      // 128 443 / 279, chunk 64 352 / 274; b1 nh24 L5000 chunk 128 (480 pairs) 26 / 20; b1 nh8 L2000 chunk 64
-      // dstate 64 (128 pairs) 6.6 / 7.7.
+      // and enough of them.  The 64-row kernel / this one, us, dstate 128, inputs from memory: b8 nh32 L8192 chunk
+      // 128 443 / 279, chunk 64 352 / 274; chunk 128 384 pairs 22.3 / 20.0, 512 25.5 / 22.4; chunk 64 384 pairs
+      // 11.5 / 12.3, 512 13.0 / 14.0, 576 17.0 / 14.2; b1 nh8 L2000 chunk 64 dstate 64 (128 pairs) 6.6 / 7.7.
       auto near = [&](const Strides3& s) { return forward_strides(s) && s.sl * d.Q < (int64_t(1) << 28); };
       const bool dense = sx.sh == P && sd.sh == P && sdx.sh == P && (d.nh / d.g) % 2 == 0;
-      if (dense && near(sx) && near(sd) && near(sB) && near(sdx) && d.batch * d.C * (d.nh / 2) >= kMidWorkgroups) {
-        if (d.Q == 128) return launch_mid<T, P, N, TS, 128>();
-        if (d.Q == 64) return launch_mid<T, P, N, TS, 64>();
+      const int64_t pairs = d.batch * d.C * (d.nh / 2);
+      if (dense && near(sx) && near(sd) && near(sB) && near(sdx)) {
+        if (d.Q == 128 && pairs >= kMidWorkgroups) return launch_mid<T, P, N, TS, 128>();
+        if (d.Q == 64 && pairs >= kMidDxPairs64) return launch_mid<T, P, N, TS, 64>();
       }
     }
     auto kernel = ssd_chunk_scan_bwd_dx_kernel<T, P, N, TS>;

@@ -67,8 +67,12 @@ inline int check_seq_chunks(const int32_t* seq_idx, int64_t seqlen, int64_t chun
 inline SeqIdx as_seq(const int32_t* p, int64_t sb, int64_t sl) { return SeqIdx{p, sb, sl}; }
 constexpr int kLdsBytes = 160 * 1024;  // LDS of one CU
 // Workgroups from which the one-tile kernels of chunks of 64 and 128 rows pay in bfloat16 (one and a half for each
-// of 256 compute units; measured at the rules that use it).
-constexpr int64_t kMidWorkgroups = 384;
+// of 256 compute units; measured at the rules that use it), and for pairs of heads and chunks of 64 rows, where the
+// 64-row kernels have only twice the workgroups: from where those no longer run at once, three on each compute unit
+// in the chunk scan and four in dx.
+constexpr int64_t kMidWorkgroups = 384, kMidScanPairs64 = 385, kMidDxPairs64 = 513;
+// Workgroups of float32 chunks of 128 rows up to which both workgroups of the 64-row kernel run at once.
+constexpr int64_t kBoth64Row = 128;
 
 template <typename K>
 int allow_smem(K kernel, int bytes) {

@@ -54,22 +54,28 @@ struct ScanLaunch {
   // Chunks of 64 or 128 rows in one tile.  Two adjacent heads of a group per workgroup where they are adjacent
   // in memory too (dense heads of 64 features): they share the fragments of cb and the rows of C.  A single
   // bfloat16 head of 64 features leaves each wave one column block for the weights it forms, and the 64-row
-  // kernel is the faster one (17 heads, L 4096, b2, chunk 128: 29.0 against 32.4 us); so it is in bfloat16 while
-  // the workgroups do not fill the chip (b1 nh8 L2000 chunk 128, 64 pairs: 8.0 against 9.6 us; b2 nh16 L1092 chunk
-  // 64, 288 pairs: 8.7 against 9.7; b1 nh24 L5000 chunk 128, 480 pairs: 27 against 17).  The 64-row kernel / this
-  // one otherwise, us at dstate 128: bfloat16 b8 nh32 L8192 hdim 64 chunk 128 437 / 260, chunk 64 334 / 240; b2
-  // nh16 L4096 hdim 128 chunk 128 41 / 38; float32 b1 nh16 L4096 chunk 128 hdim 64 35 / 26, hdim 128 70 / 40.
+  // kernel is the faster one (17 heads, L 4096, b2, chunk 128: 29.0 against 32.4 us); so it is while the workgroups
+  // do not fill the chip.  The 64-row kernel / this one, us at dstate 128, inputs from memory:
+  //   bfloat16 hdim 64, pairs   chunk 128: 64 pairs 8.0 / 9.6, 384 20.5 / 17.3, 512 27.5 / 18.8; b8 nh32 L8192 437 / 260
+  //                             chunk 64: 384 pairs 10.0 / 11.3, 416 14.1 / 11.5; b8 nh32 L8192 334 / 240
+  //   bfloat16 hdim 128         chunk 128: 384 20.9 / 17.4, 1024 51 / 39; chunk 64: 384 10.5 / 10.8, 576 16.8 / 13.9
+  //   float32 chunk 128         hdim 64: 16 11.3 / 15.8, 128 14.8 / 17.1, 192 19.0 / 17.6, 1024 74 / 54; hdim 128:
+  //                             128 20.4 / 24.4, 192 36 / 26 (two workgroups of 64 rows are the shorter chain while
+  //                             both run at once); chunk 64: level up to 128, hdim 64 256 11.8 / 10.5, 1024 31 / 25
   template <typename T, int P, int N, typename TS, int ST>
   int launch_mid_pairs(bool* taken) const {
     *taken = true;
     if constexpr (sizeof(T) == 2) {
       constexpr int HP = P == 64 ? 2 : 1;
       const bool pairs = sx.sh == P && so.sh == P && (!z || sz.sh == P) && (d.nh / d.g) % 2 == 0;
-      if ((HP == 1 || pairs) && d.batch * d.C * (d.nh / HP) >= kMidWorkgroups) return launch_mid<T, P, N, TS, HP, ST>();
+      constexpr int64_t from = HP == 2 && ST == 64 ? kMidScanPairs64 : kMidWorkgroups;
+      if ((HP == 1 || pairs) && d.batch * d.C * (d.nh / HP) >= from) return launch_mid<T, P, N, TS, HP, ST>();
       *taken = false;
       return SSD_OK;
     } else {
-      return launch_mid<T, P, N, TS, 1, ST>();
+      if (ST == 64 || d.batch * d.C * d.nh > kBoth64Row) return launch_mid<T, P, N, TS, 1, ST>();
+      *taken = false;
+      return SSD_OK;
     }
   }
   template <typename T, int P, int N, typename TS>
