@@ -205,3 +205,30 @@ def test_dx_one_tile_vs_oracle(Q, L, nh, g, N, kind, device):
         check_close("ddt", got[1], ref[1], dtype, loose=True)
         if D is not None:
             check_close("dD", got[2], ref[2], F32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("b,nh", [(1, 4), (128, 8)])  # single heads, and 1024 pairs of heads
+def test_chunk_scan_of_rows_far_apart(b, nh, device):
+    """x, z and C whose positions lie megabytes apart (position-major tensors of a large batch): strides only change
+    addresses, so the result is that of contiguous copies bit for bit."""
+    from kernels.mamba_kernels.mamba_scan_fwd import _chunk_scan_fwd
+
+    announce(f"chunk scan, rows far apart, b{b} nh{nh}")
+    L, P, N, Q, far = 300, 64, 128, 256, 1 << 21
+    gen = torch.Generator(device=device).manual_seed(3)
+    r = lambda *s: torch.randn(*s, generator=gen, device=device)
+    x, z, C = r(b, L, nh, P).to(BF16), r(b, L, nh, P).to(BF16), r(b, L, 1, N).to(BF16)
+    buf = torch.empty(L, far, device=device, dtype=BF16)
+    size = b * nh * P
+    views = []
+    for i, t in enumerate((x, z, C)):
+        v = buf[:, i * size: i * size + t[:, 0].numel()].view(L, b, *t.shape[2:]).transpose(0, 1)
+        views.append(v.copy_(t))
+        assert v.stride(1) == far
+    dA = (-torch.rand(b, nh, 2, Q, generator=gen, device=device) * 0.2).cumsum(-1)
+    cb, states, dt = r(b, 2, 1, Q, Q), r(b, 2, nh, P, N).to(BF16), torch.rand(b, nh, 2, Q, generator=gen, device=device)
+    D = r(nh)
+    want = _chunk_scan_fwd(cb, x, dt, dA, C, states, D=D, z=z)
+    got = _chunk_scan_fwd(cb, views[0], dt, dA, views[2], states, D=D, z=views[1])
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])

@@ -2012,7 +2012,6 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_scan_wide_kernel(
   const TS* pg = prev + (((b * C + c) * nh + h) * (int64_t)P) * N;
   const float* cbg = cb + (((b * C + c) * ngroups + g) * (int64_t)Q) * Q;
 
-  const unsigned xrow = (unsigned)(sx.sl * sizeof(T));
   int mrow[2];
   mrow[0] = 32 * wave;
   mrow[1] = 32 * (7 - wave);
@@ -2029,7 +2028,9 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_scan_wide_kernel(
   static_assert(S::kPrev <= (ST / 2) * S::PX * (int)sizeof(T), "the carried state must leave the upper half of the x tile free");
   constexpr bool kEarly = (ST / 2) * (PW / EPL) / 256 <= 8;  // (eight pieces per thread travel in registers)
   RowPieces<T, kEarly ? ST / 2 : 32, kEarly ? PW : EPL * 8, S::PX> upper;
-  if constexpr (kEarly) upper.template load32<true>(xg, xrow, ST / 2, limit, tid);
+  // (a pair works at the register limit: rows at 32-bit byte offsets, see the host)
+  if constexpr (kEarly && HP == 2) upper.template load32<true>(xg, (unsigned)(sx.sl * sizeof(T)), ST / 2, limit, tid);
+  else if constexpr (kEarly) upper.template load<true>(xg, sx.sl, ST / 2, limit, tid);
   // ---- phase A: C . prev, scaled by exp(dA_m)
   {
     constexpr int VPR = N / 4;

@@ -81,21 +81,23 @@ struct ScanLaunch {
   template <typename T, int P, int N, typename TS>
   int run_as() const {
     constexpr int wide_smem = WideSmem<T, P, N>::kBytes;
-    const bool close = near(sx) && near(sC) && near(so) && (!z || near(sz));
-    if (d.Q % 256 == 0 && wide_smem <= kLdsBytes && close) {  // 256-row super-tiles, no barrier inside the k loop
+    if (d.Q % 256 == 0 && wide_smem <= kLdsBytes) {  // 256-row super-tiles, no barrier inside the k loop
       // Two adjacent heads of a group per workgroup where they are adjacent in memory too (dense
-      // heads of 64 features): they share the fragments of cb and the rows of C.
+      // heads of 64 features): they share the fragments of cb and the rows of C.  Their first x tile
+      // is read at 32-bit byte offsets; single heads take any stride.
       if constexpr (P == 64 && WideSmem<T, 128, N>::bytes_for(2) <= kLdsBytes / 2) {
         // Pairs take 256 registers, two workgroups per compute unit: with fewer than 512 of them most waves a
         // compute unit could hold are missing, and single heads (twice the workgroups) are faster.  Pairs /
         // single heads, us, with gate, nh32 dstate 128 chunk 256: L2048 29.0 / 18.9, L4096 37.3 / 30.7, L8192
         // (512 pairs) 47.5 / 57.6.
         const bool dense = sx.sh == P && so.sh == P && (!z || sz.sh == P);
-        if (dense && (d.nh / d.g) % 2 == 0 && d.batch * d.C * (d.nh / 2) * (d.Q / 256) >= 512)
+        const bool offsets32 = sx.sl >= 0 && sx.sl <= (int64_t(1) << 32) / (256 * (int64_t)sizeof(T));
+        if (dense && offsets32 && (d.nh / d.g) % 2 == 0 && d.batch * d.C * (d.nh / 2) * (d.Q / 256) >= 512)
           return launch_wide<T, P, N, TS, 2>();
       }
       return launch_wide<T, P, N, TS, 1>();
     }
+    const bool close = near(sx) && near(sC) && near(so) && (!z || near(sz));
     if ((d.Q == 64 || d.Q == 128) && close) {
       bool taken;
       const int status = d.Q == 128 ? launch_mid_pairs<T, P, N, TS, 128>(&taken) : launch_mid_pairs<T, P, N, TS, 64>(&taken);
