@@ -37,6 +37,24 @@ def test_short_forward_vs_oracle(L, b, nh, d, dtype, form, device):
 
 
 @pytest.mark.parametrize("form", ["log_decay", "probability"])
+@pytest.mark.parametrize("dtype", [F32, BF16], ids=["f32", "bf16"])
+def test_short_forward_against_the_tile_kernel(dtype, form, device):
+    """Rows 1 to 8 are the tile kernel's bit for bit (the first group of rows of a wave); those beyond, which it forms
+    from the group's product and sum, agree to rounding."""
+    from kernels.ema_seq import ema_seq_fwd
+
+    b, L, nh, d = 2, 17, 3, 520
+    gen = torch.Generator(device=device).manual_seed(2)
+    x = torch.randn(b, L, nh, d, generator=gen, device=device).to(dtype)
+    coef = torch.rand(b, L, nh, generator=gen, device=device)
+    coef = -coef if form == "log_decay" else coef
+    tile, _, _ = ema_seq_fwd(coef, x, form)
+    short, _, _ = ema_seq_fwd(coef[:, :16], x[:, :16], form)
+    assert torch.equal(short[:, :8], tile[:, :8])
+    check_close("rows 9 to 16", short[:, 8:], tile[:, 8:16].cpu(), dtype)
+
+
+@pytest.mark.parametrize("form", ["log_decay", "probability"])
 @pytest.mark.parametrize("layout", ["flat", "headed", "permuted", "expanded"])
 def test_packing_in_one_launch_equals_tensor_operations(layout, form, device):
     """int32 ids take the one-launch packing, int64 ids the tensor operations: same outputs, same gradients,

@@ -131,8 +131,9 @@ def test_combined_vs_recurrence(b, L, nh, P, g, N, Q, dtype, device):
 @pytest.mark.parametrize("dtype", [F32, BF16], ids=["f32", "bf16"])
 def test_views_of_a_fused_projection(dtype, device):
     """x, B, C and z as a Mamba-2 layer holds them: slices of one projected tensor, so the position
-    stride exceeds nheads * hdim while the heads stay dense (the chunk scan then pairs heads), and
-    x with every other head of a wider tensor (head stride 2 * hdim: one head per workgroup).
+    stride exceeds nheads * hdim while the heads stay dense, and x with every other head of a wider tensor
+    (head stride 2 * hdim).  One head per workgroup throughout: the batches at which the chunk scan pairs
+    dense heads are in test_gpu_ssd_large_grids.py.
     Strides only change addresses, so the results must equal those of contiguous copies."""
     from kernels.mamba_kernels.mamba_combined_fwd import mamba_chunk_scan_combined_fwd
 

@@ -146,7 +146,7 @@ WALK_CASES = [
 
 @pytest.mark.parametrize("has_init", [False, True])
 @pytest.mark.parametrize("b,L,nh,g,Q", WALK_CASES)
-def test_dstates_and_state_passing_in_one_kernel(b, L, nh, g, Q, has_init, device):
+def test_dstates_and_state_passing_in_one_kernel(b, L, nh, g, Q, has_init, device, monkeypatch):
     """The reverse walk against the oracle's two stages with the reference's rounding, and against
     the two launchers with a float32 tensor between them (dstates bit for bit)."""
     from kernels.mamba_kernels_bwd import mamba_scan_state_passing_bwd as M
@@ -162,39 +162,49 @@ def test_dstates_and_state_passing_in_one_kernel(b, L, nh, g, Q, has_init, devic
     dfin = torch.randn(b, nh, P, N, generator=gen)
     d = lambda t: t.to(device)
 
-    fused = M._fused(d(C), d(dA_cs), d(dout), d(states), d(dfin), has_init, F32)
-    assert fused is not None, "the single kernel must take this case"
-    got = M._chunk_scan_state_passing_bwd(d(C), d(dA_cs), d(dout), d(states), dfinal_states=d(dfin),
-                                          has_initial_states=has_init, dstates_dtype=F32)
-    assert torch.equal(got[0], fused[0])
-
     dprev_ref = S.bwd_dstates(C, dA_cs, dout, round_to=BF16)
     ref = S.state_passing_bwd(states.float().reshape(b, nc, nh, P * N), dA_cs[..., -1],
                               dprev_ref.reshape(b, nc, nh, P * N), dfin.reshape(b, nh, P * N),
                               has_initial_states=has_init)
-    check_close("dstates", got[0].reshape(b, nc, nh, P * N), ref[0], BF16)
-    check_close("ddA_chunk_cumsum", got[1], ref[1], BF16)
-    if has_init:
-        check_close("dinitstates", got[2].reshape(b, nh, P * N), ref[2], BF16)
-    else:
-        assert got[2] is None
-
+    ref0 = S.state_passing_bwd(states.float().reshape(b, nc, nh, P * N), dA_cs[..., -1],
+                               dprev_ref.reshape(b, nc, nh, P * N))
     dprev = _chunk_scan_bwd_dstates(d(C), d(dA_cs), d(dout), dtype=F32)
     two = _state_passing_bwd(d(states).reshape(b, nc, nh, P * N), d(dA_cs)[..., -1], dprev.reshape(b, nc, nh, P * N),
                              dfinal_states=d(dfin).reshape(b, nh, P * N), has_initial_states=has_init,
                              dstates_dtype=F32)
-    assert torch.equal(got[0].reshape(b, nc, nh, P * N), two[0]), "dstates differ from the two launchers'"
-    check_close("ddA_chunk_cumsum against the two launchers", got[1], two[1].cpu(), F32)
-    if has_init:
-        assert torch.equal(got[2].reshape(b, nh, P * N), two[2])
+    # the walk and the two kernels without Python between them, whichever the public function chooses here
+    for form in (M._fused, M._two_launches):
+        announce(form.__name__)
+        got = form(d(C), d(dA_cs), d(dout), d(states), d(dfin), has_init, F32)
+        assert got is not None, "both forms must take this case"
+        check_close("dstates", got[0].reshape(b, nc, nh, P * N), ref[0], BF16)
+        check_close("ddA_chunk_cumsum", got[1], ref[1], BF16)
+        assert torch.equal(got[0].reshape(b, nc, nh, P * N), two[0]), "dstates differ from the two launchers'"
+        check_close("ddA_chunk_cumsum against the two launchers", got[1], two[1].cpu(), F32)
+        if has_init:
+            check_close("dinitstates", got[2].reshape(b, nh, P * N), ref[2], BF16)
+            assert torch.equal(got[2].reshape(b, nh, P * N), two[2])
+        else:
+            assert got[2] is None
 
-    # bfloat16 out (the type of the states) and no gradient of the final state
-    got16 = M._chunk_scan_state_passing_bwd(d(C), d(dA_cs), d(dout), d(states))
-    assert got16[0].dtype == BF16
-    ref0 = S.state_passing_bwd(states.float().reshape(b, nc, nh, P * N), dA_cs[..., -1],
-                               dprev_ref.reshape(b, nc, nh, P * N))
-    check_close("dstates, bfloat16, no dfinal", got16[0].reshape(b, nc, nh, P * N), ref0[0], BF16)
-    check_close("ddA_chunk_cumsum, no dfinal", got16[1], ref0[1], BF16)
+        # bfloat16 out (the type of the states) and no gradient of the final state
+        got16 = form(d(C), d(dA_cs), d(dout), d(states), None, has_init, BF16)
+        assert got16[0].dtype == BF16
+        check_close("dstates, bfloat16, no dfinal", got16[0].reshape(b, nc, nh, P * N), ref0[0], BF16)
+        check_close("ddA_chunk_cumsum, no dfinal", got16[1], S.state_passing_bwd(
+            states.float().reshape(b, nc, nh, P * N), dA_cs[..., -1], dprev_ref.reshape(b, nc, nh, P * N),
+            has_initial_states=has_init)[1], BF16)
+
+    # the public function runs one of them, with the states' type and no gradient of the final state by default
+    for choice, form in ((True, M._fused), (False, M._two_launches)):
+        monkeypatch.setattr(M, "walk_pays", lambda *a, **k: choice)
+        got = M._chunk_scan_state_passing_bwd(d(C), d(dA_cs), d(dout), d(states), dfinal_states=d(dfin),
+                                              has_initial_states=has_init, dstates_dtype=F32)
+        want = form(d(C), d(dA_cs), d(dout), d(states), d(dfin), has_init, F32)
+        assert all((a is None and w is None) or torch.equal(a, w) for a, w in zip(got, want))
+        got = M._chunk_scan_state_passing_bwd(d(C), d(dA_cs), d(dout), d(states))
+        want = form(d(C), d(dA_cs), d(dout), d(states), None, False, BF16)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]) and got[2] is None
 
 
 def test_reverse_walk_falls_back_to_the_two_launchers(device):
