@@ -432,32 +432,32 @@ int ssd_state_passing_bwd(const void* states, int states_dtype, const float* dA_
   hipStream_t st = as_stream(stream);
   float* part = static_cast<float*>(workspace);
   // the three tensors are float32 or bfloat16 independently of each other
-  const bool ahead = passing_ahead(nchunks, grid, wide ? 8 : 4);
-  auto launch_as = [&](auto kernel, auto ts, auto td, auto tg) {
+  // (packed, the form with two turns also requests a turn past the end: it needs more than two turns to pay)
+  const bool ahead = passing_ahead(seq.p ? nchunks - 4 : nchunks, grid, wide ? 8 : 4);
+  auto launch = [&](auto ts, auto td, auto tg, auto elements) {
     using TS = decltype(ts);
     using TD = decltype(td);
     using TG = decltype(tg);
+    constexpr int E = decltype(elements)::value;
+    auto kernel = seq.p ? (ahead ? ssd_state_passing_bwd_kernel<TS, TD, TG, E, true, true>
+                                 : ssd_state_passing_bwd_kernel<TS, TD, TG, E, false, true>)
+                        : (ahead ? ssd_state_passing_bwd_kernel<TS, TD, TG, E, true, false>
+                                 : ssd_state_passing_bwd_kernel<TS, TD, TG, E, false, false>);
     hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(256), 0, st,
                        (const TS*)states, dA_chunk, da_sb, da_sh, da_sc, (const TD*)dout, dfinal, (TG*)dstates, part,
                        dinit, (int)nheads, (int)nchunks, (int)dim, tiles, seq, (int)seqlen, (int)chunk);
   };
-  auto launch = [&](auto ts, auto td, auto tg) {
-    using TS = decltype(ts);
-    using TD = decltype(td);
-    using TG = decltype(tg);
-    if (ahead) launch_as(ssd_state_passing_bwd_kernel<TS, TD, TG, 4, true>, ts, td, tg);
-    else launch_as(ssd_state_passing_bwd_kernel<TS, TD, TG, 4, false>, ts, td, tg);
-  };
+  using Four = std::integral_constant<int, 4>;
+  using Eight = std::integral_constant<int, 8>;
   auto pick_g = [&](auto ts, auto td) {
-    if (dstates_dtype == SSD_BF16) launch(ts, td, bf16_t());
-    else launch(ts, td, float());
+    if (dstates_dtype == SSD_BF16) launch(ts, td, bf16_t(), Four());
+    else launch(ts, td, float(), Four());
   };
   auto pick_d = [&](auto ts) {
     if (dout_dtype == SSD_BF16) pick_g(ts, bf16_t());
     else pick_g(ts, float());
   };
-  if (wide && ahead) launch_as(ssd_state_passing_bwd_kernel<bf16_t, bf16_t, bf16_t, 8, true>, bf16_t(), bf16_t(), bf16_t());
-  else if (wide) launch_as(ssd_state_passing_bwd_kernel<bf16_t, bf16_t, bf16_t, 8, false>, bf16_t(), bf16_t(), bf16_t());
+  if (wide) launch(bf16_t(), bf16_t(), bf16_t(), Eight());
   else if (states_dtype == SSD_BF16) pick_d(bf16_t());
   else pick_d(float());
   SSD_TRY(launched());
