@@ -570,8 +570,8 @@ __global__ __launch_bounds__(256) void combine_dA_kernel(const float* __restrict
 // MODE 0 notes in starts (dense (batch, L, nh) bytes) where it did so and MODE 1 goes by that, so that the gradient
 // does not depend on what becomes of the ids in between.
 // One thread per (batch, position, head).  Bound by its launch: it stands for the eleven elementwise launches that
-// a forward and backward need in tensor operations (b6 nh2 L1777: 4.4 and 3.3 us
-// in place of 35 us of kernels and eleven times the host's part of a launch).
+// a forward and backward need in tensor operations (b6 nh2 L1777: 2.9 and 2.8 us in place of 35 us of kernels and
+// eleven times the host's part of a launch).
 // ------------------------------------------------------------------------------------
 template <int MODE>
 __global__ __launch_bounds__(256) void coef_starts_kernel(const float* src, SeqStrides ss, float* dst, SeqStrides sd,

@@ -274,7 +274,8 @@ __device__ __forceinline__ float tile_keep(float coef) {
 // requested at a time; nothing is chained, nothing is shared, so there is no workspace, no ticket and no
 // barrier.  Bound by the latency of one load and one store: b64 nh2 d1024 bf16, one row,
 // 5.5 us where the tile kernel takes 20.1.
-// The recurrence is fwd_tile_kernel's final pass from the same state, so the values are the same.
+// The recurrence is fwd_tile_kernel's final pass: the values are the same bit for bit for the first eight rows and
+// agree to rounding beyond, where that kernel starts a wave's rows from the product and the sum of the rows before.
 // ------------------------------------------------------------------------------------
 template <typename T, bool XP>
 __global__ __launch_bounds__(256) void fwd_short_kernel(const T* __restrict__ x, SeqStrides sx,
