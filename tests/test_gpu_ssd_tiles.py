@@ -170,6 +170,28 @@ def test_varlen_states_at_stage_edges(P, N, dtype, device):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [F32, BF16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("Q,length", [(64, 7), (256, 7), (64, 70), (256, 70)])  # float32 takes the matrix units in the last
+def test_varlen_states_of_many_sequences(Q, length, dtype, device):
+    from kernels.ema_chunk_state import chunk_state_varlen
+
+    announce(f"varlen states of 260 sequences of about {length}, Q={Q} {dtype}")
+    nseq, nh, g, P, N = 260, 4, 2, 64, 64
+    gen = torch.Generator().manual_seed(length)
+    cu = torch.randint(1, 2 * length, (nseq + 1,), generator=gen).cumsum(0).to(torch.int32)
+    cu -= cu[0].clone()
+    cu[-1] = max(int(cu[-1]), nseq * length)
+    L = int(cu[-1])
+    r = lambda *s: torch.randn(*s, generator=gen)
+    x, B = r(L, nh, P).to(dtype), r(L, g, N).to(dtype)
+    dA, dt = S.chunk_cumsum(torch.rand(1, L, nh, generator=gen) * 0.5, -torch.rand(nh, generator=gen), Q)
+    prev = r(-(-L // Q), nh, P, N).to(dtype)
+    ref = S.chunk_state_varlen(B, x, dt[0], dA[0], cu, prev, dtype)
+    got = chunk_state_varlen(*(t.to(device) for t in (B, x, dt[0], dA[0], cu, prev)))
+    check_close("varlen states", got, ref, dtype, regrouped=True)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["decay", "rise", "mixed"])
 @pytest.mark.parametrize("nh,g,N", [(4, 1, 128), (6, 3, 64)])
 @pytest.mark.parametrize("Q,L", [(128, 257), (128, 128), (128, 33), (64, 190), (64, 64), (64, 1)])

@@ -698,9 +698,14 @@ int varlen_states(const void* B, int64_t b_sl, int64_t b_sg, const void* x, int6
   const int64_t tiles = ((hdim + 63) / 64) * ((dstate + 63) / 64);
   const dim3 grid((unsigned)tiles, (unsigned)nseq, (unsigned)nheads);
   const int hpg = (int)(nheads / ngroups);
-  // the matrix kernel takes whole 64 x 64 tiles of the state and rows in 16-byte pieces; anything else is
-  // multiplied out in float32
-  const bool mma = hdim % 64 == 0 && dstate % 64 == 0 && check_vec(x, 0, x_sl, x_sh, dtype, hdim) == SSD_OK &&
+  // The matrix kernel takes whole 64 x 64 tiles of the state and rows in 16-byte pieces; anything else is
+  // multiplied out in float32.  So are float32 inputs where the workgroups fill the chip and the rows up to a sequence's
+  // end, about half a chunk or the sequence, leave its stages of 64 rows mostly empty: the float32 matrix
+  // instructions are no faster there and work for the padding.  Multiplied out / matrix, us, float32, 24 heads, 6000
+  // positions: 1200 sequences hdim 64 dstate 64 chunk 64 273 / 319; 60 sequences hdim 128 dstate 128 chunk 64 67 / 77,
+  // chunk 256 99 / 95; 6 sequences chunk 64 16.4 / 12.5 (bfloat16, 1200 sequences 387 / 313).
+  const bool padded = dtype == SSD_F32 && tiles * nseq * nheads > 1024 && (seqlen / nseq < 64 || chunk / 2 < 64);
+  const bool mma = !padded && hdim % 64 == 0 && dstate % 64 == 0 && check_vec(x, 0, x_sl, x_sh, dtype, hdim) == SSD_OK &&
                    check_vec(B, 0, b_sl, b_sg, dtype, dstate) == SSD_OK;
 #define SSD_VARLEN_LAUNCH(T, TS, TO)                                                                                   \
   hipLaunchKernelGGL((mma ? ssd_chunk_state_varlen_mma_kernel<T, TS, TO> : ssd_chunk_state_varlen_kernel<T, TS, TO>),  \
