@@ -1,0 +1,82 @@
+"""The kernels that walk the heads of a group (bfloat16, hdim 64, chunks of 256 rows), at the edges of their strips of 16
+rows, with each way of dealing the heads to workgroups (one head each, a share of one set, shares that run over several
+sets) and each form of the decay: one that falls (its factors apart), one that falls steeply inside a strip, one that
+rises.  The oracle looks at the first, a middle and the last element of the batch."""
+import pytest
+import torch
+
+from oracle import ssd_oracle as S
+from parity_util import announce, check_close
+from test_gpu_ssd_packed import pack_ids
+
+pytestmark = pytest.mark.gpu
+
+F32, BF16 = torch.float32, torch.bfloat16
+P, Q = 64, 256
+
+# (batch, seqlen, nheads, ngroups, dstate): 72 heads of all (batch, chunk) pairs; 276, two to a workgroup; 688 in shares of
+# four; 1200 and 3210 dealt evenly; groups that do not divide evenly
+DEALS = [(2, 527, 12, 1, 128), (23, 289, 6, 2, 128), (43, 512, 8, 1, 64), (100, 700, 4, 1, 128), (107, 513, 10, 1, 64),
+         (3, 271, 11, 1, 128)]
+
+
+def _decay(kind, b, L, nh, seed):
+    gen = torch.Generator().manual_seed(seed)
+    dt = torch.rand(b, L, nh, generator=gen) * 0.5
+    A = -torch.rand(nh, generator=gen) * 4 - 0.1
+    if kind == "steep":
+        A = A * 30
+    elif kind == "rising":
+        A = -A * 0.05
+    elif kind == "mixed":  # up and down, and one head that falls throughout
+        dt[..., 1:] -= 0.25
+    return S.chunk_cumsum(dt, A, Q)
+
+
+def _inputs(b, L, nh, g, N, kind, seed):
+    gen = torch.Generator().manual_seed(seed)
+    r = lambda *s: torch.randn(*s, generator=gen)
+    nc = -(-L // Q)
+    dA, dt = _decay(kind, b, L, nh, seed)
+    cb = r(b, nc, g, Q, Q) * 0.3
+    if L % Q:  # what lies past the sequence must not be looked at
+        cb[:, -1, :, L % Q:, :] = float("nan")
+        dA[:, :, -1, L % Q:] = dA[:, :, -1, L % Q - 1:L % Q]
+    x, y = r(b, L, nh, P).to(BF16), r(b, L, nh, P).to(BF16)
+    return x, y, r(b, L, g, N).to(BF16), dt, dA, cb, r(b, nc, nh, P, N).to(BF16), r(nh)
+
+
+def _some(b):
+    rows = sorted({0, b // 2, b - 1})
+    return rows, lambda t: None if t is None else t[rows]
+
+
+def _check_scan(case, kind, skip, gate, packed, device):
+    from kernels.mamba_kernels.mamba_scan_fwd import _chunk_scan_fwd
+
+    b, L, nh, g, N = case
+    announce(f"scan by heads {case} {kind} skip {skip} gate {gate} packed {packed}")
+    x, z, C, dt, dA, cb, states, D = _inputs(b, L, nh, g, N, kind, seed=L + nh)
+    z, D = z if gate else None, D if skip else None
+    seq = pack_ids(b, L, Q, seed=L) if packed else None
+    d = lambda t: None if t is None else t.to(device)
+    out, out_x = _chunk_scan_fwd(d(cb), d(x), d(dt), d(dA), d(C), d(states), D=d(D), z=d(z), seq_idx=d(seq))
+    rows, pick = _some(b)
+    ref, ref_x = S.chunk_scan(torch.nan_to_num(pick(cb)), pick(x), pick(dt), pick(dA), pick(C), pick(states), D=D, z=pick(z),
+                              round_to=BF16, seq_idx=pick(seq))
+    check_close("out", out[rows], ref, BF16, regrouped=True)
+    if gate:
+        check_close("out_x", out_x[rows], ref_x, BF16, regrouped=True)
+
+
+@pytest.mark.parametrize("skip,gate,packed", [(False, False, False), (True, False, True), (True, True, False), (False, True, True)])
+@pytest.mark.parametrize("case", DEALS)
+def test_scan_deals_and_options(case, skip, gate, packed, device):
+    _check_scan(case, "falling", skip, gate, packed, device)
+
+
+@pytest.mark.parametrize("gate", [False, True])
+@pytest.mark.parametrize("kind", ["falling", "steep", "rising", "mixed"])
+@pytest.mark.parametrize("L", [257, 271, 272, 273, 289, 511])
+def test_scan_strip_edges(L, kind, gate, device):
+    _check_scan((26, L, 6, 1, 128), kind, True, gate, False, device)

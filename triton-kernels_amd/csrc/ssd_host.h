@@ -74,6 +74,33 @@ constexpr int64_t kMidWorkgroups = 384, kMidScanPairs64 = 385, kMidDxPairs64 = 5
 // Workgroups of float32 chunks of 128 rows up to which both workgroups of the 64-row kernel run at once.
 constexpr int64_t kBoth64Row = 128;
 
+// How the kernels that walk the heads deal them to their workgroups, one to a compute unit: each of `sets` (batch, chunk,
+// group) sets of `per` heads to `splits` workgroups of its own, or (splits = 0) all heads evenly to 256.  What the heads of a
+// set share is fetched again by every workgroup that has some of them, at about the cost of one and a quarter heads: the
+// estimates are rounds x (heads of a workgroup and one fetch), and heads with a fetch for each set they can touch.
+// us by splits / evenly: scan 9 sets of 32 19.4 / 26.8, 60 of 6 19.9 / 27.7, 64 of 15 29.6 / 31.3, 320 of 10 97 / 88, 384 of 6
+// 78 / 72; with gate 192 of 13 113 / 106; dx 320 of 10 124 / 116.
+struct HeadsDeal {
+  unsigned workgroups;
+  int units, splits;
+};
+// Rows they take: 32-bit byte offsets within eight rows, and of a row within a chunk.
+inline bool heads_rows(const Strides3& s) { return forward_strides(s) && s.sl < (int64_t(1) << 23); }
+// dA and dt are copied in 16-byte pieces.
+inline bool heads_vectors(const float* dt, const float* dA) {
+  return (reinterpret_cast<uintptr_t>(dt) | reinterpret_cast<uintptr_t>(dA)) % 16 == 0;
+}
+inline HeadsDeal heads_deal(int64_t sets, int64_t per) {
+  const int64_t units = sets * per, each = (units + 255) / 256;  // (units: up to 2^28, see check_dims)
+  int64_t splits = 0, least = 4 * each + 5 * ((each - 2 + per) / per + 1);
+  if (units <= 256) return HeadsDeal{(unsigned)units, (int)units, (int)per};
+  for (int64_t s = 1; s <= per && sets * (s - 1) < 1024; ++s) {
+    const int64_t cost = (sets * s + 255) / 256 * (4 * ((per + s - 1) / s) + 5);
+    if (cost < least) least = cost, splits = s;
+  }
+  return HeadsDeal{splits ? (unsigned)(sets * splits) : 256u, (int)units, (int)splits};
+}
+
 template <typename K>
 int allow_smem(K kernel, int bytes) {
   if (bytes <= 64 * 1024) return SSD_OK;

@@ -3,6 +3,7 @@
 // depends on what else the unit holds (68 bytes per lane next to all the other stages, 8 here).
 #include <type_traits>
 
+#include "ssd_heads_kernels.h"
 #include "ssd_host.h"
 
 namespace {
@@ -78,8 +79,31 @@ struct ScanLaunch {
       return SSD_OK;
     }
   }
+  template <int N, bool GATED>
+  int launch_heads() const {
+    const HeadsDeal deal = heads_deal(d.batch * d.C * d.g, d.nh / d.g);
+    auto kernel = deal.splits ? ssd_chunk_scan_heads_kernel<N, GATED, false> : ssd_chunk_scan_heads_kernel<N, GATED, true>;
+    constexpr int smem = ScanHeadsSmem<N, GATED>::kBytes;
+    static_assert(smem <= kLdsBytes, "the heads under way must fit the LDS of a compute unit");
+    SSD_TRY(allow_smem(kernel, smem));
+    hipLaunchKernelGGL(kernel, dim3(deal.workgroups), dim3(512), smem, st, cb, (const bf16_t*)x, sx,
+                       (const bf16_t*)z, sz, dt, dA, (const bf16_t*)C, sC, (const bf16_t*)prev, D, (bf16_t*)out, so,
+                       (bf16_t*)out_x, (int)d.nh, (int)(d.nh / d.g), (int)d.g, (int)d.L, (int)d.C, deal.units, deal.splits, seq);
+    return launched();
+  }
   template <typename T, int P, int N, typename TS>
   int run_as() const {
+    if constexpr (std::is_same<T, bf16_t>::value && std::is_same<TS, bf16_t>::value && P == 64) {
+      // The walk over the heads, from where a workgroup has two of them or a gate hides the fetch of what they share,
+      // and groups have three heads or more.  The 256-row kernel / the walk, us, dstate 128: without gate 256 heads of
+      // all (batch, chunk) pairs 14.7 / 16.2, 288 20.9 / 19.4, 512 23.2 / 21.3, 1536 57 / 41; 512 groups of two heads 44 / 53,
+      // of three 66 / 62; with gate 16 heads 16.0 / 16.8, 64 16.9 / 17.2, 128 19.6 / 18.2, 256 22.4 / 19.1.
+      const int64_t units = d.batch * d.C * d.nh;
+      const bool pays = units > (z ? 64 : 256) && d.nh / d.g >= 3;
+      if (d.Q == 256 && pays && !(D && d_has_hdim) && heads_vectors(dt, dA) && heads_rows(sx) && heads_rows(so) &&
+          (!z || heads_rows(sz)))
+        return z ? launch_heads<N, true>() : launch_heads<N, false>();
+    }
     constexpr int wide_smem = WideSmem<T, P, N>::kBytes;
     if (d.Q % 256 == 0 && wide_smem <= kLdsBytes) {  // 256-row super-tiles, no barrier inside the k loop
       // Two adjacent heads of a group per workgroup where they are adjacent in memory too (dense
