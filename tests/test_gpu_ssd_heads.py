@@ -80,3 +80,34 @@ def test_scan_deals_and_options(case, skip, gate, packed, device):
 @pytest.mark.parametrize("L", [257, 271, 272, 273, 289, 511])
 def test_scan_strip_edges(L, kind, gate, device):
     _check_scan((26, L, 6, 1, 128), kind, True, gate, False, device)
+
+
+def _check_dx(case, kind, skip, packed, device):
+    from kernels.mamba_kernels_bwd.mamba_chunk_scan_chunk_state_bwd_dx import _chunk_scan_chunk_state_bwd_dx
+
+    b, L, nh, g, N = case
+    announce(f"dx by heads {case} {kind} skip {skip} packed {packed}")
+    x, dout, B, dt, dA, cb, ds, D = _inputs(b, L, nh, g, N, kind, seed=L + nh)
+    D = D if skip else None
+    seq = pack_ids(b, L, Q, seed=L) if packed else None
+    d = lambda t: None if t is None else t.to(device)
+    dx, ddt, dD = _chunk_scan_chunk_state_bwd_dx(d(x), d(dt), d(dA), d(B), d(cb), d(dout), d(ds), D=d(D), seq_idx=d(seq))
+    rows, pick = _some(b)
+    ref = S.chunk_scan_chunk_state_bwd_dx(pick(x), pick(dt), pick(dA), pick(B), torch.nan_to_num(pick(cb)), pick(dout), pick(ds),
+                                          D=D, round_to=BF16, seq_idx=pick(seq))
+    check_close("dx", dx[rows], ref[0], BF16, regrouped=True)
+    check_close("ddt", ddt[rows], ref[1], BF16, loose=True)
+    if skip:
+        check_close("dD", dD, (dout.float() * x.float()).sum((0, 1, 3)), F32)
+
+
+@pytest.mark.parametrize("skip,packed", [(False, False), (True, True)])
+@pytest.mark.parametrize("case", DEALS)
+def test_dx_deals_and_options(case, skip, packed, device):
+    _check_dx(case, "falling", skip, packed, device)
+
+
+@pytest.mark.parametrize("kind", ["falling", "steep", "rising", "mixed"])
+@pytest.mark.parametrize("L", [1, 15, 17, 255, 272, 289])
+def test_dx_strip_edges(L, kind, device):
+    _check_dx((2, L, 36, 1, 128), kind, True, False, device)

@@ -5,6 +5,7 @@
 #include <type_traits>
 
 #include "ema_gemm_kernels.h"
+#include "ssd_heads_kernels.h"
 #include "ssd_host.h"
 #include "ssd_kernels.h"
 
@@ -85,6 +86,21 @@ struct WalkLaunch {
   }
 };
 
+// Number of per-wave slots the dx kernels of a shape write per (batch, chunk, head): 256-row super-tiles have four waves,
+// or eight where the walk over the heads may run (the others then zero what they do not use).
+struct DxSlots {
+  int64_t Q;
+  template <typename T, int P, int N>
+  static bool wide(int64_t Q) {
+    return Q % 256 == 0 && WideSmem<T, P, N>::kBytes <= kLdsBytes;
+  }
+  template <typename T, int P, int N>
+  int run() const {
+    if (std::is_same<T, bf16_t>::value && P == 64 && Q == 256) return DxHeadsSmem<N>::kSlots;
+    return wide<T, P, N>(Q) ? (int)(4 * (Q / 256)) : (int)(4 * ((Q + 63) / 64));
+  }
+};
+
 struct DxLaunch {
   const float* cb;
   const void *x, *dout, *B;
@@ -100,11 +116,6 @@ struct DxLaunch {
   SeqIdx seq;
   float* dD_part;
   hipStream_t st;
-  // whether the 256-row kernel runs this shape (it must also fit the LDS of a CU)
-  template <typename T, int P, int N>
-  static bool wide(int64_t Q) {
-    return Q % 256 == 0 && WideSmem<T, P, N>::kBytes <= kLdsBytes;
-  }
   template <typename T, int P, int N>
   int run() const {
     if constexpr (!std::is_same<T, float>::value)
@@ -123,15 +134,34 @@ struct DxLaunch {
   }
   template <typename T, int P, int N, typename TS>
   int run_as() const {
+    if constexpr (std::is_same<T, bf16_t>::value && std::is_same<TS, bf16_t>::value && P == 64) {
+      // The walk over the heads.  The 256-row kernel / the walk, us, dstate 128: 128 heads of all (batch, chunk) pairs 16.9 /
+      // 14.1, 256 19.2 / 15.3, 512 27 / 22, 3072 121 / 91; only many groups of two or three heads, one or two to a compute unit,
+      // are behind: 256 of two 27.3 / 27.9, of three 34.4 / 35.3, of four 50 / 42.  Calls of up to 64 heads, where the launch counts
+      // for more than the kernel (15 / 12.5), give the same bits whatever the type of the states.
+      const int64_t units = d.batch * d.C * d.nh;
+      const bool pays = units > 64 && (d.nh / d.g >= 4 || d.batch * d.C * d.g < 256);
+      if (d.Q == 256 && pays && !(D && d_has_hdim) && heads_vectors(dt, dA) && heads_rows(sx) && heads_rows(sd) && heads_rows(sdx)) {
+        const HeadsDeal deal = heads_deal(d.batch * d.C * d.g, d.nh / d.g);
+        auto kernel = deal.splits ? ssd_chunk_scan_bwd_dx_heads_kernel<N, false> : ssd_chunk_scan_bwd_dx_heads_kernel<N, true>;
+        constexpr int smem = DxHeadsSmem<N>::kBytes;
+        static_assert(smem <= kLdsBytes, "the heads under way must fit the LDS of a compute unit");
+        SSD_TRY(allow_smem(kernel, smem));
+        hipLaunchKernelGGL(kernel, dim3(deal.workgroups), dim3(512), smem, st, cb, (const T*)x, sx,
+                           (const T*)dout, sd, dt, dA, (const T*)B, sB, (const TS*)dstates, D, (T*)dx, sdx, ddt,
+                           (int)d.nh, (int)(d.nh / d.g), (int)d.g, (int)d.L, (int)d.C, deal.units, deal.splits, seq, dD_part);
+        return launched();
+      }
+    }
     constexpr int wide_smem = WideSmem<T, P, N>::kBytes;
-    if (wide<T, P, N>(d.Q)) {
+    if (DxSlots::wide<T, P, N>(d.Q)) {  // (it must also fit the LDS of a CU)
       auto kernel = ssd_chunk_scan_bwd_dx_wide_kernel<T, P, N, TS>;
       SSD_TRY(allow_smem(kernel, wide_smem));
       const int stiles = (int)(d.Q / 256);
       hipLaunchKernelGGL(kernel, dim3((unsigned)(d.batch * d.C * d.nh * stiles)), dim3(256), wide_smem, st, cb,
                          (const T*)x, sx, (const T*)dout, sd, dt, dA, (const T*)B, sB, (const TS*)dstates, D,
                          d_has_hdim, (T*)dx, sdx, ddt, (int)d.nh, (int)(d.nh / d.g), (int)d.g, (int)d.L, (int)d.Q,
-                         (int)d.C, stiles, seq, dD_part);
+                         (int)d.C, stiles, seq, dD_part, DxSlots{d.Q}.template run<T, P, N>());
       return launched();
     }
     if constexpr (P == 64 && sizeof(T) == 2) {
@@ -156,15 +186,6 @@ struct DxLaunch {
                        (T*)dx, sdx, ddt, (int)d.nh, (int)(d.nh / d.g), (int)d.g, (int)d.L, (int)d.Q, (int)d.C, mtiles,
                        seq, dD_part);
     return launched();
-  }
-};
-
-// Number of per-wave slots the dx kernel of a shape writes per (batch, chunk, head).
-struct DxSlots {
-  int64_t Q;
-  template <typename T, int P, int N>
-  int run() const {
-    return DxLaunch::wide<T, P, N>(Q) ? (int)(4 * (Q / 256)) : (int)(4 * ((Q + 63) / 64));
   }
 };
 

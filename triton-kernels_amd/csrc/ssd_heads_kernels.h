@@ -489,4 +489,330 @@ __global__ __launch_bounds__(512, 2) void ssd_chunk_scan_heads_kernel(
   }
 }
 
+// Sums after a trade of registers between halves or quarters of a wave.  swap16(a, b): of two lane groups side by side
+// (0 and 1, 2 and 3) the even one receives the sum of both's a, the odd one that of both's b; swap32(a, b): the lower half
+// receives the sum of both halves' a, the upper that of both's b.
+__device__ __forceinline__ float sum_of(u32x2_t s) {
+  const unsigned a = s[0], b = s[1];
+  return __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
+}
+__device__ __forceinline__ float swap16_sum(float a, float b) {
+  return sum_of(__builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false));
+}
+__device__ __forceinline__ float swap32_sum(float a, float b) {
+  return sum_of(__builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false));
+}
+// Sum over the four groups of 16 lanes, in every lane.
+__device__ __forceinline__ float quad_sum(float v) {
+  v = swap16_sum(v, v);
+  return swap32_sum(v, v);
+}
+// Sum over the 16 lanes of a group, in every lane.
+__device__ __forceinline__ float row16_sum(float v) {
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, false));  // row_ror:8
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xf, 0xf, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x122, 0xf, 0xf, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x121, 0xf, 0xf, false));
+  return v;
+}
+
+// ------------------------------------------------------------------------------------
+// dx / ddt / the partial sums of dD (ssd_chunk_scan_bwd_dx_kernel): the mirror image of the chunk scan.  The strips'
+// positions run from the chunk's end to the diagonal, the weights are columns of cb.  us by the 256-row kernel and here,
+// dstate 128: b8 nh32 L8192 304 -> 233 (4.4 TB/s of its 1030 MB; with D 365 -> 258), b4 nh24 L8192 121 -> 91, b1 nh32 L4096 27 -> 22.
+// Alone, the copies and stores take 206 and the rest 166.
+// ------------------------------------------------------------------------------------
+template <int N>
+struct DxHeadsSmem : HeadsTile {
+  static constexpr int R = 2;  // heads in LDS
+  static constexpr int kState = P * N * (int)sizeof(bf16_t);
+  static constexpr int kHead = kRows + kState + kVec;
+  static constexpr int kBytes = R * kHead + kFactors + kRows;  // + the waves' own rows of x
+  static constexpr int kSlots = 8;                             // partial sums of dD per head: one a wave
+};
+
+template <int N, bool EVEN>
+__global__ __launch_bounds__(512, 2) void ssd_chunk_scan_bwd_dx_heads_kernel(
+    const float* __restrict__ cb, const bf16_t* __restrict__ x, Strides3 sx, const bf16_t* __restrict__ dout, Strides3 sd,
+    const float* __restrict__ dt, const float* __restrict__ dA_cs, const bf16_t* __restrict__ Bm, Strides3 sB,
+    const bf16_t* __restrict__ dstates, const float* __restrict__ D, bf16_t* __restrict__ dx, Strides3 sdx,
+    float* __restrict__ ddt, int nh, int heads_per_group, int ngroups, int L, int C, int units, int splits, SeqIdx seq,
+    float* __restrict__ dD_part) {
+  using S = DxHeadsSmem<N>;
+  using T = bf16_t;
+  constexpr int P = S::P, Q = S::Q, R = S::R, NK = N / 32;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+  HeadsWalk<EVEN> now(xcd_local_index((int)blockIdx.x, (int)gridDim.x), (int)gridDim.x, units, splits, heads_per_group, ngroups, C);
+  HeadsWalk<EVEN> ahead = now;  // the head whose copies are requested next
+  // the wave's strips of rows, their pieces of 32 positions from the end to the diagonal, their factors
+  int r0[2], steps[2];
+  float* fk[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) r0[j] = 16 * S::strip(wave, j), steps[j] = 8 - (r0[j] >> 5);
+  float* factors = reinterpret_cast<float*>(smem + R * S::kHead) + wave * 288;
+  fk[0] = factors - 32 * (8 - steps[0]);
+  fk[1] = factors + 32 * steps[0] - 32 * (8 - steps[1]);
+  unsigned char* own = smem + R * S::kHead + S::kFactors + wave * (32 * P * (int)sizeof(T));
+
+  constexpr int kXCopies = 4, kSCopies = S::kState / 8192, kCopies = kXCopies + kSCopies;
+  static_assert(8 * 8 * kXCopies == Q && 8 * 1024 * kSCopies == S::kState, "eight waves bring a head");
+  constexpr int SP = N / 8;  // pieces of a row of the state
+  auto state_key = [](int r) { return N == 128 ? r & 15 : (r >> 1) & 7; };
+  auto vec_at = [&](const HeadsWalk<EVEN>& w) { return (((int64_t)w.b * nh + w.head()) * C + w.c) * Q; };
+  auto request = [&](int u, int ln) {  // the copies of the head ahead into place u
+    const HeadsWalk<EVEN>& w = ahead;
+    const int h = w.head();
+    unsigned char* base = smem + u * S::kHead;
+    S::template copy_rows<kXCopies>(dout + w.b * sd.sb + (int64_t)w.c * Q * sd.sl + h * sd.sh, (int)sd.sl, 32 * wave,
+                                    min(Q, L - w.c * Q), base + kXCopies * wave * 1024, ln);
+    const T* sg = dstates + (((int64_t)w.b * C + w.c) * nh + h) * (P * N);
+    const int r = ln / SP;
+#pragma unroll
+    for (int j = 0; j < kSCopies; ++j) {
+      const int row0 = (kSCopies * wave + j) * (64 / SP);
+      copy16_to_lds(sg + row0 * N, (unsigned)(r * N + 8 * ((ln % SP) ^ state_key(row0 + r))) * (unsigned)sizeof(T),
+                    base + S::kRows + (kSCopies * wave + j) * 1024);
+    }
+    if (wave < 2)
+      copy16_to_lds((wave == 0 ? dA_cs : dt) + vec_at(w), 16u * (unsigned)ln, base + S::kRows + S::kState + wave * 1024);
+    ahead.next();
+  };
+  request(0, lane);
+
+  // What the heads of a set share: the rows of B, and the columns of cb from the last position on (entries before the
+  // diagonal or past the sequence zero).
+  Vec16<T> bf[2][NK];
+  float cb0[8][8], cb1[4][8];
+  bool live[2];
+  int limit = 0, stores = 0;
+  auto load_shared = [&]() {
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+    limit = min(Q, L - now.c * Q);
+    // stores of a head that can still be outstanding (a ragged chunk leaves some out: none are allowed for)
+    stores = limit < Q ? 0 : dD_part ? 7 : 6;
+    const ChunkSeq sq = chunk_seq(seq, now.b, now.c, Q);
+    const int e0 = 8 * (ln >> 4);
+    const T* Bg = Bm + now.b * sB.sb + (int64_t)now.c * Q * sB.sl + now.g * sB.sh + e0;
+    const float* cbg = cb + (((int64_t)now.b * C + now.c) * ngroups + now.g) * (Q * Q);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int m = r0[j] + (ln & 15);
+      const T* brow = Bg + (int64_t)min(m, limit - 1) * sB.sl;
+#pragma unroll
+      for (int i = 0; i < NK; ++i) bf[j][i] = load16(brow + 32 * i);
+      live[j] = !sq.on() || sq.at(min(m, limit - 1)) == sq.at(limit - 1);
+      const float* cbcol = cbg + e0 * Q + m;
+#pragma unroll
+      for (int t = 0; t < 8; ++t)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int k = 32 * (7 - t) + e;
+          if (j == 0) cb0[t][e] = cbcol[k * Q];
+          else if (t < 4) cb1[t][e] = cbcol[k * Q];
+        }
+#pragma unroll
+      for (int t = 0; t < 8; ++t)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int k = 32 * (7 - t) + e + e0;
+          const bool in = k >= m && k < limit;
+          if (j == 0) cb0[t][e] = in ? cb0[t][e] : 0.f;
+          else if (t < 4) cb1[t][e] = in ? cb1[t][e] : 0.f;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NK; ++i) asm volatile("" : "+v"(bf[0][i].raw), "+v"(bf[1][i].raw));
+#pragma unroll
+    for (int t = 0; t < 8; ++t)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        asm volatile("" : "+v"(cb0[t][e]));
+        if (t < 4) asm volatile("" : "+v"(cb1[t][e]));
+      }
+  };
+
+  if (!EVEN) load_shared();
+  for (int u = 0; !now.done(); now.next(), u ^= 1) {
+    if (EVEN && now.k == 0) load_shared();
+    const int64_t b = now.b;
+    const int c = now.c, h = now.head();
+    const bool more = now.unit + 1 < now.end;
+    wait_outstanding<7, 6>(now.k > 0 ? stores : 0);
+    __syncthreads();  // every wave's part of the head is there; every wave is done with the head before
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+    const int l16 = ln & 15, quad = ln >> 4;
+    const HeadsTile::Transposed tr(ln);
+#pragma unroll
+    for (int j = 0; j < 2; ++j)  // the wave's own rows of x
+      S::template copy_rows<kXCopies / 2>(x + b * sx.sb + (int64_t)c * Q * sx.sl + h * sx.sh, (int)sx.sl, r0[j], limit, own + j * 2048, ln);
+    if (more) request(u ^ 1, ln);
+    const unsigned char* base = smem + u * S::kHead;
+    const T* Ds = reinterpret_cast<const T*>(base);
+    const float* dAs = reinterpret_cast<const float*>(base + S::kRows + S::kState);
+    const float* dts = dAs + Q;
+
+    // The weight of (m, k) is cb[k][m] exp(dA_k - dA_m), split as in the chunk scan.
+    const float4 ak = *reinterpret_cast<const float4*>(dAs + 4 * ln);
+    const float an = dAs[min(4 * ln + 4, Q - 1)], a_end = dAs[Q - 1];
+    const bool split = __builtin_amdgcn_ballot_w64(S::falls(ak, an, ln, limit)) == ~0ull;
+    float am[2], ar[2];
+    bool narrow[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      am[j] = dAs[r0[j] + l16];
+      const float a0 = dAs[r0[j]], a1 = dAs[min(r0[j] + 7, limit - 1)], a2 = dAs[min(r0[j] + 15, limit - 1)];
+      narrow[j] = __builtin_amdgcn_readfirstlane(a0 - a1 <= 40.f && a1 - a2 <= 40.f);
+      ar[j] = narrow[j] ? a1 : a2;
+      const float4 f = make_float4(__expf(fminf(ak.x - ar[j], 40.f)), __expf(fminf(ak.y - ar[j], 40.f)),
+                                   __expf(fminf(ak.z - ar[j], 40.f)), __expf(fminf(ak.w - ar[j], 40.f)));
+      if (4 * ln >= 32 * (8 - steps[j])) *reinterpret_cast<float4*>(fk[j] + 4 * ln) = f;
+    }
+    // ---- dstates . B, features in the rows of the product: a lane's values belong to its row of each strip
+    floatx4 acc[2][4];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int pb = 0; pb < 4; ++pb) acc[j][pb] = floatx4{0.f, 0.f, 0.f, 0.f};
+    const unsigned piece0 = u * S::kHead + S::kRows + (l16 * N + 8 * (quad ^ state_key(l16))) * sizeof(T);
+#pragma unroll
+    for (int ks = 0; ks < NK; ++ks)
+#pragma unroll
+      for (int pb = 0; pb < 4; ++pb) {
+        const Vec16<T> sf = load16(reinterpret_cast<const T*>(smem + (piece0 ^ (64u * ks)) + 16 * pb * N * sizeof(T)));
+        mma16(sf, bf[0][ks], acc[0][pb]);
+        mma16(sf, bf[1][ks], acc[1][pb]);
+      }
+    float scale[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const float enter = live[j] ? __expf(fminf(a_end - (split ? ar[j] : am[j]), 0.f)) : 0.f;
+      scale[j] = split ? __expf(ar[j] - am[j]) : 1.f;
+#pragma unroll
+      for (int pb = 0; pb < 4; ++pb) acc[j][pb] *= enter;
+    }
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // the wave's own factors are visible to its own reads
+
+    // ---- the causal sum
+    if (split) {
+      struct Piece {
+        Vec16<T> xf[4];
+        float4 f0[2], f1[2];
+      };
+      auto fetch = [&](Piece& p, int t) {
+        const int k = 32 * (7 - t);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) p.f0[q] = *reinterpret_cast<const float4*>(fk[0] + k + 8 * quad + 4 * q);
+#pragma unroll
+        for (int pb = 0; pb < 4; ++pb) p.xf[pb] = tr.read(Ds + k * P, pb);
+        if (t < 4)
+#pragma unroll
+          for (int q = 0; q < 2; ++q) p.f1[q] = *reinterpret_cast<const float4*>(fk[1] + k + 8 * quad + 4 * q);
+      };
+      auto weights = [&](const float* w, const float4* f) {
+        const float t[8] = {w[0] * f[0].x, w[1] * f[0].y, w[2] * f[0].z, w[3] * f[0].w,
+                            w[4] * f[1].x, w[5] * f[1].y, w[6] * f[1].z, w[7] * f[1].w};
+        Vec16<T> wf;
+        wf.set_all(t);
+        return wf;
+      };
+      const int end0 = steps[0] - !narrow[0], end1 = steps[1] - !narrow[1];
+      Piece piece[2];
+      fetch(piece[0], 0);
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        if (t >= 4 && t >= end0) break;  // (a strip of the upper half has five pieces or more)
+        const Piece& p = piece[t & 1];
+        if (t < 7) fetch(piece[(t + 1) & 1], t + 1);
+        const Vec16<T> w0 = weights(cb0[t], p.f0);
+#pragma unroll
+        for (int pb = 0; pb < 4; ++pb) mma16(p.xf[pb], w0, acc[0][pb]);
+        if (t < 4 && t < end1) {
+          const Vec16<T> w1 = weights(cb1[t & 3], p.f1);
+#pragma unroll
+          for (int pb = 0; pb < 4; ++pb) mma16(p.xf[pb], w1, acc[1][pb]);
+        }
+      }
+    }
+    // (rare: cb is read again, which keeps the registers out of a second unrolled form)
+    if (!(split && narrow[0] && narrow[1]))
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+#pragma unroll
+      for (int pb = 0; pb < 4; ++pb) acc[j][pb] *= scale[j];
+      scale[j] = 1.f;
+      const int m = r0[j] + l16;
+      const unsigned cbcol = 4u * (8 * quad * Q + m);
+      const float* cbg = cb + (((int64_t)b * C + c) * ngroups + now.g) * (Q * Q);
+#pragma unroll 1
+      for (int t = split ? steps[j] - !narrow[j] : 0; t < steps[j]; ++t) {
+        const int k0 = 32 * (7 - t);
+        float w[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int k = k0 + 8 * quad + e;
+          const float f = *at_bytes(cbg + (k0 + e) * Q, cbcol) * __expf(fminf(dAs[k] - am[j], 0.f));
+          w[e] = k < m || k >= limit ? 0.f : f;
+        }
+        Vec16<T> wf;
+        wf.set_all(w);
+#pragma unroll
+        for (int pb = 0; pb < 4; ++pb) mma16(tr.read(Ds + k0 * P, pb), wf, acc[j][pb]);
+      }
+    }
+    // ---- row factor, the sums over the features, dt, skip; whole rows out
+    const float Dh = D ? D[h] : 0.f;
+    T* dxg = dx + b * sdx.sb + (int64_t)c * Q * sdx.sl + h * sdx.sh;
+    float* ddtp = ddt + vec_at(now);
+    wait_outstanding<kCopies>(more ? kCopies : 0);
+    floatx4 dsum[4];
+#pragma unroll
+    for (int pb = 0; pb < 4; ++pb) dsum[pb] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int m = r0[j] + l16;
+      auto at = [&](int r) {
+        return __umul24((unsigned)(r0[j] + r), (unsigned)sdx.sl * 2u) + 64u * (l16 >> 3) + 32u * (quad & 1) + 16u * (quad >> 1);
+      };
+      const float dtm = dts[m];
+      float dot = 0.f;
+#pragma unroll
+      for (int pb = 0; pb < 4; ++pb) {  // features 16 pb + 4 quad ..
+        const int piece = 8 * ((2 * pb + (quad >> 1)) ^ S::key(l16)) + 4 * (quad & 1);
+        acc[j][pb] *= scale[j];
+        const ema::bf16x4 xv = *reinterpret_cast<const ema::bf16x4*>(reinterpret_cast<const T*>(own) + (16 * j + l16) * P + piece);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) dot = fmaf(acc[j][pb][e], (float)xv[e], dot);
+        acc[j][pb] *= dtm;
+        if (D) {
+          const ema::bf16x4 dv = *reinterpret_cast<const ema::bf16x4*>(Ds + m * P + piece);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            acc[j][pb][e] = fmaf(Dh, (float)dv[e], acc[j][pb][e]);
+            dsum[pb][e] = fmaf(m < limit ? (float)dv[e] : 0.f, (float)xv[e], dsum[pb][e]);
+          }
+        }
+      }
+      dot = quad_sum(dot);
+      store_strip(dxg, join_quads(acc[j][0], acc[j][1]), join_quads(acc[j][2], acc[j][3]), l16, limit - r0[j], at);
+      if (quad == 0) ddtp[m] = m < limit ? dot : 0.f;
+    }
+    if (dD_part) {
+      floatx4 mine = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int pb = 0; pb < 4; ++pb)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float t = row16_sum(dsum[pb][e]);
+          mine[e] = l16 == pb ? t : mine[e];
+        }
+      if (l16 < 4)
+        *reinterpret_cast<floatx4*>(dD_part + (((b * C + c) * nh + h) * (int64_t)S::kSlots + wave) * P + 16 * l16 + 4 * quad) = mine;
+    }
+  }
+}
+
 }  // namespace ssd

@@ -3060,7 +3060,7 @@ __global__ __launch_bounds__(256, (P == 64 ? 3 : 2)) void ssd_chunk_scan_bwd_dx_
     const float* __restrict__ dt, const float* __restrict__ dA_cs, const T* __restrict__ Bm, Strides3 sB,
     const TS* __restrict__ dstates, const float* __restrict__ D, int d_has_hdim, T* __restrict__ dx,
     Strides3 sdx, float* __restrict__ ddt, int nh, int heads_per_group, int ngroups, int L, int Q, int C,
-    int stiles, SeqIdx seq, float* __restrict__ dD_part) {
+    int stiles, SeqIdx seq, float* __restrict__ dD_part, int slots) {
   using S = WideSmem<T, P, N>;
   constexpr int EPL = Vec16<T>::N, KG = Tile<T>::KG, PB = P / 32, ST = S::ST;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -3081,8 +3081,12 @@ __global__ __launch_bounds__(256, (P == 64 ? 3 : 2)) void ssd_chunk_scan_bwd_dx_
   const int m0 = ST * st;
   const int64_t chunk = (b * nh + h) * C + c;
   float* ddtp = ddt + chunk * Q;
-  // slot of this wave in dD_part (batch, C, nheads, 4 * stiles, hdim)
-  float* dslot = dD_part ? dD_part + ((((b * C + c) * nh + h) * (int64_t)stiles + st) * 4 + wave) * P : nullptr;
+  // slot of this wave in dD_part (batch, C, nheads, slots, hdim); slots past the waves' are zero
+  float* dslot = dD_part ? dD_part + (((b * C + c) * nh + h) * (int64_t)slots + 4 * st + wave) * P : nullptr;
+  if (dslot && lane < P / EPL)
+    for (int s = 4 * stiles; s < slots; s += 4)
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) dslot[(s - 4 * st) * P + lane * EPL + e] = 0.f;
   if (m0 >= limit) {
     ddtp[m0 + tid] = 0.f;
     if (dslot && lane < P / EPL) {
