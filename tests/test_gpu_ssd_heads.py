@@ -111,3 +111,28 @@ def test_dx_deals_and_options(case, skip, packed, device):
 @pytest.mark.parametrize("L", [1, 15, 17, 255, 272, 289])
 def test_dx_strip_edges(L, kind, device):
     _check_dx((2, L, 36, 1, 128), kind, True, False, device)
+
+
+def _check_ddA(case, kind, device):
+    from kernels.mamba_kernels_bwd.mamba_chunk_scan_bwd_da import _chunk_scan_bwd_ddAcs_stable
+
+    b, L, nh, g, N = case
+    announce(f"ddA by heads {case} {kind}")
+    x, dout, _, dt, dA, cb, _, _ = _inputs(b, L, nh, g, N, kind, seed=L + nh)
+    d = lambda t: t.to(device)
+    got = _chunk_scan_bwd_ddAcs_stable(d(x), d(dt), d(dA), d(dout), d(cb))
+    rows, pick = _some(b)
+    ref = S.chunk_scan_bwd_ddAcs_stable(pick(x), pick(dt), pick(dA), pick(dout), torch.nan_to_num(pick(cb)))
+    # (float32 throughout: products of bfloat16 values are exact in it)
+    check_close("ddA_cumsum (causal term)", got[rows], ref, F32)
+
+
+@pytest.mark.parametrize("case", DEALS)
+def test_ddA_deals(case, device):
+    _check_ddA(case, "falling", device)
+
+
+@pytest.mark.parametrize("kind", ["falling", "steep", "rising", "mixed"])
+@pytest.mark.parametrize("L", [1, 15, 17, 255, 272, 289])
+def test_ddA_strip_edges(L, kind, device):
+    _check_ddA((2, L, 4, 1, 128), kind, device)

@@ -671,6 +671,23 @@ int ssd_chunk_scan_bwd_ddAcs(const void* x, int64_t x_sb, int64_t x_sl, int64_t 
                        dt, dA_cumsum, cb, ddA_cumsum, (int)nheads, hpg, (int)ngroups, (int)seqlen, (int)chunk,  \
                        (int)d.C);                                                                               \
   } while (0)
+    if (dtype == SSD_BF16 && hdim == 64 && chunk == 256) {
+      // The walk over the heads: where each has a compute unit to itself, and for groups of eight or more.  The other
+      // kernel / the walk, us: 64 heads of all (batch, chunk) pairs 11.7 / 9.5, 256 14.3 / 11.7, 288 16.2 / 15.7; groups of six
+      // heads, 256 of them, 40 / 43, of eight 56 / 53, of 32 213 / 168; 320 of ten 89 / 85; 128 of four 18.0 / 18.6.
+      const bool pays = wgs <= 256 || hpg >= 8;
+      if (pays && heads_vectors(dt, dA_cumsum) && reinterpret_cast<uintptr_t>(ddA_cumsum) % 16 == 0 && heads_rows(sx) && heads_rows(sd)) {
+        constexpr int smem = DdaHeadsSmem::kBytes;
+        static_assert(smem <= kLdsBytes, "the heads under way must fit the LDS of a compute unit");
+        const HeadsDeal deal = heads_deal(batch * d.C * ngroups, hpg);
+        auto kernel = deal.splits ? ssd_ddA_heads_kernel<false> : ssd_ddA_heads_kernel<true>;
+        SSD_TRY(allow_smem(kernel, smem));
+        hipLaunchKernelGGL(kernel, dim3(deal.workgroups), dim3(512), smem, st, (const bf16_t*)x,
+                           sx, (const bf16_t*)dout, sd, dt, dA_cumsum, cb, ddA_cumsum, (int)nheads, hpg, (int)ngroups,
+                           (int)seqlen, (int)d.C, deal.units, deal.splits);
+        return launched();
+      }
+    }
     if (dtype == SSD_BF16) {
       if (hdim == 64) SSD_DDA_LAUNCH(bf16_t, 64);
       else SSD_DDA_LAUNCH(bf16_t, 128);

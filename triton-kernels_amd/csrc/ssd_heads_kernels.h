@@ -815,4 +815,292 @@ __global__ __launch_bounds__(512, 2) void ssd_chunk_scan_bwd_dx_heads_kernel(
   }
 }
 
+// ------------------------------------------------------------------------------------
+// Gradient of the causal term with respect to the per-position dA (ssd_ddA_causal_kernel): with
+//   W[m][n] = <dout[m], x[n]> * dt_n * cb[m][n] * exp(min(dA_m - dA_n, 0))   for n < m < limit,
+// ddA[j] = sum_{i < j} (colsum_i - rowsum_i).  A strip's blocks of 16 x 16 up to the diagonal one; the row sums stay in
+// registers, the column sums of a wave meet those of the others in LDS, and one wave, a head later, forms the prefix
+// sum.  us by the kernel of one head per workgroup and here: b8 nh32 L8192 213 -> 168 (3.6 TB/s of its 600 MB), b2 nh32 L8192 with
+// two groups 53 -> 48, b1 nh32 L2048 14.3 -> 11.7.  Alone, the copies take 119 and the rest 125.
+// ------------------------------------------------------------------------------------
+struct DdaHeadsSmem : HeadsTile {
+  static constexpr int R = 3;                                // heads in LDS, of x, dA and dt
+  static constexpr int kHead = kRows + kVec;
+  static constexpr int kSums = 8 * Q * (int)sizeof(float);   // a wave's sums of columns less those of its rows, each
+  static constexpr int kBytes = R * kHead + kRows + kFactors + 2 * kSums;  // + dout, the sums of two heads
+};
+
+template <bool EVEN>
+__global__ __launch_bounds__(512, 2) void ssd_ddA_heads_kernel(
+    const bf16_t* __restrict__ x, Strides3 sx, const bf16_t* __restrict__ dout, Strides3 sd, const float* __restrict__ dt,
+    const float* __restrict__ dA_cs, const float* __restrict__ cb, float* __restrict__ ddA, int nh, int heads_per_group,
+    int ngroups, int L, int C, int units, int splits) {
+  using S = DdaHeadsSmem;
+  using T = bf16_t;
+  constexpr int P = S::P, Q = S::Q;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+  HeadsWalk<EVEN> now(xcd_local_index((int)blockIdx.x, (int)gridDim.x), (int)gridDim.x, units, splits, heads_per_group, ngroups, C);
+  HeadsWalk<EVEN> ahead = now;  // the head whose copies are requested next
+  // the wave's strips: number `strip`, rows 16 strip .., as many blocks of columns below the diagonal one
+  int strip[2];
+  float* fk[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) strip[j] = S::strip(wave, j);
+  unsigned char* own = smem + S::R * S::kHead;  // dout, each row read by one wave only
+  fk[1] = reinterpret_cast<float*>(own + S::kRows) + wave * 288;
+  fk[0] = fk[1] + 16 * (strip[1] + 1);
+  auto sums = [&](int i) { return reinterpret_cast<float*>(own + S::kRows + S::kFactors + (i & 1) * S::kSums); };
+
+  auto vec_at = [&](const HeadsWalk<EVEN>& w) { return (((int64_t)w.b * nh + w.head()) * C + w.c) * Q; };
+  HeadsWalk<EVEN> ahead_own = now;  // the head whose rows of dout are requested next: one ahead, where the others are two
+  auto request = [&](int u, int ln) {
+    const HeadsWalk<EVEN>& w = ahead;
+    unsigned char* base = smem + u * S::kHead;
+    S::copy_rows<4>(x + w.b * sx.sb + (int64_t)w.c * Q * sx.sl + w.head() * sx.sh, (int)sx.sl, 32 * wave, min(Q, L - w.c * Q),
+                    base + 4 * wave * 1024, ln);
+    if (wave < 2) copy16_to_lds((wave == 0 ? dA_cs : dt) + vec_at(w), 16u * (unsigned)ln, base + S::kRows + wave * 1024);
+    ahead.next();
+  };
+  auto request_own = [&](int ln) {
+    const HeadsWalk<EVEN>& w = ahead_own;
+    const T* dg = dout + w.b * sd.sb + (int64_t)w.c * Q * sd.sl + w.head() * sd.sh;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) S::copy_rows<2>(dg, (int)sd.sl, 16 * strip[j], min(Q, L - w.c * Q), own + strip[j] * 2048, ln);
+    ahead_own.next();
+  };
+  request(0, lane);
+  request_own(lane);
+  if (!ahead.done()) request(1, lane);
+
+  // What the heads of a set share: the blocks of cb in the accumulator layout (rows 4 (l / 16) .. + 3, column l % 16),
+  // the diagonal one apart with its entries from the diagonal on zero; rows past the sequence zero.
+  float cb0[7][4], cb1[15][4], cbd[2][4];
+  int limit = 0;
+  auto load_shared = [&]() {
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+    limit = min(Q, L - now.c * Q);
+    const float* cbg = cb + (((int64_t)now.b * C + now.c) * ngroups + now.g) * (Q * Q);
+    const int col = ln & 15, row = 4 * (ln >> 4);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const float* p = cbg + (16 * strip[j] + row) * Q + col;
+#pragma unroll
+      for (int nb = 0; nb < 15; ++nb)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          if (j == 1) cb1[nb][v] = p[v * Q + 16 * nb];
+          else if (nb < 7) cb0[nb][v] = p[v * Q + 16 * nb];
+        }
+#pragma unroll
+      for (int v = 0; v < 4; ++v) cbd[j][v] = p[v * Q + 16 * strip[j]];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const bool in = 16 * strip[j] + row + v < limit;
+#pragma unroll
+        for (int nb = 0; nb < 15; ++nb) {
+          if (j == 1) cb1[nb][v] = in ? cb1[nb][v] : 0.f;
+          else if (nb < 7) cb0[nb][v] = in ? cb0[nb][v] : 0.f;
+        }
+        cbd[j][v] = in && col < row + v ? cbd[j][v] : 0.f;
+      }
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+#pragma unroll
+      for (int nb = 0; nb < 15; ++nb) {
+        asm volatile("" : "+v"(cb1[nb][v]));
+        if (nb < 7) asm volatile("" : "+v"(cb0[nb][v]));
+      }
+      asm volatile("" : "+v"(cbd[0][v]), "+v"(cbd[1][v]));
+    }
+  };
+
+  // delta_i = colsum_i - rowsum_i; ddA[j] = sum_{i<j} delta_i: one wave, four positions per lane
+  int64_t before = 0;  // where the head before has its dA
+  auto finish = [&](int i) {
+    const float* s = sums(i);
+    float d[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < 8; ++w) {
+      const float4 t = *reinterpret_cast<const float4*>(s + w * Q + 4 * lane);
+      d[0] += t.x, d[1] += t.y, d[2] += t.z, d[3] += t.w;
+    }
+    const float local = (d[0] + d[1]) + (d[2] + d[3]);
+    float4 o;
+    o.x = wave_inclusive_scan(local) - local;
+    o.y = o.x + d[0], o.z = o.y + d[1], o.w = o.z + d[2];
+    *reinterpret_cast<float4*>(ddA + before + 4 * lane) = o;
+  };
+
+  int i = 0;
+  if (!EVEN) load_shared();
+  for (int u = 0; !now.done(); now.next(), ++i, u = u + 1 < S::R ? u + 1 : 0) {
+    if (EVEN && now.k == 0) load_shared();
+    // the head's rows have landed once only x of the next head, requested behind them, is outstanding
+    wait_outstanding<4>(now.unit + 1 < now.end ? 4 : 0);
+    __syncthreads();  // every wave's part of the head is there; every wave is done with the head before
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+    const int l16 = ln & 15, quad = ln >> 4;
+    const unsigned char* base = smem + u * S::kHead;
+    const T* Xs = reinterpret_cast<const T*>(base);
+    const float* dAs = reinterpret_cast<const float*>(base + S::kRows);
+    const float* dts = dAs + Q;
+    float* colsum = sums(i) + wave * Q;
+    // the rows of dout go to registers and their place to the next head's
+    Vec16<T> df[2][2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+        df[j][ks] = load16(reinterpret_cast<const T*>(own) + (16 * strip[j] + l16) * P + 8 * ((4 * ks + quad) ^ S::key(l16)));
+    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(df[0][0].raw), "+v"(df[0][1].raw), "+v"(df[1][0].raw), "+v"(df[1][1].raw)::"memory");
+    if (!ahead_own.done()) request_own(ln);
+    if (!ahead.done()) request(u > 0 ? u - 1 : S::R - 1, ln);  // (the place of the head before)
+    if (i > 0 && wave == (i & 7)) finish(i - 1);
+    before = vec_at(now);
+
+    // The decay is split as in the chunk scan: a factor of the column, exp(r - dA_n) dt_n, one of the row, exp(dA_m - r).
+    const float4 ak = *reinterpret_cast<const float4*>(dAs + 4 * ln);
+    const float4 tk = S::weights_of_time(dts, ln, limit);
+    const float an = dAs[min(4 * ln + 4, Q - 1)];
+    const bool split = __builtin_amdgcn_ballot_w64(S::falls(ak, an, ln, limit) & S::finite(tk)) == ~0ull;
+    bool narrow[2];
+    float em[2][4];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int r0 = 16 * strip[j];
+      const float a0 = dAs[r0], a1 = dAs[min(r0 + 7, limit - 1)], a2 = dAs[min(r0 + 15, limit - 1)];
+      narrow[j] = __builtin_amdgcn_readfirstlane(a0 - a1 <= 40.f && a1 - a2 <= 40.f);
+      const float ar = narrow[j] ? a1 : a0;
+      const float4 f = make_float4(__expf(fminf(ar - ak.x, 40.f)) * tk.x, __expf(fminf(ar - ak.y, 40.f)) * tk.y,
+                                   __expf(fminf(ar - ak.z, 40.f)) * tk.z, __expf(fminf(ar - ak.w, 40.f)) * tk.w);
+      if (4 * ln < r0 + 16) *reinterpret_cast<float4*>(fk[j] + 4 * ln) = f;
+      const float4 am = *reinterpret_cast<const float4*>(dAs + r0 + 4 * quad);
+      em[j][0] = __expf(fminf(am.x - ar, 40.f)), em[j][1] = __expf(fminf(am.y - ar, 40.f));
+      em[j][2] = __expf(fminf(am.z - ar, 40.f)), em[j][3] = __expf(fminf(am.w - ar, 40.f));
+    }
+    const int x_lane = l16 * P + 8 * (quad ^ S::key(l16));  // (the second half of the features: bit 2 of the piece)
+    auto x_frag = [&](int nb, int ks) { return load16(Xs + (16 * nb) * P + (x_lane ^ (32 * ks))); };
+    auto product = [&](int j, const Vec16<T>* xf) {
+      floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+      mma16(df[j][0], xf[0], acc);
+      mma16(df[j][1], xf[1], acc);
+      return acc;
+    };
+    floatx4 rows[2];
+    rows[0] = rows[1] = floatx4{0.f, 0.f, 0.f, 0.f};
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // the wave's own factors are visible to its own reads
+
+    // column sums of block nb over the lane's rows; of the diagonal blocks
+    float col[16], diag[2] = {0.f, 0.f};
+#pragma unroll
+    for (int nb = 0; nb < 16; ++nb) col[nb] = 0.f;
+    const bool fast[2] = {split && narrow[0], split && narrow[1]};
+    if (split) {
+      auto block = [&](int j, const floatx4& acc, const float* w, float gn) {
+        float s = 0.f;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const float u = acc[v] * w[v];
+          rows[j][v] = fmaf(u, gn, rows[j][v]);
+          s = fmaf(u, em[j][v], s);
+        }
+        return s * gn;
+      };
+      // the diagonal blocks first (their products wait for nothing the others need), the others two ahead with their
+      // reads and one ahead with their products
+      const Vec16<T> xd0[2] = {x_frag(strip[0], 0), x_frag(strip[0], 1)}, xd1[2] = {x_frag(strip[1], 0), x_frag(strip[1], 1)};
+      const float dg0 = fk[0][16 * strip[0] + l16], dg1 = fk[1][16 * strip[1] + l16];
+      struct Piece {
+        Vec16<T> xf[2];
+        float g0, g1;
+      };
+      auto fetch = [&](Piece& p, int nb) {
+        p.xf[0] = x_frag(nb, 0), p.xf[1] = x_frag(nb, 1);
+        p.g1 = fk[1][16 * nb + l16];
+        if (nb < 7) p.g0 = fk[0][16 * nb + l16];
+      };
+      Piece piece[2];
+      fetch(piece[0], 0);
+      floatx4 d0 = product(0, xd0), d1 = product(1, xd1);
+      fetch(piece[1], 1);
+      floatx4 p0 = product(0, piece[0].xf), p1 = product(1, piece[0].xf);
+      float g0 = piece[0].g0, g1 = piece[0].g1;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {  // (a select, so that no product of an entry past the diagonal is met)
+        d0[v] = l16 < 4 * quad + v ? d0[v] : 0.f;
+        d1[v] = l16 < 4 * quad + v ? d1[v] : 0.f;
+      }
+      if (fast[0]) diag[0] = block(0, d0, cbd[0], dg0);
+      if (fast[1]) diag[1] = block(1, d1, cbd[1], dg1);
+#pragma unroll
+      for (int nb = 0; nb < 15; ++nb) {
+        if (nb >= 8 && nb >= strip[1]) break;  // (the strips of the lower half have eight blocks or more)
+        fetch(piece[nb & 1], nb + 2 < 16 ? nb + 2 : 15);
+        const floatx4 n1 = product(1, piece[(nb + 1) & 1].xf);
+        floatx4 n0;
+        if (nb < 6) n0 = product(0, piece[(nb + 1) & 1].xf);
+        const float m0 = piece[(nb + 1) & 1].g0, m1 = piece[(nb + 1) & 1].g1;
+        col[nb] = block(1, p1, cb1[nb], g1);
+        if (nb < 7 && nb < strip[0]) col[nb] += block(0, p0, cb0[nb < 7 ? nb : 0], g0);
+        p1 = n1, g1 = m1;
+        if (nb < 6) p0 = n0, g0 = m0;
+      }
+    }
+    diag[0] = quad_sum(diag[0]), diag[1] = quad_sum(diag[1]);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {  // the sums of four blocks over the groups of 16 lanes: lane group q holds block 4 i + q
+      const float lo = swap16_sum(col[4 * q], col[4 * q + 1]), hi = swap16_sum(col[4 * q + 2], col[4 * q + 3]);
+      colsum[64 * q + ln] = swap32_sum(lo, hi);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      if (quad == j) colsum[16 * strip[j] + l16] += diag[j];
+    // ---- diagonal blocks along which dA falls steeply, and everything where it rises: weights as they are defined
+    floatx4 exact[2];  // row sums that the row factor does not apply to
+    exact[0] = exact[1] = floatx4{0.f, 0.f, 0.f, 0.f};
+    if (!(fast[0] && fast[1]))
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int r0 = 16 * strip[j];
+#pragma unroll 1
+        for (int nb = split ? strip[j] + fast[j] : 0; nb <= strip[j]; ++nb) {
+          const Vec16<T> xf[2] = {x_frag(nb, 0), x_frag(nb, 1)};
+          const floatx4 acc = product(j, xf);
+          const int n = 16 * nb + l16;
+          const float* cbg = cb + (((int64_t)now.b * C + now.c) * ngroups + now.g) * (Q * Q);
+          const float an = dAs[n], tn = dts[n];
+          float s = 0.f;
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            const int m = r0 + 4 * quad + v;
+            const float f = acc[v] * cbg[m * Q + n] * tn * __expf(fminf(dAs[m] - an, 0.f));
+            const float w = n < m && m < limit ? f : 0.f;
+            exact[j][v] += w;
+            s += w;
+          }
+          s = quad_sum(s);
+          if (quad == 0) colsum[n] += s;
+        }
+      }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      float4 r;
+      r.x = row16_sum(fmaf(rows[j][0], em[j][0], exact[j][0])), r.y = row16_sum(fmaf(rows[j][1], em[j][1], exact[j][1]));
+      r.z = row16_sum(fmaf(rows[j][2], em[j][2], exact[j][2])), r.w = row16_sum(fmaf(rows[j][3], em[j][3], exact[j][3]));
+      if (l16 == 0) {
+        float4* own_rows = reinterpret_cast<float4*>(colsum + 16 * strip[j] + 4 * quad);
+        const float4 t = *own_rows;
+        *own_rows = make_float4(t.x - r.x, t.y - r.y, t.z - r.z, t.w - r.w);
+      }
+    }
+  }
+  __syncthreads();
+  if (wave == 0) finish(i - 1);
+}
+
 }  // namespace ssd
