@@ -41,6 +41,40 @@ struct StateLaunch {
   }
 };
 
+// The stages ahead of the state passing in one launch (ssd_front_kernel).
+struct FrontLaunch {
+  const void *x, *B, *C;
+  Strides3 sx, sB, sC;
+  const void* dt;
+  int dt_dtype;
+  Strides3 sd;
+  const float *A, *bias;
+  float *dA, *dt_out;
+  int softplus;
+  float dt_min, dt_max;
+  float *states, *cb;
+  Dims d;
+  SeqIdx seq;
+  hipStream_t st;
+  template <typename T, int P, int N>
+  int run() const {
+    return dt_dtype == SSD_BF16 ? run_as<T, P, N, bf16_t>() : run_as<T, P, N, float>();
+  }
+  template <typename T, int P, int N, typename TD>
+  int run_as() const {
+    auto kernel = ssd_front_kernel<T, P, N, TD>;
+    const int smem = front_smem_bytes<T, P, N>((int)d.Q);
+    SSD_TRY(allow_smem(kernel, smem));
+    const int tiles = (int)((d.Q + 63) / 64);
+    const int64_t nstate = d.batch * d.C * d.nh, grid = nstate + d.batch * d.C * d.g * tiles * tiles;
+    if (grid > 0x7fffffff) return SSD_ERR_SHAPE;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(256), smem, st, (const T*)x, sx, (const T*)B, sB, (const T*)C, sC,
+                       DtSource<TD>{(const TD*)dt, sd, A, bias, dA, dt_out, softplus, dt_min, dt_max}, states, cb, (int)d.nh,
+                       (int)d.g, (int)d.L, (int)d.Q, (int)d.C, (int)nstate, tiles, seq);
+    return launched();
+  }
+};
+
 struct WalkLaunch {
   const void *x, *B;
   Strides3 sx, sB;
@@ -799,24 +833,26 @@ int ssd_combined_fwd(const void* x, int64_t x_sb, int64_t x_sl, int64_t x_sh, in
   if (local_states) SSD_TRY(check_f32(local_states));
   if (initial) SSD_TRY(check_f32(initial));
   const int64_t C_ = d.C, tiles = (chunk + 63) / 64;
-  if (batch * C_ * nheads * tiles > 0x7fffffff || batch * C_ * ngroups * tiles * tiles > 0x7fffffff ||
+  if (batch * C_ * nheads * tiles > 0x7fffffff || batch * C_ * (nheads + ngroups * tiles * tiles) > 0x7fffffff ||
       batch * nheads * ((hdim * dstate + 1023) / 1024) > 0x7fffffff)
     return SSD_ERR_SHAPE;
-  SSD_TRY(ssd_chunk_cumsum_fwd(dt, dt_dtype, dt_sb, dt_sl, dt_sh, A, dt_bias, dA_cumsum, dt_out, batch, seqlen,
-                               nheads, chunk, dt_softplus, dt_min, dt_max, stream));
   if (local_states) {
-    SSD_TRY(ssd_chunk_state_fwd(B, b_sb, b_sl, b_sg, x, x_sb, x_sl, x_sh, dtype, dt_out, dA_cumsum, local_states,
-                                batch, seqlen, nheads, ngroups, hdim, dstate, chunk, seq_idx, seq_sb, seq_sl, stream));
+    SSD_TRY(dispatch_tpn(dtype, hdim, dstate,
+                         FrontLaunch{x, B, C, Strides3{x_sb, x_sl, x_sh}, Strides3{b_sb, b_sl, b_sg}, Strides3{c_sb, c_sl, c_sg},
+                                     dt, dt_dtype, Strides3{dt_sb, dt_sl, dt_sh}, A, dt_bias, dA_cumsum, dt_out, dt_softplus,
+                                     dt_min, dt_max, local_states, cb, d, as_seq(seq_idx, seq_sb, seq_sl), as_stream(stream)}));
     SSD_TRY(ssd_state_passing_fwd(local_states, dA_cumsum + (chunk - 1), nheads * C_ * chunk, C_ * chunk, chunk,
                                   initial, states, dtype, final_states, batch, C_, nheads, hdim * dstate, seq_idx,
                                   seq_sb, seq_sl, seqlen, chunk, stream));
   } else {
+    SSD_TRY(ssd_chunk_cumsum_fwd(dt, dt_dtype, dt_sb, dt_sl, dt_sh, A, dt_bias, dA_cumsum, dt_out, batch, seqlen,
+                                 nheads, chunk, dt_softplus, dt_min, dt_max, stream));
+    SSD_TRY(ssd_bmm_chunk_fwd(C, c_sb, c_sl, c_sg, B, b_sb, b_sl, b_sg, dtype, cb, SSD_F32, batch, seqlen, ngroups,
+                              dstate, chunk, seq_idx, seq_sb, seq_sl, stream));
     SSD_TRY(ssd_chunk_state_passing_fwd(B, b_sb, b_sl, b_sg, x, x_sb, x_sl, x_sh, dtype, dt_out, dA_cumsum, initial,
                                         states, dtype, final_states, batch, seqlen, nheads, ngroups, hdim, dstate,
                                         chunk, stream));
   }
-  SSD_TRY(ssd_bmm_chunk_fwd(C, c_sb, c_sl, c_sg, B, b_sb, b_sl, b_sg, dtype, cb, SSD_F32, batch, seqlen, ngroups,
-                            dstate, chunk, seq_idx, seq_sb, seq_sl, stream));
   SSD_TRY(ssd_chunk_scan_fwd(cb, x, x_sb, x_sl, x_sh, z, z_sb, z_sl, z_sh, dtype, dt_out, dA_cumsum, C, c_sb, c_sl,
                              c_sg, states, dtype, D, d_has_hdim, out, o_sb, o_sl, o_sh, out_x, batch, seqlen, nheads,
                              ngroups, hdim, dstate, chunk, seq_idx, seq_sb, seq_sl, stream));

@@ -327,6 +327,42 @@ __device__ __forceinline__ void stage_state(T* tile, const TS* __restrict__ g, i
 // across the chunk with DPP, each lane owning ceil(Q/64) consecutive positions.  Outputs are
 // (b, nh, C, Q) float32.  LDS: HT * (Q + 1) floats.
 // ------------------------------------------------------------------------------------
+// A step size as the stages use it: bias, softplus with the identity above 20, clamp.
+__device__ __forceinline__ float processed_dt(float t, float bias, int softplus, float dt_min, float dt_max) {
+  t += bias;
+  if (softplus && t <= 20.f) t = log1pf(__expf(t));
+  return fminf(fmaxf(t, dt_min), dt_max);
+}
+// The cumsum of row[q] * a over a chunk by one wave, each lane owning ceil(Q/64) consecutive positions; each(q, dt, cumsum)
+// receives the positions one by one, all4(q, dt, cumsum) four at a time where a lane owns four (chunks of 256).
+template <typename F, typename F4>
+__device__ __forceinline__ void cumsum_row(const float* row, float a, int Q, int lane, F each, F4 all4) {
+  const int per = (Q + 63) >> 6;
+  const int q0 = lane * per;
+  float local = 0.f;
+  for (int i = 0; i < per; ++i)
+    if (q0 + i < Q) local += row[q0 + i] * a;
+  float run = wave_inclusive_scan(local) - local;
+  if (per == 4 && Q == 256) {
+    float4 v4, c4;
+    v4.x = row[q0], v4.y = row[q0 + 1], v4.z = row[q0 + 2], v4.w = row[q0 + 3];
+    c4.x = run += v4.x * a;
+    c4.y = run += v4.y * a;
+    c4.z = run += v4.z * a;
+    c4.w = run += v4.w * a;
+    all4(q0, v4, c4);
+    return;
+  }
+  for (int i = 0; i < per; ++i) {
+    const int q = q0 + i;
+    if (q < Q) {
+      const float v = row[q];
+      run += v * a;
+      each(q, v, run);
+    }
+  }
+}
+
 template <typename TD>
 __global__ __launch_bounds__(256) void ssd_cumsum_kernel(const TD* __restrict__ dt, Strides3 sd,
                                                          const float* __restrict__ A,
@@ -357,47 +393,23 @@ __global__ __launch_bounds__(256) void ssd_cumsum_kernel(const TD* __restrict__ 
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int q = qb + u * qstep;
-        float t = v[u] + bias;
-        if (softplus && t <= 20.f) t = log1pf(__expf(t));
-        t = fminf(fmaxf(t, dt_min), dt_max);
+        const float t = processed_dt(v[u], bias, softplus, dt_min, dt_max);
         if (q < Q) tile[j * pitch + q] = q < limit ? t : 0.f;
       }
     }
   }
   __syncthreads();
-  const int per = (Q + 63) >> 6;
-  const int q0 = lane * per;
   for (int jj = wave; jj < HT && h0 + jj < nh; jj += 4) {
     const int h = h0 + jj;
-    const float a = A[h];
-    const float* row = tile + jj * pitch;
-    float local = 0.f;
-    for (int i = 0; i < per; ++i)
-      if (q0 + i < Q) local += row[q0 + i] * a;
-    float run = wave_inclusive_scan(local) - local;
     const int64_t id = (b * nh + h) * C + c;
     float* o_cs = dA_cs + id * Q;
     float* o_dt = dt_out + id * Q;
-    if (per == 4 && Q == 256) {  // the lane's four positions leave as one 16-byte store per output
-      float4 v4, c4;
-      v4.x = row[q0], v4.y = row[q0 + 1], v4.z = row[q0 + 2], v4.w = row[q0 + 3];
-      c4.x = run += v4.x * a;
-      c4.y = run += v4.y * a;
-      c4.z = run += v4.z * a;
-      c4.w = run += v4.w * a;
-      *reinterpret_cast<float4*>(o_dt + q0) = v4;
-      *reinterpret_cast<float4*>(o_cs + q0) = c4;
-      continue;
-    }
-    for (int i = 0; i < per; ++i) {
-      const int q = q0 + i;
-      if (q < Q) {
-        const float v = row[q];
-        run += v * a;
-        o_dt[q] = v;
-        o_cs[q] = run;
-      }
-    }
+    cumsum_row(
+        tile + jj * pitch, A[h], Q, lane, [&](int q, float v, float run) { o_dt[q] = v, o_cs[q] = run; },
+        [&](int q, const float4& v, const float4& run) {  // (one 16-byte store per output)
+          *reinterpret_cast<float4*>(o_dt + q) = v;
+          *reinterpret_cast<float4*>(o_cs + q) = run;
+        });
   }
 }
 
@@ -422,27 +434,42 @@ struct StateSmem {
   static constexpr int kBytes = kStage;
 };
 
-template <typename T, int P, int N, int MODE, typename TO>
-__global__ __launch_bounds__(256) void ssd_chunk_state_kernel(
+// What the body needs to form dt and dA itself (one head, one chunk), for callers that do not have them yet.
+template <typename TD>
+struct DtSource {
+  const TD* dt;
+  Strides3 sd;
+  const float *A, *bias;
+  float *dA_out, *dt_out;
+  int softplus;
+  float dt_min, dt_max;
+};
+struct NoDtSource {};
+
+// bid: the workgroup's (b, c, h).  With a DtSource the chunk's dt and dA are formed here, left in LDS behind the stage
+// (2 Q floats) and stored; dt and dA_cs are not read then.
+template <typename T, int P, int N, int MODE, typename TO, typename SRC>
+__device__ __forceinline__ void chunk_state_body(
     const T* __restrict__ x, Strides3 sx, const T* __restrict__ B, Strides3 sB,
     const float* __restrict__ dt, const float* __restrict__ dA_cs, TO* __restrict__ states, int nh,
-    int heads_per_group, int L, int Q, int C, SeqIdx seq) {
+    int heads_per_group, int L, int Q, int C, SeqIdx seq, int bid, unsigned char* smem, const SRC& src) {
+  constexpr bool FORM = !std::is_same<SRC, NoDtSource>::value;
   using S = StateSmem<T, P, N>;
   constexpr int KT = S::KT, PX = S::PX, PB = S::PB, KG = Tile<T>::KG;
   constexpr int MB = P / 32, NB = N / 32, BPW = MB * NB / 4;
   static_assert(MB * NB % 4 == 0, "output blocks must split over 4 waves");
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   T* xs = reinterpret_cast<T*>(smem);
   T* bs = xs + KT * PX;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int bid = xcd_local_index((int)blockIdx.x, (int)gridDim.x);
   const int h = bid % nh;
   const int c = (bid / nh) % C;
   const int64_t b = bid / (nh * C);
   const int limit = min(Q, L - c * Q);
-  const float* dAp = dA_cs + ((b * nh + h) * C + c) * (int64_t)Q;
-  const float* dtp = dt + ((b * nh + h) * C + c) * (int64_t)Q;
-  const float dA_last = dAp[Q - 1];
+  float* dts = reinterpret_cast<float*>(smem + S::kBytes);
+  float* dAs = dts + Q;
+  const float* dAp = FORM ? nullptr : dA_cs + ((b * nh + h) * C + c) * (int64_t)Q;
+  const float* dtp = FORM ? nullptr : dt + ((b * nh + h) * C + c) * (int64_t)Q;
+  float dA_last = FORM ? 0.f : dAp[Q - 1];
   const T* xg = x + b * sx.sb + (int64_t)c * Q * sx.sl + h * sx.sh;
   const T* Bg = B + b * sB.sb + (int64_t)c * Q * sB.sl + (h / heads_per_group) * sB.sh;
   const ChunkSeq sq = chunk_seq(seq, b, c, Q);
@@ -456,6 +483,7 @@ __global__ __launch_bounds__(256) void ssd_chunk_state_kernel(
   // Stage s + 1 is requested before the products of stage s and written to LDS after them: the
   // loads have the products to hide behind.
   auto scale_b = [&](int k, float dA_k, float dt_k) {
+    if constexpr (FORM) dA_k = dAs[k], dt_k = dts[k];
     const float w = __expf(fminf(dA_last - dA_k, 0.f)) * dt_k;
     return (sq.on() && (seq_dead || sq.at(k) != seq_ref)) ? 0.f : w;
   };
@@ -469,7 +497,34 @@ __global__ __launch_bounds__(256) void ssd_chunk_state_kernel(
     px.template load<true>(xg, sx.sl, k0, limit, tid, MODE == 1 ? dAp : nullptr);
     pb.load(Bg, sB.sl, k0, limit, tid, MODE == 0 ? dAp : nullptr, MODE == 0 ? dtp : nullptr);
   };
-  request(0);
+  if constexpr (FORM) {  // (the chunk's dt is requested ahead of the first stage and waited for behind its requests)
+    const auto* g = src.dt + b * src.sd.sb + (int64_t)c * Q * src.sd.sl + (int64_t)h * src.sd.sh;
+    const float bias = src.bias ? src.bias[h] : 0.f;
+    const float a = src.A[h];
+    float v = (float)g[(int64_t)min(tid, limit - 1) * src.sd.sl];
+    request(0);
+    for (int q = tid; q < Q; q += 256) {
+      if (q >= 256) v = (float)g[(int64_t)min(q, limit - 1) * src.sd.sl];
+      dts[q] = q < limit ? processed_dt(v, bias, src.softplus, src.dt_min, src.dt_max) : 0.f;
+    }
+    __syncthreads();
+    if (wave == 0) {
+      const int64_t at = ((b * nh + h) * C + c) * (int64_t)Q;
+      float* o_dt = src.dt_out + at;
+      float* o_cs = src.dA_out + at;
+      cumsum_row(
+          dts, a, Q, lane, [&](int q, float t, float run) { o_dt[q] = t, o_cs[q] = run, dAs[q] = run; },
+          [&](int q, const float4& t, const float4& run) {
+            *reinterpret_cast<float4*>(o_dt + q) = t;
+            *reinterpret_cast<float4*>(o_cs + q) = run;
+            *reinterpret_cast<float4*>(dAs + q) = run;
+          });
+    }
+    __syncthreads();
+    dA_last = dAs[Q - 1];
+  } else {
+    request(0);
+  }
   T* xb = xs;
   T* bb = bs;
   for (int k0 = 0; k0 < limit; k0 += KT) {
@@ -500,6 +555,16 @@ __global__ __launch_bounds__(256) void ssd_chunk_state_kernel(
     for (int v = 0; v < 16; ++v)
       __builtin_nontemporal_store((TO)acc[i][v], out + (int64_t)(32 * mi + acc_row(v, lane)) * N + 32 * ni + (lane & 31));
   }
+}
+
+template <typename T, int P, int N, int MODE, typename TO>
+__global__ __launch_bounds__(256) void ssd_chunk_state_kernel(
+    const T* __restrict__ x, Strides3 sx, const T* __restrict__ B, Strides3 sB,
+    const float* __restrict__ dt, const float* __restrict__ dA_cs, TO* __restrict__ states, int nh,
+    int heads_per_group, int L, int Q, int C, SeqIdx seq) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  chunk_state_body<T, P, N, MODE, TO>(x, sx, B, sB, dt, dA_cs, states, nh, heads_per_group, L, Q, C, seq,
+                                      xcd_local_index((int)blockIdx.x, (int)gridDim.x), smem, NoDtSource());
 }
 
 // Non-temporal 16-byte accesses for data that a kernel touches once.
@@ -1733,16 +1798,13 @@ constexpr int bmm_smem_bytes() {
 }
 
 template <typename T, typename TO, int K>
-__global__ __launch_bounds__(256) void ssd_bmm_kernel(const T* __restrict__ a, Strides3 sa,
-                                                      const T* __restrict__ bm, Strides3 sb_,
-                                                      TO* __restrict__ out, int ngroups, int L, int Q, int C,
-                                                      int tiles, SeqIdx seq) {
+__device__ __forceinline__ void bmm_body(const T* __restrict__ a, Strides3 sa, const T* __restrict__ bm, Strides3 sb_,
+                                         TO* __restrict__ out, int ngroups, int L, int Q, int C, int tiles, SeqIdx seq,
+                                         int bid, unsigned char* smem) {
   constexpr int PK = Tile<T>::pitch(K), KG = Tile<T>::KG;
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   T* as = reinterpret_cast<T*>(smem);
   T* bs = as + 64 * PK;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int bid = xcd_local_index((int)blockIdx.x, (int)gridDim.x);
   const int tn = bid % tiles;
   const int tm = (bid / tiles) % tiles;
   const int64_t bcg = bid / (tiles * tiles);
@@ -1771,6 +1833,41 @@ __global__ __launch_bounds__(256) void ssd_bmm_kernel(const T* __restrict__ a, S
     if (sq.on() && sq.at(min(row, limit - 1)) != col_id) val = 0.f;
     if (row < Q && col < Q) o[(int64_t)row * Q + col] = (TO)val;
   }
+}
+
+template <typename T, typename TO, int K>
+__global__ __launch_bounds__(256) void ssd_bmm_kernel(const T* __restrict__ a, Strides3 sa,
+                                                      const T* __restrict__ bm, Strides3 sb_,
+                                                      TO* __restrict__ out, int ngroups, int L, int Q, int C,
+                                                      int tiles, SeqIdx seq) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  bmm_body<T, TO, K>(a, sa, bm, sb_, out, ngroups, L, Q, C, tiles, seq, xcd_local_index((int)blockIdx.x, (int)gridDim.x), smem);
+}
+
+// ------------------------------------------------------------------------------------
+// The three stages ahead of the state passing in one launch: workgroups 0 .. nstate - 1 form dt and dA of their head and
+// chunk and then its local state, the others the blocks of C . B, which nothing waits for but the chunk scan.  While
+// few workgroups run each launch is the latency of one workgroup and of the launch, and those add up; when many do, the
+// short workgroups of C . B fill the gaps of the others.  The whole forward, us, three launches / one: b1 nh4 L512 chunk 64
+// float32 24.5 / 17.1, b1 nh32 L4096 chunk 256 49.7 / 41.9, b2 nh32 L8192 119 / 111, b4 nh32 L4096 hdim 128 230 / 219.
+// ------------------------------------------------------------------------------------
+template <typename T, int P, int N>
+constexpr int front_smem_bytes(int Q) {
+  const int state = StateSmem<T, P, N>::kBytes + 2 * Q * (int)sizeof(float);
+  return state > bmm_smem_bytes<T, N>() ? state : bmm_smem_bytes<T, N>();
+}
+template <typename T, int P, int N, typename TD>
+__global__ __launch_bounds__(256) void ssd_front_kernel(
+    const T* __restrict__ x, Strides3 sx, const T* __restrict__ B, Strides3 sB, const T* __restrict__ Cm, Strides3 sC,
+    DtSource<TD> src, float* __restrict__ states, float* __restrict__ cb, int nh, int ngroups, int L, int Q, int C,
+    int nstate, int tiles, SeqIdx seq) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int bid = (int)blockIdx.x;
+  if (bid < nstate)
+    chunk_state_body<T, P, N, 0, float>(x, sx, B, sB, nullptr, nullptr, states, nh, nh / ngroups, L, Q, C, seq,
+                                        xcd_local_index(bid, nstate), smem, src);
+  else
+    bmm_body<T, float, N>(Cm, sC, B, sB, cb, ngroups, L, Q, C, tiles, seq, xcd_local_index(bid - nstate, (int)gridDim.x - nstate), smem);
 }
 
 // ------------------------------------------------------------------------------------
