@@ -158,6 +158,14 @@ def on_device(dev: torch.device):
     return _NO_SWITCH if dev.index is None or torch.cuda.current_device() == dev.index else torch.cuda.device(dev)
 
 
+def untracked() -> bool:
+    """Whether nothing can differentiate through a call made now: gradients are off, no forward-mode level is open and no
+    transform is active.  What it returns is then the kernels' result alone, so the call need not go through an autograd
+    function (3.4 us of host time, a sixth of a decoding step)."""
+    return not (torch.is_grad_enabled() or torch.autograd.forward_ad._current_level >= 0
+                or torch._C._are_functorch_transforms_active())
+
+
 def seq_view(x: torch.Tensor):
     """(tensor with unit feature stride, [ptr, sb, sl, sh], batch, nheads, L, T) of a flat
     (B, L, T) or headed (b, L, nh, d) sequence tensor."""
