@@ -847,11 +847,12 @@ int ssd_combined_fwd(const void* x, int64_t x_sb, int64_t x_sl, int64_t x_sh, in
   } else {
     SSD_TRY(ssd_chunk_cumsum_fwd(dt, dt_dtype, dt_sb, dt_sl, dt_sh, A, dt_bias, dA_cumsum, dt_out, batch, seqlen,
                                  nheads, chunk, dt_softplus, dt_min, dt_max, stream));
-    SSD_TRY(ssd_bmm_chunk_fwd(C, c_sb, c_sl, c_sg, B, b_sb, b_sl, b_sg, dtype, cb, SSD_F32, batch, seqlen, ngroups,
-                              dstate, chunk, seq_idx, seq_sb, seq_sl, stream));
     SSD_TRY(ssd_chunk_state_passing_fwd(B, b_sb, b_sl, b_sg, x, x_sb, x_sl, x_sh, dtype, dt_out, dA_cumsum, initial,
                                         states, dtype, final_states, batch, seqlen, nheads, ngroups, hdim, dstate,
                                         chunk, stream));
+    // (last: the chunk scan reads it next)
+    SSD_TRY(ssd_bmm_chunk_fwd(C, c_sb, c_sl, c_sg, B, b_sb, b_sl, b_sg, dtype, cb, SSD_F32, batch, seqlen, ngroups,
+                              dstate, chunk, seq_idx, seq_sb, seq_sl, stream));
   }
   SSD_TRY(ssd_chunk_scan_fwd(cb, x, x_sb, x_sl, x_sh, z, z_sb, z_sl, z_sh, dtype, dt_out, dA_cumsum, C, c_sb, c_sl,
                              c_sg, states, dtype, D, d_has_hdim, out, o_sb, o_sl, o_sh, out_x, batch, seqlen, nheads,
