@@ -1,5 +1,6 @@
 """Calls that nothing can differentiate through skip the autograd functions: the same bits as with gradients on, and what
-an autograd function refuses (forward-mode tangents, transforms) is refused as before."""
+an autograd function refuses (forward-mode tangents, transforms) is refused as before.  A traced call runs the kernel on
+every replay."""
 import pytest
 import torch
 import torch.autograd.forward_ad as fwAD
@@ -33,7 +34,18 @@ def test_tangents_and_transforms_are_refused(name, device):
     call = _calls()[name]
     x, a = torch.randn(2, 5, 3, 64, device=device), -torch.rand(2, 5, 3, device=device)
     with torch.no_grad():
-        with fwAD.dual_level(), pytest.raises(Exception):
+        with fwAD.dual_level(), pytest.raises(NotImplementedError, match="jvp"):
             call(a, fwAD.make_dual(x, torch.ones_like(x)))
-        with pytest.raises(Exception):
+        with pytest.raises(RuntimeError, match="setup_context"):
             torch.func.vmap(call)(a[None], x[None])
+
+
+@pytest.mark.parametrize("name", ["combined", "sequence"])
+def test_traced_calls_run_the_kernel_again(name, device):
+    call = _calls()[name]
+    r = lambda: (-torch.rand(2, 5, 3, device=device), torch.randn(2, 5, 3, 64, device=device))
+    with torch.no_grad():
+        traced = torch.jit.trace(call, r(), check_trace=False)
+        for _ in range(2):
+            a, x = r()
+            assert torch.equal(traced(a, x), call(a, x))

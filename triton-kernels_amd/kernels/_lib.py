@@ -159,11 +159,12 @@ def on_device(dev: torch.device):
 
 
 def untracked() -> bool:
-    """Whether nothing can differentiate through a call made now: gradients are off, no forward-mode level is open and no
-    transform is active.  What it returns is then the kernels' result alone, so the call need not go through an autograd
-    function (3.4 us of host time, a sixth of a decoding step)."""
+    """Whether nothing looks into a call made now: gradients are off, no forward-mode level is open, no transform is
+    active and torch.jit.trace is not recording (it sees an autograd function as one call, but of a launch made through
+    ctypes only the empty tensor that it fills).  What the call returns is then the kernels' result alone, so it need
+    not go through an autograd function (3.4 us of host time, a sixth of a decoding step)."""
     return not (torch.is_grad_enabled() or torch.autograd.forward_ad._current_level >= 0
-                or torch._C._are_functorch_transforms_active())
+                or torch._C._are_functorch_transforms_active() or torch._C._get_tracing_state() is not None)
 
 
 def seq_view(x: torch.Tensor):
