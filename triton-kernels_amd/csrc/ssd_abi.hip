@@ -709,8 +709,8 @@ int ssd_chunk_scan_bwd_ddAcs(const void* x, int64_t x_sb, int64_t x_sl, int64_t 
       // The walk over the heads: where each has a compute unit to itself, and for groups of eight or more.  The other
       // kernel / the walk, us: 64 heads of all (batch, chunk) pairs 11.7 / 9.5, 256 14.3 / 11.7, 288 16.2 / 15.7; groups of six
       // heads, 256 of them, 40 / 43, of eight 56 / 53, of 32 213 / 168; 320 of ten 89 / 85; 128 of four 18.0 / 18.6.
-      // Relative error against float64, A in [-16, -1], b1 nh32 L4096: dt = softplus(n/2 - 2) 8.9e-7 / 8.8e-7, softplus(n/2)
-      // 1.22e-6 / 1.10e-6; very steep decay, softplus(n/2 + 2), 9.1e-7 / 1.15e-6: less exact there.
+      // Relative error against float64, the other kernel / the walk, A in [-16, -1], b1 nh32 L4096, mean of 12 seeds: dt =
+      // softplus(n/2 - 2) 8.8e-7 / 7.6e-7, softplus(n/2) 1.23e-6 / 9.6e-7, softplus(n/2 + 2) 9.1e-7 / 9.4e-7.
       const bool pays = wgs <= 256 || hpg >= 8;
       if (pays && heads_vectors(dt, dA_cumsum) && reinterpret_cast<uintptr_t>(ddA_cumsum) % 16 == 0 && heads_rows(sx) && heads_rows(sd)) {
         constexpr int smem = DdaHeadsSmem::kBytes;

@@ -922,12 +922,10 @@ __global__ __launch_bounds__(512, 2) void ssd_ddA_heads_kernel(
   int64_t before = 0;  // where the head before has its dA
   auto finish = [&](int i) {
     const float* s = sums(i);
-    float d[4] = {0.f, 0.f, 0.f, 0.f};
+    floatx4 t[8];
 #pragma unroll
-    for (int w = 0; w < 8; ++w) {
-      const float4 t = *reinterpret_cast<const float4*>(s + w * Q + 4 * lane);
-      d[0] += t.x, d[1] += t.y, d[2] += t.z, d[3] += t.w;
-    }
+    for (int w = 0; w < 8; ++w) t[w] = *reinterpret_cast<const floatx4*>(s + w * Q + 4 * lane);
+    const floatx4 d = ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
     const float local = (d[0] + d[1]) + (d[2] + d[3]);
     float4 o;
     o.x = wave_inclusive_scan(local) - local;
@@ -963,25 +961,24 @@ __global__ __launch_bounds__(512, 2) void ssd_ddA_heads_kernel(
     if (i > 0 && wave == (i & 7)) finish(i - 1);
     before = vec_at(now);
 
-    // The decay is split as in the chunk scan: a factor of the column, exp(r - dA_n) dt_n, one of the row, exp(dA_m - r).
+    // Below a strip the decay is split at its first row r into a factor of the column, exp(r - dA_n) dt_n, and one of the
+    // row, exp(dA_m - r).  Neither exponent is larger than their sum where dA falls, so the two are no less exact than
+    // the one they stand for (__expf is off by about 6e-8 of its exponent).  The diagonal block, where a split would need
+    // exponents of both signs, takes its weights as they are defined.
     const float4 ak = *reinterpret_cast<const float4*>(dAs + 4 * ln);
     const float4 tk = S::weights_of_time(dts, ln, limit);
     const float an = dAs[min(4 * ln + 4, Q - 1)];
     const bool split = __builtin_amdgcn_ballot_w64(S::falls(ak, an, ln, limit) & S::finite(tk)) == ~0ull;
-    bool narrow[2];
     float em[2][4];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int r0 = 16 * strip[j];
-      const float a0 = dAs[r0], a1 = dAs[min(r0 + 7, limit - 1)], a2 = dAs[min(r0 + 15, limit - 1)];
-      narrow[j] = __builtin_amdgcn_readfirstlane(a0 - a1 <= 40.f && a1 - a2 <= 40.f);
-      const float ar = narrow[j] ? a1 : a0;
-      const float4 f = make_float4(__expf(fminf(ar - ak.x, 40.f)) * tk.x, __expf(fminf(ar - ak.y, 40.f)) * tk.y,
-                                   __expf(fminf(ar - ak.z, 40.f)) * tk.z, __expf(fminf(ar - ak.w, 40.f)) * tk.w);
-      if (4 * ln < r0 + 16) *reinterpret_cast<float4*>(fk[j] + 4 * ln) = f;
+      const float ar = dAs[r0];
+      const float4 f = make_float4(__expf(ar - ak.x) * tk.x, __expf(ar - ak.y) * tk.y, __expf(ar - ak.z) * tk.z,
+                                   __expf(ar - ak.w) * tk.w);
+      if (4 * ln < r0) *reinterpret_cast<float4*>(fk[j] + 4 * ln) = f;
       const float4 am = *reinterpret_cast<const float4*>(dAs + r0 + 4 * quad);
-      em[j][0] = __expf(fminf(am.x - ar, 40.f)), em[j][1] = __expf(fminf(am.y - ar, 40.f));
-      em[j][2] = __expf(fminf(am.z - ar, 40.f)), em[j][3] = __expf(fminf(am.w - ar, 40.f));
+      em[j][0] = am.x, em[j][1] = am.y, em[j][2] = am.z, em[j][3] = am.w;
     }
     const int x_lane = l16 * P + 8 * (quad ^ S::key(l16));  // (the second half of the features: bit 2 of the piece)
     auto x_frag = [&](int nb, int ks) { return load16(Xs + (16 * nb) * P + (x_lane ^ (32 * ks))); };
@@ -999,7 +996,24 @@ __global__ __launch_bounds__(512, 2) void ssd_ddA_heads_kernel(
     float col[16], diag[2] = {0.f, 0.f};
 #pragma unroll
     for (int nb = 0; nb < 16; ++nb) col[nb] = 0.f;
-    const bool fast[2] = {split && narrow[0], split && narrow[1]};
+    floatx4 exact[2];  // row sums that the row factor does not apply to
+    // ---- the diagonal blocks
+    {
+      const Vec16<T> xd0[2] = {x_frag(strip[0], 0), x_frag(strip[0], 1)}, xd1[2] = {x_frag(strip[1], 0), x_frag(strip[1], 1)};
+      const floatx4 d[2] = {product(0, xd0), product(1, xd1)};
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int n = 16 * strip[j] + l16;
+        const float an = dAs[n], tn = n < limit ? dts[n] : 0.f;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {  // (a select, so that no product of an entry past the diagonal is met)
+          const float f = d[j][v] * cbd[j][v] * tn * __expf(fminf(em[j][v] - an, 0.f));
+          exact[j][v] = l16 < 4 * quad + v ? f : 0.f;
+          diag[j] += exact[j][v];
+          em[j][v] = __expf(fminf(em[j][v] - dAs[16 * strip[j]], 0.f));
+        }
+      }
+    }
     if (split) {
       auto block = [&](int j, const floatx4& acc, const float* w, float gn) {
         float s = 0.f;
@@ -1011,10 +1025,7 @@ __global__ __launch_bounds__(512, 2) void ssd_ddA_heads_kernel(
         }
         return s * gn;
       };
-      // the diagonal blocks first (their products wait for nothing the others need), the others two ahead with their
-      // reads and one ahead with their products
-      const Vec16<T> xd0[2] = {x_frag(strip[0], 0), x_frag(strip[0], 1)}, xd1[2] = {x_frag(strip[1], 0), x_frag(strip[1], 1)};
-      const float dg0 = fk[0][16 * strip[0] + l16], dg1 = fk[1][16 * strip[1] + l16];
+      // the blocks two ahead with their reads and one ahead with their products
       struct Piece {
         Vec16<T> xf[2];
         float g0, g1;
@@ -1026,17 +1037,9 @@ __global__ __launch_bounds__(512, 2) void ssd_ddA_heads_kernel(
       };
       Piece piece[2];
       fetch(piece[0], 0);
-      floatx4 d0 = product(0, xd0), d1 = product(1, xd1);
       fetch(piece[1], 1);
       floatx4 p0 = product(0, piece[0].xf), p1 = product(1, piece[0].xf);
       float g0 = piece[0].g0, g1 = piece[0].g1;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {  // (a select, so that no product of an entry past the diagonal is met)
-        d0[v] = l16 < 4 * quad + v ? d0[v] : 0.f;
-        d1[v] = l16 < 4 * quad + v ? d1[v] : 0.f;
-      }
-      if (fast[0]) diag[0] = block(0, d0, cbd[0], dg0);
-      if (fast[1]) diag[1] = block(1, d1, cbd[1], dg1);
 #pragma unroll
       for (int nb = 0; nb < 15; ++nb) {
         if (nb >= 8 && nb >= strip[1]) break;  // (the strips of the lower half have eight blocks or more)
@@ -1060,15 +1063,13 @@ __global__ __launch_bounds__(512, 2) void ssd_ddA_heads_kernel(
 #pragma unroll
     for (int j = 0; j < 2; ++j)
       if (quad == j) colsum[16 * strip[j] + l16] += diag[j];
-    // ---- diagonal blocks along which dA falls steeply, and everything where it rises: weights as they are defined
-    floatx4 exact[2];  // row sums that the row factor does not apply to
-    exact[0] = exact[1] = floatx4{0.f, 0.f, 0.f, 0.f};
-    if (!(fast[0] && fast[1]))
+    // ---- where dA rises: weights as they are defined
+    if (!split)
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const int r0 = 16 * strip[j];
 #pragma unroll 1
-        for (int nb = split ? strip[j] + fast[j] : 0; nb <= strip[j]; ++nb) {
+        for (int nb = 0; nb < strip[j]; ++nb) {
           const Vec16<T> xf[2] = {x_frag(nb, 0), x_frag(nb, 1)};
           const floatx4 acc = product(j, xf);
           const int n = 16 * nb + l16;
@@ -1079,7 +1080,7 @@ __global__ __launch_bounds__(512, 2) void ssd_ddA_heads_kernel(
           for (int v = 0; v < 4; ++v) {
             const int m = r0 + 4 * quad + v;
             const float f = acc[v] * cbg[m * Q + n] * tn * __expf(fminf(dAs[m] - an, 0.f));
-            const float w = n < m && m < limit ? f : 0.f;
+            const float w = m < limit ? f : 0.f;
             exact[j][v] += w;
             s += w;
           }
