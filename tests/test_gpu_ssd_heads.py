@@ -181,3 +181,59 @@ def test_ddA_is_as_exact_as_the_general_kernel(rate, shift, device):
     walk_most, general_most = (sum(c) / len(c) for c in zip(*most))
     print(f"  norm {general:.2e} / {walk:.2e}, largest {general_most:.2e} / {walk_most:.2e}", flush=True)
     assert walk <= 1.15 * general and walk_most <= 1.5 * general_most
+
+
+# ---- forms of the decay that the split has to keep its hands off
+
+WALKS = {"scan": (26, 512, 6, 1, 128), "dx": (6, 512, 6, 1, 128), "ddA": (2, 512, 6, 1, 128)}
+
+
+def _run(name, ops, dt, dA, device, ref=None):
+    """The stage's results on the device, or the oracle's for the batch elements that it looks at."""
+    x, y, BC, cb, states = ops
+    if ref is None:
+        from kernels.mamba_kernels.mamba_scan_fwd import _chunk_scan_fwd
+        from kernels.mamba_kernels_bwd.mamba_chunk_scan_bwd_da import _chunk_scan_bwd_ddAcs_stable
+        from kernels.mamba_kernels_bwd.mamba_chunk_scan_chunk_state_bwd_dx import _chunk_scan_chunk_state_bwd_dx
+
+        x, y, BC, cb, states, dt, dA = (t.to(device) for t in (x, y, BC, cb, states, dt, dA))
+        if name == "scan":
+            return [("out", _chunk_scan_fwd(cb, x, dt, dA, BC, states, z=y)[0], BF16)]
+        if name == "dx":
+            dx, ddt, _ = _chunk_scan_chunk_state_bwd_dx(x, dt, dA, BC, cb, y, states)
+            return [("dx", dx, BF16), ("ddt", ddt, BF16)]
+        return [("ddA", _chunk_scan_bwd_ddAcs_stable(x, dt, dA, y, cb), F32)]
+    x, y, BC, cb, states, dt, dA = (t[ref] for t in (x, y, BC, torch.nan_to_num(cb), states, dt, dA))
+    if name == "scan":
+        return [S.chunk_scan(cb, x, dt, dA, BC, states, z=y, round_to=BF16)[0]]
+    if name == "dx":
+        return list(S.chunk_scan_chunk_state_bwd_dx(x, dt, dA, BC, cb, y, states, round_to=BF16)[:2])
+    return [S.chunk_scan_bwd_ddAcs_stable(x, dt, dA, y, cb)]
+
+
+def _compare(name, got, ref, rows, pick=lambda t: t):
+    for (what, g, dtype), r in zip(got, ref):
+        check_close(f"{name} {what}", pick(g[rows]), pick(r), dtype, regrouped=dtype == BF16, loose=what == "ddt")
+
+
+@pytest.mark.parametrize("L", [257, 263, 271, 272, 290, 400, 511])
+def test_ddA_looks_at_nothing_past_the_sequence(L, device):
+    """dt, dA and cb past the sequence are NaN or infinite; a last position with an infinite dt, which no weight uses.
+    The general kernel does the same."""
+    case = (2, L, 6, 1, 128)
+    announce(f"ddA with anything past position {L}")
+    x, y, BC, dt, dA, cb, states, _ = _inputs(*case, "falling", seed=L)
+    ops, rows, n = (x, y, BC, cb, states), [0, 1], L % Q
+    ref = _run("ddA", ops, dt, dA, device, ref=rows)
+    for junk in (float("nan"), float("inf"), -float("inf"), 1e30):
+        cb[:, -1, :, n:, :] = junk
+        cb[:, -1, :, :, n:] = junk
+        dA[:, :, -1, n:] = junk
+        dt[:, :, -1, n:] = junk
+        for last in (0.5, float("inf")):
+            dt[:, :, -1, n - 1] = last
+            for steps in (dt.to(device), _unaligned(dt.to(device))):
+                got = _run("ddA", ops, steps, dA, device)
+                _compare("ddA", got, ref, rows, lambda t: t[:, :, :-1])
+                _compare("ddA", got, ref, rows, lambda t: t[:, :, -1, :n])
+                assert torch.isfinite(got[0][1]).all()

@@ -875,7 +875,7 @@ __global__ __launch_bounds__(512, 2) void ssd_ddA_heads_kernel(
   if (!ahead.done()) request(1, lane);
 
   // What the heads of a set share: the blocks of cb in the accumulator layout (rows 4 (l / 16) .. + 3, column l % 16),
-  // the diagonal one apart with its entries from the diagonal on zero; rows past the sequence zero.
+  // rows past the sequence zero, and the diagonal ones as they are.
   float cb0[7][4], cb1[15][4], cbd[2][4];
   int limit = 0;
   auto load_shared = [&]() {
@@ -904,7 +904,6 @@ __global__ __launch_bounds__(512, 2) void ssd_ddA_heads_kernel(
           if (j == 1) cb1[nb][v] = in ? cb1[nb][v] : 0.f;
           else if (nb < 7) cb0[nb][v] = in ? cb0[nb][v] : 0.f;
         }
-        cbd[j][v] = in && col < row + v ? cbd[j][v] : 0.f;
       }
     }
 #pragma unroll
@@ -919,13 +918,17 @@ __global__ __launch_bounds__(512, 2) void ssd_ddA_heads_kernel(
   };
 
   // delta_i = colsum_i - rowsum_i; ddA[j] = sum_{i<j} delta_i: one wave, four positions per lane
+  // (0 past the sequence, where the sums hold whatever dt and dA do)
   int64_t before = 0;  // where the head before has its dA
+  int rows_before = 0;  // its positions
   auto finish = [&](int i) {
     const float* s = sums(i);
     floatx4 t[8];
 #pragma unroll
     for (int w = 0; w < 8; ++w) t[w] = *reinterpret_cast<const floatx4*>(s + w * Q + 4 * lane);
-    const floatx4 d = ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
+    floatx4 d = ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
+#pragma unroll
+    for (int k = 0; k < 4; ++k) d[k] = 4 * lane + k < rows_before ? d[k] : 0.f;
     const float local = (d[0] + d[1]) + (d[2] + d[3]);
     float4 o;
     o.x = wave_inclusive_scan(local) - local;
@@ -959,7 +962,7 @@ __global__ __launch_bounds__(512, 2) void ssd_ddA_heads_kernel(
     if (!ahead_own.done()) request_own(ln);
     if (!ahead.done()) request(u > 0 ? u - 1 : S::R - 1, ln);  // (the place of the head before)
     if (i > 0 && wave == (i & 7)) finish(i - 1);
-    before = vec_at(now);
+    before = vec_at(now), rows_before = limit;
 
     // Below a strip the decay is split at its first row r into a factor of the column, exp(r - dA_n) dt_n, and one of the
     // row, exp(dA_m - r).  Neither exponent is larger than their sum where dA falls, so the two are no less exact than
@@ -973,9 +976,9 @@ __global__ __launch_bounds__(512, 2) void ssd_ddA_heads_kernel(
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int r0 = 16 * strip[j];
-      const float ar = dAs[r0];
-      const float4 f = make_float4(__expf(ar - ak.x) * tk.x, __expf(ar - ak.y) * tk.y, __expf(ar - ak.z) * tk.z,
-                                   __expf(ar - ak.w) * tk.w);
+      const float ar = dAs[min(r0, limit - 1)];  // (the factors of strips past the sequence meet zeros, and must be finite)
+      const float4 f = make_float4(__expf(fminf(ar - ak.x, 0.f)) * tk.x, __expf(fminf(ar - ak.y, 0.f)) * tk.y,
+                                   __expf(fminf(ar - ak.z, 0.f)) * tk.z, __expf(fminf(ar - ak.w, 0.f)) * tk.w);
       if (4 * ln < r0) *reinterpret_cast<float4*>(fk[j] + 4 * ln) = f;
       const float4 am = *reinterpret_cast<const float4*>(dAs + r0 + 4 * quad);
       em[j][0] = am.x, em[j][1] = am.y, em[j][2] = am.z, em[j][3] = am.w;
@@ -1006,9 +1009,9 @@ __global__ __launch_bounds__(512, 2) void ssd_ddA_heads_kernel(
         const int n = 16 * strip[j] + l16;
         const float an = dAs[n], tn = n < limit ? dts[n] : 0.f;
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {  // (a select, so that no product of an entry past the diagonal is met)
+        for (int v = 0; v < 4; ++v) {  // (selects, so that no product past the diagonal or the sequence is met)
           const float f = d[j][v] * cbd[j][v] * tn * __expf(fminf(em[j][v] - an, 0.f));
-          exact[j][v] = l16 < 4 * quad + v ? f : 0.f;
+          exact[j][v] = (l16 < 4 * quad + v) & (4 * quad + v < limit - 16 * strip[j]) ? f : 0.f;
           diag[j] += exact[j][v];
           em[j][v] = __expf(fminf(em[j][v] - dAs[16 * strip[j]], 0.f));
         }
