@@ -237,3 +237,37 @@ def test_ddA_looks_at_nothing_past_the_sequence(L, device):
                 _compare("ddA", got, ref, rows, lambda t: t[:, :, :-1])
                 _compare("ddA", got, ref, rows, lambda t: t[:, :, -1, :n])
                 assert torch.isfinite(got[0][1]).all()
+
+
+@pytest.mark.parametrize("at", [4, 100, 252])
+@pytest.mark.parametrize("name", list(WALKS))
+def test_infinite_decay_and_infinite_steps(name, at, device):
+    """dA of -inf from some position on lets nothing through from before it, and positions behind it see each other
+    whole; an infinite dt reaches the rows behind it only."""
+    case = WALKS[name]
+    announce(f"{name} with dA = -inf or dt = inf from position {at}")
+    x, y, BC, dt, dA, cb, states, _ = _inputs(*case, "falling", seed=at)
+    ops, rows = (x, y, BC, cb, states), _some(case[0])[0]
+    cut, far = dA.clone(), dA.clone()
+    cut[:, ::2, :, at:], far[:, ::2, :, at:] = -float("inf"), -3e4
+    _compare(name, _run(name, ops, dt, cut, device), _run(name, ops, dt, far, device, ref=rows), rows)
+    inf, zero = dt.clone(), dt.clone()
+    inf[:, 1::2, :, at], zero[:, 1::2, :, at] = float("inf"), 0
+    got, ref = _run(name, ops, inf, dA, device), _run(name, ops, zero, dA, device, ref=rows)
+    if name == "dx":  # dt scales the position's own row
+        keep = torch.arange(case[1]) % Q != at
+        pick = lambda t: t[:, keep] if t.shape[1] == case[1] else t
+    else:
+        before = lambda t, dim: t.unflatten(dim, (-1, Q)).narrow(dim + 1, 0, at)
+        pick = lambda t: before(t, 1) if name == "scan" else t[..., :at]
+    _compare(name, got, ref, rows, pick)
+
+
+# shares of four heads of one set; ragged, dealt evenly, the set changes inside the loop; groups of nine for two workgroups
+@pytest.mark.parametrize("kind", ["steep", "rising", "mixed"])
+@pytest.mark.parametrize("case", [(43, 512, 8, 1, 128), (107, 513, 10, 1, 64), (23, 289, 9, 1, 128)])
+def test_every_decay_in_workgroups_of_several_heads(case, kind, device):
+    _check_scan(case, kind, True, False, False, device)
+    _check_scan(case, kind, False, True, False, device)
+    _check_dx(case, kind, True, False, device)
+    _check_ddA(case, kind, device)

@@ -142,6 +142,11 @@ struct HeadsWalk {
   }
 };
 
+__device__ __forceinline__ void load8(float* r, const float* p) {
+  const float4 a = *reinterpret_cast<const float4*>(p), b = *reinterpret_cast<const float4*>(p + 4);
+  r[0] = a.x, r[1] = a.y, r[2] = a.z, r[3] = a.w, r[4] = b.x, r[5] = b.y, r[6] = b.z, r[7] = b.w;
+}
+
 // Waits until at most n of the wave's requests (copies, stores) are outstanding, n the same for the whole wave: the
 // first of the listed counts (falling) that n allows, or none.
 template <int FIRST, int... REST>
@@ -425,22 +430,23 @@ __global__ __launch_bounds__(512, 2) void ssd_chunk_scan_heads_kernel(
         }
       }
     }
-    // (rare: cb is read again, which keeps the registers out of a second unrolled form)
+    // weights as they are defined: last pieces along which dA falls steeply, or all of them
     if (!(split && narrow[0] && narrow[1]))
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
 #pragma unroll
       for (int pb = 0; pb < 4; ++pb) acc[j][pb] *= scale[j];
       scale[j] = 1.f;
-      const float* cbrow = cb + ((((int64_t)b * C + c) * ngroups + now.g) * Q + r0[j] + l16) * Q + 8 * quad;
-#pragma unroll 1
-      for (int t = split ? steps[j] - !narrow[j] : 0; t < steps[j]; ++t) {
-        float w[8];
+      const int begin = split ? steps[j] - !narrow[j] : 0;
+#pragma unroll
+      for (int t = 0; t < 4 + 4 * j; ++t) {
+        if (t < begin || t >= steps[j]) continue;
+        float ak[8], tk[8], w[8];
+        load8(ak, dAs + 32 * t + 8 * quad), load8(tk, dts + 32 * t + 8 * quad);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          const int k = 32 * t + 8 * quad + e;
-          const float f = cbrow[32 * t + e] * __expf(fminf(am[j] - dAs[k], 0.f)) * dts[k];
-          w[e] = k > r0[j] + l16 ? 0.f : f;
+          const float f = (j == 1 ? cb1[t][e] : cb0[t & 3][e]) * __expf(fminf(am[j] - ak[e], 0.f)) * tk[e];
+          w[e] = 32 * t + 8 * quad + e > r0[j] + l16 ? 0.f : f;
         }
         Vec16<T> wf;
         wf.set_all(w);
@@ -737,26 +743,23 @@ __global__ __launch_bounds__(512, 2) void ssd_chunk_scan_bwd_dx_heads_kernel(
         }
       }
     }
-    // (rare: cb is read again, which keeps the registers out of a second unrolled form)
+    // weights as they are defined: first pieces along which dA falls steeply, or all of them
     if (!(split && narrow[0] && narrow[1]))
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
 #pragma unroll
       for (int pb = 0; pb < 4; ++pb) acc[j][pb] *= scale[j];
       scale[j] = 1.f;
-      const int m = r0[j] + l16;
-      const unsigned cbcol = 4u * (8 * quad * Q + m);
-      const float* cbg = cb + (((int64_t)b * C + c) * ngroups + now.g) * (Q * Q);
-#pragma unroll 1
-      for (int t = split ? steps[j] - !narrow[j] : 0; t < steps[j]; ++t) {
-        const int k0 = 32 * (7 - t);
-        float w[8];
+      const int begin = split ? steps[j] - !narrow[j] : 0;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int k = k0 + 8 * quad + e;
-          const float f = *at_bytes(cbg + (k0 + e) * Q, cbcol) * __expf(fminf(dAs[k] - am[j], 0.f));
-          w[e] = k < m || k >= limit ? 0.f : f;
-        }
+      for (int t = 0; t < 8 - 4 * j; ++t) {
+        if (t < begin || t >= steps[j]) continue;
+        const int k0 = 32 * (7 - t);
+        float ak[8], w[8];
+        load8(ak, dAs + k0 + 8 * quad);
+#pragma unroll
+        for (int e = 0; e < 8; ++e)  // (the exponent is at most 0 and cb 0 where the weight is none)
+          w[e] = (j == 0 ? cb0[t][e] : cb1[t & 3][e]) * __expf(fminf(ak[e] - am[j], 0.f));
         Vec16<T> wf;
         wf.set_all(w);
 #pragma unroll
@@ -1056,6 +1059,29 @@ __global__ __launch_bounds__(512, 2) void ssd_ddA_heads_kernel(
         p1 = n1, g1 = m1;
         if (nb < 6) p0 = n0, g0 = m0;
       }
+    } else {  // where dA rises: weights as they are defined
+      const float4 a0 = *reinterpret_cast<const float4*>(dAs + 16 * strip[0] + 4 * quad);
+      const float4 a1 = *reinterpret_cast<const float4*>(dAs + 16 * strip[1] + 4 * quad);
+      auto block = [&](int j, const floatx4& acc, const float* w, const float4& am, float an, float tn) {
+        const float m[4] = {am.x, am.y, am.z, am.w};
+        float s = 0.f;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const float f = acc[v] * w[v] * tn * __expf(fminf(m[v] - an, 0.f));
+          const float u = 4 * quad + v < limit - 16 * strip[j] ? f : 0.f;
+          exact[j][v] += u;
+          s += u;
+        }
+        return s;
+      };
+#pragma unroll
+      for (int nb = 0; nb < 15; ++nb) {
+        if (nb >= 8 && nb >= strip[1]) break;
+        const Vec16<T> xf[2] = {x_frag(nb, 0), x_frag(nb, 1)};
+        const float an = dAs[16 * nb + l16], tn = dts[16 * nb + l16];
+        col[nb] = block(1, product(1, xf), cb1[nb], a1, an, tn);
+        if (nb < 7 && nb < strip[0]) col[nb] += block(0, product(0, xf), cb0[nb < 7 ? nb : 0], a0, an, tn);
+      }
     }
     diag[0] = quad_sum(diag[0]), diag[1] = quad_sum(diag[1]);
 #pragma unroll
@@ -1066,31 +1092,6 @@ __global__ __launch_bounds__(512, 2) void ssd_ddA_heads_kernel(
 #pragma unroll
     for (int j = 0; j < 2; ++j)
       if (quad == j) colsum[16 * strip[j] + l16] += diag[j];
-    // ---- where dA rises: weights as they are defined
-    if (!split)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int r0 = 16 * strip[j];
-#pragma unroll 1
-        for (int nb = 0; nb < strip[j]; ++nb) {
-          const Vec16<T> xf[2] = {x_frag(nb, 0), x_frag(nb, 1)};
-          const floatx4 acc = product(j, xf);
-          const int n = 16 * nb + l16;
-          const float* cbg = cb + (((int64_t)now.b * C + now.c) * ngroups + now.g) * (Q * Q);
-          const float an = dAs[n], tn = dts[n];
-          float s = 0.f;
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const int m = r0 + 4 * quad + v;
-            const float f = acc[v] * cbg[m * Q + n] * tn * __expf(fminf(dAs[m] - an, 0.f));
-            const float w = m < limit ? f : 0.f;
-            exact[j][v] += w;
-            s += w;
-          }
-          s = quad_sum(s);
-          if (quad == 0) colsum[n] += s;
-        }
-      }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       float4 r;
