@@ -216,6 +216,40 @@ def _compare(name, got, ref, rows, pick=lambda t: t):
         check_close(f"{name} {what}", pick(g[rows]), pick(r), dtype, regrouped=dtype == BF16, loose=what == "ddt")
 
 
+@pytest.mark.parametrize("drop", [30.0, 1000.0])
+@pytest.mark.parametrize("name", list(WALKS))
+def test_small_rises_are_clamped(name, drop, device):
+    """dA falls once and then rises by 9e-7 of itself per position, 2.3e-4 of itself in a chunk: every weight behind
+    the fall is that of exp(0)."""
+    case = WALKS[name]
+    announce(f"{name} with small rises behind {drop}")
+    x, y, BC, dt, dA, cb, states, _ = _inputs(*case, "falling", seed=5)
+    dA = (-drop * (1 - 9e-7 * torch.arange(Q))).expand(dA.shape).clone()
+    dA[..., 0] = 0
+    ops = (x, y, BC, cb, states)
+    rows, _ = _some(case[0])
+    _compare(name, _run(name, ops, dt, dA, device), _run(name, ops, dt, dA, device, ref=rows), rows)
+
+
+@pytest.mark.parametrize("rate", [0.1, 4.0, 30.0])
+@pytest.mark.parametrize("name", list(WALKS))
+def test_steps_of_zero(name, rate, device):
+    """A tenth of the steps is 0: the library's own sums rise by their rounding between some of them."""
+    from kernels.mamba_kernels.mamba_cumsum import _chunk_cumsum_fwd
+
+    case = WALKS[name]
+    b, L, nh, _, _ = case
+    announce(f"{name} with steps of zero, rate {rate}")
+    x, y, BC, _, _, cb, states, _ = _inputs(*case, "falling", seed=6)
+    gen = torch.Generator().manual_seed(7)
+    dt = torch.rand(b, L, nh, generator=gen) * (torch.rand(b, L, nh, generator=gen) > 0.1)
+    dA, dt = (t.cpu() for t in _chunk_cumsum_fwd(dt.to(device), torch.full((nh,), -rate, device=device), Q))
+    assert (dA[..., 1:] > dA[..., :-1]).any()
+    ops = (x, y, BC, cb, states)
+    rows, _ = _some(b)
+    _compare(name, _run(name, ops, dt, dA, device), _run(name, ops, dt, dA, device, ref=rows), rows)
+
+
 @pytest.mark.parametrize("L", [257, 263, 271, 272, 290, 400, 511])
 def test_ddA_looks_at_nothing_past_the_sequence(L, device):
     """dt, dA and cb past the sequence are NaN or infinite; a last position with an infinite dt, which no weight uses.
