@@ -127,7 +127,8 @@ def _check_ddA(case, kind, device):
     check_close("ddA_cumsum (causal term)", got[rows], ref, F32)
 
 
-@pytest.mark.parametrize("case", DEALS)
+# (the ddA walk takes more than 256 heads in groups of eight or more: 414 in five shares a set, 2430 dealt evenly)
+@pytest.mark.parametrize("case", DEALS + [(23, 289, 9, 1, 128), (135, 270, 9, 1, 128)])
 def test_ddA_deals(case, device):
     _check_ddA(case, "falling", device)
 
@@ -305,3 +306,44 @@ def test_every_decay_in_workgroups_of_several_heads(case, kind, device):
     _check_scan(case, kind, False, True, False, device)
     _check_dx(case, kind, True, False, device)
     _check_ddA(case, kind, device)
+
+
+# ---- rows
+
+def _rows_apart(t, stride):
+    """The same values, `stride` elements from row to row."""
+    b, L, nh, p = t.shape
+    v = torch.empty((b * L - 1) * stride + nh * p, dtype=t.dtype, device=t.device).as_strided(t.shape, (L * stride, stride, p, 1))
+    return v.copy_(t)
+
+
+# rows of a wider projection; the longest rows that the walks take (2^23 - 8 elements) and the first that they do not
+@pytest.mark.parametrize("stride", [66 * 64 + 1024, 2 ** 23 - 8, 2 ** 23])
+@pytest.mark.parametrize("L", [256, 250])
+def test_rows_apart(L, stride, device):
+    from kernels.mamba_kernels.mamba_scan_fwd import _chunk_scan_fwd
+    from kernels.mamba_kernels_bwd.mamba_chunk_scan_bwd_da import _chunk_scan_bwd_ddAcs_stable
+    from kernels.mamba_kernels_bwd.mamba_chunk_scan_chunk_state_bwd_dx import _chunk_scan_chunk_state_bwd_dx
+
+    announce(f"rows {stride} elements apart, L {L}")
+    x, y, BC, dt, dA, cb, states, D = _inputs(1, L, 66, 1, 128, "falling", seed=L)
+    cb = torch.nan_to_num(cb)  # (the general dx looks at it past the sequence)
+    ref, ref_x = S.chunk_scan(cb, x, dt, dA, BC, states, D=D, z=y, round_to=BF16)
+    ref_dx, ref_ddt, _ = S.chunk_scan_chunk_state_bwd_dx(x, dt, dA, BC, cb, y, states, D=D, round_to=BF16)
+    ref_ddA = S.chunk_scan_bwd_ddAcs_stable(x, dt, dA, y, cb)
+    x, y, BC, dt, dA, cb, states, D = (t.to(device) for t in (x, y, BC, dt, dA, cb, states, D))
+    apart = lambda t: _rows_apart(t, stride)
+    xa, ya, Ba, dxa = apart(x), apart(y), apart(BC), apart(torch.zeros_like(x))
+    out, out_x = _chunk_scan_fwd(cb, xa, dt, dA, Ba, states, D=D, z=ya)
+    dx, ddt, dD = _chunk_scan_chunk_state_bwd_dx(xa, dt, dA, Ba, cb, ya, states, D=D, dx=dxa)
+    ddA = _chunk_scan_bwd_ddAcs_stable(xa, dt, dA, ya, cb)
+    assert dx.data_ptr() == dxa.data_ptr()
+    for name, got, want in (("out", out, ref), ("out_x", out_x, ref_x), ("dx", dx, ref_dx)):
+        check_close(name, got, want, BF16, regrouped=True)
+    check_close("ddt", ddt, ref_ddt, BF16, loose=True)
+    check_close("ddA", ddA, ref_ddA, F32)
+    if stride < 2 ** 23:  # the same kernels as for dense rows
+        same = _chunk_scan_chunk_state_bwd_dx(x, dt, dA, BC, cb, y, states, D=D)
+        for got, want in ((out, _chunk_scan_fwd(cb, x, dt, dA, BC, states, D=D, z=y)[0]), (dx, same[0]), (ddt, same[1]),
+                          (dD, same[2]), (ddA, _chunk_scan_bwd_ddAcs_stable(x, dt, dA, y, cb))):
+            assert torch.equal(got, want)
