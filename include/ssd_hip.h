@@ -112,8 +112,10 @@ int ssd_bmm_chunk_fwd(const void* a, int64_t a_sb, int64_t a_sl, int64_t a_sg, c
  *          + sum_{k<=m} cb[m,k] * exp(min(dA_m - dA_k, 0)) * dt_k * x[k,p]  +  D * x[m,p],
  * then, with z: out_x = out (if out_x is not NULL) and out *= z * sigmoid(z).
  * cb float32 (batch, C, ngroups, Q, Q); prev (batch, C, nheads, hdim, dstate) in float32 or in
- * `dtype` (states_dtype; the product rounds it to `dtype` either way, so the result is the same and
- * the bfloat16 form moves half the bytes); D float32
+ * `dtype` (states_dtype; the product rounds it to `dtype` either way, and the bfloat16 form moves half the
+ * bytes.  The results have the same bits while batch * C * nheads is at most 256, with z 64; beyond, bfloat16 states of
+ * hdim 64 and chunk 256 take a kernel of their own, which rounds the same weights of the causal sum behind another
+ * product, and the results agree to the rounding of the weights); D float32
  * (nheads) or (nheads, hdim) (d_has_hdim), may be NULL; z may be NULL; out_x shares out's strides.
  * With seq_idx the first term only reaches the rows m whose id equals that of the previous
  * chunk's last position (0 for the first chunk; mamba_scan_fwd.py:77-92); cb is expected to
@@ -220,7 +222,8 @@ int ssd_chunk_scan_bwd_dc(const void* dout, int64_t d_sb, int64_t d_sl, int64_t 
  *          + sum_{k>=m} round(cb[k,m] * exp(min(dA_k - dA_m, 0))) * dout[k,p];
  * dx = acc * dt_m + D * dout (type `dtype`, dx's own strides), ddt[b,h,c,m] = sum_p acc[m,p] * x[m,p]
  * (float32, 0 past seqlen).  cb float32 (batch, C, ngroups, Q, Q), dstates float32 or `dtype`
- * (states_dtype) (batch, C, nheads, hdim, dstate), D as for ssd_chunk_scan_fwd.  dD_partial (may be NULL; needs D):
+ * (states_dtype) (batch, C, nheads, hdim, dstate), either of which gives the same bits while batch * C * nheads is at
+ * most 64 (as for ssd_chunk_scan_fwd), D as there.  dD_partial (may be NULL; needs D):
  * float32 (batch, C, nheads, S, hdim) with S = ssd_chunk_scan_chunk_state_bwd_dx_dD_slots(...),
  * every slot written: partial sums over positions of dout * x, whose sum over batch, C and S is
  * the gradient of D (nheads, hdim), summed over hdim too for a D of shape (nheads) -- the

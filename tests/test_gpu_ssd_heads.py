@@ -347,3 +347,20 @@ def test_rows_apart(L, stride, device):
         for got, want in ((out, _chunk_scan_fwd(cb, x, dt, dA, BC, states, D=D, z=y)[0]), (dx, same[0]), (ddt, same[1]),
                           (dD, same[2]), (ddA, _chunk_scan_bwd_ddAcs_stable(x, dt, dA, y, cb))):
             assert torch.equal(got, want)
+
+
+# batch * chunks * heads up to which the header promises the same bits for states of either type
+@pytest.mark.parametrize("name,b,gate", [("scan", 32, False), ("scan", 8, True), ("dx", 8, False)])
+def test_states_of_either_type_give_the_same_bits(name, b, gate, device):
+    from kernels.mamba_kernels.mamba_scan_fwd import _chunk_scan_fwd
+    from kernels.mamba_kernels_bwd.mamba_chunk_scan_chunk_state_bwd_dx import _chunk_scan_chunk_state_bwd_dx
+
+    announce(f"{name} of {8 * b} heads, gate {gate}, states of either type")
+    x, y, BC, dt, dA, cb, states, D = (t.to(device) for t in _inputs(b, 300, 4, 1, 128, "falling", seed=b))
+    cb = torch.nan_to_num(cb)
+    if name == "scan":
+        got = [_chunk_scan_fwd(cb, x, dt, dA, BC, s, D=D, z=y if gate else None) for s in (states, states.float())]
+    else:
+        got = [_chunk_scan_chunk_state_bwd_dx(x, dt, dA, BC, cb, y, s, D=D) for s in (states, states.float())]
+    for a, c in zip(*got):
+        assert a is None and c is None or torch.equal(a, c)

@@ -171,8 +171,8 @@ struct DxLaunch {
     if constexpr (std::is_same<T, bf16_t>::value && std::is_same<TS, bf16_t>::value && P == 64) {
       // The walk over the heads.  The 256-row kernel / the walk, us, dstate 128: 128 heads of all (batch, chunk) pairs 16.9 /
       // 14.1, 256 19.2 / 15.3, 512 27 / 22, 3072 121 / 91; only many groups of two or three heads, one or two to a compute unit,
-      // are behind: 256 of two 27.3 / 27.9, of three 34.4 / 35.3, of four 50 / 42.  Calls of up to 64 heads, where the launch counts
-      // for more than the kernel (15 / 12.5), give the same bits whatever the type of the states.
+      // are behind: 256 of two 27.3 / 27.9, of three 34.4 / 35.3, of four 50 / 42.  Up to 64 heads, where the walk would be faster
+      // too (15 / 12.5), the results have the same bits for states of either type, which the header promises that far.
       const int64_t units = d.batch * d.C * d.nh;
       const bool pays = units > 64 && (d.nh / d.g >= 4 || d.batch * d.C * d.g < 256);
       if (d.Q == 256 && pays && !(D && d_has_hdim) && heads_vectors(dt, dA) && heads_rows(sx) && heads_rows(sd) && heads_rows(sdx)) {

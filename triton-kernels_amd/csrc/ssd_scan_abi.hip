@@ -97,7 +97,8 @@ struct ScanLaunch {
       // The walk over the heads, from where a workgroup has two of them or a gate hides the fetch of what they share,
       // and groups have three heads or more.  The 256-row kernel / the walk, us, dstate 128: without gate 256 heads of
       // all (batch, chunk) pairs 14.7 / 16.2, 288 20.9 / 19.4, 512 23.2 / 21.3, 1536 57 / 41; 512 groups of two heads 44 / 53,
-      // of three 66 / 62; with gate 16 heads 16.0 / 16.8, 64 16.9 / 17.2, 128 19.6 / 18.2, 256 22.4 / 19.1.
+      // of three 66 / 62; with gate 16 heads 16.0 / 16.8, 64 16.9 / 17.2, 128 19.6 / 18.2, 256 22.4 / 19.1.  (The
+      // header promises the same bits for states of either type up to these lines.)
       const int64_t units = d.batch * d.C * d.nh;
       const bool pays = units > (z ? 64 : 256) && d.nh / d.g >= 3;
       if (d.Q == 256 && pays && !(D && d_has_hdim) && heads_vectors(dt, dA) && heads_rows(sx) && heads_rows(so) &&
