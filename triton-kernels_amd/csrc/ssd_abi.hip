@@ -706,16 +706,19 @@ int ssd_chunk_scan_bwd_ddAcs(const void* x, int64_t x_sb, int64_t x_sl, int64_t 
                        (int)d.C);                                                                               \
   } while (0)
     if (dtype == SSD_BF16 && hdim == 64 && chunk == 256) {
-      // The walk over the heads: where each has a compute unit to itself, and for groups of eight or more.  The other
-      // kernel / the walk, us: 64 heads of all (batch, chunk) pairs 11.7 / 9.5, 256 14.3 / 11.7, 288 16.2 / 15.7; groups of six
-      // heads, 256 of them, 40 / 43, of eight 56 / 53, of 32 213 / 168; 320 of ten 89 / 85; 128 of four 18.0 / 18.6.
+      // The walk over the heads: where each has a compute unit to itself, and for groups of eight or more (ten, where the
+      // heads are dealt evenly) from where the other kernel, 768 of whose workgroups run at once, needs a second turn; not
+      // where it fills that second turn.  The other kernel / the walk, us, inputs in turn: 64 heads of all (batch, chunk)
+      // pairs 13.2 / 10.0, 256 15.3 / 12.7; 264 15.9 / 16.5, 512 19.1 / 19.4, 640 20.5 / 22.6, 768 22.4 / 27.0; 800 30 / 27, 1024 34 /
+      // 29, 1152 36 / 34; 1280 36.3 / 37.1, 1536 40.6 / 43.3; 1568 47 / 41, 2304 57 / 56, 3072 77 / 70, 8192 186 / 155; dealt evenly
+      // 2400 of eight 67.5 / 69.5, 3072 of eight 77 / 77, 3200 of ten 85 / 82.
       // Relative error against float64, the other kernel / the walk, A in [-16, -1], b1 nh32 L4096, mean of 12 seeds: dt =
       // softplus(n/2 - 2) 8.8e-7 / 7.6e-7, softplus(n/2) 1.23e-6 / 9.6e-7, softplus(n/2 + 2) 9.1e-7 / 9.4e-7.
-      const bool pays = wgs <= 256 || hpg >= 8;
+      const HeadsDeal deal = heads_deal(batch * d.C * ngroups, hpg);
+      const bool pays = wgs <= 256 || (wgs > 768 && (wgs <= 1152 || wgs > 1536) && hpg >= (deal.splits ? 8 : 10));
       if (pays && heads_vectors(dt, dA_cumsum) && reinterpret_cast<uintptr_t>(ddA_cumsum) % 16 == 0 && heads_rows(sx) && heads_rows(sd)) {
         constexpr int smem = DdaHeadsSmem::kBytes;
         static_assert(smem <= kLdsBytes, "the heads under way must fit the LDS of a compute unit");
-        const HeadsDeal deal = heads_deal(batch * d.C * ngroups, hpg);
         auto kernel = deal.splits ? ssd_ddA_heads_kernel<false> : ssd_ddA_heads_kernel<true>;
         SSD_TRY(allow_smem(kernel, smem));
         hipLaunchKernelGGL(kernel, dim3(deal.workgroups), dim3(512), smem, st, (const bf16_t*)x,
