@@ -38,6 +38,22 @@ def test_traced_calls_run_the_kernel_again(name, off, copied):
             assert torch.equal(traced(a, x), x)
 
 
+@pytest.mark.parametrize("off", [torch.no_grad, torch.inference_mode])
+@pytest.mark.parametrize("name", ["combined", "sequence"])
+def test_tensors_left_over_from_a_transform_are_taken(name, off, copied):
+    """torch.func.grad leaves a wrapper round a tensor that outlives it, which has no memory of its own."""
+    left = []
+
+    def f(x):
+        left.append(x)
+        return (x * x).sum()
+
+    a, x = torch.zeros(2, 5), torch.arange(80.0).view(2, 5, 8)
+    torch.func.grad(f)(x)
+    with off():
+        assert torch.equal(_calls()[name](a, left[0]), x)
+
+
 def test_untracked():
     seen = []
 
