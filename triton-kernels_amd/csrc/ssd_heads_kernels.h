@@ -1032,7 +1032,7 @@ __global__ __launch_bounds__(512, 2) void ssd_ddA_heads_kernel(
 #pragma unroll
         for (int v = 0; v < 4; ++v) {  // (selects, so that no product past the diagonal or the sequence is met)
           const float f = d[j][v] * cbd[j][v] * tn * __expf(fminf(em[j][v] - an, 0.f));
-          exact[j][v] = (l16 < 4 * quad + v) & (4 * quad + v < limit - 16 * strip[j]) ? f : 0.f;
+          exact[j][v] = ((l16 < 4 * quad + v) & (4 * quad + v < limit - 16 * strip[j])) ? f : 0.f;
           diag[j] += exact[j][v];
           em[j][v] = __expf(fminf(em[j][v] - dAs[16 * strip[j]], 0.f));
         }
