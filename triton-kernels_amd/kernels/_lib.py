@@ -170,7 +170,7 @@ def untracked(*tensors) -> bool:
     if torch.is_grad_enabled() or torch.autograd.forward_ad._current_level >= 0 \
             or torch._C._are_functorch_transforms_active() or torch._C._get_tracing_state() is not None:
         return False
-    for t in () if torch.compiler.is_compiling() else tensors:  # (a compiler meets no such tensor, nor knows the question)
+    for t in () if torch.compiler.is_dynamo_compiling() else tensors:  # (a compiler meets no such tensor, nor knows the question)
         if t is not None and _wrapped(t):
             return False
     return True
