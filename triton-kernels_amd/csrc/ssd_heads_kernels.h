@@ -9,8 +9,10 @@
 // accumulators, which spills.)
 //
 // The per-head kernels these stand beside fetch cb and the rows of B / C once per head or pair of heads, a fragment at a
-// time, and wait for each.  Here a head's copies alone run at 5.0 TB/s; what keeps the kernels from that is the
-// serial chain of a head (copies landed, factors, products, sums) at two waves per SIMD, all in the same phase.
+// time, and wait for each.  Here a head's copies alone run at 5.0 to 5.2 TB/s; what keeps the kernels from that is the
+// serial chain of a head (copies landed, factors, products, sums) at two waves per SIMD.  Times below are us by the kernel
+// of one head or pair and here, at b8 nh32 L8192 dstate 128 of the three walks one after another on inputs in turn, the
+// others of a kernel by itself.
 #pragma once
 #include "ssd_kernels.h"
 
@@ -219,10 +221,11 @@ __device__ __forceinline__ void store_strip(bf16_t* g, const Vec16<bf16_t>& lo, 
 }
 
 // ------------------------------------------------------------------------------------
-// chunk_scan (ssd_chunk_scan_kernel).  us by the 256-row kernel and here, dstate 128: b8 nh32 L8192 244 -> 168 (4.4 TB/s of
-// its 742 MB; 406 -> 283 with gate and out_x), b4 nh24 L8192 95 -> 68, b1 nh32 L4096 23.2 -> 21.2 (gate 31 -> 27).  On the way:
+// chunk_scan (ssd_chunk_scan_kernel).  b8 nh32 L8192 295 -> 185 (4.0 TB/s of its 742 MB), by itself 244 -> 168 (406 -> 283
+// with gate and out_x), b4 nh24 L8192 95 -> 68, b1 nh32 L4096 23.2 -> 21.2 (gate 31 -> 27).  On the way, by itself:
 // 230 with heads in step and rows stored in 64-byte halves, 195 with the heads in turn, 184 with whole rows stored, 165 with a
-// piece's LDS reads ahead of the products of the one before.  Alone, the copies and stores take 148 and the rest 97.
+// piece's LDS reads ahead of the products of the one before.  Of the 185, the copies and stores alone take 150 and the rest
+// alone 128.
 // ------------------------------------------------------------------------------------
 template <int N, bool GATED>
 struct ScanHeadsSmem : HeadsTile {
@@ -542,9 +545,9 @@ __device__ __forceinline__ float row16_sum(float v) {
 
 // ------------------------------------------------------------------------------------
 // dx / ddt / the partial sums of dD (ssd_chunk_scan_bwd_dx_kernel): the mirror image of the chunk scan.  The strips'
-// positions run from the chunk's end to the diagonal, the weights are columns of cb.  us by the 256-row kernel and here,
-// dstate 128: b8 nh32 L8192 304 -> 233 (4.4 TB/s of its 1030 MB; with D 365 -> 258), b4 nh24 L8192 121 -> 91, b1 nh32 L4096 27 -> 22.
-// Alone, the copies and stores take 206 and the rest 166.
+// positions run from the chunk's end to the diagonal, the weights are columns of cb.  b8 nh32 L8192 317 -> 246 (4.2 TB/s of its
+// 1030 MB), by itself 304 -> 233 (with D 365 -> 258), b4 nh24 L8192 121 -> 91, b1 nh32 L4096 27 -> 22.  Of the 246, the copies
+// and stores alone take 201 and the rest alone 153.
 // ------------------------------------------------------------------------------------
 template <int N>
 struct DxHeadsSmem : HeadsTile {
@@ -841,8 +844,8 @@ __global__ __launch_bounds__(512, 2) void ssd_chunk_scan_bwd_dx_heads_kernel(
 //   W[m][n] = <dout[m], x[n]> * dt_n * cb[m][n] * exp(min(dA_m - dA_n, 0))   for n < m < limit,
 // ddA[j] = sum_{i < j} (colsum_i - rowsum_i).  A strip's blocks of 16 x 16 up to the diagonal one; the row sums stay in
 // registers, the column sums of a wave meet those of the others in LDS, and one wave, a head later, forms the prefix
-// sum.  us by the kernel of one head per workgroup and here: b8 nh32 L8192 213 -> 168 (3.6 TB/s of its 600 MB), b2 nh32 L8192 with
-// two groups 53 -> 48, b1 nh32 L2048 14.3 -> 11.7.  Alone, the copies take 119 and the rest 125.
+// sum.  b8 nh32 L8192 213 -> 196 (3.1 TB/s of its 600 MB), by itself 186 -> 155, b1 nh32 L2048 15.3 -> 12.7.  Of the 196, the
+// copies alone take 116 and the rest alone 131.
 // ------------------------------------------------------------------------------------
 struct DdaHeadsSmem : HeadsTile {
   static constexpr int R = 3;                                // heads in LDS, of x, dA and dt
