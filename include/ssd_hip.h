@@ -280,8 +280,8 @@ int ssd_chunk_state_varlen(const void* B, int64_t b_sl, int64_t b_sg, const void
 /* The five forward stages, with the results of their own entry points above: cumsum; chunk states
  * and state passing (one walk per head, or, with local_states (batch, C, nheads, hdim, dstate) float32 given, the
  * two launchers; packed batches need it); bmm; chunk scan; and, with varlen_out given (batch 1), the states at the
- * sequence ends cu_seqlens names.  With local_states the cumsum, the chunk states and bmm share one launch, with the bits
- * of their own entry points.  x, z, B, C, states and varlen_out are of `dtype`, final_states float32.  One
+ * sequence ends cu_seqlens names.  With local_states the cumsum, the chunk states and bmm share one launch (float32 of hdim
+ * 128: not where there are many of both), with the bits of their own entry points.  x, z, B, C, states and varlen_out are of `dtype`, final_states float32.  One
  * call from the host instead of five or six.  Arguments that a stage would refuse are refused before the first
  * one is enqueued. */
 int ssd_combined_fwd(const void* x, int64_t x_sb, int64_t x_sl, int64_t x_sh, int dtype, const void* dt, int dt_dtype,

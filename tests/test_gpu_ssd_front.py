@@ -1,5 +1,6 @@
 """The combined forward forms dt, dA, the chunk-local states and C . B in one launch where the states are passed on by a
-launch of their own: everything it returns is, bit for bit, what the stage launchers return one after the other."""
+launch of their own, but for many float32 states of hdim 128: everything it returns is, bit for bit, what the stage
+launchers return one after the other."""
 import pytest
 import torch
 
@@ -14,7 +15,9 @@ F32, BF16 = torch.float32, torch.bfloat16
 @pytest.mark.parametrize("dtype,dt_dtype", [(F32, F32), (BF16, F32), (BF16, BF16)])
 @pytest.mark.parametrize("packed", [False, True])
 @pytest.mark.parametrize("b,L,nh,g,P,N,Q", [(1, 1, 1, 1, 64, 64, 4), (2, 65, 3, 1, 64, 128, 64), (1, 257, 6, 2, 128, 64, 128),
-                                            (3, 511, 5, 5, 64, 128, 256), (1, 700, 2, 1, 128, 128, 200), (1, 1500, 4, 2, 64, 64, 1024)])
+                                            (3, 511, 5, 5, 64, 128, 256), (1, 700, 2, 1, 128, 128, 200), (1, 1500, 4, 2, 64, 64, 1024),
+                                            # float32: three launches again, the last block count of one and the first of three
+                                            (14, 2000, 5, 1, 128, 128, 512), (16, 2000, 4, 2, 128, 64, 512), (13, 2000, 5, 1, 128, 128, 512)])
 def test_front_equals_the_stages(b, L, nh, g, P, N, Q, packed, dtype, dt_dtype, device, monkeypatch):
     from kernels.mamba_kernels import mamba_combined_fwd as M
     from kernels.mamba_kernels.mamba_bmm import _bmm_chunk_fwd

@@ -841,8 +841,21 @@ int ssd_combined_fwd(const void* x, int64_t x_sb, int64_t x_sl, int64_t x_sh, in
   if (batch * C_ * nheads * tiles > 0x7fffffff || batch * C_ * (nheads + ngroups * tiles * tiles) > 0x7fffffff ||
       batch * nheads * ((hdim * dstate + 1023) / 1024) > 0x7fffffff)
     return SSD_ERR_SHAPE;
+  // In one launch the blocks of C . B run with the registers of the states.  Of float32 states of hdim 128 those leave one
+  // workgroup to a compute unit at dstate 128 (262 registers; C . B alone two) and three at dstate 64 (144; alone four), and
+  // where there are many of both C . B is faster in a launch of its own.  The whole forward, us, apart / in one launch: dstate
+  // 128, 256 heads of all (batch, chunk) pairs with 4096 blocks 312 / 321, with 16384 1099 / 1165, with 65536 1846 / 2157, 512
+  // heads with 2048 218 / 218, 64 with 4096 213 / 187; dstate 64, 256 heads with 4096 248 / 241, with 16384 892 / 902, with 65536
+  // 1357 / 1451, 2048 heads with 2048 235 / 235, with 8192 296 / 305.  Other types and sizes are level or gain.
+  const bool apart = dtype == SSD_F32 && hdim == 128 && batch * C_ * nheads >= 256 &&
+                     batch * C_ * ngroups * tiles * tiles >= (dstate == 128 ? 3584 : 8192);
   if (local_states) {
-    SSD_TRY(dispatch_tpn(dtype, hdim, dstate,
+    if (apart) {
+      SSD_TRY(ssd_chunk_cumsum_fwd(dt, dt_dtype, dt_sb, dt_sl, dt_sh, A, dt_bias, dA_cumsum, dt_out, batch, seqlen,
+                                   nheads, chunk, dt_softplus, dt_min, dt_max, stream));
+      SSD_TRY(ssd_chunk_state_fwd(B, b_sb, b_sl, b_sg, x, x_sb, x_sl, x_sh, dtype, dt_out, dA_cumsum, local_states,
+                                  batch, seqlen, nheads, ngroups, hdim, dstate, chunk, seq_idx, seq_sb, seq_sl, stream));
+    } else SSD_TRY(dispatch_tpn(dtype, hdim, dstate,
                          FrontLaunch{x, B, C, Strides3{x_sb, x_sl, x_sh}, Strides3{b_sb, b_sl, b_sg}, Strides3{c_sb, c_sl, c_sg},
                                      dt, dt_dtype, Strides3{dt_sb, dt_sl, dt_sh}, A, dt_bias, dA_cumsum, dt_out, dt_softplus,
                                      dt_min, dt_max, local_states, cb, d, as_seq(seq_idx, seq_sb, seq_sl), as_stream(stream)}));
@@ -855,10 +868,10 @@ int ssd_combined_fwd(const void* x, int64_t x_sb, int64_t x_sl, int64_t x_sh, in
     SSD_TRY(ssd_chunk_state_passing_fwd(B, b_sb, b_sl, b_sg, x, x_sb, x_sl, x_sh, dtype, dt_out, dA_cumsum, initial,
                                         states, dtype, final_states, batch, seqlen, nheads, ngroups, hdim, dstate,
                                         chunk, stream));
-    // (last: the chunk scan reads it next)
+  }
+  if (!local_states || apart)  // (last: the chunk scan reads it next)
     SSD_TRY(ssd_bmm_chunk_fwd(C, c_sb, c_sl, c_sg, B, b_sb, b_sl, b_sg, dtype, cb, SSD_F32, batch, seqlen, ngroups,
                               dstate, chunk, seq_idx, seq_sb, seq_sl, stream));
-  }
   SSD_TRY(ssd_chunk_scan_fwd(cb, x, x_sb, x_sl, x_sh, z, z_sb, z_sl, z_sh, dtype, dt_out, dA_cumsum, C, c_sb, c_sl,
                              c_sg, states, dtype, D, d_has_hdim, out, o_sb, o_sl, o_sh, out_x, batch, seqlen, nheads,
                              ngroups, hdim, dstate, chunk, seq_idx, seq_sb, seq_sl, stream));
