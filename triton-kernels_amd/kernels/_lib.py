@@ -158,22 +158,20 @@ def on_device(dev: torch.device):
     return _NO_SWITCH if dev.index is None or torch.cuda.current_device() == dev.index else torch.cuda.device(dev)
 
 
-_wrapped = torch._C._functorch.is_functorch_wrapped_tensor
-
-
-def untracked(*tensors) -> bool:
+def untracked() -> bool:
     """Whether nothing looks into a call made now: gradients are off, no forward-mode level is open, no transform is
     active and torch.jit.trace is not recording (it sees an autograd function as one call, but of a launch made through
-    ctypes only the empty tensor that it fills), and none of the call's tensors is still wrapped by a transform that has
-    ended (an autograd function takes those out of their wrappers).  What the call returns is then the kernels' result
-    alone, so it need not go through an autograd function (3.4 us of host time, a sixth of a decoding step)."""
-    if torch.is_grad_enabled() or torch.autograd.forward_ad._current_level >= 0 \
-            or torch._C._are_functorch_transforms_active() or torch._C._get_tracing_state() is not None:
-        return False
-    for t in () if torch.compiler.is_dynamo_compiling() else tensors:  # (a compiler meets no such tensor, nor knows the question)
-        if t is not None and _wrapped(t):
-            return False
-    return True
+    ctypes only the empty tensor that it fills).  What the call returns is then the kernels' result alone, so it need
+    not go through an autograd function (3.4 us of host time, a sixth of a decoding step)."""
+    return not (torch.is_grad_enabled() or torch.autograd.forward_ad._current_level >= 0
+                or torch._C._are_functorch_transforms_active() or torch._C._get_tracing_state() is not None)
+
+
+def left_over(*tensors) -> bool:
+    """Whether a tensor is still wrapped by a transform that has ended.  It has no memory of its own, so a call made past
+    an autograd function, which takes such tensors out of their wrappers, is refused before anything is launched; asked
+    only then, since the question costs a decoding step 0.5 us."""
+    return any(t is not None and torch._C._functorch.is_functorch_wrapped_tensor(t) for t in tensors)
 
 
 def seq_view(x: torch.Tensor):

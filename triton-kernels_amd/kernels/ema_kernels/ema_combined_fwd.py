@@ -100,8 +100,12 @@ class EMAMatmulCombinedFn(torch.autograd.Function):
 
 
 def ema_matmul_scan_combined(A_ema, X_ema, chunk_size):
-    if chunk_size % 128 == 0 and _lib.untracked(A_ema, X_ema):
+    if chunk_size % 128 == 0 and _lib.untracked():
         from kernels.ema_seq import ema_seq_fwd
 
-        return ema_seq_fwd(A_ema, X_ema, form="log_decay")[0]
+        try:
+            return ema_seq_fwd(A_ema, X_ema, form="log_decay")[0]
+        except RuntimeError:
+            if not _lib.left_over(A_ema, X_ema):
+                raise
     return EMAMatmulCombinedFn.apply(A_ema, X_ema, chunk_size)

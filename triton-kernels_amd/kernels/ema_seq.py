@@ -201,8 +201,12 @@ def ema_seq_scan(coef, x, form="log_decay", initial_states=None, return_final_st
         return (y, final) if return_final_states else y
     if seq_idx is not None:
         coef = pack_log_decay(coef, seq_idx) if form == "log_decay" else pack_probability(coef, seq_idx)
-    if _lib.untracked(coef, x, initial_states):
-        y, final, _ = ema_seq_fwd(coef, x, form, initial_states)
-    else:
-        y, final = EMASeqFn.apply(coef, x, initial_states, form)
+    if _lib.untracked():
+        try:
+            y, final, _ = ema_seq_fwd(coef, x, form, initial_states)
+            return (y, final) if return_final_states else y
+        except RuntimeError:
+            if not _lib.left_over(coef, x, initial_states):
+                raise
+    y, final = EMASeqFn.apply(coef, x, initial_states, form)
     return (y, final) if return_final_states else y
