@@ -127,9 +127,10 @@ def _check_ddA(case, kind, device):
     check_close("ddA_cumsum (causal term)", got[rows], ref, F32)
 
 
-# (beyond 256 heads the ddA walk takes more than 768, in groups of eight or more: 1600 a set each, 1664 in two shares a set,
-# 2700 dealt evenly)
-@pytest.mark.parametrize("case", DEALS + [(100, 257, 8, 1, 128), (52, 300, 16, 1, 128), (135, 270, 10, 1, 128)])
+# (beyond 256 heads the ddA walk takes more than 768 where they divide well: 1743 a set each, 816 in four shares a set, 2700
+# dealt evenly; the general kernel 1600 and 1664)
+@pytest.mark.parametrize("case", DEALS + [(100, 257, 8, 1, 128), (52, 300, 16, 1, 128), (135, 270, 10, 1, 128),
+                                          (83, 700, 7, 1, 64), (51, 250, 16, 1, 128)])
 def test_ddA_deals(case, device):
     _check_ddA(case, "falling", device)
 
@@ -299,9 +300,10 @@ def test_infinite_decay_and_infinite_steps(name, at, device):
     _compare(name, got, ref, rows, pick)
 
 
-# two shares of a set of sixteen heads; dealt evenly, the set changes inside the loop; a set each
+# two shares of a set of sixteen heads, four; dealt evenly, the set changes inside the loop; a set each (ddA: the ones behind)
 @pytest.mark.parametrize("kind", ["steep", "rising", "mixed"])
-@pytest.mark.parametrize("case", [(52, 300, 16, 1, 128), (107, 513, 10, 1, 64), (100, 257, 8, 1, 128)])
+@pytest.mark.parametrize("case", [(52, 300, 16, 1, 128), (107, 513, 10, 1, 64), (100, 257, 8, 1, 128),
+                                  (51, 250, 16, 1, 128), (135, 270, 10, 1, 128), (83, 700, 7, 1, 64)])
 def test_every_decay_in_workgroups_of_several_heads(case, kind, device):
     _check_scan(case, kind, True, False, False, device)
     _check_scan(case, kind, False, True, False, device)

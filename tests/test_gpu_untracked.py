@@ -49,3 +49,20 @@ def test_traced_calls_run_the_kernel_again(name, device):
         for _ in range(2):
             a, x = r()
             assert torch.equal(traced(a, x), call(a, x))
+
+
+@pytest.mark.parametrize("name", ["combined", "sequence"])
+def test_tensors_left_over_from_a_transform_are_taken(name, device):
+    """torch.func.grad leaves wrappers round tensors that outlive it; either operand, or both."""
+    call, left = _calls()[name], []
+
+    def f(*tensors):
+        left.extend(tensors)
+        return sum(t.sum() for t in tensors)
+
+    a, x = -torch.rand(2, 5, 3, device=device), torch.randn(2, 5, 3, 64, device=device)
+    torch.func.grad(f, argnums=(0, 1))(a, x)
+    with torch.no_grad():
+        y = call(a, x)
+        for coef, operand in ((a, left[1]), (left[0], x), left):
+            assert torch.equal(call(coef, operand), y)

@@ -169,14 +169,15 @@ struct DxLaunch {
   template <typename T, int P, int N, typename TS>
   int run_as() const {
     if constexpr (std::is_same<T, bf16_t>::value && std::is_same<TS, bf16_t>::value && P == 64) {
-      // The walk over the heads.  The 256-row kernel / the walk, us, dstate 128: 128 heads of all (batch, chunk) pairs 16.9 /
-      // 14.1, 256 19.2 / 15.3, 512 27 / 22, 3072 121 / 91; only many groups of two or three heads, one or two to a compute unit,
-      // are behind: 256 of two 27.3 / 27.9, of three 34.4 / 35.3, of four 50 / 42.  Up to 64 heads, where the walk would be faster
-      // too (15 / 12.5), the results have the same bits for states of either type, which the header promises that far.
+      // The walk over the heads, where its deal pays.  The 256-row kernel / the walk, us, dstate 128: 128 heads of all (batch,
+      // chunk) pairs 16.9 / 14.1, 256 19.2 / 15.3, 512 27 / 22, 3072 121 / 91; behind are 417 in groups of three 23.4 / 25.3,
+      // 1388 of four 59 / 68, and at dstate 64 1430 of five 50 / 57, 1885 of five 68 / 75, 3444 of four
+      // 124 / 137.  Up to 64 heads, where the walk would be faster too (15 / 12.5), the results have the same bits for states
+      // of either type, which the header promises that far.
       const int64_t units = d.batch * d.C * d.nh;
-      const bool pays = units > 64 && (d.nh / d.g >= 4 || d.batch * d.C * d.g < 256);
+      const HeadsDeal deal = heads_deal(d.batch * d.C * d.g, d.nh / d.g);
+      const bool pays = units > 64 && heads_pay(deal, 32, 28, 16);
       if (d.Q == 256 && pays && !(D && d_has_hdim) && heads_vectors(dt, dA) && heads_rows(sx) && heads_rows(sd) && heads_rows(sdx)) {
-        const HeadsDeal deal = heads_deal(d.batch * d.C * d.g, d.nh / d.g);
         auto kernel = deal.splits ? ssd_chunk_scan_bwd_dx_heads_kernel<N, false> : ssd_chunk_scan_bwd_dx_heads_kernel<N, true>;
         constexpr int smem = DxHeadsSmem<N>::kBytes;
         static_assert(smem <= kLdsBytes, "the heads under way must fit the LDS of a compute unit");
@@ -706,16 +707,15 @@ int ssd_chunk_scan_bwd_ddAcs(const void* x, int64_t x_sb, int64_t x_sl, int64_t 
                        (int)d.C);                                                                               \
   } while (0)
     if (dtype == SSD_BF16 && hdim == 64 && chunk == 256) {
-      // The walk over the heads: where each has a compute unit to itself, and for groups of eight or more (ten, where the
-      // heads are dealt evenly) from where the other kernel, 768 of whose workgroups run at once, needs a second turn; not
-      // where it fills that second turn.  The other kernel / the walk, us, inputs in turn: 64 heads of all (batch, chunk)
-      // pairs 13.2 / 10.0, 256 15.3 / 12.7; 264 15.9 / 16.5, 512 19.1 / 19.4, 640 20.5 / 22.6, 768 22.4 / 27.0; 800 30 / 27, 1024 34 /
-      // 29, 1152 36 / 34; 1280 36.3 / 37.1, 1536 40.6 / 43.3; 1568 47 / 41, 2304 57 / 56, 3072 77 / 70, 8192 186 / 155; dealt evenly
-      // 2400 of eight 67.5 / 69.5, 3072 of eight 77 / 77, 3200 of ten 85 / 82.
+      // The walk over the heads: where each has a compute unit to itself, and from where the other kernel, 768 of whose
+      // workgroups run at once, needs a second turn, if the deal pays next to its turns.  The other kernel / the walk, us,
+      // inputs in turn: 64 heads of all (batch, chunk) pairs 13.2 / 10.0, 256 15.3 / 12.7; 264 15.9 / 16.5, 512 19.1 / 19.4,
+      // 640 20.5 / 22.6, 768 22.4 / 27.0; 800 30 / 27, 1024 34 / 29; 1280 36.3 / 37.1, 1536 40.6 / 43.3; 1568 47 / 41; 2272 of
+      // sixteen 53 / 56, 2250 of ten 55 / 59; 3072 77 / 70, 8192 186 / 155.
       // Relative error against float64, the other kernel / the walk, A in [-16, -1], b1 nh32 L4096, mean of 12 seeds: dt =
       // softplus(n/2 - 2) 8.8e-7 / 7.6e-7, softplus(n/2) 1.23e-6 / 9.6e-7, softplus(n/2 + 2) 9.1e-7 / 9.4e-7.
       const HeadsDeal deal = heads_deal(batch * d.C * ngroups, hpg);
-      const bool pays = wgs <= 256 || (wgs > 768 && (wgs <= 1152 || wgs > 1536) && hpg >= (deal.splits ? 8 : 10));
+      const bool pays = wgs <= 256 || (wgs > 768 && heads_pay(deal, 38, 0, 16));
       if (pays && heads_vectors(dt, dA_cumsum) && reinterpret_cast<uintptr_t>(ddA_cumsum) % 16 == 0 && heads_rows(sx) && heads_rows(sd)) {
         constexpr int smem = DdaHeadsSmem::kBytes;
         static_assert(smem <= kLdsBytes, "the heads under way must fit the LDS of a compute unit");

@@ -83,6 +83,7 @@ constexpr int64_t kBoth64Row = 128;
 struct HeadsDeal {
   unsigned workgroups;
   int units, splits;
+  int64_t cost;  // the estimate, in quarters of a head
 };
 // Rows they take: 32-bit byte offsets within eight rows, and of a row within a chunk.
 inline bool heads_rows(const Strides3& s) { return forward_strides(s) && s.sl < (int64_t(1) << 23); }
@@ -93,12 +94,20 @@ inline bool heads_vectors(const float* dt, const float* dA) {
 inline HeadsDeal heads_deal(int64_t sets, int64_t per) {
   const int64_t units = sets * per, each = (units + 255) / 256;  // (units: up to 2^28, see check_dims)
   int64_t splits = 0, least = 4 * each + 5 * ((each - 2 + per) / per + 1);
-  if (units <= 256) return HeadsDeal{(unsigned)units, (int)units, (int)per};
+  if (units <= 256) return HeadsDeal{(unsigned)units, (int)units, (int)per, 9};
   for (int64_t s = 1; s <= per && sets * (s - 1) < 1024; ++s) {
     const int64_t cost = (sets * s + 255) / 256 * (4 * ((per + s - 1) / s) + 5);
     if (cost < least) least = cost, splits = s;
   }
-  return HeadsDeal{splits ? (unsigned)(sets * splits) : 256u, (int)units, (int)splits};
+  return HeadsDeal{splits ? (unsigned)(sets * splits) : 256u, (int)units, (int)splits, least};
+}
+// Whether that estimate is below one of the kernels of one head (or pair) per workgroup: those take `head` for each 256 heads,
+// `turn` for each 768, which is how many run at once, and `base`, in 32nds of a head of the walk.  A walk whose heads do not
+// divide well, or that fetches what a set shares too often, is behind them at any size (dx of 347 sets of four heads 59 / 68
+// us).  Fitted to 148 to 161 points a stage, sets of 1 to 64 heads, 257 to 7100 heads, each in both kernels: where it chooses
+// the walk that is 8 % behind at one of the 615 points (scan, 1884 heads in groups of six) and 2 to 4 % at five.
+inline bool heads_pay(const HeadsDeal& deal, int head, int turn, int base) {
+  return 8 * deal.cost <= head * ((deal.units + 255) / 256) + turn * ((deal.units + 767) / 768) + base;
 }
 
 template <typename K>

@@ -3283,9 +3283,10 @@ __global__ __launch_bounds__(256, (P == 64 ? 3 : 2)) void ssd_chunk_scan_bwd_dx_
         for (int u = 0; u < NS; ++u)
 #pragma unroll
           for (int e = 0; e < EPL; ++e) w[u][e] = cbcol[(int64_t)(kk0 + KG * u + EPL * half + e) * Q];
-        // the group of 32 positions that holds the diagonal takes the exact, masked form
+        // the group of 32 positions that holds the diagonal takes the exact, masked form; so does one that the sequence
+        // ends in or before, whatever cb holds there
         const int grp_first = kk0 & ~31;
-        const bool exact = diag && grp_first <= mrow[mb] + 31;
+        const bool exact = (diag && grp_first <= mrow[mb] + 31) || k0 + kk0 + NS * KG > limit;
         const float gm = __expf(fminf(dAk[grp_first] - am, 0.f));
 #pragma unroll
         for (int u = 0; u < NS; ++u) {

@@ -80,8 +80,7 @@ struct ScanLaunch {
     }
   }
   template <int N, bool GATED>
-  int launch_heads() const {
-    const HeadsDeal deal = heads_deal(d.batch * d.C * d.g, d.nh / d.g);
+  int launch_heads(const HeadsDeal& deal) const {
     auto kernel = deal.splits ? ssd_chunk_scan_heads_kernel<N, GATED, false> : ssd_chunk_scan_heads_kernel<N, GATED, true>;
     constexpr int smem = ScanHeadsSmem<N, GATED>::kBytes;
     static_assert(smem <= kLdsBytes, "the heads under way must fit the LDS of a compute unit");
@@ -98,12 +97,14 @@ struct ScanLaunch {
       // and groups have three heads or more.  The 256-row kernel / the walk, us, dstate 128: without gate 256 heads of
       // all (batch, chunk) pairs 14.7 / 16.2, 288 20.9 / 19.4, 512 23.2 / 21.3, 1536 57 / 41; 512 groups of two heads 44 / 53,
       // of three 66 / 62; with gate 16 heads 16.0 / 16.8, 64 16.9 / 17.2, 128 19.6 / 18.2, 256 22.4 / 19.1.  (The
-      // header promises the same bits for states of either type up to these lines.)
+      // header promises the same bits for states of either type up to these lines.)  And where its deal pays: 725 heads
+      // in groups of five 28.2 / 31.5, 1860 of three 66 / 71, with gate 465 of five 28.5 / 30.6.
       const int64_t units = d.batch * d.C * d.nh;
-      const bool pays = units > (z ? 64 : 256) && d.nh / d.g >= 3;
+      const HeadsDeal deal = heads_deal(d.batch * d.C * d.g, d.nh / d.g);
+      const bool pays = units > (z ? 64 : 256) && d.nh / d.g >= 3 && heads_pay(deal, 44, 8, 28);
       if (d.Q == 256 && pays && !(D && d_has_hdim) && heads_vectors(dt, dA) && heads_rows(sx) && heads_rows(so) &&
           (!z || heads_rows(sz)))
-        return z ? launch_heads<N, true>() : launch_heads<N, false>();
+        return z ? launch_heads<N, true>(deal) : launch_heads<N, false>(deal);
     }
     constexpr int wide_smem = WideSmem<T, P, N>::kBytes;
     if (d.Q % 256 == 0 && wide_smem <= kLdsBytes) {  // 256-row super-tiles, no barrier inside the k loop
